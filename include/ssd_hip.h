@@ -31,7 +31,7 @@ extern "C" {
 
 /* Bumped whenever a signature or a semantic of this header changes; ssd_abi_version() returns the value the library was built
  * with, so a consumer compiled against another header can tell (tests/abi_consumer.c does). */
-#define SSD_HIP_ABI_VERSION 8
+#define SSD_HIP_ABI_VERSION 9
 
 #define SSD_OK 0
 #define SSD_ERR_SHAPE (-1)
@@ -116,6 +116,11 @@ int ssd_gemm_parts(const void* x_frag, const void* w_frag, const void* bias, voi
 int ssd_gemm_pf_workspace_bytes(int M, int N, int K, int64_t* bytes);
 int ssd_gemm_pf(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy,
                 int epilogue, void* workspace, int64_t workspace_bytes, int splits, void* stream);
+/* The same F.linear for many token rows (csrc/gemm_big.hip): large LDS tiles, any M; N % 16 == 0 (% 64 with SSD_EPI_SILU_FRAG), K % 32 == 0,
+ * K >= 96, ldy % 4 == 0.  `workspace` (may be NULL): room for the fp32 slabs of products with too few tiles to fill the chip, which are
+ * split along K as far as workspace_bytes allow. */
+int ssd_gemm_big(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
+                 void* workspace, int64_t workspace_bytes, void* stream);
 /* Fused decode-layer GEMM for M <= 16 (csrc/gemm_fused.hip): [residual add + RMSNorm] -> F.linear ->
  * [RoPE + paged KV store | SiLU*mul | rows] in ONE launch; replaces add_norm_forward (layernorm.py:76-88) + F.linear
  * (linear.py:97-98) + RotaryEmbedding.forward (rotary_embedding.py:40-60) + store_kvcache (attention.py:10-41), or

@@ -24,6 +24,12 @@ int ssd_gemm_pf_cfg(const void* x_frag, const void* w_frag, const void* bias, vo
                     int epilogue, void* workspace, int64_t workspace_bytes, int nt, int splits, void* stream);
 
 
+/* ssd_gemm_big with an explicit decomposition: shape = 0 256 x 128, 1 128 x 256, 2 128 x 128, 3 128 x 64 (features x tokens), splits of K
+ * (1..8, at least three k-steps of 32 each). */
+int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
+                     void* workspace, int64_t workspace_bytes, int shape, int splits, void* stream);
+
+
 /* A/B facility (bench.py --tune-deep, profiles/): ssd_gemm_wf's default dispatch for the 70B-class matrices -- 1 (default) the DEEP
  * form, 0 the plain kernels of rounds 1-5.
  * Process-wide; call before any hipGraph is captured. */

@@ -1,0 +1,204 @@
+// GEMM  y[M,N] = x[M,K] . W[N,K]^T  of many token rows (prompts, large decode batches) over the fragment-major layout of common.h, with
+// the epilogues of gemm.hip (bf16 rows + bias | SiLU(gate) * up -> fragment-major).  Same reference call sites as gemm.hip.
+//
+// The <= 128-row kernels (gemm.hip, gemm_pf.hip) are built to stream W once per launch, so a prompt of T rows streamed every matrix
+// T / 128 times, and matrices under 100 MB ran the skinny kernel at 128 rows (150 TFLOP/s).  Here the products are bound by the matrix
+// cores (gemm_tile.h).  Measured on MI355X, us per product, 128-row chunks -> this kernel:
+//   T = 2594 (Llama-3.2-1B): qkv 3072 x 2048  530 -> 36, gate_up 16384 x 2048  570 -> 160, down 2048 x 8192  960 -> 100
+//   T = 2163 (Llama-3.1-8B): qkv 6144 x 4096  460 -> 110, gate_up 28672 x 4096  875 -> 440, down 4096 x 14336  590 -> 300
+//   T = 16384 (8B): gate_up 6900 -> 3100 (1240 TFLOP/s), down 4600 -> 1540
+#include "common.h"
+#include "gemm_tile.h"
+
+enum { BIG_ROWS = 0, BIG_SILU_FRAG = 1, BIG_PARTS = 2 };
+
+namespace {
+
+template <int WN, int WM, int NT, int MT, int STAGES, int EPI>
+__global__ void __launch_bounds__(64 * WN * WM, 2)
+gemm_big_kernel(const char* __restrict__ Wf, const char* __restrict__ Xf, const bf16_t* __restrict__ bias, void* __restrict__ Yv, int M, int N,
+                int K, int ldy, int tn, int tm, int splits) {
+  typedef TileLoop<WN, WM, NT, MT, STAGES> L;
+  __shared__ __attribute__((aligned(1024))) char smem[L::LDS];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const TileAt t = tile_at(blockIdx.x, tn, tm);
+  const int z = blockIdx.y, kb = (int)((long)(K >> 5) * z / splits), nk = (int)((long)(K >> 5) * (z + 1) / splits) - kb;
+  const int KT = K >> 5, g0 = t.n * L::WG, h0 = t.m * L::XG;
+  const int gl = (N >> 4) - 1, hl = (M - 1) >> 4;                 // last 16-row groups: tiles past them read those again and store nothing
+  uint32_t voff[L::PER], soff[L::PER];
+#pragma unroll
+  for (int i = 0; i < L::PER; ++i) {
+    const int c = wave * L::PER + i;
+    voff[i] = lane * 16;
+    soff[i] = (uint32_t)(c < L::WG ? min(c, gl - g0) : min(c - L::WG, hl - h0)) * (uint32_t)KT * 1024u + (uint32_t)kb * 1024u;
+  }
+  f32x4_t acc[NT][MT];
+  L::run(smem, tile_rsrc(Wf + (size_t)g0 * KT * 1024, (uint32_t)(min(L::WG, gl + 1 - g0) * KT) * 1024u),
+         tile_rsrc(Xf + (size_t)h0 * KT * 1024, (uint32_t)(min(L::XG, hl + 1 - h0) * KT) * 1024u), voff, soff, 1024, 1024, nk, acc);
+
+  const int wn = wave / WM, wm = wave % WM;
+  const int gw = g0 + wn * NT, m0 = (h0 + wm * MT) * 16 + (lane & 15), nrow = (lane >> 4) * 4;
+  if constexpr (EPI == BIG_PARTS) {
+    float* out = reinterpret_cast<float*>(Yv) + (size_t)z * M * N;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      if (gw + i > gl) continue;
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        if (m0 + j * 16 < M) *reinterpret_cast<f32x4_t*>(out + (size_t)(m0 + j * 16) * N + (gw + i) * 16 + nrow) = acc[i][j];
+    }
+  } else if constexpr (EPI == BIG_ROWS) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      if (gw + i > gl) continue;
+      const int n = (gw + i) * 16 + nrow;
+      float bb[4] = {0.f, 0.f, 0.f, 0.f};
+      if (bias) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bb[r] = bf2f(bias[n + r]);
+      }
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        const int m = m0 + j * 16;
+        if (m < M) {
+          const u32x2_t v = {pack_bf2_hw(acc[i][j][0] + bb[0], acc[i][j][1] + bb[1]), pack_bf2_hw(acc[i][j][2] + bb[2], acc[i][j][3] + bb[3])};
+          *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(Yv) + (size_t)m * ldy + n) = v;
+        }
+      }
+    }
+  } else {
+    const int KT2 = N >> 6;
+    u32x2_t* out = reinterpret_cast<u32x2_t*>(Yv);
+#pragma unroll
+    for (int i = 0; i < NT; i += 2) {
+      if (gw + i > gl) continue;
+      const int f = ((gw + i) >> 1) * 16 + nrow, ng = (gw + i) * 16 + nrow, nu = ng + 16;
+      float bg[4] = {0.f, 0.f, 0.f, 0.f}, bu[4] = {0.f, 0.f, 0.f, 0.f};
+      if (bias) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) { bg[r] = bf2f(bias[ng + r]); bu[r] = bf2f(bias[nu + r]); }
+      }
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        const int m = m0 + j * 16;
+        float o[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float g = round_bf_hw(acc[i][j][r] + bg[r]), u = round_bf_hw(acc[i + 1][j][r] + bu[r]);
+          o[r] = (g / (1.0f + __expf(-g))) * u;
+        }
+        if (m < M) out[frag_chunk(m, f >> 3, KT2) * 2 + ((f >> 2) & 1)] = u32x2_t{pack_bf2_hw(o[0], o[1]), pack_bf2_hw(o[2], o[3])};
+      }
+    }
+  }
+}
+
+// The sum of a split product's slabs [splits][M][N] in order, then the epilogue of an unsplit one.
+template <int EPI>
+__global__ void __launch_bounds__(256)
+gemm_big_sum_kernel(const float* __restrict__ ws, const bf16_t* __restrict__ bias, void* __restrict__ Yv, int M, int N, int splits, int ldy) {
+  const size_t MN = (size_t)M * N, i4 = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  auto sum = [&](size_t at, int n) {
+    f32x4_t s = *reinterpret_cast<const f32x4_t*>(ws + at);
+    for (int z = 1; z < splits; ++z) s += *reinterpret_cast<const f32x4_t*>(ws + z * MN + at);
+    if (bias) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[r] += bf2f(bias[n + r]);
+    }
+    return s;
+  };
+  if constexpr (EPI == BIG_ROWS) {
+    if (i4 >= MN) return;
+    const int m = (int)(i4 / N), n = (int)(i4 % N);
+    const f32x4_t s = sum(i4, n);
+    *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(Yv) + (size_t)m * ldy + n) = u32x2_t{pack_bf2_hw(s[0], s[1]), pack_bf2_hw(s[2], s[3])};
+  } else {
+    const int half = N >> 1;
+    if (i4 >= (size_t)M * half) return;
+    const int m = (int)(i4 / half), f = (int)(i4 % half), ng = (f >> 4) * 32 + (f & 15);
+    const f32x4_t g = sum((size_t)m * N + ng, ng), u = sum((size_t)m * N + ng + 16, ng + 16);
+    float o[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float a = round_bf_hw(g[r]), b = round_bf_hw(u[r]);
+      o[r] = (a / (1.0f + __expf(-a))) * b;
+    }
+    reinterpret_cast<u32x2_t*>(Yv)[frag_chunk(m, f >> 3, half >> 5) * 2 + ((f >> 2) & 1)] = u32x2_t{pack_bf2_hw(o[0], o[1]), pack_bf2_hw(o[2], o[3])};
+  }
+}
+
+template <int WN, int WM, int NT, int MT, int STAGES>
+int go(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue, int splits, void* ws, hipStream_t st) {
+  typedef TileLoop<WN, WM, NT, MT, STAGES> L;
+  const int tn = (N / 16 + L::WG - 1) / L::WG, tm = ((M + 15) / 16 + L::XG - 1) / L::XG;
+#define GO(EPI, OUT)                                                                                                              \
+  hipLaunchKernelGGL((gemm_big_kernel<WN, WM, NT, MT, STAGES, EPI>), dim3(tn * tm, splits), dim3(64 * L::WAVES), 0, st, (const char*)w, \
+                     (const char*)x, (const bf16_t*)bias, OUT, M, N, K, ldy, tn, tm, splits)
+  if (splits > 1) GO(BIG_PARTS, ws);
+  else if (epilogue == BIG_ROWS) GO(BIG_ROWS, y);
+  else GO(BIG_SILU_FRAG, y);
+#undef GO
+  if (hipGetLastError() != hipSuccess) return SSD_ERR_LAUNCH;
+  if (splits > 1) {
+    const unsigned blocks = (unsigned)(((size_t)M * (epilogue == BIG_ROWS ? N : N / 2) / 4 + 255) / 256);
+    if (epilogue == BIG_ROWS)
+      hipLaunchKernelGGL((gemm_big_sum_kernel<BIG_ROWS>), dim3(blocks), dim3(256), 0, st, (const float*)ws, (const bf16_t*)bias, y, M, N, splits, ldy);
+    else
+      hipLaunchKernelGGL((gemm_big_sum_kernel<BIG_SILU_FRAG>), dim3(blocks), dim3(256), 0, st, (const float*)ws, (const bf16_t*)bias, y, M, N, splits, ldy);
+  }
+  return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
+}
+
+// Tile shapes (features x tokens) and what a k-step of 32 takes when n workgroups share a CU, in us (MI355X; fits of
+// T = 130 .. 16384 over the 1B / 8B / 70B matrices, within 15 %).  Large tiles read less LDS per product; small ones leave fewer CUs idle.
+struct Shape { int features, tokens; float step[3], full; };       // step[n - 1] for n <= 3 workgroups on a CU; n * full beyond
+constexpr Shape SHAPES[] = {{256, 128, {0.40f, 0.76f, 1.25f}, 0.42f},
+                            {128, 256, {0.40f, 0.76f, 1.25f}, 0.43f},
+                            {128, 128, {0.29f, 0.45f, 0.66f}, 0.242f},
+                            {128, 64, {0.21f, 0.29f, 0.42f}, 0.167f}};
+struct Plan { int shape, splits; };
+
+// The shape and the number of K splits with the least estimated time: k-steps of the fullest CU, plus, for a split product, a launch
+// (5 us) and its slabs' way to memory and back.  A product with fewer tiles than CUs gains from splits as long as the slabs stay small:
+// 500 x 4096 x 14336 runs 134 us unsplit (128 workgroups), 69 us in four (measured), 99 us as 64-token tiles.
+Plan pick(int M, int N, int K, long ws_bytes) {
+  Plan best{0, 1};
+  float least = 1e30f;
+  for (int c = 0; c < 4; ++c)
+    for (int s = 1; s <= 8; ++s) {
+      const int steps = (K / 32 + s - 1) / s;
+      if (s > 1 && (steps < 8 || (long)s * M * N * 4 > ws_bytes)) break;
+      const long tiles = (long)((N + SHAPES[c].features - 1) / SHAPES[c].features) * ((M + SHAPES[c].tokens - 1) / SHAPES[c].tokens) * s;
+      const long n = (tiles + 255) / 256;
+      const float est = steps * (n <= 3 ? SHAPES[c].step[n - 1] : n * SHAPES[c].full) + (s > 1 ? 5.0f + (float)s * M * N * 8 / 5e6f : 0.f);
+      if (est < least) { least = est; best = Plan{c, s}; }
+    }
+  return best;
+}
+
+}  // namespace
+
+extern "C" int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
+                                void* workspace, int64_t workspace_bytes, int shape, int splits, void* stream) {
+  if (!x_frag || !w_frag || !y) return SSD_ERR_ARG;
+  if (epilogue != BIG_ROWS && epilogue != BIG_SILU_FRAG) return SSD_ERR_ARG;
+  if (M <= 0 || N <= 0 || K < 64 || N % 16 || K % 32 || (epilogue == BIG_SILU_FRAG && N % 64) || K > (1 << 22)) return SSD_ERR_SHAPE;
+  if (epilogue == BIG_ROWS && (ldy < N || ldy % 4)) return SSD_ERR_SHAPE;
+  if (shape < 0 || shape > 3 || splits < 1 || splits > 8 || K / 32 / splits < 3) return SSD_ERR_ARG;
+  if (splits > 1 && (!workspace || workspace_bytes < (int64_t)splits * M * N * 4)) return SSD_ERR_ARG;
+  hipStream_t st = (hipStream_t)stream;
+#define BIG_ARGS x_frag, w_frag, bias, y, M, N, K, ldy, epilogue, splits, workspace, st
+  if (shape == 0) return go<4, 2, 4, 4, 3>(BIG_ARGS);
+  if (shape == 1) return go<2, 4, 4, 4, 3>(BIG_ARGS);
+  if (shape == 2) return go<2, 2, 4, 4, 3>(BIG_ARGS);
+  return go<2, 2, 4, 2, 4>(BIG_ARGS);
+#undef BIG_ARGS
+}
+
+extern "C" int ssd_gemm_big(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
+                            void* workspace, int64_t workspace_bytes, void* stream) {
+  if (M <= 0 || N <= 0 || K < 96) return SSD_ERR_SHAPE;
+  const Plan p = pick(M, N, K, workspace ? workspace_bytes : 0);
+  return ssd_gemm_big_cfg(x_frag, w_frag, bias, y, M, N, K, ldy, epilogue, workspace, workspace_bytes, p.shape, p.splits, stream);
+}

@@ -1,0 +1,92 @@
+// The main loop of the large-tile bf16 GEMMs (many token rows: prefill): a workgroup owns (WN * NT) 16-row groups of W and (WM * MT)
+// 16-row groups of x, its WN x WM waves NT x MT of them each, and leaves the fp32 products in acc[NT][MT].
+//
+// What bounds it is the matrix cores, as long as they are fed: a wave with 8 x 4 accumulator tiles reads 12 KiB of LDS per 32 MFMAs
+// (96 of the 128 bytes a CU's LDS delivers per cycle), so both operands travel HBM / L2 -> LDS by DMA (buffer_load ... lds: no
+// registers, no LDS write instructions), one 1 KiB MFMA operand per instruction, into a ring of STAGES k-steps of 32.  A k-step's
+// loads are issued STAGES - 1 steps ahead, and ONE barrier per step both publishes the step and frees the buffer of the one before.
+// Every accumulator is one chain over ascending k-steps, whatever the tile: a row's result does not depend on the rows beside it.
+#pragma once
+#include "common.h"
+
+// Buffer descriptor of `bytes` bytes at p (raw, unswizzled; reads past the end return zero).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00020000);
+}
+
+// 64 lanes x 16 bytes: memory at rsrc + voff (per lane) + soff -> LDS at lds (wave-uniform) + 16 * lane.
+__device__ __forceinline__ void tile_dma(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, char* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)lds, 16, (int)voff, (int)soff, 0, 0);
+}
+template <int N>
+__device__ __forceinline__ void tile_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int WN, int WM, int NT, int MT, int STAGES>
+struct TileLoop {
+  static constexpr int WAVES = WN * WM, WG = WN * NT, XG = WM * MT;          // waves; 16-row groups of W, of x
+  static constexpr int STEP = (WG + XG) * 1024;                              // LDS bytes of a k-step
+  static constexpr int PER = (WG + XG) / WAVES;                              // 1 KiB operands each wave fetches per k-step
+  static constexpr int LDS = STAGES * STEP;
+  static_assert((WG + XG) % WAVES == 0, "every wave fetches as many operands");
+
+  // wr / xr: descriptors.  Operand i of this wave (i < PER; W's groups first, then x's) comes from voff[i] (per lane) + soff[i] + step * kstep[i].
+  // nk >= STAGES - 1 k-steps.
+  static __device__ __forceinline__ void run(char* smem, __amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t xr, const uint32_t (&voff)[PER], const uint32_t (&soff)[PER],
+                                             uint32_t wk, uint32_t xk, int nk, f32x4_t (&acc)[NT][MT]) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wn = wave / WM, wm = wave % WM;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto fetch = [&](int step, uint32_t buf) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int c = wave * PER + i;
+        const bool w = c < WG;
+        tile_dma(w ? wr : xr, voff[i], soff[i] + (uint32_t)step * (w ? wk : xk), smem + buf * STEP + c * 1024);
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
+    uint32_t cur = 0;
+    const char* ap = smem + wn * NT * 1024 + lane * 16;
+    const char* bp = smem + (WG + wm * MT) * 1024 + lane * 16;
+    for (int k = 0; k < nk; ++k) {
+      tile_wait<PER * (STAGES - 2)>();                 // this wave's share of step k is in LDS
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // everybody's is, and nobody reads step k - 1 any more
+      // (past the end the last step is fetched again: into the buffer nobody reads, so that the count of loads in flight stays static)
+      const int ahead = k + STAGES - 1;
+      fetch(ahead < nk ? ahead : nk - 1, cur == 0 ? STAGES - 1 : cur - 1);
+      const char* a0 = ap + cur * STEP;
+      const char* b0 = bp + cur * STEP;
+      u32x4_t a[NT], b[MT];
+#pragma unroll
+      for (int j = 0; j < MT; ++j) b[j] = *reinterpret_cast<const u32x4_t*>(b0 + j * 1024);
+#pragma unroll
+      for (int i = 0; i < NT; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(a0 + i * 1024);
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+      cur = cur + 1 == STAGES ? 0 : cur + 1;
+    }
+    tile_wait<0>();                                    // nothing may land in LDS after the workgroup has ended
+  }
+};
+
+// Workgroup -> tile: the 8 XCDs (each with an L2 of its own) take workgroups in turn; every XCD gets one contiguous run of the tile
+// list, and the list walks `GM` token tiles for every feature tile, so that the W and x tiles a run shares stay in its L2.
+struct TileAt { int n, m; };
+__device__ __forceinline__ TileAt tile_at(int bid, int tn, int tm) {
+  constexpr int XCDS = 8, GM = 4;
+  const int total = tn * tm, per = total / XCDS, rem = total % XCDS;
+  const int x = bid % XCDS, i = bid / XCDS;
+  const int t = x * per + (x < rem ? x : rem) + i;
+  const int band = t / (GM * tn), in = t % (GM * tn);
+  const int rows = min(GM, tm - band * GM);
+  return TileAt{in / rows, band * GM + in % rows};
+}

@@ -116,6 +116,19 @@ def gemm_pf(x_frag, w_frag, y, M: int, N: int, K: int, ldy: int, workspace, epil
                                           wb, splits, _stream()), "ssd_gemm_pf")
 
 
+def gemm_big(x_frag, w_frag, y, M: int, N: int, K: int, ldy: int, epilogue: int = EPI_ROWS, bias=None, workspace=None, shape: int = -1,
+             splits: int = 1):
+    """GEMM of many token rows; workspace: an optional float32 device tensor for products that are split along K.  shape >= 0: an explicit
+    decomposition (ssd_gemm_big_cfg)."""
+    wb = workspace.numel() * workspace.element_size() if workspace is not None else 0
+    if shape >= 0:
+        _check(load_library().ssd_gemm_big_cfg(_p(x_frag), _p(w_frag), _p(bias), _p(y), M, N, K, ldy, epilogue, _p(workspace), wb, shape,
+                                               splits, _stream()), "ssd_gemm_big_cfg")
+    else:
+        _check(load_library().ssd_gemm_big(_p(x_frag), _p(w_frag), _p(bias), _p(y), M, N, K, ldy, epilogue, _p(workspace), wb, _stream()),
+               "ssd_gemm_big")
+
+
 def rope_store_kv(qkv_rows, positions, cos_sin, slot_mapping, q_out, k_cache, v_cache, T, nh, nkv, hd, block_size,
                   q_norm_w=None, k_norm_w=None, eps: float = 0.0, qkv_perm: int = 0):
     _check(load_library().ssd_rope_store_kv(_p(qkv_rows), _p(positions), _p(cos_sin), _p(slot_mapping), _p(q_out),

@@ -165,6 +165,8 @@ class HipDecoder:
         pf_shapes = [(self.qkv_n, self.h), (self.h, self.qn), (2 * self.I, self.h), (self.h, self.I), (self.V, self.h)]
         need = max([H.gemm_pf_workspace_bytes(128, n, k) // 4 for n, k in pf_shapes if self._pf_eligible(n, k)], default=0)
         self._ws_pf = z(need, dtype=torch.float32) if need and max_tokens > 32 else None
+        # slabs of larger batches' products that are split along K (csrc/gemm_big.hip; no plan uses more than is here)
+        self._ws_big = z(self.BIG_WORKSPACE_BYTES // 4, dtype=torch.float32) if max_tokens > 32 else None
         st = min(T, max_split_tokens)
         self.ws_o = z(st * self.nh * self.max_splits * self.hd, dtype=torch.float32)
         self.ws_ml = z(st * self.nh * self.max_splits * 2, dtype=torch.float32)
@@ -252,18 +254,28 @@ class HipDecoder:
 
     # ---------------------------------------------------------------------------------------------
     PF_MIN_WEIGHT_BYTES = 100 << 20
+    PF_ALWAYS_WEIGHT_BYTES = 300 << 20
+    BIG_MIN_WEIGHT_BYTES = 16 << 20
+    BIG_SMALLEST_WEIGHT_BYTES = 1 << 20
+    BIG_WORKSPACE_BYTES = 48 << 20
 
     @classmethod
     def _pf_eligible(cls, N: int, K: int) -> bool:
         return 2 * N * K >= cls.PF_MIN_WEIGHT_BYTES and N % 128 == 0 and K % 128 == 0
 
     def _gemm_chunk(self, xf, K, w, N, y, m, ldy, epi, bias):
-        """One <= 128-row chunk.  Prefill-sized chunks of a big matrix go to the LDS-shared / split-K kernel
-        (csrc/gemm_pf.hip): measured on MI355X at M = 128, 70B layer GEMMs 611 -> 383 us, 8B gate_up 83 -> 62 us; small
-        matrices (<100 MB: too few workgroups without deep K-splits) stay on the skinny kernel."""
-        if m > 32 and self._pf_eligible(N, K):
+        """At most 128 token rows.  65..128: gemm_pf for a matrix of 100 MB and more (70B layer GEMMs 611 -> 383 us, 8B gate_up 83 -> 62 at
+        128 rows), the skinny kernel below.  33..64, by the weight's size (MI355X, 64 rows, us: skinny | gemm_pf | gemm_big): gemm_pf from
+        300 MB (70B gate_up 248 | 144 | 168), the large-tile kernel with its K splits from 16 MB (8B gate_up 71 | 49 | 45, down_proj
+        51 | 32 | 28, o_proj 17 | 17 | 14; 1B down_proj 28 | 18 | 14), the skinny one for what it reads in one go (1B qkv 11 | 13 | 11;
+        4096 x 1024 8 | 12 | 10).  (The large-tile kernel also wins at 65..128 rows of 16..100 MB -- 8B o_proj 26 -> 15 us -- but prompts
+        of that length are what the recorded full-size token streams start from, and another order of summation moves their near-ties.)"""
+        size = 2 * N * K
+        if m > 32 and self._pf_eligible(N, K) and (m > 64 or size >= self.PF_ALWAYS_WEIGHT_BYTES):
             assert self._ws_pf is not None and self._ws_pf.numel() * 4 >= H.gemm_pf_workspace_bytes(128, N, K), (N, K)
             H.gemm_pf(xf, w, y, m, N, K, ldy, self._ws_pf, epilogue=epi, bias=bias)
+        elif 32 < m <= 64 and K >= 96 and size >= self.BIG_MIN_WEIGHT_BYTES:
+            H.gemm_big(xf, w, y, m, N, K, ldy, epi, bias, self._ws_big)
         else:
             H.gemm(xf, w, y, m, N, K, ldy, epi, bias)
 
@@ -283,15 +295,18 @@ class HipDecoder:
         return S
 
     def _gemm(self, xf, K, w, N, y, T, ldy, epi=H.EPI_ROWS, bias=None):
+        # (a couple of hundred rows of a matrix under 1 MB -- models of a few hundred channels -- stay with the 128-row kernels that such a
+        #  model uses for everything else: 13 us against 5 at 220 rows, launch overhead either way.  K < 96: fewer k-steps than a ring has stages)
+        if T > 128 and K >= 96 and (T > 256 or 2 * N * K >= self.BIG_SMALLEST_WEIGHT_BYTES):
+            H.gemm_big(xf, w, y, T, N, K, ldy, epi, bias, self._ws_big)
+            return
         if T <= 128:
             self._gemm_chunk(xf, K, w, N, y, T, ldy, epi, bias)
             return
         yf = y.view(-1)
         for m0 in range(0, T, 128):
-            m = min(128, T - m0)
-            x_off = (m0 // 16) * (K // 32) * 512
             y_off = (m0 // 16) * ((N // 2) // 32) * 512 if epi == H.EPI_SILU_FRAG else m0 * ldy
-            self._gemm_chunk(xf[x_off:], K, w, N, yf[y_off:], m, ldy, epi, bias)
+            self._gemm_chunk(xf[(m0 // 16) * (K // 32) * 512:], K, w, N, yf[y_off:], min(128, T - m0), ldy, epi, bias)
 
     def _allreduce(self, t):
         if not self.use_coll:
