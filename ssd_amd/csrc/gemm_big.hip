@@ -23,19 +23,22 @@ gemm_big_kernel(const char* __restrict__ Wf, const char* __restrict__ Xf, const 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const TileAt t = tile_at(blockIdx.x, tn, tm);
-  const int z = blockIdx.y, kb = (int)((long)(K >> 5) * z / splits), nk = (int)((long)(K >> 5) * (z + 1) / splits) - kb;
+  const int z = blockIdx.y, kb = (K >> 5) * z / splits, nk = (K >> 5) * (z + 1) / splits - kb;
   const int KT = K >> 5, g0 = t.n * L::WG, h0 = t.m * L::XG;
   const int gl = (N >> 4) - 1, hl = (M - 1) >> 4;                 // last 16-row groups: tiles past them read those again and store nothing
-  uint32_t voff[L::PER], soff[L::PER];
+  uint32_t soff[L::PER];
 #pragma unroll
   for (int i = 0; i < L::PER; ++i) {
     const int c = wave * L::PER + i;
-    voff[i] = lane * 16;
     soff[i] = (uint32_t)(c < L::WG ? min(c, gl - g0) : min(c - L::WG, hl - h0)) * (uint32_t)KT * 1024u + (uint32_t)kb * 1024u;
   }
+  const auto wr = tile_rsrc(Wf + (size_t)g0 * KT * 1024, (uint32_t)(min(L::WG, gl + 1 - g0) * KT) * 1024u);
+  const auto xr = tile_rsrc(Xf + (size_t)h0 * KT * 1024, (uint32_t)(min(L::XG, hl + 1 - h0) * KT) * 1024u);
   f32x4_t acc[NT][MT];
-  L::run(smem, tile_rsrc(Wf + (size_t)g0 * KT * 1024, (uint32_t)(min(L::WG, gl + 1 - g0) * KT) * 1024u),
-         tile_rsrc(Xf + (size_t)h0 * KT * 1024, (uint32_t)(min(L::XG, hl + 1 - h0) * KT) * 1024u), voff, soff, 1024, 1024, nk, acc);
+  const uint32_t at[1] = {(uint32_t)lane * 16u};
+  L::run(smem, nk, at, acc, [&](int i, int step, char* lds) {
+    tile_dma(wave * L::PER + i < L::WG ? wr : xr, lane * 16, soff[i] + (uint32_t)step * 1024u, lds);
+  });
 
   const int wn = wave / WM, wm = wave % WM;
   const int gw = g0 + wn * NT, m0 = (h0 + wm * MT) * 16 + (lane & 15), nrow = (lane >> 4) * 4;

@@ -12,6 +12,7 @@
 //   batched: G independent products in one launch (blockIdx.z / blockIdx.y = g): x + g * gsx with row stride ldx, w + g * N * K,
 //   y + g * gsy with row stride ldy -- per-head products whose operands are column slices of token-major rows.
 #include "common.h"
+#include "gemm_tile.h"
 
 namespace {
 
@@ -283,7 +284,132 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, v
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------------
+// Large-tile form (bf16, K % 64 == 0, 16-byte aligned rows, more rows than the skinny form takes: prompts, larger batches): the main loop
+// of gemm_tile.h over row-major operands, k-steps of 64.  An operand's DMA covers 8 rows x 128 bytes -- whole cache lines; 16 rows x 64
+// bytes, the MFMA operand itself, ran at 60 % -- and lane l fetches chunk (l & 7) ^ (l >> 3) of row l >> 3, so that the eight lanes which an LDS
+// read serves at a time find their chunks in different banks.  The rows of a grouped product are gathered by the same loads.  The
+// accumulators go through LDS once more, 16 or 32 token rows at a time: a wave then stores whole runs of a row, whatever the epilogue.
+// Bound by the matrix cores.  MI355X, against the 64 x 64 form below (which re-stages both operands through registers, two barriers per 32-wide
+// k-step): 4000 x 14720 x 4096 1516 -> 452 us (1070 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 41.
+// ---------------------------------------------------------------------------------------------------------------------
+template <int WN, int WM, int NT, int MT, bool GROUPED>
+__global__ void __launch_bounds__(64 * WN * WM, 2)
+gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
+                      const int* __restrict__ offsets, int E, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx,
+                      long gsy, GluClamp gc, DecayGate dg, int tn, int tm, bool vec_out) {
+  typedef TileLoop<WN, WM, NT, MT, 2, 2> L;
+  constexpr int LDT = NT * 16 + 4, PASS = L::WAVES * 32 * LDT * 4 <= L::LDS ? 32 : 16;                       // a wave's epilogue rows (floats), token rows per pass
+  static_assert(MT * 16 % PASS == 0 && L::WAVES * PASS * LDT * 4 <= L::LDS, "the epilogue rows fit the ring");
+  __shared__ __attribute__((aligned(1024))) char smem[L::LDS];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const TileAt t = tile_at(blockIdx.x, tn, tm);
+  const int n0 = t.n * L::WG * 16;
+  int row0 = t.m * L::XG * 16, row_end = M;
+  const bf16_t* wg = w + (size_t)blockIdx.y * N * K;
+  x += (size_t)blockIdx.y * gsx;
+  const long ycol = (long)blockIdx.y * gsy;
+  if constexpr (GROUPED) {
+    int tile = t.m, e = 0;
+    for (; e < E; ++e) {
+      const int nt = (offsets[e + 1] - offsets[e] + L::XG * 16 - 1) / (L::XG * 16);
+      if (tile < nt) break;
+      tile -= nt;
+    }
+    if (e >= E) return;
+    row0 = offsets[e] + tile * L::XG * 16;
+    row_end = offsets[e + 1];
+    wg = w + (size_t)e * N * K;
+  }
+  // (rows past the edge read the last row again: their products are never stored)
+  const auto wr = tile_rsrc(wg + (size_t)n0 * K, (uint32_t)min(L::WG * 16, N - n0) * (uint32_t)K * 2u);
+  uint32_t woff[L::PER];
+  const bf16_t* xp[L::PER];
+#pragma unroll
+  for (int i = 0; i < L::PER; ++i) {
+    const int c = wave * L::PER + i, r = (c & 1) * 8 + (lane >> 3), k8 = (lane & 7) ^ (lane >> 3);
+    woff[i] = (uint32_t)min((c >> 1) * 16 + r, N - 1 - n0) * (uint32_t)K * 2u + k8 * 16;
+    const int m = min(row0 + ((c >> 1) < L::WG ? 0 : (c >> 1) - L::WG) * 16 + r, row_end - 1);
+    xp[i] = x + (GROUPED && row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx + k8 * 8;
+  }
+  const uint32_t at0 = (uint32_t)(((lane >> 3) & 1) * 1024 + ((lane & 7) * 8 + ((lane >> 4) ^ (lane & 7))) * 16), at[2] = {at0, at0 ^ 64u};
+  f32x4_t acc[NT][MT];
+  L::run(smem, K >> 6, at, acc, [&](int i, int step, char* lds) {
+    if (wave * L::PER + i < 2 * L::WG)
+      tile_dma(wr, woff[i], (uint32_t)step * 128u, lds);
+    else
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp[i] + step * 64), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+  });
+  __syncthreads();
+
+  const int wn = wave / WM, wm = wave % WM;
+  float* rows = reinterpret_cast<float*>(smem) + wave * PASS * LDT;
+  const bool pairs = epi_pairs(epi);
+#pragma unroll
+  for (int p = 0; p < MT * 16 / PASS; ++p) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < PASS / 16; ++j)
+        *reinterpret_cast<f32x4_t*>(rows + (j * 16 + (lane & 15)) * LDT + i * 16 + (lane >> 4) * 4) = acc[i][p * (PASS / 16) + j];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // (rows of this wave alone)
+#pragma unroll 1
+    for (int c = lane; c < PASS * NT * 4; c += 64) {
+      const int r = c / (NT * 4), q = (c % (NT * 4)) * 4;
+      const int m = row0 + wm * MT * 16 + p * PASS + r, n = n0 + wn * NT * 16 + q;
+      if (m >= row_end || n >= N) continue;
+      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(rows + r * LDT + q);
+      if (pairs) {
+        const float rs = epi == 6 && gc.row_scale ? gc.row_scale[row_idx ? row_idx[m] : m] : 1.0f;
+        bf16_t* o = reinterpret_cast<bf16_t*>(y) + (long)m * ldy + ycol + (n >> 1);
+        const float a = glu_act(v[0], v[1], epi, rs, gc.limit, gc.alpha);
+        if (n + 3 < N && vec_out) {
+          *reinterpret_cast<uint32_t*>(o) = pack_bf2(a, glu_act(v[2], v[3], epi, rs, gc.limit, gc.alpha));
+        } else {
+          o[0] = (bf16_t)f2bf(a);
+          if (n + 3 < N) o[1] = (bf16_t)f2bf(glu_act(v[2], v[3], epi, rs, gc.limit, gc.alpha));
+        }
+      } else if (vec_out && n + 3 < N && (epi == 0 || epi == 8)) {
+        f32x4_t o = v;
+        if (epi == 8) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] += dg.bias[n + e];
+        }
+        *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(y) + (long)m * ldy + ycol + n) = o;
+      } else if (vec_out && n + 3 < N && (epi == 1 || epi == 2)) {
+        f32x4_t o = v;
+        if (epi == 1) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { o[e] = o[e] > 0.f ? o[e] : 0.f; o[e] = o[e] * o[e]; }
+        }
+        *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(y) + (long)m * ldy + ycol + n) = u32x2_t{pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3])};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) store_out<bf16_t>(y, m, ldy, ycol + n + e, v[e], epi, dg);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+
 constexpr int SKINNY_MAX_ROWS = 16, SKINNY_MAX_GROUPED_ROWS = 64;
+
+// The tile shape (256 x 256, 128 x 128 or 128 x 64 features x tokens) with the least estimated time: k-steps of the fullest CU, in us per
+// step of 64 when n workgroups share it (MI355X, fits of 20 .. 4000 rows over 4096 .. 14720-wide matrices).  A grouped product's runs
+// leave half a tile empty each.
+int tile_shape(int M, int N, int G, int E) {
+  constexpr int FEATURES[3] = {256, 128, 128}, TOKENS[3] = {256, 128, 64};
+  constexpr float STEP[3][3] = {{1.55f, 3.5f, 5.3f}, {0.66f, 1.0f, 1.5f}, {0.55f, 0.75f, 1.05f}}, FULL[3] = {1.77f, 0.48f, 0.33f};
+  int best = 0;
+  float least = 1e30f;
+  for (int c = 0; c < 3; ++c) {
+    const long tiles = (long)((N + FEATURES[c] - 1) / FEATURES[c]) * ((M + TOKENS[c] - 1) / TOKENS[c] + (E + 1) / 2) * G, n = (tiles + 255) / 256;
+    const float est = n <= 3 ? STEP[c][n - 1] : n * FULL[c];
+    if (est < least) { least = est; best = c; }
+  }
+  return best;
+}
 
 int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, const int* offsets, int E, const int* row_idx,
            int idx_div, int f32, void* stream, int G = 1, long ldx = 0, long gsx = 0, long ldy = 0, long gsy = 0,
@@ -316,6 +442,31 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
     else
       hipLaunchKernelGGL(gemm_skinny_kernel<4>, sg, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)w, y, M, N, K,
                          epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, gc, dg);
+    return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
+  }
+  if (!f32 && K % 64 == 0 && K >= 128 && K <= (1 << 22) && x_vec && (uintptr_t)w % 16 == 0) {
+    const int shape = tile_shape(M, N, G, offsets ? E : 0);
+    // what a store of four (paired: two) neighbouring outputs needs: their address a multiple of its size
+    const int width = epi_pairs(epi) ? 4 : (epi == 0 || epi == 8 ? 16 : 8), esz = epi == 0 || epi == 8 ? 4 : 2;
+    const bool vec_out = (uintptr_t)y % width == 0 && (size_t)ldy * esz % width == 0 && (size_t)gsy * esz % width == 0;
+    const int id = idx_div < 1 ? 1 : idx_div;
+#define TILE_GO(WN, WM, NT, MT, GROUPED)                                                                                              \
+  {                                                                                                                                   \
+    typedef TileLoop<WN, WM, NT, MT, 2, 2> L;                                                                                            \
+    const int tn = (N + L::WG * 16 - 1) / (L::WG * 16), tm = (M + L::XG * 16 - 1) / (L::XG * 16) + (offsets ? E : 0);                 \
+    hipLaunchKernelGGL((gemm_rows_tile_kernel<WN, WM, NT, MT, GROUPED>), dim3(tn * tm, G), dim3(64 * L::WAVES), 0,                    \
+                       (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)w, y, M, N, K, epi, offsets, E, row_idx, id, ldx, ldy,   \
+                       gsx, gsy, gc, dg, tn, tm, vec_out);                                                                            \
+  }
+#define TILE_SHAPES(GROUPED)                                  \
+  {                                                           \
+    if (shape == 0) TILE_GO(2, 4, 8, 4, GROUPED)              \
+    else if (shape == 1) TILE_GO(2, 2, 4, 4, GROUPED)         \
+    else TILE_GO(2, 2, 4, 2, GROUPED)                         \
+  }
+    if (offsets) TILE_SHAPES(true) else TILE_SHAPES(false)
+#undef TILE_SHAPES
+#undef TILE_GO
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
   const int tiles_m = (M + BM - 1) / BM + (offsets ? E : 0);

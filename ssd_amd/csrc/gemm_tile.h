@@ -2,10 +2,10 @@
 // 16-row groups of x, its WN x WM waves NT x MT of them each, and leaves the fp32 products in acc[NT][MT].
 //
 // What bounds it is the matrix cores, as long as they are fed: a wave with 8 x 4 accumulator tiles reads 12 KiB of LDS per 32 MFMAs
-// (96 of the 128 bytes a CU's LDS delivers per cycle), so both operands travel HBM / L2 -> LDS by DMA (buffer_load ... lds: no
-// registers, no LDS write instructions), one 1 KiB MFMA operand per instruction, into a ring of STAGES k-steps of 32.  A k-step's
-// loads are issued STAGES - 1 steps ahead, and ONE barrier per step both publishes the step and frees the buffer of the one before.
-// Every accumulator is one chain over ascending k-steps, whatever the tile: a row's result does not depend on the rows beside it.
+// (96 of the 128 bytes a CU's LDS delivers per cycle), so both operands travel HBM / L2 -> LDS by DMA (loads to LDS: no registers, no
+// LDS write instructions), 1 KiB per instruction, into a ring of STAGES steps of KS x 32 k.  A step's loads are issued STAGES - 1 steps
+// ahead, and ONE barrier per step both publishes the step and frees the buffer of the one before.
+// Every accumulator is one chain over ascending k, whatever the tile: a row's result does not depend on the rows beside it.
 #pragma once
 #include "common.h"
 
@@ -23,19 +23,18 @@ __device__ __forceinline__ void tile_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int WN, int WM, int NT, int MT, int STAGES>
+template <int WN, int WM, int NT, int MT, int STAGES, int KS = 1>
 struct TileLoop {
   static constexpr int WAVES = WN * WM, WG = WN * NT, XG = WM * MT;          // waves; 16-row groups of W, of x
-  static constexpr int STEP = (WG + XG) * 1024;                              // LDS bytes of a k-step
-  static constexpr int PER = (WG + XG) / WAVES;                              // 1 KiB operands each wave fetches per k-step
+  static constexpr int STEP = (WG + XG) * KS * 1024;                              // LDS bytes of a k-step
+  static constexpr int PER = (WG + XG) * KS / WAVES;                             // 1 KiB operands each wave fetches per k-step
   static constexpr int LDS = STAGES * STEP;
-  static_assert((WG + XG) % WAVES == 0, "every wave fetches as many operands");
+  static_assert((WG + XG) * KS % WAVES == 0, "every wave fetches as many operands");
 
-  // wr / xr: descriptors.  Operand i of this wave (i < PER; W's groups first, then x's) comes from voff[i] (per lane) + soff[i] + step * kstep[i].
-  // nk >= STAGES - 1 k-steps.
-  static __device__ __forceinline__ void run(char* smem, __amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t xr, const uint32_t (&voff)[PER], const uint32_t (&soff)[PER],
-                                             uint32_t wk, uint32_t xk, int nk, f32x4_t (&acc)[NT][MT]) {
-    const int lane = threadIdx.x & 63;
+  // fetch_one(i, step, lds): KiB i of this wave's PER (KiB wave * PER + i of the workgroup's step: W's groups first, KS each, then x's) of
+  // step `step` on its way to LDS.  at[s]: where in a group's KS KiB this lane finds its part of the s-th MFMA operand.  nk >= STAGES - 1.
+  template <typename Fetch>
+  static __device__ __forceinline__ void run(char* smem, int nk, const uint32_t (&at)[KS], f32x4_t (&acc)[NT][MT], const Fetch& fetch_one) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave / WM, wm = wave % WM;
 #pragma unroll
@@ -44,34 +43,31 @@ struct TileLoop {
       for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     auto fetch = [&](int step, uint32_t buf) {
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int c = wave * PER + i;
-        const bool w = c < WG;
-        tile_dma(w ? wr : xr, voff[i], soff[i] + (uint32_t)step * (w ? wk : xk), smem + buf * STEP + c * 1024);
-      }
+      for (int i = 0; i < PER; ++i) fetch_one(i, step, smem + buf * STEP + (wave * PER + i) * 1024);
     };
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
     uint32_t cur = 0;
-    const char* ap = smem + wn * NT * 1024 + lane * 16;
-    const char* bp = smem + (WG + wm * MT) * 1024 + lane * 16;
     for (int k = 0; k < nk; ++k) {
       tile_wait<PER * (STAGES - 2)>();                 // this wave's share of step k is in LDS
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // everybody's is, and nobody reads step k - 1 any more
       // (past the end the last step is fetched again: into the buffer nobody reads, so that the count of loads in flight stays static)
       const int ahead = k + STAGES - 1;
       fetch(ahead < nk ? ahead : nk - 1, cur == 0 ? STAGES - 1 : cur - 1);
-      const char* a0 = ap + cur * STEP;
-      const char* b0 = bp + cur * STEP;
-      u32x4_t a[NT], b[MT];
 #pragma unroll
-      for (int j = 0; j < MT; ++j) b[j] = *reinterpret_cast<const u32x4_t*>(b0 + j * 1024);
+      for (int s = 0; s < KS; ++s) {
+        const char* a0 = smem + cur * STEP + wn * NT * KS * 1024 + at[s];
+        const char* b0 = smem + cur * STEP + (WG + wm * MT) * KS * 1024 + at[s];
+        u32x4_t a[NT], b[MT];
 #pragma unroll
-      for (int i = 0; i < NT; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(a0 + i * 1024);
+        for (int j = 0; j < MT; ++j) b[j] = *reinterpret_cast<const u32x4_t*>(b0 + j * KS * 1024);
 #pragma unroll
-      for (int i = 0; i < NT; ++i)
+        for (int i = 0; i < NT; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(a0 + i * KS * 1024);
 #pragma unroll
-        for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+          for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+      }
       cur = cur + 1 == STAGES ? 0 : cur + 1;
     }
     tile_wait<0>();                                    // nothing may land in LDS after the workgroup has ended

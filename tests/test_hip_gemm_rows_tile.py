@@ -1,0 +1,97 @@
+"""Large-tile form of the row-major GEMM (csrc/gemm_rows.hip) against fp64 products: edges of its three tile shapes, every epilogue, strided
+and unaligned outputs, gathered rows and empty groups."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def H():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ssd_amd.hip import ops
+    return ops
+
+
+def operands(M, N, K, seed, E=None):
+    g = torch.Generator().manual_seed(seed)
+    w = torch.randn(*([E] if E else []), N, K, generator=g) / K ** 0.5
+    return torch.randn(M, K, generator=g).to(BF).cuda(), w.to(BF).cuda()
+
+
+# |result - fp64| <= rounding of the output (2^-8 of it for bf16, nothing for fp32) + fp32 sums of K unit-variance terms of size K^-1/2:
+# K roundings of 2^-24 of a partial sum of at most about 5 (values are N(0, 1)), K <= 4096 -> below 2^-10; times the epilogue's slope
+def check(y, ref, what, bf16, slope=1.0):
+    d = (y.double() - ref).abs()
+    tol = (2.0 ** -8 * ref.abs() if bf16 else 0.0) + slope * 2.0 ** -10
+    assert bool((d <= tol).all()), (what, float((d - tol).max()))
+
+
+def act(z, epi):
+    a, u = z[..., 0::2], z[..., 1::2]
+    if epi == 3:
+        return a * torch.sigmoid(a) * u
+    return 0.5 * a * (1 + torch.tanh(math.sqrt(2 / math.pi) * (a + 0.044715 * a ** 3))) * u
+
+
+# sizes: 256-token tiles are chosen for the third, 128 for the fourth, 64 for the others; features off every tile and vector width
+@pytest.mark.parametrize("M,N,K", [(17, 128, 128), (65, 131, 192), (4000, 4050, 128), (2001, 4098, 128), (129, 386, 4096)])
+def test_dense_epilogues(H, M, N, K):
+    x, w = operands(M, N, K, M + N + K)
+    z = x.double() @ w.double().T
+    for epi in (0, 1, 2, 3, 4, 5):
+        if epi in (3, 4) and N % 2:
+            continue
+        out = N // 2 if epi in (3, 4) else N
+        y = torch.full((M, out), 7.0, dtype=torch.float32 if epi == 0 else BF, device="cuda")
+        H.gemm_rows(x, w, y, M, N, K, False, epi)
+        ref = {0: lambda: z, 1: lambda: z.relu() ** 2, 2: lambda: z, 5: lambda: torch.tanh(z)}.get(epi, lambda: act(z, epi))()
+        check(y, ref, (M, N, K, epi), epi != 0, slope={1: 12.0, 3: 12.0, 4: 12.0}.get(epi, 1.0))
+    b = torch.randn(N, device="cuda")
+    y = torch.zeros(M, N, device="cuda")
+    H.gemm_rows_bias(x, w, y, M, N, K, b, False)
+    check(y, z + b.double(), (M, N, K, "bias"), False)
+    rate, nd = torch.rand(N, device="cuda") + 0.1, N // 3
+    H.gemm_rows_decay_gate(x, w, y, M, N, K, rate, b, nd, False)
+    check(y, torch.cat([torch.exp(-rate[:nd].double() * torch.nn.functional.softplus(z[:, :nd] + b[:nd].double())), torch.sigmoid(z[:, nd:])], 1),
+          (M, N, K, "decay"), False)
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 100, 128), (300, 257, 256)])
+def test_batched_columns(H, M, N, K):
+    """Three products on column slices of the same rows, outputs between other columns; an output that four-wide stores may not touch."""
+    G, ldx, ldy = 3, 3 * K + 64, 3 * N + 5
+    g = torch.Generator().manual_seed(N)
+    x = torch.randn(M, ldx, generator=g).to(BF).cuda()
+    w = (torch.randn(G, N, K, generator=g) / K ** 0.5).to(BF).cuda()
+    for off in (0, 1):
+        y = torch.full((M * ldy + 8,), 7.0, device="cuda")
+        H.gemm_rows_batched(x, w, y[off:], M, N, K, G, ldx, K, ldy, N, False)
+        rows = y[off:off + M * ldy].view(M, ldy)
+        for i in range(G):
+            check(rows[:, i * N:(i + 1) * N], x[:, i * K:(i + 1) * K].double() @ w[i].double().T, (M, N, K, i, off), False)
+        assert bool((rows[:, G * N:] == 7.0).all()) and bool((y[:off] == 7.0).all())
+
+
+@pytest.mark.parametrize("counts,N,K,div", [([70, 0, 1, 129, 0, 64], 200, 128, 1), ([300, 213, 0, 511], 130, 192, 2)])
+def test_grouped(H, counts, N, K, div):
+    R, E = sum(counts), len(counts)
+    x, w = operands(-(-R // div), N, K, R, E)
+    perm = torch.randperm(R, generator=torch.Generator().manual_seed(R)).to(torch.int32)
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    ref = torch.cat([x[(perm[off[e]:off[e + 1]].long() // div).cuda()].double() @ w[e].double().T for e in range(E)])
+    for epi in (0, 1, 3):
+        y = torch.zeros(R, N // 2 if epi == 3 else N, dtype=torch.float32 if epi == 0 else BF, device="cuda")
+        H.gemm_rows_grouped(x, w, y, off, E, R, N, K, False, epi, row_idx=perm.cuda(), idx_div=div)
+        check(y, ref if epi == 0 else ref.relu() ** 2 if epi == 1 else act(ref, 3), (counts, epi), epi != 0, slope=1.0 if epi == 0 else 12.0)
+    scale = torch.rand(R, device="cuda") + 0.5
+    y = torch.zeros(R, N // 2, dtype=BF, device="cuda")
+    H.gemm_rows_grouped_glu_clamp(x, w, y, off, E, R, N, K, 1.5, 1.702, row_idx=perm.cuda(), idx_div=div, row_scale=scale)
+    z = ref * scale[perm.long().cuda()].double().unsqueeze(1)
+    a, u = z[:, 0::2].clamp(max=1.5), z[:, 1::2].clamp(-1.5, 1.5)
+    check(y, a * torch.sigmoid(1.702 * a) * (u + 1), (counts, "clamp"), True, slope=12.0)
