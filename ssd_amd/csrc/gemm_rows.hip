@@ -293,12 +293,14 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, v
 // Bound by the matrix cores.  MI355X, against the 64 x 64 form below (which re-stages both operands through registers, two barriers per 32-wide
 // k-step): 4000 x 14720 x 4096 1516 -> 452 us (1070 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 41.
 // ---------------------------------------------------------------------------------------------------------------------
-template <int WN, int WM, int NT, int MT, bool GROUPED>
+template <typename T, int WN, int WM, int NT, int MT, bool GROUPED>
 __global__ void __launch_bounds__(64 * WN * WM, 2)
-gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
+gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
                       const int* __restrict__ offsets, int E, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx,
                       long gsy, GluClamp gc, DecayGate dg, int tn, int tm, bool vec_out) {
-  typedef TileLoop<WN, WM, NT, MT, 2, 2> L;
+  constexpr bool F32 = sizeof(T) == 4;
+  constexpr int VEC = 16 / sizeof(T), ROWB = sizeof(T);              // elements of a 16-byte chunk; bytes of an element
+  typedef TileLoop<WN, WM, NT, MT, 2, 2, F32> L;
   constexpr int LDT = NT * 16 + 4, PASS = L::WAVES * 32 * LDT * 4 <= L::LDS ? 32 : 16;                       // a wave's epilogue rows (floats), token rows per pass
   static_assert(MT * 16 % PASS == 0 && L::WAVES * PASS * LDT * 4 <= L::LDS, "the epilogue rows fit the ring");
   __shared__ __attribute__((aligned(1024))) char smem[L::LDS];
@@ -306,7 +308,7 @@ gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w
   const TileAt t = tile_at(blockIdx.x, tn, tm);
   const int n0 = t.n * L::WG * 16;
   int row0 = t.m * L::XG * 16, row_end = M;
-  const bf16_t* wg = w + (size_t)blockIdx.y * N * K;
+  const T* wg = w + (size_t)blockIdx.y * N * K;
   x += (size_t)blockIdx.y * gsx;
   const long ycol = (long)blockIdx.y * gsy;
   if constexpr (GROUPED) {
@@ -322,23 +324,23 @@ gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w
     wg = w + (size_t)e * N * K;
   }
   // (rows past the edge read the last row again: their products are never stored)
-  const auto wr = tile_rsrc(wg + (size_t)n0 * K, (uint32_t)min(L::WG * 16, N - n0) * (uint32_t)K * 2u);
+  const auto wr = tile_rsrc(wg + (size_t)n0 * K, (uint32_t)min(L::WG * 16, N - n0) * (uint32_t)K * ROWB);
   uint32_t woff[L::PER];
-  const bf16_t* xp[L::PER];
+  const T* xp[L::PER];
 #pragma unroll
   for (int i = 0; i < L::PER; ++i) {
     const int c = wave * L::PER + i, r = (c & 1) * 8 + (lane >> 3), k8 = (lane & 7) ^ (lane >> 3);
-    woff[i] = (uint32_t)min((c >> 1) * 16 + r, N - 1 - n0) * (uint32_t)K * 2u + k8 * 16;
+    woff[i] = (uint32_t)min((c >> 1) * 16 + r, N - 1 - n0) * (uint32_t)K * ROWB + k8 * 16;
     const int m = min(row0 + ((c >> 1) < L::WG ? 0 : (c >> 1) - L::WG) * 16 + r, row_end - 1);
-    xp[i] = x + (GROUPED && row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx + k8 * 8;
+    xp[i] = x + (GROUPED && row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx + k8 * VEC;
   }
   const uint32_t at0 = (uint32_t)(((lane >> 3) & 1) * 1024 + ((lane & 7) * 8 + ((lane >> 4) ^ (lane & 7))) * 16), at[2] = {at0, at0 ^ 64u};
   f32x4_t acc[NT][MT];
-  L::run(smem, K >> 6, at, acc, [&](int i, int step, char* lds) {
+  L::run(smem, K / (8 * VEC), at, acc, [&](int i, int step, char* lds) {
     if (wave * L::PER + i < 2 * L::WG)
       tile_dma(wr, woff[i], (uint32_t)step * 128u, lds);
     else
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp[i] + step * 64), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp[i] + step * 8 * VEC), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
   });
   __syncthreads();
 
@@ -359,7 +361,7 @@ gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w
       const int m = row0 + wm * MT * 16 + p * PASS + r, n = n0 + wn * NT * 16 + q;
       if (m >= row_end || n >= N) continue;
       const f32x4_t v = *reinterpret_cast<const f32x4_t*>(rows + r * LDT + q);
-      if (pairs) {
+      if (!F32 && pairs) {
         const float rs = epi == 6 && gc.row_scale ? gc.row_scale[row_idx ? row_idx[m] : m] : 1.0f;
         bf16_t* o = reinterpret_cast<bf16_t*>(y) + (long)m * ldy + ycol + (n >> 1);
         const float a = glu_act(v[0], v[1], epi, rs, gc.limit, gc.alpha);
@@ -369,11 +371,12 @@ gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w
           o[0] = (bf16_t)f2bf(a);
           if (n + 3 < N) o[1] = (bf16_t)f2bf(glu_act(v[2], v[3], epi, rs, gc.limit, gc.alpha));
         }
-      } else if (vec_out && n + 3 < N && (epi == 0 || epi == 8)) {
+      } else if (vec_out && n + 3 < N && (epi == 0 || epi == 8 || (F32 && epi < 3))) {
         f32x4_t o = v;
-        if (epi == 8) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] += dg.bias[n + e];
+        for (int e = 0; e < 4; ++e) {
+          if (epi == 8) o[e] += dg.bias[n + e];
+          if (epi == 1) { o[e] = o[e] > 0.f ? o[e] : 0.f; o[e] = o[e] * o[e]; }
         }
         *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(y) + (long)m * ldy + ycol + n) = o;
       } else if (vec_out && n + 3 < N && (epi == 1 || epi == 2)) {
@@ -386,10 +389,85 @@ gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (n + e < N) store_out<bf16_t>(y, m, ldy, ycol + n + e, v[e], epi, dg);
+          if (n + e < N) store_out<T>(y, m, ldy, ycol + n + e, v[e], epi, dg);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Skinny form in fp32 (K % 32 == 0, aligned rows, few token rows or few features): a workgroup owns 16 features and its 8 waves take the
+// segments of K in turn, so that eight segments of the 16 weight rows are in flight together; after every round wave 0 adds the segments'
+// sums in their order (gemm_tile.h).  Bound by the weights' way from HBM.  MI355X, against the 64 x 64 form of FMA chains: 3 x 3088 x 2048
+// 139 -> 11 us, 3 x 32000 x 2048 214 -> 74 us (3.5 TB/s); large: 2000 x 4096 x 4096 1021 -> 524 us (tile form).  Error against fp64, relative:
+// 8e-7 -> 3e-7 at K = 2048, 1.1e-6 -> 3e-7 at 4096 (segments shorten the chains).
+// ---------------------------------------------------------------------------------------------------------------------
+constexpr int SKINNY32_WAVES = 8;
+__global__ void __launch_bounds__(SKINNY32_WAVES * 64)
+gemm_skinny_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int M, int N, int K, int epi,
+                       const int* __restrict__ offsets, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx, long gsy,
+                       DecayGate dg) {
+  constexpr int NW = SKINNY32_WAVES, U = 8;
+  __shared__ f32x4_t red[NW][64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  int m_begin = 0, m_end = M;
+  const float* wg = w + (size_t)blockIdx.y * N * K;
+  long ycol = 0;
+  if (offsets) {
+    m_begin = offsets[blockIdx.y];
+    m_end = offsets[blockIdx.y + 1];
+    if (m_begin >= m_end) return;
+  } else {                 // batched (or a single product: blockIdx.y == 0)
+    x += (size_t)blockIdx.y * gsx;
+    ycol = (long)blockIdx.y * gsy;
+  }
+  const float* wp = wg + (size_t)min(n0 + r, N - 1) * K + qd * 4;
+  const int segs = (K + F32_SEG - 1) / F32_SEG;
+  for (int m0 = m_begin + 16 * blockIdx.z; m0 < m_end; m0 += 16 * gridDim.z) {
+    const int mrow = m0 + r;
+    const bool mvalid = mrow < m_end;
+    const float* xp = x + (mvalid ? (row_idx ? (long)(row_idx[mrow] / idx_div) : (long)mrow) : 0) * ldx + qd * 4;
+    f32x4_t total = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < segs; s0 += NW) {
+      const int seg = s0 + wave;
+      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+      if (seg < segs) {
+        const int k0 = seg * F32_SEG, blocks = (min(K - k0, F32_SEG)) >> 4;
+        for (int b0 = 0; b0 < blocks; b0 += U) {
+          u32x4_t a[U], b[U];
+#pragma unroll
+          for (int i = 0; i < U; ++i) {
+            a[i] = b[i] = u32x4_t{0u, 0u, 0u, 0u};
+            const bool ok = b0 + i < blocks;
+            if (ok) a[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp + k0 + (b0 + i) * 16));
+            if (ok && mvalid) b[i] = *reinterpret_cast<const u32x4_t*>(xp + k0 + (b0 + i) * 16);
+          }
+#pragma unroll
+          for (int i = 0; i < U; ++i)
+            if (b0 + i < blocks) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc = mfma_f32(a[i][e], b[i][e], acc);
+            }
+        }
+      }
+      red[wave][lane] = acc;
+      __syncthreads();
+      if (wave == 0) {
+#pragma unroll
+        for (int v = 0; v < NW; ++v)
+          if (s0 + v < segs) total += red[v][lane];
+      }
+      __syncthreads();
+    }
+    if (wave == 0 && mvalid) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = n0 + qd * 4 + e;
+        if (n < N) store_out<float>(y, mrow, ldy, ycol + n, total[e], epi, dg);
+      }
+    }
   }
 }
 
@@ -409,6 +487,13 @@ int tile_shape(int M, int N, int G, int E) {
     if (est < least) { least = est; best = c; }
   }
   return best;
+}
+
+// fp32: 128 x 128 (0) or 64 x 64 (1) -- bound by the matrix cores either way (a 64 x 64 tile reads a quarter of what LDS and L2 deliver), so the
+// shape that keeps the fullest CU shortest: 514 x 3088 x 2048 147 | 79 us, 4000 x 14720 x 4096 3866 | 3903.
+int tile_shape_f32(int M, int N, int G, int E) {
+  const long t0 = (long)((N + 127) / 128) * ((M + 127) / 128 + (E + 1) / 2) * G, t1 = (long)((N + 63) / 64) * ((M + 63) / 64 + (E + 1) / 2) * G;
+  return (t0 + 255) / 256 * 4 <= (t1 + 255) / 256 ? 0 : 1;
 }
 
 int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, const int* offsets, int E, const int* row_idx,
@@ -444,25 +529,39 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
                          epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, gc, dg);
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
-  if (!f32 && K % 64 == 0 && K >= 128 && K <= (1 << 22) && x_vec && (uintptr_t)w % 16 == 0) {
-    const int shape = tile_shape(M, N, G, offsets ? E : 0);
-    // what a store of four (paired: two) neighbouring outputs needs: their address a multiple of its size
-    const int width = epi_pairs(epi) ? 4 : (epi == 0 || epi == 8 ? 16 : 8), esz = epi == 0 || epi == 8 ? 4 : 2;
-    const bool vec_out = (uintptr_t)y % width == 0 && (size_t)ldy * esz % width == 0 && (size_t)gsy * esz % width == 0;
-    const int id = idx_div < 1 ? 1 : idx_div;
-#define TILE_GO(WN, WM, NT, MT, GROUPED)                                                                                              \
-  {                                                                                                                                   \
-    typedef TileLoop<WN, WM, NT, MT, 2, 2> L;                                                                                            \
-    const int tn = (N + L::WG * 16 - 1) / (L::WG * 16), tm = (M + L::XG * 16 - 1) / (L::XG * 16) + (offsets ? E : 0);                 \
-    hipLaunchKernelGGL((gemm_rows_tile_kernel<WN, WM, NT, MT, GROUPED>), dim3(tn * tm, G), dim3(64 * L::WAVES), 0,                    \
-                       (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)w, y, M, N, K, epi, offsets, E, row_idx, id, ldx, ldy,   \
-                       gsx, gsy, gc, dg, tn, tm, vec_out);                                                                            \
+  // (fp32: which of the two orders of summation a product gets -- gemm_tile.h's, or the plain chain of the form for everything else -- may
+  //  depend on sizes and alignment that do not change with the number of rows only)
+  const bool tiled = (f32 ? K % 32 == 0 && K >= 64 : K % 64 == 0 && K >= 128) && K <= (1 << 22) && x_vec && (uintptr_t)w % 16 == 0;
+  const int id = idx_div < 1 ? 1 : idx_div;
+  // few rows, or few features: 16-row chunks over the grid as long as that is about what the chip holds at once (64 x 2048 x 2048: 49 us as a
+  // tile, a serial walk of K by few workgroups; a router's 1000 x 8 x 2048 the same 48 us)
+  const int chunks = (M + 15) / 16;
+  if (tiled && f32 && (offsets ? M <= SKINNY_MAX_GROUPED_ROWS : M <= SKINNY_MAX_ROWS || (long)chunks * ((N + 15) / 16) * G <= 1024)) {
+    hipLaunchKernelGGL(gemm_skinny_f32_kernel, dim3((N + 15) / 16, offsets ? E : G, offsets ? 1 : chunks), dim3(64 * SKINNY32_WAVES), 0, (hipStream_t)stream,
+                       (const float*)x, (const float*)w, (float*)y, M, N, K, epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, dg);
+    return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
-#define TILE_SHAPES(GROUPED)                                  \
-  {                                                           \
-    if (shape == 0) TILE_GO(2, 4, 8, 4, GROUPED)              \
-    else if (shape == 1) TILE_GO(2, 2, 4, 4, GROUPED)         \
-    else TILE_GO(2, 2, 4, 2, GROUPED)                         \
+  if (tiled) {
+    const int shape = f32 ? tile_shape_f32(M, N, G, offsets ? E : 0) : tile_shape(M, N, G, offsets ? E : 0);
+    // what a store of four (paired: two) neighbouring outputs needs: their address a multiple of its size
+    const bool out32 = f32 || epi == 0 || epi == 8;
+    const int width = epi_pairs(epi) ? 4 : (out32 ? 16 : 8), osz = out32 ? 4 : 2;
+    const bool vec_out = (uintptr_t)y % width == 0 && (size_t)ldy * osz % width == 0 && (size_t)gsy * osz % width == 0;
+#define TILE_GO(T, WN, WM, NT, MT, GROUPED)                                                                                           \
+  {                                                                                                                                   \
+    typedef TileLoop<WN, WM, NT, MT, 2, 2, sizeof(T) == 4> L;                                                                         \
+    const int tn = (N + L::WG * 16 - 1) / (L::WG * 16), tm = (M + L::XG * 16 - 1) / (L::XG * 16) + (offsets ? E : 0);                 \
+    hipLaunchKernelGGL((gemm_rows_tile_kernel<T, WN, WM, NT, MT, GROUPED>), dim3(tn * tm, G), dim3(64 * L::WAVES), 0,                 \
+                       (hipStream_t)stream, (const T*)x, (const T*)w, y, M, N, K, epi, offsets, E, row_idx, id, ldx, ldy, gsx, gsy,   \
+                       gc, dg, tn, tm, vec_out);                                                                                      \
+  }
+#define TILE_SHAPES(GROUPED)                                          \
+  {                                                                   \
+    if (f32 && shape == 0) TILE_GO(float, 2, 2, 4, 4, GROUPED)        \
+    else if (f32) TILE_GO(float, 2, 2, 2, 2, GROUPED)                 \
+    else if (shape == 0) TILE_GO(bf16_t, 2, 4, 8, 4, GROUPED)         \
+    else if (shape == 1) TILE_GO(bf16_t, 2, 2, 4, 4, GROUPED)         \
+    else TILE_GO(bf16_t, 2, 2, 4, 2, GROUPED)                         \
   }
     if (offsets) TILE_SHAPES(true) else TILE_SHAPES(false)
 #undef TILE_SHAPES

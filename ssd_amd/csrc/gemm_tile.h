@@ -23,7 +23,17 @@ __device__ __forceinline__ void tile_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int WN, int WM, int NT, int MT, int STAGES, int KS = 1>
+// fp32 products (mfma 16x16x4: a lane holds ONE k of its row; peak 157 TFLOP/s, twice the vector unit's without packed fp32).  The order of
+// a sum is part of what the fp32 mode promises -- a row's result is the same bits whichever kernel computes it -- and is defined here:
+// segments of F32_SEG k (the last one shorter), each a chain from zero over its blocks of 16 k, a block being four MFMAs, the e-th over
+// k = e, 4 + e, 8 + e, 12 + e (lane q of a row holds 4 consecutive k: one 16-byte load); the segments' sums are added in order, from zero.
+constexpr int F32_SEG = 256, F32_SEG_STEPS = F32_SEG / 32;
+__device__ __forceinline__ f32x4_t mfma_f32(uint32_t a, uint32_t b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a), __uint_as_float(b), c, 0, 0, 0);
+}
+
+// F32: operands are floats, a step is 32 k (KS = 2), `acc` the sum over segments.
+template <int WN, int WM, int NT, int MT, int STAGES, int KS = 1, bool F32 = false>
 struct TileLoop {
   static constexpr int WAVES = WN * WM, WG = WN * NT, XG = WM * MT;          // waves; 16-row groups of W, of x
   static constexpr int STEP = (WG + XG) * KS * 1024;                              // LDS bytes of a k-step
@@ -48,6 +58,13 @@ struct TileLoop {
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
     uint32_t cur = 0;
+    f32x4_t part[F32 ? NT : 1][F32 ? MT : 1];
+    if constexpr (F32) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
     for (int k = 0; k < nk; ++k) {
       tile_wait<PER * (STAGES - 2)>();                 // this wave's share of step k is in LDS
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // everybody's is, and nobody reads step k - 1 any more
@@ -66,7 +83,25 @@ struct TileLoop {
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
-          for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+          for (int j = 0; j < MT; ++j) {
+            if constexpr (!F32) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+          }
+        if constexpr (F32) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+              for (int j = 0; j < MT; ++j) part[i][j] = mfma_f32(a[i][e], b[j][e], part[i][j]);
+        }
+      }
+      if constexpr (F32) {
+        if ((k + 1) % F32_SEG_STEPS == 0 || k + 1 == nk) {
+#pragma unroll
+          for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) { acc[i][j] += part[i][j]; part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f}; }
+        }
       }
       cur = cur + 1 == STAGES ? 0 : cur + 1;
     }

@@ -1,5 +1,5 @@
-"""Large-tile form of the row-major GEMM (csrc/gemm_rows.hip) against fp64 products: edges of its three tile shapes, every epilogue, strided
-and unaligned outputs, gathered rows and empty groups."""
+"""Large-tile and fp32 forms of the row-major GEMM (csrc/gemm_rows.hip) against fp64 products: edges of the tile shapes, every epilogue,
+strided and unaligned outputs, gathered rows and empty groups; in fp32 the same bits for a row whichever form computes it."""
 import math
 
 import pytest
@@ -95,3 +95,45 @@ def test_grouped(H, counts, N, K, div):
     z = ref * scale[perm.long().cuda()].double().unsqueeze(1)
     a, u = z[:, 0::2].clamp(max=1.5), z[:, 1::2].clamp(-1.5, 1.5)
     check(y, a * torch.sigmoid(1.702 * a) * (u + 1), (counts, "clamp"), True, slope=12.0)
+
+
+# fp32: a segment of 256 is a chain of 256 roundings (2^-24 each of a partial sum below 5), then one per segment: 272 * 5 * 2^-24 < 1e-4 at worst
+@pytest.mark.parametrize("M,N,K", [(3, 131, 64), (70, 66, 288), (200, 1030, 544), (1300, 8, 2048), (2100, 2200, 96)])
+def test_fp32_forms_agree(H, M, N, K):
+    g = torch.Generator().manual_seed(M + K)
+    x, w = torch.randn(M, K, generator=g).cuda(), (torch.randn(N, K, generator=g) / K ** 0.5).cuda()
+    z = x.double() @ w.double().T
+    for epi in (0, 1, 2, 5):
+        y = torch.full((M, N), 7.0, device="cuda")
+        H.gemm_rows(x, w, y, M, N, K, True, epi)
+        ref = {0: z, 1: z.relu() ** 2, 2: z, 5: torch.tanh(z)}[epi]
+        assert bool(((y.double() - ref).abs() <= 1e-4 * (12.0 if epi == 1 else 1.0)).all()), (M, N, K, epi)
+        for rows in (1, 17, 65, 130, M):
+            for at in (0, M - min(rows, M)):
+                n = min(rows, M)
+                part = torch.zeros(n, N, device="cuda")
+                H.gemm_rows(x[at:at + n], w, part, n, N, K, True, epi)
+                assert torch.equal(part, y[at:at + n]), (M, N, K, epi, rows, at)
+    b = torch.randn(N, device="cuda")
+    y, part = torch.zeros(M, N, device="cuda"), torch.zeros(1, N, device="cuda")
+    H.gemm_rows_bias(x, w, y, M, N, K, b, True)
+    H.gemm_rows_bias(x[M - 1:], w, part, 1, N, K, b, True)
+    assert torch.equal(part, y[M - 1:]) and bool(((y.double() - z - b.double()).abs() <= 1e-4).all())
+
+
+@pytest.mark.parametrize("counts,N,K", [([3, 0, 40, 1], 70, 96), ([70, 0, 1, 200, 5], 130, 320)])
+def test_fp32_grouped(H, counts, N, K):
+    R, E = sum(counts), len(counts)
+    g = torch.Generator().manual_seed(R)
+    x, w = torch.randn(-(-R // 2), K, generator=g).cuda(), (torch.randn(E, N, K, generator=g) / K ** 0.5).cuda()
+    perm = torch.randperm(R, generator=g).to(torch.int32).cuda()
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    y = torch.zeros(R, N, device="cuda")
+    H.gemm_rows_grouped(x, w, y, off, E, R, N, K, True, 0, row_idx=perm, idx_div=2)
+    for e in range(E):
+        rows = x[(perm[off[e]:off[e + 1]].long() // 2)].contiguous()
+        if len(rows):
+            alone = torch.zeros(len(rows), N, device="cuda")
+            H.gemm_rows(rows, w[e].contiguous(), alone, len(rows), N, K, True, 0)
+            assert torch.equal(alone, y[off[e]:off[e + 1]])
+            assert bool(((alone.double() - rows.double() @ w[e].double().T).abs() <= 1e-4).all())
