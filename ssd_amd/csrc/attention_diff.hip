@@ -15,6 +15,7 @@
 //   A token's position and sequence come from positions[] / cu_q[] (varlen batches: prompt portions beside single tokens) or from
 //   q_per_seq (fixed rows per sequence); it sees keys 0 .. position of ITS sequence, through that sequence's block table.
 #include "common.h"
+#include "gemm_tile.h"      // mfma_f32
 
 namespace {
 
@@ -209,8 +210,9 @@ __device__ __forceinline__ float quad_sum(float v) { v += __shfl_xor(v, 16, 64);
 constexpr int DM_WS_SLOT = 64 + 2 * DM_DVT * 64 * 4;      // floats per (sequence, kv head, key slice): max / sum rows, then the O fragments
 
 // Combine the maps, norm over the head's values, scale, gate; lane (row r, values i*16 + qd*4 ..+3) holds acc[m][i][0..3].
+template <typename T>
 __device__ __forceinline__ void diff_finalize(f32x4_t (&acc)[2][DM_DVT], const float (&ls)[2], int DVT, int Dv, float lambda,
-                                              float out_scale, float gate, float eps, bool valid, bf16_t* orow) {
+                                              float out_scale, float gate, float eps, bool valid, T* orow) {
   const float i1 = 1.0f / ls[0], i2 = lambda / ls[1];
   float ss = 0.f;
 #pragma unroll
@@ -226,8 +228,12 @@ __device__ __forceinline__ void diff_finalize(f32x4_t (&acc)[2][DM_DVT], const f
 #pragma unroll
     for (int i = 0; i < DM_DVT; ++i)
       if (i < DVT) {
-        const u32x2_t o = {pack_bf2(acc[0][i][0] * rn, acc[0][i][1] * rn), pack_bf2(acc[0][i][2] * rn, acc[0][i][3] * rn)};
-        *reinterpret_cast<u32x2_t*>(orow + i * 16) = o;
+        if constexpr (sizeof(T) == 4) {
+          *reinterpret_cast<f32x4_t*>(orow + i * 16) = acc[0][i] * rn;
+        } else {
+          const u32x2_t o = {pack_bf2(acc[0][i][0] * rn, acc[0][i][1] * rn), pack_bf2(acc[0][i][2] * rn, acc[0][i][3] * rn)};
+          *reinterpret_cast<u32x2_t*>(orow + i * 16) = o;
+        }
       }
   }
 }
@@ -522,6 +528,216 @@ diffattn_merge_kernel(const float* __restrict__ ws, int nsplit, const float* __r
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------------
+// MFMA form in fp32 (D % 16 == 0, D <= 64, Dv % 16 == 0, Dv <= 128, block_size % 16 == 0): rows as above, products by mfma 16x16x4, whose
+// operands are single floats -- a lane's 16-byte load is four of them, and the score fragment (lane: row r, keys 4 qd + e) is the second
+// product's operand as it stands.  The keys are scanned in segments of 64 from key 0 (steps of 16, online softmax inside a segment), and a
+// segment's (max, sum, O) joins the row's total in order: the same steps for a prompt's row and for a decoded token, so a row's bits do not
+// depend on the schedule.  Steps and segments behind a row's position leave its values as they are.
+// tile mode:  workgroup = 4 waves of 16 rows; a wave's totals lie in LDS (registers hold the segment's O and the step's K and V).
+// split mode: 8 waves share the <= 16 rows and take the segments in turn; after a round, wave w adds value tile w of the segments in order.
+// Bound by the chain of a segment's steps (a memory round trip and 96 MFMAs each).  MI355X, 16 heads in 4 groups, dim 64, vdim 128: a portion
+// of 512 rows up to key 1000 3070 -> 198 us, single tokens of three sequences at up to 1000 keys 131 -> 49 us (before: the scalar form
+// above, a workgroup per token and head whose lanes each read a whole K row).
+// ---------------------------------------------------------------------------------------------------------------------
+constexpr int DF_KS = 4, DF_SEG = 64, DF_SPLIT_WAVES = 8;
+
+struct DiffPart { float mx[2], ls[2]; f32x4_t acc[2][DM_DVT]; };
+
+// the factors of total <- total + a later segment's part, and its new maximum and sum
+__device__ __forceinline__ void diff_factors(float (&M)[2], float (&L)[2], const float (&mx)[2], const float (&ls)[2], float (&fo)[2], float (&fn)[2]) {
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const float top = fmaxf(M[m], mx[m]);
+    fo[m] = M[m] == -INFINITY ? 0.f : __expf(M[m] - top);
+    fn[m] = mx[m] == -INFINITY ? 0.f : __expf(mx[m] - top);
+    L[m] = L[m] * fo[m] + ls[m] * fn[m];
+    M[m] = top;
+  }
+}
+
+// keys [k_begin, k_end) of one segment for the 16 rows of a wave (k_end past a row's position, or past the cache, is masked)
+__device__ __forceinline__ void diff_segment(DiffPart& p, const u32x4_t (&qreg)[2][DF_KS], const float* __restrict__ kc, const float* __restrict__ vt,
+                                             const int32_t* __restrict__ table, int G, int g, int D, int Dv, int bs, int r, int qd, int k_begin,
+                                             int k_end, int pos, int ctx, float scale) {
+  const int KS = D >> 4, DVT = Dv >> 4;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    p.mx[m] = -INFINITY;
+    p.ls[m] = 0.f;
+#pragma unroll
+    for (int i = 0; i < DM_DVT; ++i) p.acc[m][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int k0 = k_begin; k0 < k_end; k0 += 16) {
+    const size_t pg = (size_t)table[k0 / bs] * G + g;
+    const int koff = k0 % bs;
+    u32x4_t kreg[2][DF_KS], v[DM_DVT];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int ks = 0; ks < DF_KS; ++ks) {
+        kreg[m][ks] = u32x4_t{0u, 0u, 0u, 0u};
+        if (ks < KS) kreg[m][ks] = *reinterpret_cast<const u32x4_t*>(kc + (pg * bs + koff + r) * 2 * D + m * D + ks * 16 + qd * 4);
+      }
+#pragma unroll
+    for (int i = 0; i < DM_DVT; ++i) {
+      v[i] = u32x4_t{0u, 0u, 0u, 0u};
+      if (i < DVT) v[i] = *reinterpret_cast<const u32x4_t*>(vt + (pg * Dv + i * 16 + r) * bs + koff + qd * 4);
+    }
+    f32x4_t s[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int ks = 0; ks < DF_KS; ++ks)
+      if (ks < KS) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int m = 0; m < 2; ++m) s[m] = mfma_f32(kreg[m][ks][e], qreg[m][ks][e], s[m]);
+      }
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      float top = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[m][e] = k0 + qd * 4 + e <= pos ? s[m][e] * scale : -INFINITY;
+        top = fmaxf(top, s[m][e]);
+      }
+      top = fmaxf(p.mx[m], quad_max(top));
+      const float safe = top == -INFINITY ? 0.f : top, corr = __expf(p.mx[m] - safe);
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { s[m][e] = __expf(s[m][e] - safe); sum += s[m][e]; }
+      p.ls[m] = p.ls[m] * corr + quad_sum(sum);
+      p.mx[m] = top;
+#pragma unroll
+      for (int i = 0; i < DM_DVT; ++i) p.acc[m][i] *= corr;
+    }
+    if (k0 + 16 > ctx) {        // keys past the sequence: whatever the page holds there must not meet a zero weight as NaN
+#pragma unroll
+      for (int i = 0; i < DM_DVT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (k0 + qd * 4 + e >= ctx) v[i][e] = 0u;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < DM_DVT; ++i)
+        if (i < DVT) {
+#pragma unroll
+          for (int m = 0; m < 2; ++m) p.acc[m][i] = mfma_f32(v[i][e], __float_as_uint(s[m][e]), p.acc[m][i]);
+        }
+  }
+}
+
+template <bool SPLIT>
+__global__ void __launch_bounds__(SPLIT ? 64 * DF_SPLIT_WAVES : 256, 2)
+diffattn_f32_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vt, const float* __restrict__ gate,
+                    const int32_t* __restrict__ bt, int max_blocks, const int64_t* __restrict__ positions,
+                    const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ cu_q, int q_per_seq, int B, int H, int G, int D, int Dv,
+                    int bs, float scale, float lambda, float out_scale, float eps, float* __restrict__ out) {
+  // tile mode: [wave][map][tile][lane] totals; split mode: [wave][map][tile][lane] of a round's segments, then their (max, sum)
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
+  const int g = blockIdx.y, R = H / G, DVT = Dv >> 4, KS = D >> 4;
+  int b = 0, tile = blockIdx.x, tok0 = 0, qb = 0;
+  if (SPLIT) {
+    b = blockIdx.x;
+    tile = 0;
+    tok0 = cu_q ? cu_q[b] : b * q_per_seq;
+    qb = cu_q ? cu_q[b + 1] - cu_q[b] : q_per_seq;
+    if (qb <= 0) return;
+  } else {
+    for (; b < B; ++b) {
+      tok0 = cu_q ? cu_q[b] : b * q_per_seq;
+      qb = cu_q ? cu_q[b + 1] - cu_q[b] : q_per_seq;
+      const int nt = (qb * R + 63) >> 6;
+      if (tile < nt) break;
+      tile -= nt;
+    }
+    if (b >= B) return;
+  }
+  const int nrows = qb * R, row0 = SPLIT ? 0 : tile * 64 + wave * 16;
+  if (!SPLIT && row0 >= nrows) return;                 // (tile mode has no workgroup barriers)
+  const bool valid = row0 + r < nrows;
+  const int rr = valid ? row0 + r : row0;
+  const int token = tok0 + rr / R, head = g * R + rr % R;
+  const int pos = (int)positions[token], ctx = ctx_lens[b];
+  int maxpos = pos;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) maxpos = max(maxpos, __shfl_xor(maxpos, o, 64));
+  const int32_t* table = bt + (size_t)b * max_blocks;
+  u32x4_t qreg[2][DF_KS];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int ks = 0; ks < DF_KS; ++ks) {
+      qreg[m][ks] = u32x4_t{0u, 0u, 0u, 0u};
+      if (ks < KS && valid) qreg[m][ks] = *reinterpret_cast<const u32x4_t*>(q + ((size_t)token * H + head) * 2 * D + m * D + ks * 16 + qd * 4);
+    }
+  const int keys = maxpos + 1, nseg = (keys + DF_SEG - 1) / DF_SEG;
+  float M[2] = {-INFINITY, -INFINITY}, L[2] = {0.f, 0.f};
+  f32x4_t* mine = reinterpret_cast<f32x4_t*>(smem) + (size_t)wave * 2 * DVT * 64 + lane;
+  DiffPart p;
+  if constexpr (!SPLIT) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int i = 0; i < DM_DVT; ++i)
+        if (i < DVT) mine[(m * DVT + i) * 64] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int sg = 0; sg < nseg; ++sg) {
+      diff_segment(p, qreg, kc, vt, table, G, g, D, Dv, bs, r, qd, sg * DF_SEG, min(keys, (sg + 1) * DF_SEG), pos, ctx, scale);
+      float fo[2], fn[2];
+      diff_factors(M, L, p.mx, p.ls, fo, fn);
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int i = 0; i < DM_DVT; ++i)
+          if (i < DVT) mine[(m * DVT + i) * 64] = mine[(m * DVT + i) * 64] * fo[m] + p.acc[m][i] * fn[m];
+    }
+  } else {
+    float* sml = smem + (size_t)DF_SPLIT_WAVES * 2 * DVT * 256;         // [wave][map][max, sum][16 rows]
+    const f32x4_t* all = reinterpret_cast<const f32x4_t*>(smem) + lane;
+    f32x4_t total[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};       // value tile `wave`
+    for (int s0 = 0; s0 < nseg; s0 += DF_SPLIT_WAVES) {
+      const int sg = s0 + wave;
+      if (sg < nseg) {
+        diff_segment(p, qreg, kc, vt, table, G, g, D, Dv, bs, r, qd, sg * DF_SEG, min(keys, (sg + 1) * DF_SEG), pos, ctx, scale);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+#pragma unroll
+          for (int i = 0; i < DM_DVT; ++i)
+            if (i < DVT) mine[(m * DVT + i) * 64] = p.acc[m][i];
+          if (qd == 0) { sml[((wave * 2 + m) * 2 + 0) * 16 + r] = p.mx[m]; sml[((wave * 2 + m) * 2 + 1) * 16 + r] = p.ls[m]; }
+        }
+      }
+      __syncthreads();
+      for (int v = 0; v < DF_SPLIT_WAVES && s0 + v < nseg; ++v) {
+        float fo[2], fn[2];
+        const float mx[2] = {sml[((v * 2 + 0) * 2 + 0) * 16 + r], sml[((v * 2 + 1) * 2 + 0) * 16 + r]};
+        const float ls[2] = {sml[((v * 2 + 0) * 2 + 1) * 16 + r], sml[((v * 2 + 1) * 2 + 1) * 16 + r]};
+        diff_factors(M, L, mx, ls, fo, fn);
+        if (wave < DVT) {
+#pragma unroll
+          for (int m = 0; m < 2; ++m) total[m] = total[m] * fo[m] + all[((v * 2 + m) * DVT + wave) * 64] * fn[m];
+        }
+      }
+      __syncthreads();
+    }
+    if (wave < DVT) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) reinterpret_cast<f32x4_t*>(smem)[(m * DVT + wave) * 64 + lane] = total[m];
+    }
+    __syncthreads();
+    if (wave != 0) return;
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int i = 0; i < DM_DVT; ++i) p.acc[m][i] = i < DVT ? mine[(m * DVT + i) * 64] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  diff_finalize<float>(p.acc, L, DVT, Dv, lambda, out_scale, gate[(size_t)token * H + head], eps, valid,
+                       out + ((size_t)token * H + head) * Dv + qd * 4);
+}
+
 }  // namespace
 
 #define LAUNCH_OK() (hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH)
@@ -578,6 +794,26 @@ extern "C" int ssd_diffattn_paged(const void* q_rows, const void* k_cache, const
     if (nsplit > 1)
       hipLaunchKernelGGL(diffattn_merge_kernel, dim3(B, G), dim3(256), 0, (hipStream_t)stream, (const float*)workspace, nsplit,
                          (const float*)gate, cu_q, q_per_seq, H, G, Dv, lambda, out_scale, eps, (bf16_t*)out_rows);
+    return LAUNCH_OK();
+  }
+  // fp32: which form a model gets may depend on its sizes only (a row's bits are the same whatever the schedule)
+  if (f32 && context_lens && max_q > 0 && D % 16 == 0 && D <= 16 * DF_KS && Dv % 16 == 0 && Dv <= 16 * DM_DVT && block_size % 16 == 0 &&
+      (((uintptr_t)q_rows | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out_rows) & 15) == 0) {
+    const int R = H / G;
+    const size_t per_wave = (size_t)2 * (Dv / 16) * 64 * 16;
+#define DF_ARGS (const float*)q_rows, (const float*)k_cache, (const float*)v_cache, (const float*)gate, block_tables, max_blocks, positions,  \
+                context_lens, cu_q, q_per_seq, B, H, G, D, Dv, block_size, scale, lambda, out_scale, eps, (float*)out_rows
+    if (max_q * R <= 16) {
+      const size_t lds = DF_SPLIT_WAVES * (per_wave + 2 * 2 * 16 * 4);
+      if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)diffattn_f32_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
+                                 hipSuccess)
+        return SSD_ERR_LAUNCH;
+      hipLaunchKernelGGL(diffattn_f32_kernel<true>, dim3(B, G), dim3(64 * DF_SPLIT_WAVES), lds, (hipStream_t)stream, DF_ARGS);
+    } else {
+      hipLaunchKernelGGL(diffattn_f32_kernel<false>, dim3((unsigned)(((long)T * R + 63) / 64 + B), G), dim3(256), 4 * per_wave,
+                         (hipStream_t)stream, DF_ARGS);
+    }
+#undef DF_ARGS
     return LAUNCH_OK();
   }
   const size_t lds = (size_t)(2 * D + 4 * 2 * 64) * 4 + 4 * 64 * 8 + (size_t)(4 * 2 * Dv + 16 + 4) * 4 + 8;
