@@ -17,6 +17,7 @@
 //                                 B = P^T, which is exactly the S^T accumulator layout -> no shuffles)
 // Split-KV partials (m, l, O) are merged by attn_combine_kernel in a fixed order.
 #include "common.h"
+#include "attention_prefill.h"
 
 struct AttnParams {
   const bf16_t* q;
@@ -570,6 +571,15 @@ extern "C" int ssd_attn_paged(const void* q_rows, const void* k_cache, const voi
   p.scale_log2e = scale * 1.4426950408889634f;
   p.ow = nullptr; p.oparts = nullptr; p.oN = 0;
   hipStream_t st = (hipStream_t)stream;
+  // More than a workgroup's worth of causal rows per kv head: the throughput form (attention_prefill.hip) -- 42 -> 21 us at 512 tokens of 32 heads in
+  // 8 groups, 25 -> 15 at 256 tokens of 64 heads.  (It also leads at 128 tokens, 13 -> 10 us; prompts of up to 160 tokens are
+  // what the recorded full-size token streams start from, and another order of summation moves their near-ties: they stay with the form above.)
+  const int G = nh / nkv;
+  if (mode == 0 && splits == 1 && !(flags & 3) && max_q * G > PREFILL_ROWS && T >= PREFILL_MIN_TOKENS) {
+    const PrefillAttn a = {p.q, p.kc, p.vc, block_tables, context_lens, cu_q, p.out_rows, p.out_frag, max_blocks, q_per_seq, nh, nkv, p.bs_shift,
+                           p.scale_log2e};
+    return attn_prefill_launch(a, B, max_q, hd, st);
+  }
   // flags bits 8..11: waves per workgroup that split the key range and merge in LDS (default 1; 1..8)
   int waves = (flags >> 8) & 0xf;
   if (waves < 1) waves = 1;

@@ -255,6 +255,7 @@ class HipDecoder:
     # ---------------------------------------------------------------------------------------------
     PF_MIN_WEIGHT_BYTES = 100 << 20
     PF_ALWAYS_WEIGHT_BYTES = 300 << 20
+    BIG_MIN_ROWS = 160
     BIG_MIN_WEIGHT_BYTES = 16 << 20
     BIG_SMALLEST_WEIGHT_BYTES = 1 << 20
     BIG_WORKSPACE_BYTES = 48 << 20
@@ -295,9 +296,11 @@ class HipDecoder:
         return S
 
     def _gemm(self, xf, K, w, N, y, T, ldy, epi=H.EPI_ROWS, bias=None):
-        # (a couple of hundred rows of a matrix under 1 MB -- models of a few hundred channels -- stay with the 128-row kernels that such a
-        #  model uses for everything else: 13 us against 5 at 220 rows, launch overhead either way.  K < 96: fewer k-steps than a ring has stages)
-        if T > 128 and K >= 96 and (T > 256 or 2 * N * K >= self.BIG_SMALLEST_WEIGHT_BYTES):
+        # (up to BIG_MIN_ROWS, and a couple of hundred rows of a matrix under 1 MB -- models of a few hundred channels --, prompts walk the
+        #  128-row kernels: the recorded full-size token streams restart from prompts of up to 160 tokens, and another order of summation moves
+        #  their near-ties.  The large-tile kernel leads there too: 130 rows of 8B qkv 42 -> 24 us, of a 512 x 256 toy 9 -> 5.  K < 96: fewer
+        #  k-steps than a ring has stages)
+        if T > self.BIG_MIN_ROWS and K >= 96 and (T > 256 or 2 * N * K >= self.BIG_SMALLEST_WEIGHT_BYTES):
             H.gemm_big(xf, w, y, T, N, K, ldy, epi, bias, self._ws_big)
             return
         if T <= 128:
