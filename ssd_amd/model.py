@@ -345,6 +345,11 @@ class HipDecoder:
         splits = 1 if ctx <= 1024 else max(1, min(self.max_splits, ctx // 512))
         if base >= 256 or T > self.max_split_tokens:
             splits = 1
+            if meta.cu_q is None:
+                # a decoding batch that fills the grid by itself: its scans are chains of tile loads, as long as the longest context --
+                # more waves per (sequence, kv head), not grid splits (MI355X, 1 | 4 | 8 waves: 48 sequences of 190 .. 3000 keys, 8 kv heads of
+                # 128: 204 | 64 | 50 us, with 4 | 8 waves x 2 splits 54 | 55; 64 of 12 .. 200: 20 | 12 | 16; 32 of 60 .. 1000: 40 | 24 | 20)
+                waves = 4 if ctx <= 1024 and base > 256 else 8
         return splits, waves
 
     def _attn_flags(self, meta: AttnMeta) -> int:
