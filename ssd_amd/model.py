@@ -164,16 +164,18 @@ class HipDecoder:
         # path (layer matrices and the LM head): prefill hipGraphs bake this pointer, so it must never be reallocated
         pf_shapes = [(self.qkv_n, self.h), (self.h, self.qn), (2 * self.I, self.h), (self.h, self.I), (self.V, self.h)]
         need = max([H.gemm_pf_workspace_bytes(128, n, k) // 4 for n, k in pf_shapes if self._pf_eligible(n, k)], default=0)
-        self._ws_pf = z(need, dtype=torch.float32) if need and max_tokens > 32 else None
+        self._ws_pf = z(need, dtype=torch.float32) if need and max_tokens > 16 else None
         # slabs of larger batches' products that are split along K (csrc/gemm_big.hip; no plan uses more than is here)
-        self._ws_big = z(self.BIG_WORKSPACE_BYTES // 4, dtype=torch.float32) if max_tokens > 32 else None
+        self._ws_big = z(self.BIG_WORKSPACE_BYTES // 4, dtype=torch.float32) if max_tokens > 16 else None
         st = min(T, max_split_tokens)
         self.ws_o = z(st * self.nh * self.max_splits * self.hd, dtype=torch.float32)
         self.ws_ml = z(st * self.nh * self.max_splits * 2, dtype=torch.float32)
         # LM-head argmax candidates (csrc/gemm.hip EPI_ROWS_ARGMAX): one (value, index) per token row and workgroup, finished
         # by ssd_argmax_parts* -- on the greedy path for up to 32 logit rows (decode / verify / tree step)
         self.argmax_fused = True
-        self.ap_rows = min(self.max_logit_rows, 32)
+        # (a head of 1.2 GB and more: up to 16 rows.  From there gemm_pf + the argmax of its rows is faster: 151936 x 5120, 32 rows: 314 us with
+        #  candidates, 253 + 13 without)
+        self.ap_rows = min(self.max_logit_rows, 32 if 2 * self.V * self.h < self.AP_WIDE_HEAD_BYTES else 16)
         self.ap_stride = max(H.gemm_argmax_nparts(m, self.V, self.h) for m in ({1, self.ap_rows} if self.ap_rows > 16 else {1}))
         self.ap_val = z(self.ap_rows, self.ap_stride, dtype=torch.float32)
         self.ap_idx = z(self.ap_rows, self.ap_stride, dtype=torch.int32)
@@ -256,6 +258,8 @@ class HipDecoder:
     PF_MIN_WEIGHT_BYTES = 100 << 20
     PF_ALWAYS_WEIGHT_BYTES = 300 << 20
     BIG_MIN_ROWS = 160
+    AP_WIDE_HEAD_BYTES = 1200 << 20
+    PARTS_WIDE_WEIGHT_BYTES = 64 << 20
     BIG_MIN_WEIGHT_BYTES = 16 << 20
     BIG_SMALLEST_WEIGHT_BYTES = 1 << 20
     BIG_WORKSPACE_BYTES = 48 << 20
@@ -265,17 +269,20 @@ class HipDecoder:
         return 2 * N * K >= cls.PF_MIN_WEIGHT_BYTES and N % 128 == 0 and K % 128 == 0
 
     def _gemm_chunk(self, xf, K, w, N, y, m, ldy, epi, bias):
-        """At most 128 token rows.  65..128: gemm_pf for a matrix of 100 MB and more (70B layer GEMMs 611 -> 383 us, 8B gate_up 83 -> 62 at
-        128 rows), the skinny kernel below.  33..64, by the weight's size (MI355X, 64 rows, us: skinny | gemm_pf | gemm_big): gemm_pf from
-        300 MB (70B gate_up 248 | 144 | 168), the large-tile kernel with its K splits from 16 MB (8B gate_up 71 | 49 | 45, down_proj
-        51 | 32 | 28, o_proj 17 | 17 | 14; 1B down_proj 28 | 18 | 14), the skinny one for what it reads in one go (1B qkv 11 | 13 | 11;
-        4096 x 1024 8 | 12 | 10).  (The large-tile kernel also wins at 65..128 rows of 16..100 MB -- 8B o_proj 26 -> 15 us -- but prompts
-        of that length are what the recorded full-size token streams start from, and another order of summation moves their near-ties.)"""
+        """At most 128 token rows.  Up to 16: the skinny kernel, which a second 16-row token tile slows down where K is long.
+        65..128: gemm_pf for a matrix of 100 MB and more (70B layer GEMMs 611 -> 383 us, 8B gate_up 83 -> 62 at 128 rows), the skinny kernel
+        below.  (The large-tile kernel also wins there for 16..100 MB -- 8B o_proj 26 -> 15 us -- but prompts of that length are what the
+        recorded full-size token streams start from, and another order of summation moves their near-ties.)
+        17..64, by the weight's size (MI355X, us: skinny | gemm_pf | gemm_big): gemm_pf from 300 MB (64 rows of 70B gate_up 248 | 144 | 168; 32
+        rows 153 | 139 | 164, down_proj 119 | 80 | 86, 32B gate_up 95 | 86 | 96); the large-tile kernel with its K splits from 16 MB (64 rows of
+        8B gate_up 71 | 49 | 45, down_proj 51 | 32 | 28, o_proj 17 | 17 | 14, 1B down_proj 28 | 18 | 14; 32 rows of 8B down_proj
+        34 | 29 | 26, 70B o_proj 39 | 31 | 31, 32B qkv 34 | 32 | 27), up to 32 rows not for gate_up, whose K is short (8B 44 | 48 | 51);
+        the skinny one for what it reads in one go (64 rows of 1B qkv 11 | 13 | 11; 4096 x 1024 8 | 12 | 10)."""
         size = 2 * N * K
-        if m > 32 and self._pf_eligible(N, K) and (m > 64 or size >= self.PF_ALWAYS_WEIGHT_BYTES):
+        if m > 16 and self._pf_eligible(N, K) and (m > 64 or size >= self.PF_ALWAYS_WEIGHT_BYTES):
             assert self._ws_pf is not None and self._ws_pf.numel() * 4 >= H.gemm_pf_workspace_bytes(128, N, K), (N, K)
             H.gemm_pf(xf, w, y, m, N, K, ldy, self._ws_pf, epilogue=epi, bias=bias)
-        elif 32 < m <= 64 and K >= 96 and size >= self.BIG_MIN_WEIGHT_BYTES:
+        elif 16 < m <= 64 and K >= 96 and size >= self.BIG_MIN_WEIGHT_BYTES and (m > 32 or epi == H.EPI_ROWS):
             H.gemm_big(xf, w, y, m, N, K, ldy, epi, bias, self._ws_big)
         else:
             H.gemm(xf, w, y, m, N, K, ldy, epi, bias)
@@ -394,8 +401,9 @@ class HipDecoder:
 
     def parts_plan(self, T: int) -> bool:
         """o_proj / down_proj as split-K partial slabs consumed by the next norm: single-rank models with < 256 row groups at
-        decode-sized T (the draft's chain / glue / tree forwards)."""
-        return self.use_parts and not self.use_coll and T <= 32
+        decode-sized T (the draft's chain / glue / tree forwards).  A down_proj of 64 MB and more: up to 16 rows only -- with two token tiles its
+        slabs cost more than the large-tile GEMM's rows (32B, 32 rows, with the norm: 80 -> 55 us)."""
+        return self.use_parts and not self.use_coll and T <= (32 if 2 * self.h * self.I < self.PARTS_WIDE_WEIGHT_BYTES else 16)
 
     def attn_o_plan(self, T: int, meta: AttnMeta, splits: int) -> bool:
         """Attention + o_proj as ONE launch (csrc/attention.hip OPROJ variant): single-rank models on the slab path, one
