@@ -6,7 +6,7 @@
 // cores (gemm_tile.h).  Measured on MI355X, us per product, 128-row chunks -> this kernel:
 //   T = 2594 (Llama-3.2-1B): qkv 3072 x 2048  530 -> 36, gate_up 16384 x 2048  570 -> 160, down 2048 x 8192  960 -> 100
 //   T = 2163 (Llama-3.1-8B): qkv 6144 x 4096  460 -> 110, gate_up 28672 x 4096  875 -> 440, down 4096 x 14336  590 -> 300
-//   T = 16384 (8B): gate_up 6900 -> 3100 (1240 TFLOP/s), down 4600 -> 1540
+//   T = 16384 (8B): gate_up 6900 -> 2900 (1330 TFLOP/s), down 4600 -> 1400
 #include "common.h"
 #include "gemm_tile.h"
 
@@ -15,7 +15,7 @@ enum { BIG_ROWS = 0, BIG_SILU_FRAG = 1, BIG_PARTS = 2 };
 namespace {
 
 template <int WN, int WM, int NT, int MT, int STAGES, int EPI>
-__global__ void __launch_bounds__(64 * WN * WM, 2)
+__global__ void __launch_bounds__(64 * WN * WM, WN * WM <= 8 ? 2 : 4)
 gemm_big_kernel(const char* __restrict__ Wf, const char* __restrict__ Xf, const bf16_t* __restrict__ bias, void* __restrict__ Yv, int M, int N,
                 int K, int ldy, int tn, int tm, int splits) {
   typedef TileLoop<WN, WM, NT, MT, STAGES> L;
@@ -153,13 +153,16 @@ int go(const void* x, const void* w, const void* bias, void* y, int M, int N, in
   return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
 }
 
-// Tile shapes (features x tokens) and what a k-step of 32 takes when n workgroups share a CU, in us (MI355X; fits of
-// T = 130 .. 16384 over the 1B / 8B / 70B matrices, within 15 %).  Large tiles read less LDS per product; small ones leave fewer CUs idle.
-struct Shape { int features, tokens; float step[3], full; };       // step[n - 1] for n <= 3 workgroups on a CU; n * full beyond
-constexpr Shape SHAPES[] = {{256, 128, {0.40f, 0.76f, 1.25f}, 0.42f},
-                            {128, 256, {0.40f, 0.76f, 1.25f}, 0.43f},
-                            {128, 128, {0.29f, 0.45f, 0.66f}, 0.242f},
-                            {128, 64, {0.21f, 0.29f, 0.42f}, 0.167f}};
+// Tile shapes (features x tokens) and what a k-step of 32 takes when n workgroups share a CU, in us (MI355X, operands not in the caches; fits
+// of T = 130 .. 16384 over the 1B / 8B / 70B matrices).  Large tiles read less of L2 and LDS per product -- 256 x 256 on sixteen waves reaches
+// 1.4 PFLOP/s where 256 x 128 on eight stays at 1.28 (16384 x 4096 x 14336: 1390 | 1510 us), but is alone on its CU while it starts and stores
+// (K = 2048 gains nothing) --; small ones leave fewer CUs idle.
+struct Shape { int features, tokens; float step[3], full, ends; };       // step[n - 1] for n <= 3 workgroups on a CU, n * full beyond; filling the ring, storing
+constexpr Shape SHAPES[] = {{256, 128, {0.46f, 0.85f, 1.27f}, 0.42f, 1.0f},
+                            {128, 256, {0.46f, 0.85f, 1.27f}, 0.43f, 1.0f},
+                            {128, 128, {0.29f, 0.44f, 0.75f}, 0.26f, 1.0f},
+                            {128, 64, {0.21f, 0.31f, 0.54f}, 0.20f, 1.0f},
+                            {256, 256, {0.68f, 1.55f, 2.35f}, 0.79f, 4.0f}};
 struct Plan { int shape, splits; };
 
 // The shape and the number of K splits with the least estimated time: k-steps of the fullest CU, plus, for a split product, a launch
@@ -168,13 +171,13 @@ struct Plan { int shape, splits; };
 Plan pick(int M, int N, int K, long ws_bytes) {
   Plan best{0, 1};
   float least = 1e30f;
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < 5; ++c)
     for (int s = 1; s <= 8; ++s) {
       const int steps = (K / 32 + s - 1) / s;
       if (s > 1 && (steps < 8 || (long)s * M * N * 4 > ws_bytes)) break;
       const long tiles = (long)((N + SHAPES[c].features - 1) / SHAPES[c].features) * ((M + SHAPES[c].tokens - 1) / SHAPES[c].tokens) * s;
       const long n = (tiles + 255) / 256;
-      const float est = steps * (n <= 3 ? SHAPES[c].step[n - 1] : n * SHAPES[c].full) + (s > 1 ? 5.0f + (float)s * M * N * 8 / 5e6f : 0.f);
+      const float est = steps * (n <= 3 ? SHAPES[c].step[n - 1] : n * SHAPES[c].full) + n * SHAPES[c].ends + (s > 1 ? 5.0f + (float)s * M * N * 8 / 5e6f : 0.f);
       if (est < least) { least = est; best = Plan{c, s}; }
     }
   return best;
@@ -188,14 +191,15 @@ extern "C" int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const vo
   if (epilogue != BIG_ROWS && epilogue != BIG_SILU_FRAG) return SSD_ERR_ARG;
   if (M <= 0 || N <= 0 || K < 64 || N % 16 || K % 32 || (epilogue == BIG_SILU_FRAG && N % 64) || K > (1 << 22)) return SSD_ERR_SHAPE;
   if (epilogue == BIG_ROWS && (ldy < N || ldy % 4)) return SSD_ERR_SHAPE;
-  if (shape < 0 || shape > 3 || splits < 1 || splits > 8 || K / 32 / splits < 3) return SSD_ERR_ARG;
+  if (shape < 0 || shape > 4 || splits < 1 || splits > 8 || K / 32 / splits < 3) return SSD_ERR_ARG;
   if (splits > 1 && (!workspace || workspace_bytes < (int64_t)splits * M * N * 4)) return SSD_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
 #define BIG_ARGS x_frag, w_frag, bias, y, M, N, K, ldy, epilogue, splits, workspace, st
   if (shape == 0) return go<4, 2, 4, 4, 3>(BIG_ARGS);
   if (shape == 1) return go<2, 4, 4, 4, 3>(BIG_ARGS);
   if (shape == 2) return go<2, 2, 4, 4, 3>(BIG_ARGS);
-  return go<2, 2, 4, 2, 4>(BIG_ARGS);
+  if (shape == 3) return go<2, 2, 4, 2, 4>(BIG_ARGS);
+  return go<4, 4, 4, 4, 4>(BIG_ARGS);
 #undef BIG_ARGS
 }
 

@@ -291,10 +291,11 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, v
 // read serves at a time find their chunks in different banks.  The rows of a grouped product are gathered by the same loads.  The
 // accumulators go through LDS once more, 16 or 32 token rows at a time: a wave then stores whole runs of a row, whatever the epilogue.
 // Bound by the matrix cores.  MI355X, against the 64 x 64 form below (which re-stages both operands through registers, two barriers per 32-wide
-// k-step): 4000 x 14720 x 4096 1516 -> 452 us (1070 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 41.
+// k-step): 4000 x 14720 x 4096 1516 -> 418 us (1150 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 41.
+// (The 256 x 256 tile runs sixteen waves of 64 x 64: with eight of 128 x 64 the first took 452 us.)
 // ---------------------------------------------------------------------------------------------------------------------
 template <typename T, int WN, int WM, int NT, int MT, bool GROUPED>
-__global__ void __launch_bounds__(64 * WN * WM, 2)
+__global__ void __launch_bounds__(64 * WN * WM, WN * WM <= 8 ? 2 : 4)
 gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
                       const int* __restrict__ offsets, int E, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx,
                       long gsy, GluClamp gc, DecayGate dg, int tn, int tm, bool vec_out) {
@@ -478,7 +479,7 @@ constexpr int SKINNY_MAX_ROWS = 16, SKINNY_MAX_GROUPED_ROWS = 64;
 // leave half a tile empty each.
 int tile_shape(int M, int N, int G, int E) {
   constexpr int FEATURES[3] = {256, 128, 128}, TOKENS[3] = {256, 128, 64};
-  constexpr float STEP[3][3] = {{1.55f, 3.5f, 5.3f}, {0.66f, 1.0f, 1.5f}, {0.55f, 0.75f, 1.05f}}, FULL[3] = {1.77f, 0.48f, 0.33f};
+  constexpr float STEP[3][3] = {{1.6f, 3.2f, 4.9f}, {0.66f, 1.0f, 1.5f}, {0.55f, 0.75f, 1.05f}}, FULL[3] = {1.63f, 0.48f, 0.33f};
   int best = 0;
   float least = 1e30f;
   for (int c = 0; c < 3; ++c) {
@@ -559,7 +560,7 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   {                                                                   \
     if (f32 && shape == 0) TILE_GO(float, 2, 2, 4, 4, GROUPED)        \
     else if (f32) TILE_GO(float, 2, 2, 2, 2, GROUPED)                 \
-    else if (shape == 0) TILE_GO(bf16_t, 2, 4, 8, 4, GROUPED)         \
+    else if (shape == 0) TILE_GO(bf16_t, 4, 4, 4, 4, GROUPED)         \
     else if (shape == 1) TILE_GO(bf16_t, 2, 2, 4, 4, GROUPED)         \
     else TILE_GO(bf16_t, 2, 2, 4, 2, GROUPED)                         \
   }

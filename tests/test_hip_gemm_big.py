@@ -36,7 +36,7 @@ def check(y, ref, what):
     assert bool(((y - ref).abs() <= tol).all()), (what, float(((y - ref).abs() - tol).max()))
 
 
-@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3])
+@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3, 4])
 @pytest.mark.parametrize("M,N,K,splits", [(1, 16, 96, 1), (129, 272, 96, 1), (257, 144, 352, 3), (255, 512, 1024, 8), (64, 4112, 160, 1), (700, 128, 2080, 2)])
 def test_rows(H, shape, M, N, K, splits):
     x, w, b = operands(M, N, K, M + N + K)
@@ -50,7 +50,7 @@ def test_rows(H, shape, M, N, K, splits):
         assert bool((y[:, N:] == 7.0).all())
 
 
-@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3])
+@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3, 4])
 @pytest.mark.parametrize("M,I,K,splits", [(130, 96, 96, 1), (257, 160, 416, 2)])
 def test_silu(H, shape, M, I, K, splits):
     x, w, _ = operands(M, 2 * I, K, M + I)
