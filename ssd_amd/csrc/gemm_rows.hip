@@ -205,65 +205,161 @@ gemm_rows_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restr
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
-// Skinny form (bf16, K % 8 == 0, few token rows: decoding): a weight-streaming product.  A workgroup owns 16 features; its NW waves take
-// the 32-wide k-tiles round-robin in runs of U, so the workgroup as a whole walks its 16 weight rows linearly; both MFMA operands are
-// 16-byte loads straight from the row-major matrices (lane = (row & 15) + 16 * (k chunk)); the waves' partial tiles are summed through
-// LDS in wave order.  Grouped: blockIdx.y is the group; a group with no rows exits at once, one with more than 16 rows loops over
-// 16-row chunks.
+// Skinny form (few token rows, or few features: decoding, routers; 16-byte aligned rows; bf16 K % 8 == 0, fp32 K % 32 == 0): a weight-streaming
+// product, bound by the weights' way from HBM.  A workgroup owns 16 features; its four waves take K in turn, in runs of 256 k, each through a ring
+// of its own that DMA fills (no barrier: only the wave itself waits for it).  A stage is 256 bytes of 16 weight rows and of the token rows:
+// one instruction fetches four whole 256-byte pieces, whose 16-byte chunks are rotated by the row so that the 16 lanes of an operand read hit
+// different banks.  (16-byte loads straight into the MFMA layout fetch 64 bytes of a row at a time, and a wave has nothing in flight while it
+// multiplies.)  Two workgroups share a CU, one's loads covering the other's start and end; more waves or deeper rings gained nothing.
+//   bf16: a wave's runs are one chain of 16x16x32 MFMAs, the waves' sums are added in wave order.
+//   fp32: a run is a segment of gemm_tile.h's order; after every round of four, wave 0 adds the segments' sums in theirs.
+// MI355X, weights not in the caches, direct loads -> this: bf16, 4 rows: 14720 x 4096 36.6 -> 21.3 us (5.7 TB/s), 4096 x 14720 31.5 -> 19.3,
+// 4096 x 4096 11.6 -> 7.9, 2048 x 7424 18.9 -> 8.8; fp32, 4 rows: 32000 x 2048 77 -> 40 us (6.6 TB/s), 3088 x 2048 11.4 -> 6.8, 2048 x 3072
+// 16.9 -> 8.8.  fp32 error against fp64, relative: 3e-7 at K = 2048 .. 4096.
+// Grouped: blockIdx.y is the group; a group with no rows exits at once.  16-row chunks are dealt out over blockIdx.z.
 // ---------------------------------------------------------------------------------------------------------------------
-template <int NW>
-__global__ void __launch_bounds__(NW * 64)
-gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
+constexpr int SKINNY_WAVES = 4;
+template <typename T>
+struct Skinny {
+  static constexpr bool F32 = sizeof(T) == 4;
+  static constexpr int SPR = F32 ? F32_SEG * 4 / 256 : 2;                    // stages of a run
+  static constexpr int RING = 16 * 1024;                                      // LDS bytes of a wave's ring: the largest of stages() x stage_bytes()
+  static constexpr int stage_bytes(int xi) { return (4 + xi) * 1024; }
+  static constexpr int stages(int xi) { return xi == 1 ? 3 : 2; }
+
+  // Up to 4 * XI token rows at xr (this lane's four-row pieces) against the 16 weight rows at wr: wave 0 returns the sums.
+  template <int XI>
+  static __device__ __forceinline__ f32x4_t chunk(char* ring, f32x4_t (*red)[SKINNY_WAVES][64], uint32_t& turn, const char* const (&wr)[4],
+                                                  const char* const (&xr)[XI], long row_bytes) {
+    constexpr int NW = SKINNY_WAVES, R = stages(XI), STAGE = stage_bytes(XI), PER = 4 + XI;
+    static_assert(R * STAGE <= RING, "the ring holds the stages");
+    const int lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4, xrow = r & (4 * XI - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int S = (int)((row_bytes + 255) >> 8), runs = (S + SPR - 1) / SPR;
+    const bool ragged = (row_bytes & 255) != 0;                              // the last stage is a part of one
+    const int mine = runs > wave ? (runs - wave + NW - 1) / NW : 0;
+    const int n = mine * SPR - (mine && wave + (mine - 1) * NW == runs - 1 ? runs * SPR - S : 0);       // this wave's stages
+    auto stage_of = [&](int l) { return ((l / SPR) * NW + wave) * SPR + l % SPR; };
+    auto fetch = [&](int l, int slot) {
+      const long off = (long)stage_of(l) * 256;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int row = (i < 4 ? i : i - 4) * 4 + qd;
+        long at = off + (r ^ row) * 16;
+        if (ragged) at = at < row_bytes ? at : row_bytes - 16;
+        const char* src = (i < 4 ? wr[i < 4 ? i : 0] : xr[i < 4 ? 0 : i - 4]) + at;
+        auto* dst = (__attribute__((address_space(3))) void*)(ring + slot * STAGE + i * 1024);
+        if (i < 4) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, dst, 16, 0, 2);        // (weights: non-temporal)
+        else __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, dst, 16, 0, 0);
+      }
+    };
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                       // the ring is free: what was read of it has arrived
+#pragma unroll
+    for (int s = 0; s < R - 1; ++s)
+      if (s < n) fetch(s, s);
+    f32x4_t total = {0.f, 0.f, 0.f, 0.f};
+    int cur = 0, l = 0;
+    const int rounds = F32 ? (runs + NW - 1) / NW : 1;
+    for (int round = 0; round < rounds; ++round, ++turn) {
+      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+      const int end = F32 ? min(n, (round + 1) * SPR) : n;
+      for (; l < end; ++l) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                   // (the stage before is in registers)
+        const int ahead = n - 1 - l;
+        if (ahead >= R - 1) {
+          fetch(l + R - 1, cur == 0 ? R - 1 : cur - 1);
+          tile_wait<(R - 1) * PER>();
+        } else if (R > 2 && ahead == 1) {
+          tile_wait<PER>();
+        } else {
+          tile_wait<0>();
+        }
+        const char* p = ring + cur * STAGE;
+        cur = cur + 1 == R ? 0 : cur + 1;
+        u32x4_t a[4], b[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          a[j] = *reinterpret_cast<const u32x4_t*>(p + r * 256 + ((j * 4 + qd) ^ r) * 16);
+          b[j] = *reinterpret_cast<const u32x4_t*>(p + 4096 + xrow * 256 + ((j * 4 + qd) ^ xrow) * 16);
+        }
+        const long left = row_bytes - (long)stage_of(l) * 256;               // bytes of the rows from this stage on
+        if (ragged && left < 256) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if ((j * 4 + qd) * 16 >= left) a[j] = b[j] = u32x4_t{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (j && j * 64 >= left) break;
+          if constexpr (F32) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = mfma_f32(a[j][e], b[j][e], acc);
+          } else {
+            acc = mfma16(a[j], b[j], acc);
+          }
+        }
+      }
+      // (two sets of sums in turn: one barrier per round both publishes a set and tells that the one before has been read)
+      red[turn & 1][wave][lane] = acc;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (wave == 0) {
+#pragma unroll
+        for (int v = 0; v < NW; ++v)
+          if (round * NW + v < runs) total += red[turn & 1][v][lane];
+      }
+    }
+    return total;
+  }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(SKINNY_WAVES * 64)
+gemm_skinny_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
                    const int* __restrict__ offsets, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx,
                    long gsy, GluClamp gc, DecayGate dg) {
-  constexpr int U = 8;
-  __shared__ f32x4_t red[NW * 64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
+  typedef Skinny<T> L;
+  __shared__ __attribute__((aligned(1024))) char smem[SKINNY_WAVES * L::RING];
+  __shared__ f32x4_t red[2][SKINNY_WAVES][64];
+  const int lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = blockIdx.x * 16;
   int m_begin = 0, m_end = M;
-  const bf16_t* wg = w;
   long ycol = 0;
-  if (!offsets) {          // batched (or a single product: blockIdx.y == 0)
-    wg = w + (size_t)blockIdx.y * N * K;
-    x += (size_t)blockIdx.y * gsx;
-    ycol = (long)blockIdx.y * gsy;
-  }
   if (offsets) {
     m_begin = offsets[blockIdx.y];
     m_end = offsets[blockIdx.y + 1];
     if (m_begin >= m_end) return;
-    wg = w + (size_t)blockIdx.y * N * K;
+  } else {                 // batched (or a single product: blockIdx.y == 0)
+    x += (size_t)blockIdx.y * gsx;
+    ycol = (long)blockIdx.y * gsy;
   }
-  const int nrow = min(n0 + r, N - 1);
-  const bf16_t* wp = wg + (size_t)nrow * K + qd * 8;
-  const int KT = (K + 31) >> 5;
-  for (int m0 = m_begin; m0 < m_end; m0 += 16) {
-    const int mrow = m0 + r;
-    const bool mvalid = mrow < m_end;
-    const long xrow = mvalid ? (row_idx ? (long)(row_idx[mrow] / idx_div) : (long)mrow) : 0;
-    const bf16_t* xp = x + xrow * ldx + qd * 8;
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    for (int kt0 = wave * U; kt0 < KT; kt0 += NW * U) {
-      u32x4_t a[U], b[U];
+  const long row_bytes = (long)K * (long)sizeof(T);
+  const char* wr[4];
 #pragma unroll
-      for (int i = 0; i < U; ++i) {
-        const int kt = kt0 + i;
-        const bool ok = kt < KT && kt * 32 + qd * 8 < K;
-        a[i] = u32x4_t{0u, 0u, 0u, 0u};
-        b[i] = u32x4_t{0u, 0u, 0u, 0u};
-        if (ok) a[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp + kt * 32));
-        if (ok && mvalid) b[i] = *reinterpret_cast<const u32x4_t*>(xp + kt * 32);
-      }
-#pragma unroll
-      for (int i = 0; i < U; ++i) acc = mfma16(a[i], b[i], acc);
+  for (int i = 0; i < 4; ++i)
+    wr[i] = reinterpret_cast<const char*>(w) + ((size_t)blockIdx.y * N + min(n0 + i * 4 + qd, N - 1)) * row_bytes;
+  char* ring = smem + wave * L::RING;
+  uint32_t turn = 0;
+  for (int m0 = m_begin + 16 * blockIdx.z; m0 < m_end; m0 += 16 * gridDim.z) {
+    const int rows = min(m_end - m0, 16);
+    auto token = [&](int i) {
+      const int m = m0 + min(i * 4 + qd, rows - 1);
+      return reinterpret_cast<const char*>(x + (row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx);
+    };
+    f32x4_t sum;
+    if (rows <= 4) {
+      const char* const xr[1] = {token(0)};
+      sum = L::template chunk<1>(ring, red, turn, wr, xr, row_bytes);
+    } else if (rows <= 8) {
+      const char* const xr[2] = {token(0), token(1)};
+      sum = L::template chunk<2>(ring, red, turn, wr, xr, row_bytes);
+    } else {
+      const char* const xr[4] = {token(0), token(1), token(2), token(3)};
+      sum = L::template chunk<4>(ring, red, turn, wr, xr, row_bytes);
     }
-    red[wave * 64 + lane] = acc;
-    __syncthreads();
-    if (wave == 0) {
-      f32x4_t sum = red[lane];
-#pragma unroll
-      for (int wv = 1; wv < NW; ++wv) sum += red[wv * 64 + lane];
-      if (mvalid && epi_pairs(epi)) {
+    const int mrow = m0 + r;
+    if (wave == 0 && r < rows) {
+      if (!L::F32 && epi_pairs(epi)) {
         const float rs = epi == 6 && gc.row_scale ? gc.row_scale[row_idx ? row_idx[mrow] : mrow] : 1.0f;
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
@@ -272,15 +368,14 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, v
             reinterpret_cast<bf16_t*>(y)[(long)mrow * ldy + ycol + (n >> 1)] =
                 (bf16_t)f2bf(glu_act(sum[e], sum[e + 1], epi, rs, gc.limit, gc.alpha));
         }
-      } else if (mvalid) {
+      } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int n = n0 + qd * 4 + e;
-          if (n < N) store_out<bf16_t>(y, mrow, ldy, ycol + n, sum[e], epi, dg);
+          if (n < N) store_out<T>(y, mrow, ldy, ycol + n, sum[e], epi, dg);
         }
       }
     }
-    __syncthreads();
   }
 }
 
@@ -397,81 +492,6 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
   }
 }
 
-// ---------------------------------------------------------------------------------------------------------------------
-// Skinny form in fp32 (K % 32 == 0, aligned rows, few token rows or few features): a workgroup owns 16 features and its 8 waves take the
-// segments of K in turn, so that eight segments of the 16 weight rows are in flight together; after every round wave 0 adds the segments'
-// sums in their order (gemm_tile.h).  Bound by the weights' way from HBM.  MI355X, against the 64 x 64 form of FMA chains: 3 x 3088 x 2048
-// 139 -> 11 us, 3 x 32000 x 2048 214 -> 74 us (3.5 TB/s); large: 2000 x 4096 x 4096 1021 -> 524 us (tile form).  Error against fp64, relative:
-// 8e-7 -> 3e-7 at K = 2048, 1.1e-6 -> 3e-7 at 4096 (segments shorten the chains).
-// ---------------------------------------------------------------------------------------------------------------------
-constexpr int SKINNY32_WAVES = 8;
-__global__ void __launch_bounds__(SKINNY32_WAVES * 64)
-gemm_skinny_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int M, int N, int K, int epi,
-                       const int* __restrict__ offsets, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx, long gsy,
-                       DecayGate dg) {
-  constexpr int NW = SKINNY32_WAVES, U = 8;
-  __shared__ f32x4_t red[NW][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  int m_begin = 0, m_end = M;
-  const float* wg = w + (size_t)blockIdx.y * N * K;
-  long ycol = 0;
-  if (offsets) {
-    m_begin = offsets[blockIdx.y];
-    m_end = offsets[blockIdx.y + 1];
-    if (m_begin >= m_end) return;
-  } else {                 // batched (or a single product: blockIdx.y == 0)
-    x += (size_t)blockIdx.y * gsx;
-    ycol = (long)blockIdx.y * gsy;
-  }
-  const float* wp = wg + (size_t)min(n0 + r, N - 1) * K + qd * 4;
-  const int segs = (K + F32_SEG - 1) / F32_SEG;
-  for (int m0 = m_begin + 16 * blockIdx.z; m0 < m_end; m0 += 16 * gridDim.z) {
-    const int mrow = m0 + r;
-    const bool mvalid = mrow < m_end;
-    const float* xp = x + (mvalid ? (row_idx ? (long)(row_idx[mrow] / idx_div) : (long)mrow) : 0) * ldx + qd * 4;
-    f32x4_t total = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < segs; s0 += NW) {
-      const int seg = s0 + wave;
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-      if (seg < segs) {
-        const int k0 = seg * F32_SEG, blocks = (min(K - k0, F32_SEG)) >> 4;
-        for (int b0 = 0; b0 < blocks; b0 += U) {
-          u32x4_t a[U], b[U];
-#pragma unroll
-          for (int i = 0; i < U; ++i) {
-            a[i] = b[i] = u32x4_t{0u, 0u, 0u, 0u};
-            const bool ok = b0 + i < blocks;
-            if (ok) a[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp + k0 + (b0 + i) * 16));
-            if (ok && mvalid) b[i] = *reinterpret_cast<const u32x4_t*>(xp + k0 + (b0 + i) * 16);
-          }
-#pragma unroll
-          for (int i = 0; i < U; ++i)
-            if (b0 + i < blocks) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc = mfma_f32(a[i][e], b[i][e], acc);
-            }
-        }
-      }
-      red[wave][lane] = acc;
-      __syncthreads();
-      if (wave == 0) {
-#pragma unroll
-        for (int v = 0; v < NW; ++v)
-          if (s0 + v < segs) total += red[v][lane];
-      }
-      __syncthreads();
-    }
-    if (wave == 0 && mvalid) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int n = n0 + qd * 4 + e;
-        if (n < N) store_out<float>(y, mrow, ldy, ycol + n, total[e], epi, dg);
-      }
-    }
-  }
-}
-
 constexpr int SKINNY_MAX_ROWS = 16, SKINNY_MAX_GROUPED_ROWS = 64;
 
 // The tile shape (256 x 256, 128 x 128 or 128 x 64 features x tokens) with the least estimated time: k-steps of the fullest CU, in us per
@@ -513,21 +533,8 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   const bool x_vec = ((size_t)ldx * esz0) % 16 == 0 && ((size_t)gsx * esz0) % 16 == 0 && (uintptr_t)x % 16 == 0;
   if (!f32 && K % 8 == 0 && x_vec && (uintptr_t)w % 16 == 0 &&
       M <= (offsets ? SKINNY_MAX_GROUPED_ROWS : SKINNY_MAX_ROWS)) {
-    const int groups = (N + 15) / 16;
-    const dim3 sg(groups, offsets ? E : G);
-    const int id = idx_div < 1 ? 1 : idx_div;
-    const long wgs = (long)groups * (offsets ? (M < E ? M : E) : G);          // workgroups that have rows
-    // few workgroups: more waves each (a CU pulls from HBM what its waves have in flight), as long as every wave gets k-tiles
-    const int kt = (K + 31) / 32;
-    if (wgs < 256 && kt >= 64)
-      hipLaunchKernelGGL(gemm_skinny_kernel<16>, sg, dim3(1024), 0, (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)w, y, M, N, K,
-                         epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, gc, dg);
-    else if (wgs < 1024 && kt >= 32)
-      hipLaunchKernelGGL(gemm_skinny_kernel<8>, sg, dim3(512), 0, (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)w, y, M, N, K,
-                         epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, gc, dg);
-    else
-      hipLaunchKernelGGL(gemm_skinny_kernel<4>, sg, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)w, y, M, N, K,
-                         epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, gc, dg);
+    hipLaunchKernelGGL(gemm_skinny_kernel<bf16_t>, dim3((N + 15) / 16, offsets ? E : G), dim3(64 * SKINNY_WAVES), 0, (hipStream_t)stream,
+                       (const bf16_t*)x, (const bf16_t*)w, y, M, N, K, epi, offsets, row_idx, idx_div < 1 ? 1 : idx_div, ldx, ldy, gsx, gsy, gc, dg);
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
   // (fp32: which of the two orders of summation a product gets -- gemm_tile.h's, or the plain chain of the form for everything else -- may
@@ -538,8 +545,8 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   // tile, a serial walk of K by few workgroups; a router's 1000 x 8 x 2048 the same 48 us)
   const int chunks = (M + 15) / 16;
   if (tiled && f32 && (offsets ? M <= SKINNY_MAX_GROUPED_ROWS : M <= SKINNY_MAX_ROWS || (long)chunks * ((N + 15) / 16) * G <= 1024)) {
-    hipLaunchKernelGGL(gemm_skinny_f32_kernel, dim3((N + 15) / 16, offsets ? E : G, offsets ? 1 : chunks), dim3(64 * SKINNY32_WAVES), 0, (hipStream_t)stream,
-                       (const float*)x, (const float*)w, (float*)y, M, N, K, epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, dg);
+    hipLaunchKernelGGL(gemm_skinny_kernel<float>, dim3((N + 15) / 16, offsets ? E : G, offsets ? 1 : chunks), dim3(64 * SKINNY_WAVES), 0,
+                       (hipStream_t)stream, (const float*)x, (const float*)w, y, M, N, K, epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, gc, dg);
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
   if (tiled) {
