@@ -380,24 +380,24 @@ gemm_skinny_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __res
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
-// Large-tile form (bf16, K % 64 == 0, 16-byte aligned rows, more rows than the skinny form takes: prompts, larger batches): the main loop
+// Large-tile form (bf16, K % 64 == 0; fp32, K % 32 == 0; 16-byte aligned rows, more rows than the skinny form takes: prompts, larger batches): the main loop
 // of gemm_tile.h over row-major operands, k-steps of 64.  An operand's DMA covers 8 rows x 128 bytes -- whole cache lines; 16 rows x 64
 // bytes, the MFMA operand itself, ran at 60 % -- and lane l fetches chunk (l & 7) ^ (l >> 3) of row l >> 3, so that the eight lanes which an LDS
 // read serves at a time find their chunks in different banks.  The rows of a grouped product are gathered by the same loads.  The
 // accumulators go through LDS once more, 16 or 32 token rows at a time: a wave then stores whole runs of a row, whatever the epilogue.
 // Bound by the matrix cores.  MI355X, against the 64 x 64 form below (which re-stages both operands through registers, two barriers per 32-wide
-// k-step): 4000 x 14720 x 4096 1516 -> 418 us (1150 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 41.
+// k-step): 4000 x 14720 x 4096 1516 -> 418 us (1150 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 35.
 // (The 256 x 256 tile runs sixteen waves of 64 x 64: with eight of 128 x 64 the first took 452 us.)
 // ---------------------------------------------------------------------------------------------------------------------
-template <typename T, int WN, int WM, int NT, int MT, bool GROUPED>
+template <typename T, int WN, int WM, int NT, int MT, int STAGES, bool GROUPED>
 __global__ void __launch_bounds__(64 * WN * WM, WN * WM <= 8 ? 2 : 4)
 gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
                       const int* __restrict__ offsets, int E, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx,
                       long gsy, GluClamp gc, DecayGate dg, int tn, int tm, bool vec_out) {
   constexpr bool F32 = sizeof(T) == 4;
   constexpr int VEC = 16 / sizeof(T), ROWB = sizeof(T);              // elements of a 16-byte chunk; bytes of an element
-  typedef TileLoop<WN, WM, NT, MT, 2, 2, F32> L;
-  constexpr int LDT = NT * 16 + 4, PASS = L::WAVES * 32 * LDT * 4 <= L::LDS ? 32 : 16;                       // a wave's epilogue rows (floats), token rows per pass
+  typedef TileLoop<WN, WM, NT, MT, STAGES, 2, F32> L;
+  constexpr int LDT = NT * 16 + 4, PASS = MT % 2 == 0 && L::WAVES * 32 * LDT * 4 <= L::LDS ? 32 : 16;                       // a wave's epilogue rows (floats), token rows per pass
   static_assert(MT * 16 % PASS == 0 && L::WAVES * PASS * LDT * 4 <= L::LDS, "the epilogue rows fit the ring");
   __shared__ __attribute__((aligned(1024))) char smem[L::LDS];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -494,27 +494,28 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
 
 constexpr int SKINNY_MAX_ROWS = 16, SKINNY_MAX_GROUPED_ROWS = 64;
 
-// The tile shape (256 x 256, 128 x 128 or 128 x 64 features x tokens) with the least estimated time: k-steps of the fullest CU, in us per
-// step of 64 when n workgroups share it (MI355X, fits of 20 .. 4000 rows over 4096 .. 14720-wide matrices).  A grouped product's runs
-// leave half a tile empty each.
-int tile_shape(int M, int N, int G, int E) {
-  constexpr int FEATURES[3] = {256, 128, 128}, TOKENS[3] = {256, 128, 64};
-  constexpr float STEP[3][3] = {{1.6f, 3.2f, 4.9f}, {0.66f, 1.0f, 1.5f}, {0.55f, 0.75f, 1.05f}}, FULL[3] = {1.63f, 0.48f, 0.33f};
+// The tile shape with the least estimated time: k-steps of the fullest CU, in us per step of 128 bytes of a row when n workgroups share it
+// (MI355X, fits of 20 .. 7000 rows over 2048 .. 14720-wide matrices).  A grouped product's runs leave half a tile empty each.
+//   bf16: 256 x 256 (features x tokens) has the highest rate, 192 x 192 comes next and divides other sizes (4228 x 4096 x 14720: 506 tiles on
+//   256 CUs, 478 us, where 272 of 256 x 256 take 663 and 1088 of 128 x 128 610); 128 x 64 has a third stage, as it is chosen where a CU
+//   has one or two workgroups (500 x 4096 x 4096: 39 -> 33 us).
+//   fp32, bound by the matrix cores: 64 x 32 fills the chip with a few hundred rows (562 x 2048 x 2048 80 -> 64 us, 568 gathered rows of 8 experts
+//   x 3072 x 2048 146 -> 106).
+struct RowTile { int features, tokens; float step[3], full; };       // step[n - 1] for n <= 3, n * full beyond
+constexpr RowTile TILES_BF16[] = {{256, 256, {1.45f, 3.2f, 4.9f}, 1.66f}, {192, 192, {1.05f, 2.15f, 3.2f}, 1.06f}, {128, 128, {0.70f, 1.03f, 1.5f}, 0.51f},
+                                  {128, 64, {0.48f, 0.75f, 1.15f}, 0.38f}};
+constexpr RowTile TILES_F32[] = {{128, 128, {2.25f, 4.4f, 6.3f}, 2.03f}, {64, 64, {0.77f, 1.27f, 1.8f}, 0.54f}, {64, 32, {0.45f, 0.71f, 1.0f}, 0.33f}};
+template <int COUNT>
+int tile_shape(const RowTile (&tiles)[COUNT], int M, int N, int G, int E) {
   int best = 0;
   float least = 1e30f;
-  for (int c = 0; c < 3; ++c) {
-    const long tiles = (long)((N + FEATURES[c] - 1) / FEATURES[c]) * ((M + TOKENS[c] - 1) / TOKENS[c] + (E + 1) / 2) * G, n = (tiles + 255) / 256;
-    const float est = n <= 3 ? STEP[c][n - 1] : n * FULL[c];
+  for (int c = 0; c < COUNT; ++c) {
+    const long count = (long)((N + tiles[c].features - 1) / tiles[c].features) * ((M + tiles[c].tokens - 1) / tiles[c].tokens + (E + 1) / 2) * G;
+    const long n = (count + 255) / 256;
+    const float est = n <= 3 ? tiles[c].step[n - 1] : n * tiles[c].full;
     if (est < least) { least = est; best = c; }
   }
   return best;
-}
-
-// fp32: 128 x 128 (0) or 64 x 64 (1) -- bound by the matrix cores either way (a 64 x 64 tile reads a quarter of what LDS and L2 deliver), so the
-// shape that keeps the fullest CU shortest: 514 x 3088 x 2048 147 | 79 us, 4000 x 14720 x 4096 3866 | 3903.
-int tile_shape_f32(int M, int N, int G, int E) {
-  const long t0 = (long)((N + 127) / 128) * ((M + 127) / 128 + (E + 1) / 2) * G, t1 = (long)((N + 63) / 64) * ((M + 63) / 64 + (E + 1) / 2) * G;
-  return (t0 + 255) / 256 * 4 <= (t1 + 255) / 256 ? 0 : 1;
 }
 
 int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, const int* offsets, int E, const int* row_idx,
@@ -550,26 +551,28 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
   if (tiled) {
-    const int shape = f32 ? tile_shape_f32(M, N, G, offsets ? E : 0) : tile_shape(M, N, G, offsets ? E : 0);
+    const int shape = f32 ? tile_shape(TILES_F32, M, N, G, offsets ? E : 0) : tile_shape(TILES_BF16, M, N, G, offsets ? E : 0);
     // what a store of four (paired: two) neighbouring outputs needs: their address a multiple of its size
     const bool out32 = f32 || epi == 0 || epi == 8;
     const int width = epi_pairs(epi) ? 4 : (out32 ? 16 : 8), osz = out32 ? 4 : 2;
     const bool vec_out = (uintptr_t)y % width == 0 && (size_t)ldy * osz % width == 0 && (size_t)gsy * osz % width == 0;
-#define TILE_GO(T, WN, WM, NT, MT, GROUPED)                                                                                           \
+#define TILE_GO(T, WN, WM, NT, MT, STAGES, GROUPED)                                                                                       \
   {                                                                                                                                   \
-    typedef TileLoop<WN, WM, NT, MT, 2, 2, sizeof(T) == 4> L;                                                                         \
+    typedef TileLoop<WN, WM, NT, MT, STAGES, 2, sizeof(T) == 4> L;                                                                    \
     const int tn = (N + L::WG * 16 - 1) / (L::WG * 16), tm = (M + L::XG * 16 - 1) / (L::XG * 16) + (offsets ? E : 0);                 \
-    hipLaunchKernelGGL((gemm_rows_tile_kernel<T, WN, WM, NT, MT, GROUPED>), dim3(tn * tm, G), dim3(64 * L::WAVES), 0,                 \
+    hipLaunchKernelGGL((gemm_rows_tile_kernel<T, WN, WM, NT, MT, STAGES, GROUPED>), dim3(tn * tm, G), dim3(64 * L::WAVES), 0,                 \
                        (hipStream_t)stream, (const T*)x, (const T*)w, y, M, N, K, epi, offsets, E, row_idx, id, ldx, ldy, gsx, gsy,   \
                        gc, dg, tn, tm, vec_out);                                                                                      \
   }
-#define TILE_SHAPES(GROUPED)                                          \
-  {                                                                   \
-    if (f32 && shape == 0) TILE_GO(float, 2, 2, 4, 4, GROUPED)        \
-    else if (f32) TILE_GO(float, 2, 2, 2, 2, GROUPED)                 \
-    else if (shape == 0) TILE_GO(bf16_t, 4, 4, 4, 4, GROUPED)         \
-    else if (shape == 1) TILE_GO(bf16_t, 2, 2, 4, 4, GROUPED)         \
-    else TILE_GO(bf16_t, 2, 2, 4, 2, GROUPED)                         \
+#define TILE_SHAPES(GROUPED)                                                \
+  {                                                                         \
+    if (f32 && shape == 0) TILE_GO(float, 2, 2, 4, 4, 2, GROUPED)           \
+    else if (f32 && shape == 1) TILE_GO(float, 2, 2, 2, 2, 2, GROUPED)      \
+    else if (f32) TILE_GO(float, 2, 2, 2, 1, 4, GROUPED)                    \
+    else if (shape == 0) TILE_GO(bf16_t, 4, 4, 4, 4, 2, GROUPED)            \
+    else if (shape == 1) TILE_GO(bf16_t, 4, 4, 3, 3, 3, GROUPED)            \
+    else if (shape == 2) TILE_GO(bf16_t, 2, 2, 4, 4, 2, GROUPED)            \
+    else TILE_GO(bf16_t, 2, 2, 4, 2, 3, GROUPED)                            \
   }
     if (offsets) TILE_SHAPES(true) else TILE_SHAPES(false)
 #undef TILE_SHAPES

@@ -42,7 +42,7 @@ struct TileLoop {
   static_assert((WG + XG) * KS % WAVES == 0, "every wave fetches as many operands");
 
   // fetch_one(i, step, lds): KiB i of this wave's PER (KiB wave * PER + i of the workgroup's step: W's groups first, KS each, then x's) of
-  // step `step` on its way to LDS.  at[s]: where in a group's KS KiB this lane finds its part of the s-th MFMA operand.  nk >= STAGES - 1.
+  // step `step` on its way to LDS.  at[s]: where in a group's KS KiB this lane finds its part of the s-th MFMA operand.
   template <typename Fetch>
   static __device__ __forceinline__ void run(char* smem, int nk, const uint32_t (&at)[KS], f32x4_t (&acc)[NT][MT], const Fetch& fetch_one) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -56,7 +56,7 @@ struct TileLoop {
       for (int i = 0; i < PER; ++i) fetch_one(i, step, smem + buf * STEP + (wave * PER + i) * 1024);
     };
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) fetch(s, s);
+    for (int s = 0; s < STAGES - 1; ++s) fetch(s < nk ? s : nk - 1, s);
     uint32_t cur = 0;
     f32x4_t part[F32 ? NT : 1][F32 ? MT : 1];
     if constexpr (F32) {

@@ -39,8 +39,8 @@ def act(z, epi):
     return 0.5 * a * (1 + torch.tanh(math.sqrt(2 / math.pi) * (a + 0.044715 * a ** 3))) * u
 
 
-# sizes: 256-token tiles are chosen for the third, 128 for the fourth, 64 for the others; features off every tile and vector width
-@pytest.mark.parametrize("M,N,K", [(17, 128, 128), (65, 131, 192), (4000, 4050, 128), (2001, 4098, 128), (129, 386, 4096)])
+# sizes: 256-token tiles are chosen for the third, 192 for the fourth, 128 for the fifth, 64 for the others; features off every tile and vector width
+@pytest.mark.parametrize("M,N,K", [(17, 128, 128), (65, 131, 192), (4000, 4050, 128), (2001, 4098, 128), (700, 6002, 128), (129, 386, 4096)])
 def test_dense_epilogues(H, M, N, K):
     x, w = operands(M, N, K, M + N + K)
     z = x.double() @ w.double().T
@@ -98,7 +98,7 @@ def test_grouped(H, counts, N, K, div):
 
 
 # fp32: a segment of 256 is a chain of 256 roundings (2^-24 each of a partial sum below 5), then one per segment: 272 * 5 * 2^-24 < 1e-4 at worst
-@pytest.mark.parametrize("M,N,K", [(3, 131, 64), (70, 66, 288), (200, 1030, 544), (1300, 8, 2048), (2100, 2200, 96)])
+@pytest.mark.parametrize("M,N,K", [(3, 131, 64), (70, 66, 288), (200, 1030, 544), (1300, 8, 2048), (2100, 2200, 96), (4000, 4096, 64)])
 def test_fp32_forms_agree(H, M, N, K):
     g = torch.Generator().manual_seed(M + K)
     x, w = torch.randn(M, K, generator=g).cuda(), (torch.randn(N, K, generator=g) / K ** 0.5).cuda()
