@@ -534,13 +534,18 @@ diffattn_merge_kernel(const float* __restrict__ ws, int nsplit, const float* __r
 // product's operand as it stands.  The keys are scanned in segments of 64 from key 0 (steps of 16, online softmax inside a segment), and a
 // segment's (max, sum, O) joins the row's total in order: the same steps for a prompt's row and for a decoded token, so a row's bits do not
 // depend on the schedule.  Steps and segments behind a row's position leave its values as they are.
-// tile mode:  workgroup = 4 waves of 16 rows; a wave's totals lie in LDS (registers hold the segment's O and the step's K and V).
-// split mode: 8 waves share the <= 16 rows and take the segments in turn; after a round, wave w adds value tile w of the segments in order.
-// Bound by the chain of a segment's steps (a memory round trip and 96 MFMAs each).  MI355X, 16 heads in 4 groups, dim 64, vdim 128: a portion
-// of 512 rows up to key 1000 3070 -> 198 us, single tokens of three sequences at up to 1000 keys 131 -> 49 us (before: the scalar form
-// above, a workgroup per token and head whose lanes each read a whole K row).
+// A workgroup owns 16 rows; its NW waves take the segments in turn, and after a round of NW the waves add the round's parts in order, each its
+// share of the value tiles.  A step's K comes while the step before computes, its V while its own scores are.
+//   prompt portions: four waves, two workgroups to a CU: bound by the fp32 matrix cores (96 MFMAs of 32 cycles per step) and a chip that
+//   a few hundred rows do not fill evenly.  (Four waves of 16 rows each, every wave the whole scan, left the chip half empty.)
+//   decoding (at most 16 rows per sequence): eight waves; with more than one round of segments and a workspace, one launch leaves the parts
+//   of the first `slots` segments of every sequence there, segments over the grid, and a second one adds them and scans what is left.
+// MI355X, 16 heads in 4 groups, dim 64, vdim 128, against four waves of 16 rows each with every scan its own: a
+// portion of 512 rows up to key 1000 201 -> 92 us, single tokens of three sequences at up to 1000 keys 50 -> 18 + 9 us
+// (the scalar form above, a workgroup per token and head whose lanes each read a whole K row: 3070 and 131 us).
 // ---------------------------------------------------------------------------------------------------------------------
-constexpr int DF_KS = 4, DF_SEG = 64, DF_SPLIT_WAVES = 8;
+constexpr int DF_KS = 4, DF_SEG = 64, DF_PROMPT_WAVES = 4, DF_DECODE_WAVES = 8;
+enum { DF_ALL = 0, DF_PARTS = 1, DF_REST = 2 };            // every segment; parts of the first segments to the workspace; those parts and the rest
 
 struct DiffPart { float mx[2], ls[2]; f32x4_t acc[2][DM_DVT]; };
 
@@ -556,10 +561,31 @@ __device__ __forceinline__ void diff_factors(float (&M)[2], float (&L)[2], const
   }
 }
 
-// keys [k_begin, k_end) of one segment for the 16 rows of a wave (k_end past a row's position, or past the cache, is masked)
-__device__ __forceinline__ void diff_segment(DiffPart& p, const u32x4_t (&qreg)[2][DF_KS], const float* __restrict__ kc, const float* __restrict__ vt,
-                                             const int32_t* __restrict__ table, int G, int g, int D, int Dv, int bs, int r, int qd, int k_begin,
-                                             int k_end, int pos, int ctx, float scale) {
+struct DiffKeys {                      // where 16 keys lie, and their K rows as they come
+  size_t pg;
+  int koff;
+  u32x4_t k[2][DF_KS];
+};
+
+__device__ __forceinline__ void diff_keys(DiffKeys& t, const float* __restrict__ kc, const int32_t* __restrict__ table, int G, int g, int D, int bs,
+                                          int r, int qd, int k0) {
+  const int KS = D >> 4;
+  t.pg = (size_t)table[k0 / bs] * G + g;
+  t.koff = k0 % bs;
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int ks = 0; ks < DF_KS; ++ks) {
+      t.k[m][ks] = u32x4_t{0u, 0u, 0u, 0u};
+      if (ks < KS) t.k[m][ks] = *reinterpret_cast<const u32x4_t*>(kc + (t.pg * bs + t.koff + r) * 2 * D + m * D + ks * 16 + qd * 4);
+    }
+}
+
+// keys [k_begin, k_end) of one segment for 16 rows (k_end past a row's position, or past the cache, is masked).  `t` holds the first keys, and
+// those at k_next (if not negative) when the segment is done.
+__device__ __forceinline__ void diff_segment(DiffPart& p, DiffKeys& t, const u32x4_t (&qreg)[2][DF_KS], const float* __restrict__ kc,
+                                             const float* __restrict__ vt, const int32_t* __restrict__ table, int G, int g, int D, int Dv, int bs,
+                                             int r, int qd, int k_begin, int k_end, int k_next, int pos, int ctx, float scale) {
   const int KS = D >> 4, DVT = Dv >> 4;
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
@@ -569,21 +595,15 @@ __device__ __forceinline__ void diff_segment(DiffPart& p, const u32x4_t (&qreg)[
     for (int i = 0; i < DM_DVT; ++i) p.acc[m][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   for (int k0 = k_begin; k0 < k_end; k0 += 16) {
-    const size_t pg = (size_t)table[k0 / bs] * G + g;
-    const int koff = k0 % bs;
-    u32x4_t kreg[2][DF_KS], v[DM_DVT];
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-      for (int ks = 0; ks < DF_KS; ++ks) {
-        kreg[m][ks] = u32x4_t{0u, 0u, 0u, 0u};
-        if (ks < KS) kreg[m][ks] = *reinterpret_cast<const u32x4_t*>(kc + (pg * bs + koff + r) * 2 * D + m * D + ks * 16 + qd * 4);
-      }
+    u32x4_t v[DM_DVT];
 #pragma unroll
     for (int i = 0; i < DM_DVT; ++i) {
       v[i] = u32x4_t{0u, 0u, 0u, 0u};
-      if (i < DVT) v[i] = *reinterpret_cast<const u32x4_t*>(vt + (pg * Dv + i * 16 + r) * bs + koff + qd * 4);
+      if (i < DVT) v[i] = *reinterpret_cast<const u32x4_t*>(vt + (t.pg * Dv + i * 16 + r) * bs + t.koff + qd * 4);
     }
+    DiffKeys next = t;
+    const int kn = k0 + 16 < k_end ? k0 + 16 : k_next;
+    if (kn >= 0) diff_keys(next, kc, table, G, g, D, bs, r, qd, kn);
     f32x4_t s[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int ks = 0; ks < DF_KS; ++ks)
@@ -591,8 +611,9 @@ __device__ __forceinline__ void diff_segment(DiffPart& p, const u32x4_t (&qreg)[
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int m = 0; m < 2; ++m) s[m] = mfma_f32(kreg[m][ks][e], qreg[m][ks][e], s[m]);
+          for (int m = 0; m < 2; ++m) s[m] = mfma_f32(t.k[m][ks][e], qreg[m][ks][e], s[m]);
       }
+    t = next;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       float top = -INFINITY;
@@ -629,35 +650,31 @@ __device__ __forceinline__ void diff_segment(DiffPart& p, const u32x4_t (&qreg)[
   }
 }
 
-template <bool SPLIT>
-__global__ void __launch_bounds__(SPLIT ? 64 * DF_SPLIT_WAVES : 256, 2)
+// slots, ws (DF_PARTS, DF_REST): one slot of DM_WS_SLOT floats per (workgroup's rows, kv head, segment below `slots`): [map][max, sum][16 rows], then
+// [map][tile][lane][4]; workgroup z of DF_PARTS writes the slots z * NW .. + NW - 1.
+template <int NW, int MODE>
+__global__ void __launch_bounds__(64 * NW, 2)
 diffattn_f32_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vt, const float* __restrict__ gate,
                     const int32_t* __restrict__ bt, int max_blocks, const int64_t* __restrict__ positions,
                     const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ cu_q, int q_per_seq, int B, int H, int G, int D, int Dv,
-                    int bs, float scale, float lambda, float out_scale, float eps, float* __restrict__ out) {
-  // tile mode: [wave][map][tile][lane] totals; split mode: [wave][map][tile][lane] of a round's segments, then their (max, sum)
+                    int bs, float scale, float lambda, float out_scale, float eps, float* __restrict__ out, int slots, float* __restrict__ ws) {
+  // [wave][map][tile][lane] of a round's segments, [wave][map][max, sum][16 rows]
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
-  const int g = blockIdx.y, R = H / G, DVT = Dv >> 4, KS = D >> 4;
-  int b = 0, tile = blockIdx.x, tok0 = 0, qb = 0;
-  if (SPLIT) {
-    b = blockIdx.x;
-    tile = 0;
+  constexpr int TPW = (DM_DVT + NW - 1) / NW;                          // value tiles of a wave: wave, wave + NW, ...
+  const int lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = blockIdx.y, R = H / G, DVT = Dv >> 4;
+  // (the last tiles, whose scans are the longest, start first)
+  int b = 0, tile = (int)(gridDim.x - 1 - blockIdx.x), tok0 = 0, qb = 0;
+  for (; b < B; ++b) {
     tok0 = cu_q ? cu_q[b] : b * q_per_seq;
     qb = cu_q ? cu_q[b + 1] - cu_q[b] : q_per_seq;
-    if (qb <= 0) return;
-  } else {
-    for (; b < B; ++b) {
-      tok0 = cu_q ? cu_q[b] : b * q_per_seq;
-      qb = cu_q ? cu_q[b + 1] - cu_q[b] : q_per_seq;
-      const int nt = (qb * R + 63) >> 6;
-      if (tile < nt) break;
-      tile -= nt;
-    }
-    if (b >= B) return;
+    const int nt = (qb * R + 15) >> 4;
+    if (tile < nt) break;
+    tile -= nt;
   }
-  const int nrows = qb * R, row0 = SPLIT ? 0 : tile * 64 + wave * 16;
-  if (!SPLIT && row0 >= nrows) return;                 // (tile mode has no workgroup barriers)
+  if (b >= B) return;
+  const int nrows = qb * R, row0 = tile * 16;
   const bool valid = row0 + r < nrows;
   const int rr = valid ? row0 + r : row0;
   const int token = tok0 + rr / R, head = g * R + rr % R;
@@ -665,75 +682,117 @@ diffattn_f32_kernel(const float* __restrict__ q, const float* __restrict__ kc, c
   int maxpos = pos;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) maxpos = max(maxpos, __shfl_xor(maxpos, o, 64));
+  maxpos = __builtin_amdgcn_readfirstlane(maxpos);
+  const int keys = maxpos + 1, nseg = (keys + DF_SEG - 1) / DF_SEG;
   const int32_t* table = bt + (size_t)b * max_blocks;
+  float* slot = ws + ((size_t)(gridDim.x - 1 - blockIdx.x) * G + g) * slots * DM_WS_SLOT;
+  const int first = MODE == DF_PARTS ? (int)blockIdx.z * NW : MODE == DF_REST ? slots : 0;       // of the segments scanned here
+  const int last = MODE == DF_PARTS ? min(nseg, slots) : nseg;
+  if (MODE == DF_PARTS && first >= last) return;
+
   u32x4_t qreg[2][DF_KS];
 #pragma unroll
   for (int m = 0; m < 2; ++m)
 #pragma unroll
     for (int ks = 0; ks < DF_KS; ++ks) {
       qreg[m][ks] = u32x4_t{0u, 0u, 0u, 0u};
-      if (ks < KS && valid) qreg[m][ks] = *reinterpret_cast<const u32x4_t*>(q + ((size_t)token * H + head) * 2 * D + m * D + ks * 16 + qd * 4);
+      if (ks < D >> 4 && valid) qreg[m][ks] = *reinterpret_cast<const u32x4_t*>(q + ((size_t)token * H + head) * 2 * D + m * D + ks * 16 + qd * 4);
     }
-  const int keys = maxpos + 1, nseg = (keys + DF_SEG - 1) / DF_SEG;
-  float M[2] = {-INFINITY, -INFINITY}, L[2] = {0.f, 0.f};
-  f32x4_t* mine = reinterpret_cast<f32x4_t*>(smem) + (size_t)wave * 2 * DVT * 64 + lane;
+  DiffKeys t;
+  t.pg = 0;
+  t.koff = 0;
+  if (first + wave < last) diff_keys(t, kc, table, G, g, D, bs, r, qd, (first + wave) * DF_SEG);
   DiffPart p;
-  if constexpr (!SPLIT) {
+  if constexpr (MODE == DF_PARTS) {
+    const int sg = first + wave;
+    if (sg >= last) return;
+    diff_segment(p, t, qreg, kc, vt, table, G, g, D, Dv, bs, r, qd, sg * DF_SEG, min(keys, (sg + 1) * DF_SEG), -1, pos, ctx, scale);
+    float* o = slot + (size_t)sg * DM_WS_SLOT;
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+    for (int m = 0; m < 2; ++m) {
+      if (qd == 0) { o[(m * 2 + 0) * 16 + r] = p.mx[m]; o[(m * 2 + 1) * 16 + r] = p.ls[m]; }
 #pragma unroll
       for (int i = 0; i < DM_DVT; ++i)
-        if (i < DVT) mine[(m * DVT + i) * 64] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int sg = 0; sg < nseg; ++sg) {
-      diff_segment(p, qreg, kc, vt, table, G, g, D, Dv, bs, r, qd, sg * DF_SEG, min(keys, (sg + 1) * DF_SEG), pos, ctx, scale);
+        if (i < DVT) *reinterpret_cast<f32x4_t*>(o + 64 + ((m * DM_DVT + i) * 64 + lane) * 4) = p.acc[m][i];
+    }
+    return;
+  }
+
+  float M[2] = {-INFINITY, -INFINITY}, L[2] = {0.f, 0.f};
+  f32x4_t total[2][TPW];                               // value tiles wave + NW * i
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) total[m][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if constexpr (MODE == DF_REST) {
+    static_assert(TPW == 1, "a value tile per wave");
+    constexpr int U = 8;                               // parts on their way together
+    const int n = min(nseg, slots), at = min(wave, DVT - 1);
+    for (int v0 = 0; v0 < n; v0 += U) {
+      float mx[U][2], ls[U][2];
+      f32x4_t part[U][2];
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const float* o = slot + (size_t)min(v0 + j, n - 1) * DM_WS_SLOT;
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          mx[j][m] = o[m * 32 + r];
+          ls[j][m] = o[m * 32 + 16 + r];
+          part[j][m] = *reinterpret_cast<const f32x4_t*>(o + 64 + ((m * DM_DVT + at) * 64 + lane) * 4);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        if (v0 + j >= n) break;
+        float fo[2], fn[2];
+        diff_factors(M, L, mx[j], ls[j], fo, fn);
+#pragma unroll
+        for (int m = 0; m < 2; ++m) total[m][0] = total[m][0] * fo[m] + part[j][m] * fn[m];
+      }
+    }
+  }
+  f32x4_t* mine = reinterpret_cast<f32x4_t*>(smem) + (size_t)wave * 2 * DVT * 64 + lane;
+  const f32x4_t* all = reinterpret_cast<const f32x4_t*>(smem) + lane;
+  float* sml = smem + (size_t)NW * 2 * DVT * 256;
+  for (int s0 = first; s0 < nseg; s0 += NW) {
+    const int sg = s0 + wave;
+    if (sg < nseg) {
+      diff_segment(p, t, qreg, kc, vt, table, G, g, D, Dv, bs, r, qd, sg * DF_SEG, min(keys, (sg + 1) * DF_SEG),
+                   sg + NW < nseg ? (sg + NW) * DF_SEG : -1, pos, ctx, scale);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+#pragma unroll
+        for (int i = 0; i < DM_DVT; ++i)
+          if (i < DVT) mine[(m * DVT + i) * 64] = p.acc[m][i];
+        if (qd == 0) { sml[((wave * 2 + m) * 2 + 0) * 16 + r] = p.mx[m]; sml[((wave * 2 + m) * 2 + 1) * 16 + r] = p.ls[m]; }
+      }
+    }
+    // (barriers that do not wait for the keys on their way)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    for (int v = 0; v < NW && s0 + v < nseg; ++v) {
       float fo[2], fn[2];
-      diff_factors(M, L, p.mx, p.ls, fo, fn);
+      const float mx[2] = {sml[((v * 2 + 0) * 2 + 0) * 16 + r], sml[((v * 2 + 1) * 2 + 0) * 16 + r]};
+      const float ls[2] = {sml[((v * 2 + 0) * 2 + 1) * 16 + r], sml[((v * 2 + 1) * 2 + 1) * 16 + r]};
+      diff_factors(M, L, mx, ls, fo, fn);
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int i = 0; i < DM_DVT; ++i)
-          if (i < DVT) mine[(m * DVT + i) * 64] = mine[(m * DVT + i) * 64] * fo[m] + p.acc[m][i] * fn[m];
+        for (int i = 0; i < TPW; ++i)
+          if (wave + i * NW < DVT) total[m][i] = total[m][i] * fo[m] + all[((v * 2 + m) * DVT + wave + i * NW) * 64] * fn[m];
     }
-  } else {
-    float* sml = smem + (size_t)DF_SPLIT_WAVES * 2 * DVT * 256;         // [wave][map][max, sum][16 rows]
-    const f32x4_t* all = reinterpret_cast<const f32x4_t*>(smem) + lane;
-    f32x4_t total[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};       // value tile `wave`
-    for (int s0 = 0; s0 < nseg; s0 += DF_SPLIT_WAVES) {
-      const int sg = s0 + wave;
-      if (sg < nseg) {
-        diff_segment(p, qreg, kc, vt, table, G, g, D, Dv, bs, r, qd, sg * DF_SEG, min(keys, (sg + 1) * DF_SEG), pos, ctx, scale);
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-#pragma unroll
-          for (int i = 0; i < DM_DVT; ++i)
-            if (i < DVT) mine[(m * DVT + i) * 64] = p.acc[m][i];
-          if (qd == 0) { sml[((wave * 2 + m) * 2 + 0) * 16 + r] = p.mx[m]; sml[((wave * 2 + m) * 2 + 1) * 16 + r] = p.ls[m]; }
-        }
-      }
-      __syncthreads();
-      for (int v = 0; v < DF_SPLIT_WAVES && s0 + v < nseg; ++v) {
-        float fo[2], fn[2];
-        const float mx[2] = {sml[((v * 2 + 0) * 2 + 0) * 16 + r], sml[((v * 2 + 1) * 2 + 0) * 16 + r]};
-        const float ls[2] = {sml[((v * 2 + 0) * 2 + 1) * 16 + r], sml[((v * 2 + 1) * 2 + 1) * 16 + r]};
-        diff_factors(M, L, mx, ls, fo, fn);
-        if (wave < DVT) {
-#pragma unroll
-          for (int m = 0; m < 2; ++m) total[m] = total[m] * fo[m] + all[((v * 2 + m) * DVT + wave) * 64] * fn[m];
-        }
-      }
-      __syncthreads();
-    }
-    if (wave < DVT) {
-#pragma unroll
-      for (int m = 0; m < 2; ++m) reinterpret_cast<f32x4_t*>(smem)[(m * DVT + wave) * 64 + lane] = total[m];
-    }
-    __syncthreads();
-    if (wave != 0) return;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
 #pragma unroll
   for (int m = 0; m < 2; ++m)
 #pragma unroll
-    for (int i = 0; i < DM_DVT; ++i) p.acc[m][i] = i < DVT ? mine[(m * DVT + i) * 64] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < TPW; ++i)
+      if (wave + i * NW < DVT) reinterpret_cast<f32x4_t*>(smem)[(m * DVT + wave + i * NW) * 64 + lane] = total[m][i];
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int i = 0; i < DM_DVT; ++i) p.acc[m][i] = i < DVT ? all[(m * DVT + i) * 64] : f32x4_t{0.f, 0.f, 0.f, 0.f};
   diff_finalize<float>(p.acc, L, DVT, Dv, lambda, out_scale, gate[(size_t)token * H + head], eps, valid,
                        out + ((size_t)token * H + head) * Dv + qd * 4);
 }
@@ -800,20 +859,33 @@ extern "C" int ssd_diffattn_paged(const void* q_rows, const void* k_cache, const
   if (f32 && context_lens && max_q > 0 && D % 16 == 0 && D <= 16 * DF_KS && Dv % 16 == 0 && Dv <= 16 * DM_DVT && block_size % 16 == 0 &&
       (((uintptr_t)q_rows | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out_rows) & 15) == 0) {
     const int R = H / G;
-    const size_t per_wave = (size_t)2 * (Dv / 16) * 64 * 16;
-#define DF_ARGS (const float*)q_rows, (const float*)k_cache, (const float*)v_cache, (const float*)gate, block_tables, max_blocks, positions,  \
-                context_lens, cu_q, q_per_seq, B, H, G, D, Dv, block_size, scale, lambda, out_scale, eps, (float*)out_rows
-    if (max_q * R <= 16) {
-      const size_t lds = DF_SPLIT_WAVES * (per_wave + 2 * 2 * 16 * 4);
-      if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)diffattn_f32_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
-                                 hipSuccess)
-        return SSD_ERR_LAUNCH;
-      hipLaunchKernelGGL(diffattn_f32_kernel<true>, dim3(B, G), dim3(64 * DF_SPLIT_WAVES), lds, (hipStream_t)stream, DF_ARGS);
-    } else {
-      hipLaunchKernelGGL(diffattn_f32_kernel<false>, dim3((unsigned)(((long)T * R + 63) / 64 + B), G), dim3(256), 4 * per_wave,
-                         (hipStream_t)stream, DF_ARGS);
+    const unsigned tiles = max_q * R <= 16 ? (unsigned)B : (unsigned)(((long)T * R + 15) / 16 + B);
+    const size_t per_wave = (size_t)2 * (Dv / 16) * 64 * 16 + 2 * 2 * 16 * 4;
+#define DF_GO(NW, MODE, Z, LDS)                                                                                                            \
+  {                                                                                                                                        \
+    if ((LDS) > 64 * 1024 && hipFuncSetAttribute((const void*)diffattn_f32_kernel<NW, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,  \
+                                                 (int)(LDS)) != hipSuccess)                                                                \
+      return SSD_ERR_LAUNCH;                                                                                                               \
+    hipLaunchKernelGGL((diffattn_f32_kernel<NW, MODE>), dim3(tiles, G, Z), dim3(64 * NW), LDS, (hipStream_t)stream, (const float*)q_rows,     \
+                       (const float*)k_cache, (const float*)v_cache, (const float*)gate, block_tables, max_blocks, positions, context_lens,   \
+                       cu_q, q_per_seq, B, H, G, D, Dv, block_size, scale, lambda, out_scale, eps, (float*)out_rows, slots, (float*)workspace); \
+  }
+    // decoding of contexts of more than one round of segments: the parts of as many as the hint promises and the workspace holds over the grid
+    int slots = 0;
+    if (max_q * R <= 16 && workspace && (uintptr_t)workspace % 16 == 0 && ctx_hint > DF_SEG * DF_DECODE_WAVES) {
+      const long held = workspace_bytes / ((long)B * G * DM_WS_SLOT * 4), want = (ctx_hint + DF_SEG - 1) / DF_SEG;
+      slots = (int)(held < want ? held : want);
+      if (slots <= DF_DECODE_WAVES || slots > 65535) slots = 0;
     }
-#undef DF_ARGS
+    if (slots) {
+      DF_GO(DF_PROMPT_WAVES, DF_PARTS, (slots + DF_PROMPT_WAVES - 1) / DF_PROMPT_WAVES, 0)
+      DF_GO(DF_DECODE_WAVES, DF_REST, 1, DF_DECODE_WAVES * per_wave)
+    } else if (max_q * R <= 16) {
+      DF_GO(DF_DECODE_WAVES, DF_ALL, 1, DF_DECODE_WAVES * per_wave)
+    } else {
+      DF_GO(DF_PROMPT_WAVES, DF_ALL, 1, DF_PROMPT_WAVES * per_wave)
+    }
+#undef DF_GO
     return LAUNCH_OK();
   }
   const size_t lds = (size_t)(2 * D + 4 * 2 * 64) * 4 + 4 * 64 * 8 + (size_t)(4 * 2 * Dv + 16 + 4) * 4 + 8;

@@ -1,6 +1,6 @@
 """The matrix-core form of the fp32 differential attention (csrc/attention_diff.hip): the last rows of sequences whose lengths lie at the edges of
-steps (16 keys), segments (64) and rounds (512), against fp64 -- and the same bits whether a row comes alone, in a small batch, or inside
-a prompt portion."""
+steps (16 keys), segments (64) and rounds (512), against fp64 -- and the same bits whether a row comes alone, in a small batch, inside
+a prompt portion, or with its segments over the grid."""
 import pytest
 import torch
 
@@ -49,12 +49,14 @@ def test_rows_alone_and_in_portions(Hh, G, D, Dv, bs):
         q, gate = rnd(rows, Hh, 2, D), torch.sigmoid(rnd(rows, Hh))
         ctx = torch.tensor([n], dtype=torch.int32).cuda()
 
-        def attend(a, b):
+        def attend(a, b, slots=0, hint=0):
             T = b - a
             out = torch.zeros(T, Hh * Dv, device="cuda")
+            ws = torch.full((G * slots * 4160,), float("nan"), device="cuda") if slots else None
             pos = torch.arange(n - rows + a, n - rows + b).cuda()
             H.diffattn_paged(q[a:b].contiguous(), kc, vc, gate[a:b].contiguous(), bt, len(pages), pos, 1, T, Hh, G, D, Dv, bs, scale, lam, osc,
-                             eps, out, True, cu_q=torch.tensor([0, T], dtype=torch.int32).cuda(), context_lens=ctx, max_q=T)
+                             eps, out, True, cu_q=torch.tensor([0, T], dtype=torch.int32).cuda(), context_lens=ctx, max_q=T,
+                             workspace=ws, ctx_hint=hint)
             return out
 
         whole = attend(0, rows)
@@ -64,3 +66,6 @@ def test_rows_alone_and_in_portions(Hh, G, D, Dv, bs):
         for i in {0, rows // 2, rows - 1}:
             assert torch.equal(attend(i, i + 1), whole[i:i + 1]), (n, i)
         assert torch.equal(attend(max(0, rows - 3), rows), whole[max(0, rows - 3):]), n
+        # segments over the grid: room for all of them, for the first nine, a hint that falls short of the context
+        for slots, hint in ((18, 1152), (9, 1152), (18, 640)):
+            assert torch.equal(attend(rows - 1, rows, slots, hint), whole[rows - 1:]), (n, slots, hint)
