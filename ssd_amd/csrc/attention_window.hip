@@ -11,7 +11,7 @@
 //                         the window's first key (so a row's summation order is a function of its own position only); a lane owns a
 //                         KEY for the scores and a VALUE COLUMN for the sums; partial (max, sum, accumulator) triples merge in LDS in
 //                         wave order, then the sink joins the denominator.
-//                         MFMA form (bf16, D % 32 == 0, D <= 256, Dv % 16 == 0, Dv <= 256, block_size % 32 == 0; the caller gives
+//                         MFMA forms (bf16, D % 32 == 0, D <= 256, Dv % 16 == 0, Dv <= 256, block_size % 32 == 0; the caller gives
 //                         max_q, an upper bound of the rows a sequence brings): see below.
 //   * ssd_winattn_store_rope  the store of a rotary variant: RMS norm with weights over the WHOLE q and the whole k projection (before
 //                         the heads are split), rotary positions on the first rot_dims entries of every q / k head, and (v_freqs given)
@@ -343,6 +343,73 @@ winattn_paged_kernel(const T* __restrict__ q, const T* __restrict__ kc, const T*
   }
 }
 
+// The end of a row (lane: row r, columns i * 16 + qd * 4 + e of its sum): the sink joins the denominator, the output turns, the gate.
+template <int MV>
+__device__ __forceinline__ void win_finish(f32x4_t (&acc)[MV], float mx, float ls, int DVT, int Dv, float sink, int pos, int qd,
+                                           const float* __restrict__ out_freqs, const float* __restrict__ gate, float out_scale,
+                                           bf16_t* __restrict__ out) {
+  const float M = fmaxf(mx, sink);
+  const float fo = ls > 0.f ? __expf(mx - M) : 0.f;
+  const float den = ls * fo + (sink == -INFINITY ? 0.f : __expf(sink - M));
+  const float rs = fo / den;
+#pragma unroll
+  for (int i = 0; i < MV; ++i)
+    if (i < DVT) acc[i] *= rs;
+  if (out_freqs) {
+    // the head's output turns back by the query's position; Dv % 32 == 0 here, so the partner of column i * 16 + qd * 4 + e (the
+    // column Dv / 2 further) is element e of tile i + DVT / 2 of the SAME lane
+    const int HT = DVT >> 1;
+    if (DVT == MV) {
+#pragma unroll
+      for (int i = 0; i < MV / 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float sn, c;
+          sincosf((float)pos * out_freqs[i * 16 + qd * 4 + e], &sn, &c);
+          const float a = acc[i][e], b = acc[i + MV / 2][e];
+          acc[i][e] = a * c + b * sn;
+          acc[i + MV / 2][e] = b * c - a * sn;
+        }
+    } else {          // fewer value tiles than the register array holds: the partner tile's index is not a constant; select it
+#pragma unroll
+      for (int i = 0; i < MV / 2; ++i)
+        if (i < HT) {
+          f32x4_t pb = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = 0; k < MV; ++k) pb = (k == i + HT) ? acc[k] : pb;
+          f32x4_t na, nb;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float sn, c;
+            sincosf((float)pos * out_freqs[i * 16 + qd * 4 + e], &sn, &c);
+            na[e] = acc[i][e] * c + pb[e] * sn;
+            nb[e] = pb[e] * c - acc[i][e] * sn;
+          }
+          acc[i] = na;
+#pragma unroll
+          for (int k = 0; k < MV; ++k) acc[k] = (k == i + HT) ? nb : acc[k];
+        }
+    }
+  }
+  if (gate) {
+    const float* gr = gate + qd * 4;
+#pragma unroll
+    for (int i = 0; i < MV; ++i)
+      if (i < DVT)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] = acc[i][e] / (1.0f + __expf(-gr[i * 16 + e])) * out_scale;
+  }
+  bf16_t* orow = out + qd * 4;
+#pragma unroll
+  for (int i = 0; i < MV; ++i)
+    if (i < DVT) {
+      u32x2_t o2;
+      o2[0] = pack_bf2_hw(acc[i][0], acc[i][1]);
+      o2[1] = pack_bf2_hw(acc[i][2], acc[i][3]);
+      *reinterpret_cast<u32x2_t*>(orow + i * 16) = o2;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------------------
 // MFMA form (bf16, D % 32 == 0, D <= 256, Dv % 16 == 0, Dv <= 256, block_size % 32 == 0).  For one kv head, the query ROWS of a
 // sequence are its (token, head of the group) pairs, token-major; a wave owns 16 rows and walks the keys in steps of 32 that start
@@ -534,68 +601,222 @@ winattn_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
       return;
     }
   }
-  if (!valid) return;
-  const float sink = sinks ? sinks[head] : -INFINITY;
-  const float M = fmaxf(mx, sink);
-  const float fo = ls > 0.f ? __expf(mx - M) : 0.f;
-  const float den = ls * fo + (sinks ? __expf(sink - M) : 0.f);
-  const float rs = fo / den;
+  if (valid)
+    win_finish<MV>(acc, mx, ls, DVT, Dv, sinks ? sinks[head] : -INFINITY, pos, qd, out_freqs, gate ? gate + (size_t)token * ldg + head * Dv : nullptr,
+                   out_scale, out + (size_t)token * ldo + head * Dv);
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// Prompt form (more than 256 rows a sequence and kv head; D = 64 or 128, Dv <= 128): the same products, for throughput: a workgroup = 4 waves of 32 (or
+// 16) rows shares every 64-key tile of K and V through LDS, filled by DMA one tile ahead, one barrier per tile; a row keeps its reference maximum until
+// some score exceeds it by 2^8 (exact: sum and denominator both carry it); only tiles at a row's first or last key are masked.  A key's 16-byte
+// chunks of K are rotated by its index, a value column's chunks of 8 keys by the column, so that operand reads hit different banks.
+// Bound by the exponentials and conversions between the two products.  (The form above reads every K and V tile once per 16 rows from L2.)
+// MI355X, 32 heads of 128 in 8 groups, the form above -> this: prompts of 1800, 1500, 600 and 328 tokens 610 -> 201 us, behind a window of 512
+// 340 -> 101, 500 tokens 52 -> 43, 16384 tokens 23.1 -> 4.9 ms; 32 heads of 64 in 8, 2000 tokens 316 -> 116 us.
+// ---------------------------------------------------------------------------------------------------------------------
+constexpr int WP_KEYS = 64;
+
+template <int MK, int MV, int RT>            // D = 32 MK, Dv <= 16 MV; a wave owns 16 RT rows
+__global__ void __launch_bounds__(256, 2)
+winattn_prompt_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vt,
+                      const float* __restrict__ slopes, const float* __restrict__ sinks, const int32_t* __restrict__ bt, int max_blocks,
+                      const int64_t* __restrict__ positions, const int32_t* __restrict__ cu_q, int q_per_seq, int H, int G, int Dv,
+                      int bs, int window, int keep_first, float scale, float cap, const float* __restrict__ out_freqs,
+                      const float* __restrict__ gate, long ldg, float out_scale, bf16_t* __restrict__ out, long ldo) {
+  constexpr int D = MK * 32, CH = D / 8, KPI = 64 / CH, ROWS = 64 * RT, KB = WP_KEYS * D * 2;       // chunks of a key, keys per DMA
+  constexpr float LOG2E = 1.4426950408889634f;
+  extern __shared__ __attribute__((aligned(1024))) char wsm[];                 // [buffer][K, V]
+  const int TILE = KB + Dv * WP_KEYS * 2;
+  const int lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.z, g = blockIdx.y, R = H / G, DVT = Dv >> 4;
+  const int tok0 = cu_q ? cu_q[b] : b * q_per_seq;
+  const int nrows = (cu_q ? cu_q[b + 1] - tok0 : q_per_seq) * R;
+  const int row_wg = (int)(gridDim.x - 1 - blockIdx.x) * ROWS;                 // the longest scans start first
+  if (row_wg >= nrows) return;
+  const int32_t* table = bt + (size_t)b * max_blocks;
+  auto first_key = [&](int pos) { return window > 0 && pos + 1 > window ? pos + 1 - window : 0; };
+
+  // ---- keys of the workgroup, and of this wave's rows ----
+  int kmin = 0x7fffffff, kmax = -1;
 #pragma unroll
-  for (int i = 0; i < MV; ++i)
-    if (i < DVT) acc[i] *= rs;
-  if (out_freqs) {
-    // the head's output turns back by the query's position; Dv % 32 == 0 here, so the partner of column i * 16 + qd * 4 + e (the
-    // column Dv / 2 further) is element e of tile i + DVT / 2 of the SAME lane
-    const int HT = DVT >> 1;
-    if (DVT == MV) {
+  for (int i = 0; i < RT; ++i) {
+    const int row = row_wg + i * 64 + lane, pos = row < nrows ? (int)positions[tok0 + row / R] : -1;
+    kmax = max(kmax, pos);
+    kmin = min(kmin, row < nrows ? first_key(pos) : 0x7fffffff);
+  }
+  u32x4_t qf[RT][MK];
+  int pos[RT], first[RT], wmax = -1, wmin = 0x7fffffff, wfirst = 0, wlast = 0x7fffffff;       // (wfirst, wlast: keys that every row of the wave sees)
+  float slope[RT];
 #pragma unroll
-      for (int i = 0; i < MV / 2; ++i)
+  for (int t = 0; t < RT; ++t) {
+    const int row = row_wg + (wave * RT + t) * 16 + r, rr = min(row, nrows - 1), token = tok0 + rr / R, head = g * R + rr % R;
+    pos[t] = row < nrows ? (int)positions[token] : -1;
+    first[t] = row < nrows ? first_key(pos[t]) : 0x7fffffff;
+    slope[t] = slopes ? slopes[head] * LOG2E : 0.f;
+    wmax = max(wmax, pos[t]);
+    wmin = min(wmin, first[t]);
+    wfirst = max(wfirst, first[t]);
+    wlast = min(wlast, pos[t]);
+#pragma unroll
+    for (int ks = 0; ks < MK; ++ks) qf[t][ks] = *reinterpret_cast<const u32x4_t*>(q + ((size_t)token * H + head) * D + ks * 32 + qd * 8);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    kmax = max(kmax, __shfl_xor(kmax, o, 64));
+    kmin = min(kmin, __shfl_xor(kmin, o, 64));
+    wmax = max(wmax, __shfl_xor(wmax, o, 64));
+    wmin = min(wmin, __shfl_xor(wmin, o, 64));
+    wfirst = max(wfirst, __shfl_xor(wfirst, o, 64));
+    wlast = min(wlast, __shfl_xor(wlast, o, 64));
+  }
+  kmax = __builtin_amdgcn_readfirstlane(kmax); kmin = __builtin_amdgcn_readfirstlane(kmin);
+  wmax = __builtin_amdgcn_readfirstlane(wmax); wmin = __builtin_amdgcn_readfirstlane(wmin);
+  wfirst = __builtin_amdgcn_readfirstlane(wfirst); wlast = __builtin_amdgcn_readfirstlane(wlast);
+  // (Q arrives before the loop: a wait for it inside would be one for the DMA in flight as well)
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int ks = 0; ks < MK; ++ks) asm volatile("" : "+v"(qf[t][ks]));
+
+  const int s_first = kmin / WP_KEYS, s_last = kmax / WP_KEYS;
+  const int n_kept = min((keep_first + WP_KEYS - 1) / WP_KEYS, s_first);        // tiles of kept first tokens that lie before the window's
+  const int tiles = kmax < 0 ? 0 : n_kept + s_last - s_first + 1;
+  auto key_of = [&](int i) { return (i < n_kept ? i : s_first + i - n_kept) * WP_KEYS; };
+
+  // ---- DMA of a tile: its two halves of 32 keys lie in a page each.  A half that no row needs is not touched (its page may not exist any
+  //      more): the other half's data comes twice, and the second product passes over it ----
+  auto needed = [&](int k) { return k <= kmax && (k + 31 >= kmin || k < keep_first); };
+  auto fetch = [&](int i, int buf) {
+    const int k0 = key_of(i);
+    const int h0 = needed(k0) ? k0 : k0 + 32, h1 = needed(k0 + 32) ? k0 + 32 : h0;
+    const size_t p0 = (size_t)table[h0 / bs] * G + g, p1 = (size_t)table[h1 / bs] * G + g;
+    const int o0 = h0 % bs, o1 = h1 % bs;
+    char* kl = wsm + buf * TILE;
+#pragma unroll
+    for (int j = 0; j < CH / 4; ++j) {
+      const int c = wave * (CH / 4) + j, key = c * KPI + lane / CH, ch = (lane % CH) ^ (key & 7);
+      const size_t row = (key < 32 ? p0 : p1) * bs + (key < 32 ? o0 : o1) + (key & 31);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kc + row * D + ch * 8),
+                                       (__attribute__((address_space(3))) void*)(kl + c * 1024), 16, 0, 0);
+    }
+    for (int c = wave; c < Dv / 8; c += 4) {
+      const int col = c * 8 + (lane >> 3), ch = (lane & 7) ^ (col & 7);
+      const bf16_t* src = vt + ((ch < 4 ? p0 : p1) * Dv + col) * bs + (ch < 4 ? o0 : o1) + (ch & 3) * 8;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)(kl + KB + c * 1024), 16, 0, 0);
+    }
+  };
+
+  float m[RT], lsum[RT];                               // the row's reference maximum (log2 units) and sum
+  f32x4_t acc[RT][MV];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    m[t] = -INFINITY;
+    lsum[t] = 0.f;
+#pragma unroll
+    for (int i = 0; i < MV; ++i) acc[t][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  const float inv_cap = cap > 0.f ? 1.0f / cap : 0.f;
+  if (tiles > 0) fetch(0, 0);
+  for (int it = 0; it < tiles; ++it) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");       // the tile is in LDS; nobody reads the one before any more
+    if (it + 1 < tiles) fetch(it + 1, (it + 1) & 1);
+    const int k0 = key_of(it);
+    if (k0 > wmax || (k0 + WP_KEYS <= wmin && k0 >= keep_first)) continue;             // (a wave without rows here still meets the barriers)
+    const char* kl = wsm + (it & 1) * TILE;
+    const char* vl = kl + KB;
+    f32x4_t st[WP_KEYS / 16][RT];
+#pragma unroll
+    for (int kb = 0; kb < WP_KEYS / 16; ++kb) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t) st[kb][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < MK; ++ks) {
+        const u32x4_t a = *reinterpret_cast<const u32x4_t*>(kl + ((kb * 16 + r) * CH + ((ks * 4 + qd) ^ (r & 7))) * 16);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) st[kb][t] = mfma16(a, qf[t][ks], st[kb][t]);
+      }
+    }
+    const bool edge = k0 + WP_KEYS - 1 > wlast || k0 < wfirst;
+    u32x4_t pb[WP_KEYS / 32][RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      float top = -INFINITY;
+#pragma unroll
+      for (int kb = 0; kb < WP_KEYS / 16; ++kb)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          float sn, c;
-          sincosf((float)pos * out_freqs[i * 16 + qd * 4 + e], &sn, &c);
-          const float a = acc[i][e], b = acc[i + MV / 2][e];
-          acc[i][e] = a * c + b * sn;
-          acc[i + MV / 2][e] = b * c - a * sn;
+          float v = st[kb][t][e];
+          const int key = k0 + kb * 16 + qd * 4 + e;
+          if (cap > 0.f) v = cap * LOG2E * (1.0f - 2.0f / (1.0f + __expf(2.0f * (v * scale) * inv_cap)));
+          else v *= scale * LOG2E;
+          if (slopes) v -= slope[t] * (float)(pos[t] - key);
+          if (edge) v = key <= pos[t] && (key >= first[t] || key < keep_first) ? v : -INFINITY;
+          st[kb][t][e] = v;
+          top = fmaxf(top, v);
         }
-    } else {          // fewer value tiles than the register array holds: the partner tile's index is not a constant; select it
+      if (__any(top > m[t] + 8.0f)) {
+        top = fmaxf(top, __shfl_xor(top, 16, 64));
+        top = fmaxf(m[t], fmaxf(top, __shfl_xor(top, 32, 64)));
+        const float alpha = top == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[t] - top);
+        m[t] = top;
+        lsum[t] *= alpha;
 #pragma unroll
-      for (int i = 0; i < MV / 2; ++i)
-        if (i < HT) {
-          f32x4_t pb = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < MV; ++i) acc[t][i] *= alpha;
+      }
+      const float ref = m[t] == -INFINITY ? 0.f : m[t];       // (a row that has seen no key yet: all weights are zero)
+      float sum = 0.f;
 #pragma unroll
-          for (int k = 0; k < MV; ++k) pb = (k == i + HT) ? acc[k] : pb;
-          f32x4_t na, nb;
+      for (int kb = 0; kb < WP_KEYS / 16; ++kb) {
+        float w[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float sn, c;
-            sincosf((float)pos * out_freqs[i * 16 + qd * 4 + e], &sn, &c);
-            na[e] = acc[i][e] * c + pb[e] * sn;
-            nb[e] = pb[e] * c - acc[i][e] * sn;
-          }
-          acc[i] = na;
+        for (int e = 0; e < 4; ++e) {
+          w[e] = __builtin_amdgcn_exp2f(st[kb][t][e] - ref);
+          sum += w[e];
+        }
+        pb[kb / 2][t][(kb & 1) * 2] = pack_bf2_hw(w[0], w[1]);
+        pb[kb / 2][t][(kb & 1) * 2 + 1] = pack_bf2_hw(w[2], w[3]);
+      }
+      lsum[t] += sum;
+    }
 #pragma unroll
-          for (int k = 0; k < MV; ++k) acc[k] = (k == i + HT) ? nb : acc[k];
+    for (int c = 0; c < WP_KEYS / 32; ++c) {
+      if (!needed(k0 + c * 32)) continue;
+      // keys past the last row's position were never stored: whatever lies there must not meet a zero weight
+      const int ka = k0 + c * 32 + qd * 4;
+      const bool past = k0 + c * 32 + 31 > kmax;
+      const uint32_t l0 = (ka <= kmax ? 0xffffu : 0u) | (ka + 1 <= kmax ? 0xffff0000u : 0u);
+      const uint32_t l1 = (ka + 2 <= kmax ? 0xffffu : 0u) | (ka + 3 <= kmax ? 0xffff0000u : 0u);
+      const uint32_t u0 = (ka + 16 <= kmax ? 0xffffu : 0u) | (ka + 17 <= kmax ? 0xffff0000u : 0u);
+      const uint32_t u1 = (ka + 18 <= kmax ? 0xffffu : 0u) | (ka + 19 <= kmax ? 0xffff0000u : 0u);
+#pragma unroll
+      for (int i = 0; i < MV; ++i)
+        if (i < DVT) {
+          const char* row = vl + (i * 16 + r) * 128 + (qd & 1) * 8;
+          const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(row + (((c * 4 + (qd >> 1)) ^ (r & 7)) * 16));
+          const u32x2_t hi = *reinterpret_cast<const u32x2_t*>(row + (((c * 4 + 2 + (qd >> 1)) ^ (r & 7)) * 16));
+          u32x4_t va = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+          if (past) { va[0] &= l0; va[1] &= l1; va[2] &= u0; va[3] &= u1; }
+#pragma unroll
+          for (int t = 0; t < RT; ++t) acc[t][i] = mfma16(va, pb[c][t], acc[t][i]);
         }
     }
   }
-  if (gate) {
-    const float* gr = gate + (size_t)token * ldg + head * Dv + qd * 4;
-#pragma unroll
-    for (int i = 0; i < MV; ++i)
-      if (i < DVT)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][e] = acc[i][e] / (1.0f + __expf(-gr[i * 16 + e])) * out_scale;
-  }
-  bf16_t* orow = out + (size_t)token * ldo + head * Dv + qd * 4;
-#pragma unroll
-  for (int i = 0; i < MV; ++i)
-    if (i < DVT) {
-      u32x2_t o2;
-      o2[0] = pack_bf2_hw(acc[i][0], acc[i][1]);
-      o2[1] = pack_bf2_hw(acc[i][2], acc[i][3]);
-      *reinterpret_cast<u32x2_t*>(orow + i * 16) = o2;
+  auto finish = [&](f32x4_t (&o)[MV], float mx, float sum, int at, int t) {
+    float ls = sum + __shfl_xor(sum, 16, 64);
+    ls += __shfl_xor(ls, 32, 64);
+    const int row = row_wg + (wave * RT + t) * 16 + r;
+    if (row < nrows) {
+      const int token = tok0 + row / R, head = g * R + row % R;
+      win_finish<MV>(o, mx / LOG2E, ls, DVT, Dv, sinks ? sinks[head] : -INFINITY, at, qd, out_freqs,
+                     gate ? gate + (size_t)token * ldg + head * Dv : nullptr, out_scale, out + (size_t)token * ldo + head * Dv);
     }
+  };
+  static_assert(RT <= 2, "written out: a loop over t is too long to be unrolled, and would index the sums in memory");
+  finish(acc[0], m[0], lsum[0], pos[0], 0);
+  if constexpr (RT == 2) finish(acc[1], m[1], lsum[1], pos[1], 1);
 }
 
 // One wave per row of the decode launch: the slices' partial rows in slice order, the sink, the output's turn, the gate.
@@ -741,6 +962,32 @@ extern "C" int ssd_winattn_paged(const void* q_rows, const void* k_cache, const 
   if (!f32 && max_q > 0 && D % 32 == 0 && D <= 256 && Dv % (out_freqs ? 32 : 16) == 0 && Dv <= 256 && block_size % 32 == 0 && G <= 65535 &&
       B <= 65535 && ldo % 4 == 0 && (uintptr_t)out_rows % 8 == 0) {
     const int R = H / G;
+    // 32 workgroups of 128 rows: fewer leave so much of the chip idle that the smaller units of the form below win (700 rows in 4 kv heads of 128
+    // behind a window of 100: 26 | 20 us; 300 tokens of 16 heads in 4: 29 | 33).  Heads of 64: 64 rows a workgroup as long as those of 128
+    // do not fill the chip (900 and 60 tokens of 16 heads in 4: 42 | 61 us; four of 1800 behind a window of 128: 42 | 36).
+    const long units = ((long)max_q * R + 127) / 128 * G * B;
+    if ((long)max_q * R > 256 && units >= 32 && (((uintptr_t)q_rows | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0 &&
+        (D == 64 || D == 128) && Dv <= 128) {
+      const int rows = D == 64 && Dv <= 64 && units < 384 ? 64 : 128;
+      const dim3 pg((unsigned)(((long)max_q * R + rows - 1) / rows), G, B);
+      const size_t plds = 2 * (size_t)WP_KEYS * 2 * (D + Dv);
+#define WIN_PROMPT(MK, MV, RT)                                                                                                       \
+  {                                                                                                                                  \
+    if (plds > 64 * 1024 && hipFuncSetAttribute((const void*)winattn_prompt_kernel<MK, MV, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                                (int)plds) != hipSuccess)                                                             \
+      return SSD_ERR_LAUNCH;                                                                                                         \
+    hipLaunchKernelGGL((winattn_prompt_kernel<MK, MV, RT>), pg, dim3(256), plds, (hipStream_t)stream, (const bf16_t*)q_rows,          \
+                       (const bf16_t*)k_cache, (const bf16_t*)v_cache, slopes, sinks, block_tables, max_blocks, positions, cu_q,      \
+                       q_per_seq, H, G, Dv, block_size, window, keep_first, scale, cap, out_freqs, gate_rows, ldg, out_scale,          \
+                       (bf16_t*)out_rows, ldo);                                                                                       \
+    return LAUNCH_OK();                                                                                                              \
+  }
+      if (rows == 64) WIN_PROMPT(2, 4, 1)
+      if (D == 64 && Dv <= 64) WIN_PROMPT(2, 4, 2)
+      if (D == 64) WIN_PROMPT(2, 8, 2)
+      WIN_PROMPT(4, 8, 2)
+#undef WIN_PROMPT
+    }
     dim3 grid((unsigned)(((long)max_q * R + 63) / 64), G, B);
     int dtiles = 0, slices = 1;
     if (workspace && (long)max_q * R <= 64) {          // decode: cut the keys over the grid when the rows alone do not fill the chip

@@ -1,0 +1,95 @@
+"""Prompt form of the windowed attention (csrc/attention_window.hip) against fp64: ragged prompts behind cached keys around the tiles of 128 rows and
+64 keys, windows, kept first tokens, sinks, penalties, caps, gates and turned outputs, pages of 32 to 128 keys.  Unwritten slots hold NaN, and
+so do the pages that every row's window has left behind."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+
+CASES = [  # H, G, D, Dv, bs, window, keep, options
+    (8, 2, 128, 128, 64, 0, 0, ()),
+    (8, 2, 128, 128, 32, 100, 0, ("sink",)),
+    (4, 4, 64, 64, 128, 77, 40, ("sink", "slopes", "cap")),
+    (6, 2, 64, 96, 32, 130, 0, ("gate", "slopes")),
+    (8, 1, 128, 80, 64, 300, 33, ("gate", "cap")),
+    (4, 1, 128, 128, 32, 64, 0, ("freqs", "sink")),
+    (4, 2, 64, 64, 64, 1, 0, ()),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_against_fp64(case):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ssd_amd.hip import ops as K
+    H, G, D, Dv, bs, window, keep, opt = case
+    R = H // G
+    g = torch.Generator().manual_seed(D + Dv + bs + window)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    news, pasts = [128 // R + 1, 600, 65, 1], [0, 213, 700, 90]
+    nb = sum(-(-(n + c) // bs) for n, c in zip(news, pasts)) + 1
+    order = torch.randperm(nb, generator=g).tolist()
+    kc = torch.full((nb, G, bs, D), float("nan")).to(BF)
+    vc = torch.full((nb, G, Dv, bs), float("nan")).to(BF)
+    tables, Ks, Vs = [], [], []
+    for n, c in zip(news, pasts):
+        L = n + c
+        pages = [order.pop() for _ in range(-(-L // bs))]
+        Kd, Vd = rnd(L, G, D).to(BF), rnd(L, G, Dv).to(BF)
+        for j, p in enumerate(pages):
+            lo, hi = j * bs, min(L, (j + 1) * bs)
+            if window and hi <= c + 1 - window and lo >= keep:
+                continue                                   # no row sees any of its keys
+            kc[p, :, :hi - lo] = Kd[lo:hi].transpose(0, 1)
+            vc[p, :, :, :hi - lo] = Vd[lo:hi].permute(1, 2, 0)
+        tables.append(pages)
+        Ks.append(Kd)
+        Vs.append(Vd)
+    mb = max(map(len, tables)) + 1
+    bt = torch.tensor([t + [-1] * (mb - len(t)) for t in tables], dtype=torch.int32).cuda()
+    T = sum(news)
+    q = (rnd(T, H, D) * 1.5).to(BF)
+    slopes = torch.rand(H, generator=g) * 0.1 if "slopes" in opt else None
+    sinks = rnd(H) if "sink" in opt else None
+    gate = rnd(T, H * Dv + 4) if "gate" in opt else None
+    freqs = torch.rand(Dv // 2, generator=g) if "freqs" in opt else None
+    cap, scale, osc = (20.0 if "cap" in opt else 0.0), D ** -0.5, (1.5 if "gate" in opt else 1.0)
+    pos = torch.cat([torch.arange(c, c + n) for n, c in zip(news, pasts)])
+    cu = torch.tensor([0] + news).cumsum(0).to(torch.int32)
+    ldo = H * Dv + 8
+    out = torch.full((T, ldo), 7.0, dtype=BF, device="cuda")
+    dev = lambda t: None if t is None else t.cuda()
+    K.winattn_paged(q.cuda(), kc.cuda(), vc.cuda(), dev(slopes), dev(sinks), bt, mb, pos.cuda(), len(news), T, H, G, D, Dv, bs, window, scale, cap,
+                    out, False, cu_q=cu.cuda(), max_q=max(news), keep_first=keep, out_freqs=dev(freqs), gate=dev(gate), ldg=H * Dv + 4,
+                    out_scale=osc, ldo=ldo)
+    out = out.cpu()
+    assert bool((out[:, H * Dv:] == 7.0).all())
+    out = out[:, :H * Dv].double().view(T, H, Dv)
+    for b, (n, c) in enumerate(zip(news, pasts)):
+        Kd, Vd = Ks[b].double().repeat_interleave(R, 1), Vs[b].double().repeat_interleave(R, 1)
+        for i in {0, 1, n // 2, n - 1} & set(range(n)):
+            t, p = int(cu[b]) + i, c + i
+            s = torch.einsum("hd,khd->hk", q[t].double(), Kd[:p + 1]) * scale
+            if cap:
+                s = cap * torch.tanh(s / cap)
+            key = torch.arange(p + 1)
+            if slopes is not None:
+                s = s - slopes.double().unsqueeze(1) * (p - key)
+            if window:
+                s = s.masked_fill(~((key > p - window) | (key < keep)), float("-inf"))
+            z = torch.cat([s, sinks.double().unsqueeze(1)], 1) if sinks is not None else s
+            w = torch.softmax(z, 1)[:, :p + 1]
+            o, mag = torch.einsum("hk,khv->hv", w, Vd[:p + 1]), torch.einsum("hk,khv->hv", w, Vd[:p + 1].abs())
+            if freqs is not None:
+                a, hv = p * freqs.double(), Dv // 2
+                o = torch.cat([o[:, :hv] * a.cos() + o[:, hv:] * a.sin(), o[:, hv:] * a.cos() - o[:, :hv] * a.sin()], 1)
+                mag = (mag[:, :hv] + mag[:, hv:]).repeat(1, 2) + 2.0 ** -8       # (an angle of up to 800 in fp32: 800 * 2^-24 of the pair)
+            if gate is not None:
+                f = torch.sigmoid(gate[t, :H * Dv].double()).view(H, Dv) * osc
+                o, mag = o * f, mag * f
+            # the output's rounding; the weights' rounding to bf16 (2^-9 each) with 1e-4 for scores in fp32 and the hardware exponential
+            tol = 2.0 ** -8 * o.abs() + (2.0 ** -9 + 1e-4) * mag + 1e-5
+            d = (out[t] - o).abs() - tol
+            assert bool((d <= 0).all()), (case, b, i, float(d.max()))
