@@ -418,9 +418,11 @@ int ssd_diffattn_store(const void* qkvg_rows, const void* q_norm_w, const void* 
 /* out[t][h] = out_scale * gate[t][h] * rms_noweight(a_1 - lambda * a_2), a_m = softmax(scale * q_m . k_m) v over keys
  * 0 .. positions[t] of the token's sequence (cu_q int32 [B+1] row ranges, or q_per_seq rows per sequence when cu_q is NULL).
  * context_lens int32 [B] (keys each sequence holds) and max_q (most rows of one sequence) are optional (NULL / 0); with them, bf16,
- * D % 8 == 0, D <= 128, Dv % 16 == 0, Dv <= 128 and block_size % 32 == 0 the MFMA form runs, else the fp32 scalar form.
+ * D % 8 == 0, D <= 128, Dv % 16 == 0, Dv <= 128 and block_size % 32 == 0 the MFMA form runs, and in fp32 with D % 16 == 0, D <= 64,
+ * Dv % 16 == 0, Dv <= 128, block_size % 16 == 0 and 16-byte aligned rows its fp32 form; else the scalar form.
  * workspace (optional, fp32, workspace_bytes) + ctx_hint (host-side bound of the context lengths): decoding rows cut their keys
- * over up to 16 workgroups per (sequence, kv head); 4160 floats per (sequence, kv head, slice). */
+ * over up to 16 workgroups per (sequence, kv head); 4160 floats per (sequence, kv head, slice).  fp32: a slice is a segment of 64 keys
+ * (workspace 16-byte aligned; what it does not hold, or lies behind ctx_hint, is scanned by the second launch). */
 int ssd_diffattn_paged(const void* q_rows, const void* k_cache, const void* v_cache, const void* gate, const int32_t* block_tables,
                        int max_blocks, const int64_t* positions, const int32_t* context_lens, const int32_t* cu_q, int q_per_seq,
                        int max_q, int B, int T, int H, int G, int D, int Dv, int block_size, float scale, float lambda, float out_scale,

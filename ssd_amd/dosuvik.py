@@ -25,7 +25,7 @@ projections permuted at load (Rotary.to_halves): q and k parts permuted alike le
 
 Arithmetic: residual rows and their sums, the history and its average, norms, rope angles, scores, softmax, router, decays, the recurrent
 state, gates and every GEMM accumulator are fp32 in both modes.  dtype "bfloat16": weights, GEMM-input rows and the caches are bf16;
-"float32": they are fp32 and products are FMA chains.
+"float32": they are fp32 and products are fp32 throughout.
 """
 from __future__ import annotations
 

@@ -17,7 +17,7 @@ over pre-allocated buffers (nothing is allocated during a forward).  Same interf
 
 Arithmetic: residual rows and their sums, norms, rotation angles, scores, softmax, convolutions, unit norms, step sizes, decays, recurrent
 states, gates and every GEMM accumulator are fp32 in both modes.  dtype "bfloat16": weights, GEMM-input rows (also the inner rows of the
-low-rank projections) and the KV cache are bf16; "float32": they are fp32 and products are FMA chains.
+low-rank projections) and the KV cache are bf16; "float32": they are fp32 and products are fp32 throughout.
 """
 from __future__ import annotations
 

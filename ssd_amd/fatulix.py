@@ -11,7 +11,7 @@ Same interface as ssd_amd.model.HipDecoder towards the ModelRunner: forward / co
 
 Arithmetic: residual rows, norm statistics, q / k norms, scores, softmax weights, router logits and the expert mix are fp32 always.
 dtype "bfloat16": weights, GEMM-input rows and the KV cache are bf16 (MFMA, fp32 accumulation); "float32": they are fp32 and
-the products are FMA chains.  Every layer run has KV pages of its own (a repeated pass attends to ITS pass's keys).
+the products are fp32 throughout.  Every layer run has KV pages of its own (a repeated pass attends to ITS pass's keys).
 """
 from __future__ import annotations
 

@@ -19,7 +19,7 @@ over pre-allocated buffers (nothing is allocated during a forward).  Same interf
 
 Arithmetic: residual rows, norms, scores, softmax, router, decays, step sizes, recurrent states, gates of the recurrences and every GEMM
 accumulator are fp32 in both modes.  dtype "bfloat16": weights, GEMM-input rows and the KV cache are bf16; "float32": they are fp32 and
-products are FMA chains.
+products are fp32 throughout.
 """
 from __future__ import annotations
 

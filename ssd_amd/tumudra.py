@@ -21,7 +21,7 @@ its q and k projections and their norms' weights are permuted at load (Rotary.to
 
 Arithmetic: residual rows and their sums, norms, rotation angles, scores, softmax, gates and decays, recurrent states and normalisers,
 biases and every GEMM accumulator are fp32 in both modes.  dtype "bfloat16": weights, GEMM-input rows and the KV cache are bf16;
-"float32": they are fp32 and products are FMA chains.
+"float32": they are fp32 and products are fp32 throughout.
 """
 from __future__ import annotations
 

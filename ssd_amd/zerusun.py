@@ -15,7 +15,7 @@ Launches per layer run (T token rows):
 over pre-allocated buffers (nothing is allocated during a forward).  Same interface as ssd_amd.model.HipDecoder towards the ModelRunner.
 
 Arithmetic: residual rows, norms, rope angles, scores, softmax, router, recurrent state, gates and every GEMM accumulator are fp32 in
-both modes.  dtype "bfloat16": weights, GEMM-input rows and the latent cache are bf16; "float32": they are fp32 and products are FMA chains.
+both modes.  dtype "bfloat16": weights, GEMM-input rows and the latent cache are bf16; "float32": they are fp32 and products are fp32 throughout.
 """
 from __future__ import annotations
 
