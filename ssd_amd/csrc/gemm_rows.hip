@@ -1,11 +1,13 @@
-// Row-major GEMM for ANY M, N, K, in bf16 (MFMA 16x16x32, fp32 accumulation) or in true fp32 (FMA), dense or grouped:
+// Row-major GEMM for ANY M, N, K, in bf16 (MFMA 16x16x32, fp32 accumulation) or in true fp32 (MFMA 16x16x4, or FMA), dense or grouped:
 //   y[m][n] = sum_k x[row(m)][k] * w[g(m)][n][k]
-// The skinny / prefill GEMMs of gemm.hip and gemm_pf.hip need fragment-major operands with N % 16 == 0 and K % 32 == 0; models whose
-// sizes do not meet that, grouped (per-expert) products over gathered token rows, and the fp32 arithmetic mode use this kernel.
-// Few token rows in bf16 take the skinny weight-streaming form below; otherwise a 256-thread workgroup owns a 64 x 64 output tile; a K step of 32 is staged through LDS with bounds guards (rows or columns past
-// the edge read as zero), so no operand needs padding.  Wave w multiplies token rows 16w..16w+15 by the tile's four 16-feature
-// groups.  Every output element is the sum over k in ascending 32-wide steps, whatever M, the tile or the group is: a row's result does not
-// depend on which other rows share its launch.
+// The skinny / prefill GEMMs of gemm.hip, gemm_pf.hip and gemm_big.hip need fragment-major operands with N % 16 == 0 and K % 32 == 0; models
+// whose sizes do not meet that, grouped (per-expert) products over gathered token rows, and the fp32 arithmetic mode use this file:
+// few token rows the skinny weight-streaming form, more rows the large-tile form (both below), and what is unaligned or of odd K the kernel that
+// follows: a 256-thread workgroup owns a 64 x 64 output tile; a K step of 32 is staged through LDS with bounds guards (rows or columns past the
+// edge read as zero), so no operand needs padding; wave w multiplies token rows 16w..16w+15 by the tile's four 16-feature groups.
+// In the tile forms every bf16 output element is the sum over k in ascending 32-wide steps, whatever M, the tile or the group is; in fp32 the order
+// (gemm_tile.h; FMA chains in the guarded kernel) is a function of K and the alignment alone: a row's result does not depend on which other
+// rows share its launch.
 //   grouped: offsets[E+1] cuts the (sorted) rows into E runs, run e multiplies by w + e * N * K; row_idx (optional) names the x row
 //   of every sorted row as row_idx[r] / idx_div; tiles never straddle two runs (blockIdx.y walks a list of at most
 //   ceil(rows / 64) + E tiles, found by a scan of offsets).
