@@ -87,8 +87,10 @@ attn_prefill_kernel(const PrefillAttn p) {
     for (int dt = 0; dt < DT; ++dt) o[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  look_up(0);
-  fetch(0, 0);
+  if (tiles > 0) {                                   // (no key for any row: a padded sequence, or more rows than keys)
+    look_up(0);
+    fetch(0, 0);
+  }
   for (int t = 0; t < tiles; ++t) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");       // tile t is in LDS; nobody reads tile t - 1 any more
     if (t + 1 < tiles) {
@@ -134,19 +136,20 @@ attn_prefill_kernel(const PrefillAttn p) {
       if (__any(top > m[rt] + 8.0f)) {
         top = fmaxf(top, __shfl_xor(top, 16, 64));
         top = fmaxf(m[rt], fmaxf(top, __shfl_xor(top, 32, 64)));
-        const float alpha = __builtin_amdgcn_exp2f(m[rt] - top);        // (first tile: exp2(-inf) = 0; key 0 is visible to every row)
+        const float alpha = top == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[rt] - top);       // (a row's first key: exp2(-inf) = 0)
         m[rt] = top;
         lsum[rt] *= alpha;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[rt][dt] *= alpha;
       }
+      const float ref = m[rt] == -INFINITY ? 0.f : m[rt];       // (a row that has seen no key yet: all weights are zero)
       float sum = 0.f;
 #pragma unroll
       for (int kb = 0; kb < KEYS / 16; ++kb) {
         float w[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          w[e] = __builtin_amdgcn_exp2f(fmaf(st[kb][rt][e], p.scale_log2e, -m[rt]));
+          w[e] = __builtin_amdgcn_exp2f(fmaf(st[kb][rt][e], p.scale_log2e, -ref));
           sum += w[e];
         }
         const uint32_t h0 = pack_bf2_hw(w[0], w[1]), h1 = pack_bf2_hw(w[2], w[3]);

@@ -66,3 +66,34 @@ def test_prompts(nh, nkv, hd, bs, new, old):
     back = torch.zeros(T, nh * hd, dtype=BF, device="cuda")
     H.frag_to_rows(frag, back, T, nh * hd)
     assert torch.equal(back, rows)
+
+
+@pytest.mark.parametrize("scale,ctx,fixed", [(0.125, [0, 30, 200], True), (0.125, [0, 30, 200], False)])
+def test_rows_without_keys(scale, ctx, fixed):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ssd_amd.hip import ops as H
+    nh, nkv, hd, bs, new = 8, 2, 64, 16, 64
+    g = torch.Generator().manual_seed(sum(ctx))
+    rnd = lambda *s: torch.randn(*s, generator=g).to(BF).cuda()
+    need = [-(-c // bs) for c in ctx]
+    kc = torch.full((sum(need), nkv, bs, hd), float("nan"), dtype=BF, device="cuda")
+    vc = kc.clone()
+    bt, at, refs = torch.full((len(ctx), max(need)), -1, dtype=torch.int32), 0, []
+    T = new * len(ctx)
+    q = 4.0 * rnd(T, nh, hd)
+    for b, c in enumerate(ctx):
+        bt[b, :need[b]] = torch.arange(at, at + need[b], dtype=torch.int32)
+        K, V = rnd(c, nkv, hd), rnd(c, nkv, hd)
+        for j in range(need[b]):
+            part = slice(j * bs, min(c, (j + 1) * bs))
+            kc[at + j, :, :part.stop - part.start], vc[at + j, :, :part.stop - part.start] = K[part].transpose(0, 1), V[part].transpose(0, 1)
+        at += need[b]
+        refs.append(reference(q[b * new:(b + 1) * new].double(), K.double(), V.double(), scale).nan_to_num(0.0))       # (no key: zeros)
+    ref = torch.cat(refs).flatten(1)
+    cu = None if fixed else torch.arange(0, T + 1, new, dtype=torch.int32, device="cuda")
+    rows = torch.full((T, nh * hd), 7.0, dtype=BF, device="cuda")
+    H.attn_paged(q, kc, vc, bt.cuda(), bt.shape[1], torch.tensor(ctx, dtype=torch.int32).cuda(), len(ctx), T, new, nh, nkv, hd, bs, scale, cu_q=cu,
+                 q_per_seq=new, out_rows=rows)
+    d = (rows.double() - ref).abs()
+    assert bool((d <= 2.0 ** -8 * ref.abs() + 2.0 ** -13).all()), float(d.max())          # (bounds as above)
