@@ -68,8 +68,10 @@ def test_prompts(nh, nkv, hd, bs, new, old):
     assert torch.equal(back, rows)
 
 
-@pytest.mark.parametrize("scale,ctx,fixed", [(0.125, [0, 30, 200], True), (0.125, [0, 30, 200], False)])
-def test_rows_without_keys(scale, ctx, fixed):
+@pytest.mark.parametrize("scale,ctx,fixed", [
+    (0.125, [0, 30, 200], True), (0.125, [0, 30, 200], False),       # a sequence without keys, one with fewer keys than rows
+    (-0.125, [64, 70, 300], False), (0.0, [64, 64, 100], True)])      # scores that fall with the products; equal weights
+def test_rows_without_keys_and_any_scale(scale, ctx, fixed):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     from ssd_amd.hip import ops as H
