@@ -430,26 +430,16 @@ __device__ __forceinline__ void win_finish(f32x4_t (&acc)[MV], float mx, float l
 // V of keys past the last row's position is zeroed (a weight of zero times whatever an unwritten slot holds must stay zero).
 // The sink joins the denominator at the end.  The cap's tanh is 1 - 2 / (1 + exp(2x)) on the fast exponential.
 // ---------------------------------------------------------------------------------------------------------------------
+// One wave's part of it: the 16 rows from row0 (split: the workgroup's, of which this wave takes every fourth step of its slice).
 template <int MK, int MV>        // upper bounds of D / 32 and Dv / 16 (register arrays)
-__global__ void __launch_bounds__(256)
-winattn_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vt,
-                    const float* __restrict__ slopes, const float* __restrict__ sinks, const int32_t* __restrict__ bt, int max_blocks,
-                    const int64_t* __restrict__ positions, const int32_t* __restrict__ cu_q, int q_per_seq, int H, int G, int D, int Dv,
-                    int bs, int window, int keep_first, float scale, float cap, const float* __restrict__ out_freqs,
-                    const float* __restrict__ gate, long ldg, float out_scale, bf16_t* __restrict__ out, long ldo, int dtiles,
-                    float* __restrict__ part) {
-  extern __shared__ float smem[];
+__device__ __forceinline__ void
+win_rows(float* __restrict__ smem, const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vt,
+         const float* __restrict__ slopes, const float* __restrict__ sinks, const int32_t* __restrict__ bt, int max_blocks,
+         const int64_t* __restrict__ positions, int H, int G, int D, int Dv, int bs, int window, int keep_first, float scale, float cap,
+         const float* __restrict__ out_freqs, const float* __restrict__ gate, long ldg, float out_scale, bf16_t* __restrict__ out, long ldo,
+         float* __restrict__ part, int b, int g, int tok0, int nrows, int row0, bool split, int tile, int dtiles, int slice, int slices) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
-  const int b = blockIdx.z, g = blockIdx.y, R = H / G;
-  const int KS = D >> 5, DVT = Dv >> 4;
-  const int tok0 = cu_q ? cu_q[b] : b * q_per_seq;
-  const int nrows = (cu_q ? cu_q[b + 1] - tok0 : q_per_seq) * R;
-  const bool split = dtiles > 0 || nrows <= 16;
-  const int tile = dtiles > 0 ? blockIdx.x % dtiles : 0, slice = dtiles > 0 ? blockIdx.x / dtiles : 0;
-  const int slices = dtiles > 0 ? gridDim.x / dtiles : 1;
-  if ((dtiles > 0 ? tile * 16 : (int)blockIdx.x * 64) >= nrows) return;
-  const int row0 = split ? tile * 16 : blockIdx.x * 64 + wave * 16;
-  if (!split && row0 >= nrows) return;                 // (tile mode has no workgroup barriers)
+  const int R = H / G, KS = D >> 5, DVT = Dv >> 4;
   const int row = row0 + r;
   const bool valid = row < nrows;
   const int rr = valid ? row : row0;
@@ -606,12 +596,37 @@ winattn_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                    out_scale, out + (size_t)token * ldo + head * Dv);
 }
 
+template <int MK, int MV>
+__global__ void __launch_bounds__(256)
+winattn_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vt,
+                    const float* __restrict__ slopes, const float* __restrict__ sinks, const int32_t* __restrict__ bt, int max_blocks,
+                    const int64_t* __restrict__ positions, const int32_t* __restrict__ cu_q, int q_per_seq, int H, int G, int D, int Dv,
+                    int bs, int window, int keep_first, float scale, float cap, const float* __restrict__ out_freqs,
+                    const float* __restrict__ gate, long ldg, float out_scale, bf16_t* __restrict__ out, long ldo, int dtiles,
+                    float* __restrict__ part) {
+  extern __shared__ float smem[];
+  const int wave = threadIdx.x >> 6, b = blockIdx.z, g = blockIdx.y, R = H / G;
+  const int tok0 = cu_q ? cu_q[b] : b * q_per_seq;
+  const int nrows = (cu_q ? cu_q[b + 1] - tok0 : q_per_seq) * R;
+  const bool split = dtiles > 0 || nrows <= 16;
+  const int tile = dtiles > 0 ? blockIdx.x % dtiles : 0, slice = dtiles > 0 ? blockIdx.x / dtiles : 0;
+  const int slices = dtiles > 0 ? gridDim.x / dtiles : 1;
+  if ((dtiles > 0 ? tile * 16 : (int)blockIdx.x * 64) >= nrows) return;
+  const int row0 = split ? tile * 16 : blockIdx.x * 64 + wave * 16;
+  if (!split && row0 >= nrows) return;                 // (tile mode has no workgroup barriers)
+  win_rows<MK, MV>(smem, q, kc, vt, slopes, sinks, bt, max_blocks, positions, H, G, D, Dv, bs, window, keep_first, scale, cap, out_freqs, gate, ldg,
+                   out_scale, out, ldo, part, b, g, tok0, nrows, row0, split, tile, dtiles, slice, slices);
+}
+
 // ---------------------------------------------------------------------------------------------------------------------
 // Prompt form (more than 256 rows a sequence and kv head; D = 64 or 128, Dv <= 128): the same products, for throughput: a workgroup = 4 waves of 32 (or
 // 16) rows shares every 64-key tile of K and V through LDS, filled by DMA one tile ahead, one barrier per tile; a row keeps its reference maximum until
 // some score exceeds it by 2^8 (exact: sum and denominator both carry it); only tiles at a row's first or last key are masked.  A key's 16-byte
 // chunks of K are rotated by its index, a value column's chunks of 8 keys by the column, so that operand reads hit different banks.
 // Bound by the exponentials and conversions between the two products.  (The form above reads every K and V tile once per 16 rows from L2.)
+// A sequence of at most 16 rows beside prompts (a decoded token) would leave one wave to scan its whole context: its workgroup takes the form above,
+// the steps over all four waves.  MI355X, 32 heads of 128 in 8 groups, the form above alone | one wave | this: 300 tokens and one at key 16000
+// 420 | 1149 | 391 us, 512 tokens and two at keys 2000 and 1500 87 | 151 | 58.
 // MI355X, 32 heads of 128 in 8 groups, the form above -> this: prompts of 1800, 1500, 600 and 328 tokens 610 -> 201 us, behind a window of 512
 // 340 -> 101, 500 tokens 52 -> 43, 16384 tokens 23.1 -> 4.9 ms; 32 heads of 64 in 8, 2000 tokens 316 -> 116 us.
 // ---------------------------------------------------------------------------------------------------------------------
@@ -635,6 +650,11 @@ winattn_prompt_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
   const int nrows = (cu_q ? cu_q[b + 1] - tok0 : q_per_seq) * R;
   const int row_wg = (int)(gridDim.x - 1 - blockIdx.x) * ROWS;                 // the longest scans start first
   if (row_wg >= nrows) return;
+  if (nrows <= 16) {                     // a decoded token beside the prompts: its steps over the four waves, as in split mode
+    win_rows<MK, MV>(reinterpret_cast<float*>(wsm), q, kc, vt, slopes, sinks, bt, max_blocks, positions, H, G, D, Dv, bs, window, keep_first, scale, cap,
+                     out_freqs, gate, ldg, out_scale, out, ldo, nullptr, b, g, tok0, nrows, 0, true, 0, 0, 0, 1);
+    return;
+  }
   const int32_t* table = bt + (size_t)b * max_blocks;
   auto first_key = [&](int pos) { return window > 0 && pos + 1 > window ? pos + 1 - window : 0; };
 

@@ -93,3 +93,38 @@ def test_against_fp64(case):
             tol = 2.0 ** -8 * o.abs() + (2.0 ** -9 + 1e-4) * mag + 1e-5
             d = (out[t] - o).abs() - tol
             assert bool((d <= 0).all()), (case, b, i, float(d.max()))
+
+
+@pytest.mark.parametrize("H,G,D,Dv,window,keep", [(8, 2, 128, 128, 0, 0), (8, 2, 64, 64, 300, 20), (4, 1, 64, 128, 0, 0), (16, 4, 128, 64, 500, 0)])
+def test_single_tokens_beside_a_prompt(H, G, D, Dv, window, keep):
+    """Decoded tokens in a prompt's batch give the bits that they give among themselves: the same keys over the same four waves."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ssd_amd.hip import ops as K
+    bs, news, pasts = 64, [600, 1, 16 // (H // G), 700, 1], [30, 2111, 1500, 0, 63]
+    g = torch.Generator().manual_seed(D + Dv + window)
+    need = [-(-(n + c) // bs) for n, c in zip(news, pasts)]
+    order, at = torch.randperm(sum(need), generator=g).to(torch.int32), 0
+    bt = torch.full((len(news), max(need)), -1, dtype=torch.int32)
+    for b, n in enumerate(need):
+        bt[b, :n] = order[at:at + n]
+        at += n
+    bt = bt.cuda()
+    kc, vc = (torch.randn(sum(need), G, *s, generator=g).to(BF).cuda() for s in ((bs, D), (Dv, bs)))
+    q = torch.randn(sum(news), H, D, generator=g).to(BF).cuda()
+    sinks = torch.randn(H, generator=g).cuda()
+    cu = torch.tensor([0] + news).cumsum(0).to(torch.int32)
+    pos = torch.cat([torch.arange(c, c + n) for n, c in zip(news, pasts)]).cuda()
+
+    def attend(rows, seqs):
+        out = torch.zeros(len(rows), H * Dv, dtype=BF, device="cuda")
+        n = [news[b] for b in seqs]
+        K.winattn_paged(q[rows].contiguous(), kc, vc, None, sinks, bt[seqs].contiguous(), bt.shape[1], pos[rows].contiguous(), len(seqs), len(rows), H, G,
+                        D, Dv, bs, window, D ** -0.5, 0.0, out, False, cu_q=torch.tensor([0] + n).cumsum(0).to(torch.int32).cuda(), max_q=max(n),
+                        keep_first=keep)
+        return out
+
+    both = attend(list(range(len(q))), list(range(len(news))))
+    for b in (1, 2, 4):
+        rows = list(range(int(cu[b]), int(cu[b + 1])))
+        assert torch.equal(attend(rows, [b]), both[rows]), b
