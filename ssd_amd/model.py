@@ -353,10 +353,17 @@ class HipDecoder:
         if base >= 256 or T > self.max_split_tokens:
             splits = 1
             if meta.cu_q is None:
-                # a decoding batch that fills the grid by itself: its scans are chains of tile loads, as long as the longest context --
-                # more waves per (sequence, kv head), not grid splits (MI355X, 1 | 4 | 8 waves: 48 sequences of 190 .. 3000 keys, 8 kv heads of
-                # 128: 204 | 64 | 50 us, with 4 | 8 waves x 2 splits 54 | 55; 64 of 12 .. 200: 20 | 12 | 16; 32 of 60 .. 1000: 40 | 24 | 20)
-                waves = 4 if ctx <= 1024 and base > 256 else 8
+                # A decoding batch that fills the grid by itself: its scans are chains of tile loads, as long as the longest context -- more waves
+                # per (sequence, kv head), not grid splits, as long as they are resident together: 2048 waves of 128-wide heads, twice as
+                # many of 64-wide ones.  (MI355X, 8 kv heads of 128, contexts of a sixteenth to the whole of the longest, us with 1 | 2 | 4 | 8
+                # waves: 48 sequences, up to 3000 keys 204 | 120 | 90 | 76, up to 150 17 | 15 | 13 | 16; 64 x 8 rows, 64 heads, up to 3000 keys
+                # 256 | 311 | 355 | 369, up to 150 23 | 32 | 40 | 58; 48 x 8 rows, 32 heads, up to 3000 keys 210 | 126 | 118 | 132.  2 waves at
+                # fill 900 .. 1024: 0.98 of one wave's time at 150 keys, 0.84 at 1000; at 1025 .. 1535 1.17 and 0.82.)
+                fill = base * self.hd // 128
+                if ctx <= 1024:
+                    waves = 8 if base <= 256 else 4 if fill <= 512 else 2 if fill <= 1024 else 1
+                else:
+                    waves = 8 if fill <= 512 else 4 if fill <= 768 else 2 if fill < 1536 else 1
         return splits, waves
 
     def _attn_flags(self, meta: AttnMeta) -> int:
