@@ -260,6 +260,7 @@ class HipDecoder:
     BIG_MIN_ROWS = 160
     AP_WIDE_HEAD_BYTES = 1200 << 20
     PARTS_WIDE_WEIGHT_BYTES = 64 << 20
+    PARTS_WIDE_OUTPUTS = 2560
     BIG_MIN_WEIGHT_BYTES = 16 << 20
     BIG_SMALLEST_WEIGHT_BYTES = 1 << 20
     BIG_WORKSPACE_BYTES = 48 << 20
@@ -408,9 +409,13 @@ class HipDecoder:
 
     def parts_plan(self, T: int) -> bool:
         """o_proj / down_proj as split-K partial slabs consumed by the next norm: single-rank models with < 256 row groups at
-        decode-sized T (the draft's chain / glue / tree forwards).  A down_proj of 64 MB and more: up to 16 rows only -- with two token tiles its
-        slabs cost more than the large-tile GEMM's rows (32B, 32 rows, with the norm: 80 -> 55 us)."""
-        return self.use_parts and not self.use_coll and T <= (32 if 2 * self.h * self.I < self.PARTS_WIDE_WEIGHT_BYTES else 16)
+        decode-sized T (the draft's chain / glue / tree forwards).  A down_proj of 64 MB and more with 2560 outputs and more: up to 16 rows only --
+        with two token tiles its slabs cost more than the large-tile GEMM's rows (MI355X, 32 | 17 rows with the norm, slabs -> rows: 5120 x 25600
+        81 | 74 -> 54 | 53 us, 5120 x 13824 49 | 43 -> 34 | 33, 3584 x 18944 55 | 51 -> 34 | 34, 3072 x 12288 30 | 28 -> 25 | 25; level at
+        2560 x 16384 32 | 29 -> 30 | 30; the other way at 2048 x 16384 24 | 23 -> 29 | 28, 1536 x 24576 29 | 26 -> 34 | 34, and of 48 MB
+        3072 x 8192 20 | 18 -> 21 | 20)."""
+        wide = self.h >= self.PARTS_WIDE_OUTPUTS and 2 * self.h * self.I >= self.PARTS_WIDE_WEIGHT_BYTES
+        return self.use_parts and not self.use_coll and T <= (16 if wide else 32)
 
     def attn_o_plan(self, T: int, meta: AttnMeta, splits: int) -> bool:
         """Attention + o_proj as ONE launch (csrc/attention.hip OPROJ variant): single-rank models on the slab path, one

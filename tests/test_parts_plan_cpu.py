@@ -37,6 +37,13 @@ def test_unfused_consumer_plans_fit_for_arbitrary_shapes():
             assert t <= 8 or K // 32 > 16 * 16 * 8, (N, K, t)
 
 
+def test_wide_down_projections_leave_the_slabs_at_two_token_tiles():
+    for h, I, rows in ((5120, 25600, 16), (3584, 18944, 16), (3072, 12288, 16), (3072, 8192, 32), (2048, 16384, 32), (2048, 24576, 32), (1024, 3072, 32)):
+        d = HipDecoder.__new__(HipDecoder)
+        d.h, d.I, d.use_parts, d.use_coll = h, I, True, False
+        assert [d.parts_plan(T) for T in (1, 16, 17, 32, 33)] == [True, True, rows == 32, rows == 32, False], (h, I)
+
+
 def test_peaky_recipe_scales_the_same_tokens_in_target_and_eagle_draft():
     """bench.py --workload c4e builds its EAGLE pair with the "peaky" recipe (ssd_amd/weights.py peaky_rows): the LM-head rows
     of the same few tokens -- draft-vocabulary ids pushed through the draft's d2t -- are scaled in BOTH models, everything
