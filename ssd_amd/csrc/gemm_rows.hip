@@ -208,20 +208,22 @@ gemm_rows_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restr
 
 // ---------------------------------------------------------------------------------------------------------------------
 // Skinny form (few token rows, or few features: decoding, routers; 16-byte aligned rows; bf16 K % 8 == 0, fp32 K % 32 == 0): a weight-streaming
-// product, bound by the weights' way from HBM.  A workgroup owns 16 features; its four waves take K in turn, in runs of 256 k, each through a ring
-// of its own that DMA fills (no barrier: only the wave itself waits for it).  A stage is 256 bytes of 16 weight rows and of the token rows:
+// product, bound by the weights' way from HBM.  A workgroup owns 16 features; its four or eight waves take K in turn, in runs of 256 k, each through
+// a ring of its own that DMA fills (no barrier: only the wave itself waits for it).  A stage is 256 bytes of 16 weight rows and of the token rows:
 // one instruction fetches four whole 256-byte pieces, whose 16-byte chunks are rotated by the row so that the 16 lanes of an operand read hit
 // different banks.  (16-byte loads straight into the MFMA layout fetch 64 bytes of a row at a time, and a wave has nothing in flight while it
-// multiplies.)  Two workgroups share a CU, one's loads covering the other's start and end; more waves or deeper rings gained nothing.
+// multiplies.)  With four waves two workgroups share a CU, one's loads covering the other's start and end; where no CU gets a second one, eight waves
+// halve the chain of stages.  Deeper rings gained nothing.
 //   bf16: a wave's runs are one chain of 16x16x32 MFMAs, the waves' sums are added in wave order.
 //   fp32: a run is a segment of gemm_tile.h's order; after every round of four, wave 0 adds the segments' sums in theirs.
-// MI355X, weights not in the caches, direct loads -> this: bf16, 4 rows: 14720 x 4096 36.6 -> 21.3 us (5.7 TB/s), 4096 x 14720 31.5 -> 19.3,
-// 4096 x 4096 11.6 -> 7.9, 2048 x 7424 18.9 -> 8.8; fp32, 4 rows: 32000 x 2048 77 -> 40 us (6.6 TB/s), 3088 x 2048 11.4 -> 6.8, 2048 x 3072
-// 16.9 -> 8.8.  fp32 error against fp64, relative: 3e-7 at K = 2048 .. 4096.
+// MI355X, weights not in the caches, direct loads -> four waves: bf16, 4 rows: 14720 x 4096 36.6 -> 21.3 us (5.7 TB/s), 4096 x 14720 31.5 -> 19.3,
+// 2048 x 7424 18.9 -> 8.8; fp32, 4 rows: 32000 x 2048 77 -> 40 us (6.6 TB/s), 3088 x 2048 11.4 -> 6.8, 2048 x 3072 16.9 -> 8.8.  fp32 error against
+// fp64, relative: 3e-7 at K = 2048 .. 4096.
+// Weights of many matrices in turn (partly from the Infinity Cache), one row, direct loads with 16 waves | four | eight waves: N = 8, K = 4096 7.7 | 8.1 |
+// 5.6 us, K = 14720 16.3 | 25.6 | 14.6; 4096 x 4096 10.3 | 11.3 | 9.4, 4096 x 14720 30.4 | 32.5 | 22.7, 64 x 2048 6.7 | 5.4 | 4.7.
 // Grouped: blockIdx.y is the group; a group with no rows exits at once.  16-row chunks are dealt out over blockIdx.z.
 // ---------------------------------------------------------------------------------------------------------------------
-constexpr int SKINNY_WAVES = 4;
-template <typename T>
+template <typename T, int NW>             // NW waves
 struct Skinny {
   static constexpr bool F32 = sizeof(T) == 4;
   static constexpr int SPR = F32 ? F32_SEG * 4 / 256 : 2;                    // stages of a run
@@ -231,9 +233,9 @@ struct Skinny {
 
   // Up to 4 * XI token rows at xr (this lane's four-row pieces) against the 16 weight rows at wr: wave 0 returns the sums.
   template <int XI>
-  static __device__ __forceinline__ f32x4_t chunk(char* ring, f32x4_t (*red)[SKINNY_WAVES][64], uint32_t& turn, const char* const (&wr)[4],
+  static __device__ __forceinline__ f32x4_t chunk(char* ring, f32x4_t (*red)[NW][64], uint32_t& turn, const char* const (&wr)[4],
                                                   const char* const (&xr)[XI], long row_bytes) {
-    constexpr int NW = SKINNY_WAVES, R = stages(XI), STAGE = stage_bytes(XI), PER = 4 + XI;
+    constexpr int R = stages(XI), STAGE = stage_bytes(XI), PER = 4 + XI;
     static_assert(R * STAGE <= RING, "the ring holds the stages");
     const int lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4, xrow = r & (4 * XI - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -314,14 +316,14 @@ struct Skinny {
   }
 };
 
-template <typename T>
-__global__ void __launch_bounds__(SKINNY_WAVES * 64)
+template <typename T, int NW>
+__global__ void __launch_bounds__(NW * 64)
 gemm_skinny_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
                    const int* __restrict__ offsets, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx,
                    long gsy, GluClamp gc, DecayGate dg) {
-  typedef Skinny<T> L;
-  __shared__ __attribute__((aligned(1024))) char smem[SKINNY_WAVES * L::RING];
-  __shared__ f32x4_t red[2][SKINNY_WAVES][64];
+  typedef Skinny<T, NW> L;
+  __shared__ __attribute__((aligned(1024))) char smem[NW * L::RING];
+  __shared__ f32x4_t red[2][NW][64];
   const int lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = blockIdx.x * 16;
@@ -536,8 +538,13 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   const bool x_vec = ((size_t)ldx * esz0) % 16 == 0 && ((size_t)gsx * esz0) % 16 == 0 && (uintptr_t)x % 16 == 0;
   if (!f32 && K % 8 == 0 && x_vec && (uintptr_t)w % 16 == 0 &&
       M <= (offsets ? SKINNY_MAX_GROUPED_ROWS : SKINNY_MAX_ROWS)) {
-    hipLaunchKernelGGL(gemm_skinny_kernel<bf16_t>, dim3((N + 15) / 16, offsets ? E : G), dim3(64 * SKINNY_WAVES), 0, (hipStream_t)stream,
-                       (const bf16_t*)x, (const bf16_t*)w, y, M, N, K, epi, offsets, row_idx, idx_div < 1 ? 1 : idx_div, ldx, ldy, gsx, gsy, gc, dg);
+#define SKINNY_GO(T, NW, Z)                                                                                                              \
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, NW>), dim3((N + 15) / 16, offsets ? E : G, Z), dim3(64 * NW), 0, (hipStream_t)stream, (const T*)x, \
+                     (const T*)w, y, M, N, K, epi, offsets, row_idx, idx_div < 1 ? 1 : idx_div, ldx, ldy, gsx, gsy, gc, dg)
+    // at most a workgroup per CU: eight waves, whose rings fill its LDS, as long as each gets a run (K = 1024: level)
+    const long wgs = (long)((N + 15) / 16) * (offsets ? (M < E ? M : E) : G);          // those that have rows
+    if (wgs <= 256 && K >= 2048) SKINNY_GO(bf16_t, 8, 1);
+    else SKINNY_GO(bf16_t, 4, 1);
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
   // (fp32: which of the two orders of summation a product gets -- gemm_tile.h's, or the plain chain of the form for everything else -- may
@@ -548,8 +555,8 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   // tile, a serial walk of K by few workgroups; a router's 1000 x 8 x 2048 the same 48 us)
   const int chunks = (M + 15) / 16;
   if (tiled && f32 && (offsets ? M <= SKINNY_MAX_GROUPED_ROWS : M <= SKINNY_MAX_ROWS || (long)chunks * ((N + 15) / 16) * G <= 1024)) {
-    hipLaunchKernelGGL(gemm_skinny_kernel<float>, dim3((N + 15) / 16, offsets ? E : G, offsets ? 1 : chunks), dim3(64 * SKINNY_WAVES), 0,
-                       (hipStream_t)stream, (const float*)x, (const float*)w, y, M, N, K, epi, offsets, row_idx, id, ldx, ldy, gsx, gsy, gc, dg);
+    SKINNY_GO(float, 4, offsets ? 1 : chunks);
+#undef SKINNY_GO
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
   if (tiled) {

@@ -43,6 +43,23 @@ def test_rows_of_every_ring_shape(H, K, f32):
         assert torch.equal(one[0], y[M - 1]), (M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K,G", [(3, 4096, 2048, 1), (3, 4097, 2048, 1), (16, 4096, 2056, 1), (5, 4112, 2056, 1), (9, 2048, 4104, 2), (9, 2049, 4104, 2),
+                                     (4, 40, 2040, 3), (1, 8, 14720, 1)])
+def test_bf16_four_and_eight_waves(H, M, N, K, G):
+    """Both sides of the line between them, a workgroup per CU (256 of 16 features) and K = 2048, with the last run a part of one."""
+    g = torch.Generator().manual_seed(M + N + K)
+    w = (torch.randn(G, N, K, generator=g) / K ** 0.5).to(BF).cuda()
+    x = torch.randn(M, G * K, generator=g).to(BF).cuda()
+    y = torch.full((M, G * N), 7.0, device="cuda")
+    H.gemm_rows_batched(x, w, y, M, N, K, G, G * K, K, G * N, N, False)
+    one = torch.zeros(1, G * N, device="cuda")
+    H.gemm_rows_batched(x[M - 1:], w, one, 1, N, K, G, G * K, K, G * N, N, False)
+    assert torch.equal(one[0], y[M - 1])
+    for i in range(G):
+        d = float((y[:, i * N:(i + 1) * N].double() - x[:, i * K:(i + 1) * K].double() @ w[i].double().T).abs().max())
+        assert d <= tol(False) * max(1.0, K / 2 ** 13), (M, N, K, i, d)
+
+
 @pytest.mark.parametrize("K", [8, 24, 40, 136, 264, 1032])
 def test_bf16_ends_inside_an_operand(H, K):
     """What lies behind a row's end is not part of its sum, whatever it holds."""
@@ -56,10 +73,10 @@ def test_bf16_ends_inside_an_operand(H, K):
         assert d <= tol(False), (M, N, K, d)
 
 
-@pytest.mark.parametrize("f32", [False, True])
-def test_grouped_chunks(H, f32):
+@pytest.mark.parametrize("f32,K", [(False, 320), (True, 320), (False, 2056), (True, 2080)])
+def test_grouped_chunks(H, f32, K):
     """Runs of 0, 1, 4, 7 and 33 gathered rows: one, two and four row pieces, and three 16-row chunks in turn."""
-    K, N, runs = 320, 70, [1, 0, 4, 7, 33]
+    N, runs = 70, [1, 0, 4, 7, 33]
     offs = [0]
     for c in runs:
         offs.append(offs[-1] + c)
