@@ -16,6 +16,8 @@ CASES = [  # H, G, D, Dv, bs, window, keep, options
     (8, 1, 128, 80, 64, 300, 33, ("gate", "cap")),
     (4, 1, 128, 128, 32, 64, 0, ("freqs", "sink")),
     (4, 2, 64, 64, 64, 1, 0, ()),
+    (32, 8, 64, 64, 64, 0, 0, ("sink",)),             # 608 units of 128 rows: heads of 64 in workgroups of 128 rows
+    (32, 8, 64, 48, 32, 200, 10, ("gate", "cap")),
 ]
 
 
@@ -89,8 +91,9 @@ def test_against_fp64(case):
             if gate is not None:
                 f = torch.sigmoid(gate[t, :H * Dv].double()).view(H, Dv) * osc
                 o, mag = o * f, mag * f
-            # the output's rounding; the weights' rounding to bf16 (2^-9 each) with 1e-4 for scores in fp32 and the hardware exponential
-            tol = 2.0 ** -8 * o.abs() + (2.0 ** -9 + 1e-4) * mag + 1e-5
+            # bf16 has 8 significant bits: rounding moves a number by half a last place, at most 2^-8 of it.  Once for the output, once for every
+            # weight (which their sum does not see), with 1e-4 for scores in fp32 and the hardware exponential
+            tol = 2.0 ** -8 * o.abs() + (2.0 ** -8 + 1e-4) * mag + 1e-5
             d = (out[t] - o).abs() - tol
             assert bool((d <= 0).all()), (case, b, i, float(d.max()))
 
