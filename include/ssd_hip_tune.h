@@ -30,6 +30,13 @@ int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const void* bias, v
                      void* workspace, int64_t workspace_bytes, int shape, int splits, void* stream);
 
 
+/* ssd_gemm_rows, or with offsets ssd_gemm_rows_grouped, on a large tile of the caller's choice whatever the number of rows: shape = 0 256 x 256,
+ * 1 192 x 192, 2 128 x 128, 3 128 x 64 (features x tokens); fp32: 0 128 x 128, 1 64 x 64, 2 64 x 32.  Sizes that no large tile takes (K, alignment)
+ * are refused.  All shapes of a type give the same bits. */
+int ssd_gemm_rows_cfg(const void* x_rows, const void* w_rows, void* y, const int32_t* offsets, int E, const int32_t* row_idx, int idx_div, int rows,
+                      int N, int K, int epilogue, int f32, int shape, void* stream);
+
+
 /* A/B facility (bench.py --tune-deep, profiles/): ssd_gemm_wf's default dispatch for the 70B-class matrices -- 1 (default) the DEEP
  * form, 0 the plain kernels of rounds 1-5.
  * Process-wide; call before any hipGraph is captured. */

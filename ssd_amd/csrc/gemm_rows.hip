@@ -524,7 +524,7 @@ int tile_shape(const RowTile (&tiles)[COUNT], int M, int N, int G, int E) {
 
 int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, const int* offsets, int E, const int* row_idx,
            int idx_div, int f32, void* stream, int G = 1, long ldx = 0, long gsx = 0, long ldy = 0, long gsy = 0,
-           GluClamp gc = GluClamp{nullptr, 0.f, 0.f}, DecayGate dg = DecayGate{nullptr, nullptr, 0}) {
+           GluClamp gc = GluClamp{nullptr, 0.f, 0.f}, DecayGate dg = DecayGate{nullptr, nullptr, 0}, int shape = -1) {
   if (!x || !w || !y) return SSD_ERR_ARG;
   if (M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > 8) return SSD_ERR_SHAPE;
   if ((epi == 7 && !dg.rate) || (epi == 8 && !dg.bias)) return SSD_ERR_SHAPE;
@@ -536,7 +536,7 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   if (ldx < K || ldy < (epi_pairs(epi) ? N / 2 : N)) return SSD_ERR_SHAPE;
   const int esz0 = f32 ? 4 : 2;
   const bool x_vec = ((size_t)ldx * esz0) % 16 == 0 && ((size_t)gsx * esz0) % 16 == 0 && (uintptr_t)x % 16 == 0;
-  if (!f32 && K % 8 == 0 && x_vec && (uintptr_t)w % 16 == 0 &&
+  if (shape < 0 && !f32 && K % 8 == 0 && x_vec && (uintptr_t)w % 16 == 0 &&
       M <= (offsets ? SKINNY_MAX_GROUPED_ROWS : SKINNY_MAX_ROWS)) {
 #define SKINNY_GO(T, NW, Z)                                                                                                              \
   hipLaunchKernelGGL((gemm_skinny_kernel<T, NW>), dim3((N + 15) / 16, offsets ? E : G, Z), dim3(64 * NW), 0, (hipStream_t)stream, (const T*)x, \
@@ -554,13 +554,14 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   // few rows, or few features: 16-row chunks over the grid as long as that is about what the chip holds at once (64 x 2048 x 2048: 49 us as a
   // tile, a serial walk of K by few workgroups; a router's 1000 x 8 x 2048 the same 48 us)
   const int chunks = (M + 15) / 16;
-  if (tiled && f32 && (offsets ? M <= SKINNY_MAX_GROUPED_ROWS : M <= SKINNY_MAX_ROWS || (long)chunks * ((N + 15) / 16) * G <= 1024)) {
+  if (shape >= 0 && (!tiled || shape >= (f32 ? 3 : 4))) return SSD_ERR_SHAPE;
+  if (shape < 0 && tiled && f32 && (offsets ? M <= SKINNY_MAX_GROUPED_ROWS : M <= SKINNY_MAX_ROWS || (long)chunks * ((N + 15) / 16) * G <= 1024)) {
     SKINNY_GO(float, 4, offsets ? 1 : chunks);
 #undef SKINNY_GO
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
   if (tiled) {
-    const int shape = f32 ? tile_shape(TILES_F32, M, N, G, offsets ? E : 0) : tile_shape(TILES_BF16, M, N, G, offsets ? E : 0);
+    if (shape < 0) shape = f32 ? tile_shape(TILES_F32, M, N, G, offsets ? E : 0) : tile_shape(TILES_BF16, M, N, G, offsets ? E : 0);
     // what a store of four (paired: two) neighbouring outputs needs: their address a multiple of its size
     const bool out32 = f32 || epi == 0 || epi == 8;
     const int width = epi_pairs(epi) ? 4 : (out32 ? 16 : 8), osz = out32 ? 4 : 2;
@@ -613,6 +614,13 @@ extern "C" int ssd_gemm_rows_grouped(const void* x_rows, const void* w_rows, voi
                                      void* stream) {
   if (!offsets) return SSD_ERR_ARG;
   return launch(x_rows, w_rows, y, rows, N, K, epilogue, offsets, E, row_idx, idx_div, f32, stream);
+}
+
+extern "C" int ssd_gemm_rows_cfg(const void* x_rows, const void* w_rows, void* y, const int32_t* offsets, int E, const int32_t* row_idx, int idx_div,
+                                 int rows, int N, int K, int epilogue, int f32, int shape, void* stream) {
+  if (shape < 0) return SSD_ERR_ARG;
+  return launch(x_rows, w_rows, y, rows, N, K, epilogue, offsets, E, row_idx, idx_div, f32, stream, 1, 0, 0, 0, 0, GluClamp{nullptr, 0.f, 0.f},
+                DecayGate{nullptr, nullptr, 0}, shape);
 }
 
 extern "C" int ssd_gemm_rows_grouped_glu_clamp(const void* x_rows, const void* w_rows, void* y, const int32_t* offsets, int E,

@@ -438,6 +438,13 @@ def gemm_rows_grouped(x, w, y, offsets, E: int, rows: int, N: int, K: int, f32: 
                                                 int(f32), _stream()), "ssd_gemm_rows_grouped")
 
 
+def gemm_rows_cfg(x, w, y, rows: int, N: int, K: int, f32: bool, shape: int, epilogue: int = GR_F32, offsets=None, E: int = 0, row_idx=None,
+                  idx_div: int = 1):
+    """gemm_rows (offsets None) or gemm_rows_grouped on a large tile of the caller's choice (include/ssd_hip_tune.h)."""
+    _check(load_library().ssd_gemm_rows_cfg(_p(x), _p(w), _p(y), _p(offsets), E, _p(row_idx), idx_div, rows, N, K, epilogue, int(f32), shape,
+                                            _stream()), "ssd_gemm_rows_cfg")
+
+
 def diffattn_store(qkvg, q_norm_w, k_norm_w, eps: float, slots, q_out, gate_out, k_cache, v_cache, T, H, G, D, Dv, block_size,
                    f32: bool):
     _check(load_library().ssd_diffattn_store(_p(qkvg), _p(q_norm_w), _p(k_norm_w), eps, _p(slots), _p(q_out), _p(gate_out),

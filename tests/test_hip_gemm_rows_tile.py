@@ -137,3 +137,38 @@ def test_fp32_grouped(H, counts, N, K):
             H.gemm_rows(rows, w[e].contiguous(), alone, len(rows), N, K, True, 0)
             assert torch.equal(alone, y[off[e]:off[e + 1]])
             assert bool(((alone.double() - rows.double() @ w[e].double().T).abs() <= 1e-4).all())
+
+
+@pytest.mark.parametrize("f32,shape", [(False, s) for s in range(4)] + [(True, s) for s in range(3)])
+def test_every_shape(H, f32, shape):
+    """Every tile shape of either type, dense and grouped (empty runs, runs of one row, of a tile, of a tile and one; rows gathered), whatever shape the
+    sizes would be given: within the bounds of the tests above, and the bits of the shape that they are given."""
+    counts, N, K, div = [257, 0, 1, 64, 300, 0, 33], 390, 320 if f32 else 192, 2
+    R, E = sum(counts), len(counts)
+    g = torch.Generator().manual_seed(shape)
+    dt = torch.float32 if f32 else BF
+    x, w = torch.randn(-(-R // div), K, generator=g).to(dt).cuda(), (torch.randn(E, N, K, generator=g) / K ** 0.5).to(dt).cuda()
+    perm = torch.randperm(R, generator=g).to(torch.int32).cuda()
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32).cuda()
+    ref = torch.cat([x[(perm[off[e]:off[e + 1]].long() // div)].double() @ w[e].double().T for e in range(E)])
+    dense = x.double() @ w[0].double().T
+    for epi in ((0, 1) if f32 else (0, 1, 2, 3)):
+        y, z = (torch.full((n, N // 2 if epi == 3 else N), 7.0, dtype=torch.float32 if f32 or epi == 0 else BF, device="cuda") for n in (R, len(x)))
+        y2, z2 = y.clone(), z.clone()
+        H.gemm_rows_cfg(x, w, y, R, N, K, f32, shape, epi, offsets=off, E=E, row_idx=perm, idx_div=div)
+        H.gemm_rows_grouped(x, w, y2, off, E, R, N, K, f32, epi, row_idx=perm, idx_div=div)
+        H.gemm_rows_cfg(x, w[0].contiguous(), z, len(x), N, K, f32, shape, epi)
+        H.gemm_rows(x, w[0].contiguous(), z2, len(x), N, K, f32, epi)
+        assert torch.equal(y, y2) and torch.equal(z, z2), epi
+        for got, want in ((y, ref), (z, dense)):
+            want = {0: want, 1: want.relu() ** 2, 2: want, 3: act(want, 3)}[epi]
+            if f32:
+                assert bool(((got.double() - want).abs() <= 1e-4 * (12.0 if epi else 1.0)).all()), epi
+            else:
+                check(got, want, epi, epi != 0, slope=12.0 if epi in (1, 3) else 1.0)
+    from ssd_amd.hip.lib import SsdHipError
+    for bad in (-1, 3 if f32 else 4):
+        with pytest.raises(SsdHipError):
+            H.gemm_rows_cfg(x, w[0].contiguous(), z, len(x), N, K, f32, bad)
+    with pytest.raises(SsdHipError):
+        H.gemm_rows_cfg(x[:, :K - 8].contiguous(), w[0, :, :K - 8].contiguous(), z, len(x), N, K - 8, f32, shape)
