@@ -114,9 +114,18 @@ extern "C" int ssd_topk_rows(const void* logits, long ld, int T, int V, int k, i
 // The draw of one slice of a row.  A candidate costs two 64-bit hashes and two logarithms -- 128256 of them kept one CU busy for 82 us, most of a
 // single token's sampling -- so a row is cut into slices over the grid; out[row] holds the best (value, lowest index) so far as one ordered
 // 64-bit key (sample_init_kernel: below every candidate), which the slices raise, and sample_finish_kernel turns into the token.
-// MI355X, vocabulary 128256, the three launches: 1 row 82 -> 10 us, 48 rows 84 -> 19; 32000: 23 -> 10.  A vocabulary of a few thousand (and a batch of
-// more rows than four workgroups per CU) takes one workgroup per row and one launch (`direct`): 513 tokens 5 us, three launches 11.
+// MI355X, vocabulary 128256, the three launches: 1 row 82 -> 7 us, 48 rows 84 -> 19; 32000: 23 -> 7.  One workgroup per row and one launch (`direct`)
+// where that is as fast: a vocabulary of a few thousand (4096: 5 us, in three launches 7), and rows that fill the chip by themselves (below).
 constexpr int SAMPLE_THREADS = 256, SAMPLE_DIRECT_VOCAB = 8192;
+
+// One workgroup per row takes 0.6 ns per candidate as long as each has a CU to itself, 1.1 ns with two to a CU, and starts over after 512 rows; slices
+// spread all candidates evenly, 0.0020 ns each (0.0023 from unaligned rows), behind two more launches (3.4 us).  (MI355X, us, direct | slices: 256 rows of 16000 12 | 14, of 128256
+// 76 | 70; 192 of 8200 8 | 10, of 32000 21 | 18; 512 of 8200 12 | 15, of 50257 62 | 70; 300 of 32000 38 | 26.)
+static bool sample_direct(int T, int V, bool aligned) {
+  const int rest = T % 512;
+  const double row = 1.1e-3 * (T / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.6e-3 : 1.1e-3);
+  return V <= SAMPLE_DIRECT_VOCAB || V * (row - (aligned ? 2.03e-6 : 2.3e-6) * T) < 3.4;
+}
 
 __device__ __forceinline__ unsigned long long best_key(Best b) {
   const uint32_t u = __float_as_uint(b.v + 0.0f);                       // (-0 counts as 0)
@@ -186,8 +195,8 @@ extern "C" int ssd_sample_rows(const void* logits, long ld, int T, int V, const 
     per *= (slices + most - 1) / most;
     slices = (V + per - 1) / per;
   }
-  const bool direct = slices == 1 || V <= SAMPLE_DIRECT_VOCAB;
-  const bool vec = ld % 8 == 0 && ((uintptr_t)logits & 15) == 0 && V > SAMPLE_DIRECT_VOCAB;
+  const bool aligned = ld % 8 == 0 && ((uintptr_t)logits & 15) == 0, vec = aligned && V > SAMPLE_DIRECT_VOCAB;
+  const bool direct = slices == 1 || sample_direct(T, V, aligned);
   const float log_x = boost_idx ? logf(boost_x) : 0.f;
 #define SAMPLE_GO(THREADS, BOOST, SLICES, PER)                                                                                               \
   hipLaunchKernelGGL((sample_slices_kernel<THREADS, BOOST>), dim3(T, SLICES), dim3(THREADS), 0, st, (const bf16_t*)logits, ld, V, PER, temps, \

@@ -31,7 +31,8 @@ def scores(x, T, seed, salt, row, boost, log_x):
     return s
 
 
-@pytest.mark.parametrize("T,V,ld", [(1, 128256, 128256), (3, 8193, 8200), (2, 20011, 20011), (70, 9000, 9000), (1, 8192, 8192), (5, 37, 40), (1100, 8200, 8200)])
+@pytest.mark.parametrize("T,V,ld", [(1, 128256, 128256), (3, 8193, 8200), (2, 20011, 20011), (70, 9000, 9000), (1, 8192, 8192), (5, 37, 40), (1100, 8200, 8200), (192, 8200, 8200),
+                                    (256, 20011, 20011), (257, 8200, 8208), (512, 9000, 9000), (600, 8200, 8200)])
 def test_the_draw_is_the_hosts(T, V, ld):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
