@@ -40,7 +40,8 @@ def act(z, epi):
 
 
 # sizes: 256-token tiles are chosen for the third, 192 for the fourth, 128 for the fifth, 64 for the others; features off every tile and vector width
-@pytest.mark.parametrize("M,N,K", [(17, 128, 128), (65, 131, 192), (4000, 4050, 128), (2001, 4098, 128), (700, 6002, 128), (129, 386, 4096)])
+@pytest.mark.parametrize("M,N,K", [(17, 128, 128), (65, 131, 192), (4000, 4050, 128), (2001, 4098, 128), (700, 6002, 128), (129, 386, 4096),
+                                   (40, 8, 128), (300, 32, 192), (40, 34, 192), (70, 24, 256)])       # few features: the guarded kernel, large tiles
 def test_dense_epilogues(H, M, N, K):
     x, w = operands(M, N, K, M + N + K)
     z = x.double() @ w.double().T
