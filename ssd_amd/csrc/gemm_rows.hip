@@ -220,7 +220,8 @@ gemm_rows_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restr
 // 2048 x 7424 18.9 -> 8.8; fp32, 4 rows: 32000 x 2048 77 -> 40 us (6.6 TB/s), 3088 x 2048 11.4 -> 6.8, 2048 x 3072 16.9 -> 8.8.  fp32 error against
 // fp64, relative: 3e-7 at K = 2048 .. 4096.
 // Weights of many matrices in turn (partly from the Infinity Cache), one row, direct loads with 16 waves | four | eight waves: N = 8, K = 4096 7.7 | 8.1 |
-// 5.6 us, K = 14720 16.3 | 25.6 | 14.6; 4096 x 4096 10.3 | 11.3 | 9.4, 4096 x 14720 30.4 | 32.5 | 22.7, 64 x 2048 6.7 | 5.4 | 4.7.
+// 5.6 us, K = 14720 16.3 | 25.6 | 14.6; 4096 x 4096 10.3 | 11.3 | 9.4, 4096 x 14720 30.4 | 32.5 | 22.7, 64 x 2048 6.7 | 5.4 | 4.7; direct loads with
+// eight, four, eight: 4096 x 1280 5.2 | 5.8 | 5.0, 64 x 1536 4.6 | 5.0 | 4.2.
 // Grouped: blockIdx.y is the group; a group with no rows exits at once.  16-row chunks are dealt out over blockIdx.z.
 // ---------------------------------------------------------------------------------------------------------------------
 template <typename T, int NW>             // NW waves
@@ -541,9 +542,9 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
 #define SKINNY_GO(T, NW, Z)                                                                                                              \
   hipLaunchKernelGGL((gemm_skinny_kernel<T, NW>), dim3((N + 15) / 16, offsets ? E : G, Z), dim3(64 * NW), 0, (hipStream_t)stream, (const T*)x, \
                      (const T*)w, y, M, N, K, epi, offsets, row_idx, idx_div < 1 ? 1 : idx_div, ldx, ldy, gsx, gsy, gc, dg)
-    // at most a workgroup per CU: eight waves, whose rings fill its LDS, as long as each gets a run (K = 1024: level)
+    // at most a workgroup per CU: eight waves, whose rings fill its LDS, as long as four have more than a run each (K = 1024: level)
     const long wgs = (long)((N + 15) / 16) * (offsets ? (M < E ? M : E) : G);          // those that have rows
-    if (wgs <= 256 && K >= 2048) SKINNY_GO(bf16_t, 8, 1);
+    if (wgs <= 256 && K > 1024) SKINNY_GO(bf16_t, 8, 1);
     else SKINNY_GO(bf16_t, 4, 1);
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
