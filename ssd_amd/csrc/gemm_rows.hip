@@ -208,7 +208,7 @@ gemm_rows_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restr
 
 // ---------------------------------------------------------------------------------------------------------------------
 // Skinny form (few token rows, or few features: decoding, routers; 16-byte aligned rows; bf16 K % 8 == 0, fp32 K % 32 == 0): a weight-streaming
-// product, bound by the weights' way from HBM.  A workgroup owns 16 features; its four or eight waves take K in turn, in runs of 256 k, each through
+// product, bound by the weights' way from HBM.  A workgroup owns 16 features; its one, four or eight waves take K in turn, in runs of 256 k, each through
 // a ring of its own that DMA fills (no barrier: only the wave itself waits for it).  A stage is 256 bytes of 16 weight rows and of the token rows:
 // one instruction fetches four whole 256-byte pieces, whose 16-byte chunks are rotated by the row so that the 16 lanes of an operand read hit
 // different banks.  (16-byte loads straight into the MFMA layout fetch 64 bytes of a row at a time, and a wave has nothing in flight while it
@@ -542,9 +542,13 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
 #define SKINNY_GO(T, NW, Z)                                                                                                              \
   hipLaunchKernelGGL((gemm_skinny_kernel<T, NW>), dim3((N + 15) / 16, offsets ? E : G, Z), dim3(64 * NW), 0, (hipStream_t)stream, (const T*)x, \
                      (const T*)w, y, M, N, K, epi, offsets, row_idx, idx_div < 1 ? 1 : idx_div, ldx, ldy, gsx, gsy, gc, dg)
-    // at most a workgroup per CU: eight waves, whose rings fill its LDS, as long as four have more than a run each (K = 1024: level)
+    // how many waves: a run of K is one wave's work, and four hold the LDS of four (2 workgroups to a CU instead of 8), so one wave for K <= 256, and for
+    // twice that where there are workgroups to go round (us, direct loads | four waves | one: 128 x 512 x 128 in a batch, one row 13.6 | 20.1 | 6.9,
+    // 64 x 512 x 512 12.8 | 13.3 | 8.5; 2048 x 512 3.2 | 3.4 | 3.9, two waves 3.5).  At most a workgroup per CU: eight waves, whose rings fill its LDS, as
+    // long as four have more than a run each (K = 1024: level).
     const long wgs = (long)((N + 15) / 16) * (offsets ? (M < E ? M : E) : G);          // those that have rows
-    if (wgs <= 256 && K > 1024) SKINNY_GO(bf16_t, 8, 1);
+    if (K <= 256 || (K <= 512 && wgs > 512)) SKINNY_GO(bf16_t, 1, 1);
+    else if (wgs <= 256 && K > 1024) SKINNY_GO(bf16_t, 8, 1);
     else SKINNY_GO(bf16_t, 4, 1);
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }

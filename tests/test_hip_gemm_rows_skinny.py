@@ -44,9 +44,11 @@ def test_rows_of_every_ring_shape(H, K, f32):
 
 
 @pytest.mark.parametrize("M,N,K,G", [(3, 4096, 1024, 1), (3, 4096, 1032, 1), (3, 4097, 1032, 1), (16, 4096, 2056, 1), (5, 4112, 2056, 1), (9, 2048, 4104, 2), (9, 2049, 4104, 2),
-                                     (4, 40, 1000, 3), (1, 8, 14720, 1)])
-def test_bf16_four_and_eight_waves(H, M, N, K, G):
-    """Both sides of the line between them, a workgroup per CU (256 of 16 features) and K = 1024, with the last run a part of one."""
+                                     (4, 40, 1000, 3), (1, 8, 14720, 1), (4, 50, 128, 3), (16, 33, 256, 2), (5, 33, 264, 2),
+                                     (7, 8192, 512, 1), (7, 8193, 512, 1), (16, 8208, 264, 1)])
+def test_bf16_one_four_and_eight_waves(H, M, N, K, G):
+    """Both sides of the lines between them -- 512 workgroups of 16 features and K = 256 or 512, 256 workgroups and K = 1024 -- with the last run a part of
+    one."""
     g = torch.Generator().manual_seed(M + N + K)
     w = (torch.randn(G, N, K, generator=g) / K ** 0.5).to(BF).cuda()
     x = torch.randn(M, G * K, generator=g).to(BF).cuda()
