@@ -982,11 +982,16 @@ extern "C" int ssd_winattn_paged(const void* q_rows, const void* k_cache, const 
   if (!f32 && max_q > 0 && D % 32 == 0 && D <= 256 && Dv % (out_freqs ? 32 : 16) == 0 && Dv <= 256 && block_size % 32 == 0 && G <= 65535 &&
       B <= 65535 && ldo % 4 == 0 && (uintptr_t)out_rows % 8 == 0) {
     const int R = H / G;
-    // 32 workgroups of 128 rows: fewer leave so much of the chip idle that the smaller units of the form below win (700 rows in 4 kv heads of 128
-    // behind a window of 100: 26 | 20 us; 300 tokens of 16 heads in 4: 29 | 33).  Heads of 64: 64 rows a workgroup as long as those of 128
-    // do not fill the chip (900 and 60 tokens of 16 heads in 4: 42 | 61 us; four of 1800 behind a window of 128: 42 | 36).
-    const long units = ((long)max_q * R + 127) / 128 * G * B;
-    if ((long)max_q * R > 256 && units >= 32 && (((uintptr_t)q_rows | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0 &&
+    // The prompt form from 192 workgroups of 128 rows on, and from 32 on where a row sees some hundred keys and more: fewer leave so much of the chip
+    // idle that the form below, with its smaller units, wins on short scans (MI355X, that form | this, us: 500 tokens of 8 heads in 8 behind 2000, heads
+    // of 128, window 64 16 | 25, 256 34 | 39, 512 56 | 58, none 236 | 198; 1000 of 32 in 8, none 172 | 74).  A window of fewer keys than a workgroup's
+    // tokens: its waves fetch what only the others need (3000 tokens of 16 in 16, heads of 64, window 64: 21 | 25).  Counted from all rows of the
+    // batch, not from its longest sequence.
+    // Heads of 64: 64 rows a workgroup as long as those of 128 do not fill the chip (900 and 60 tokens of 16 heads in 4: 42 | 61 us; four of
+    // 1800 behind a window of 128: 42 | 36).
+    const long units = ((long)T * R + 127) / 128 * G;
+    const bool prompt = units >= 192 ? window == 0 || (long)window * R >= 128 : units >= 32 && (window == 0 || window >= 512) && max_q >= 256;
+    if (prompt && (long)max_q * R > 256 && (((uintptr_t)q_rows | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0 &&
         (D == 64 || D == 128) && Dv <= 128) {
       const int rows = D == 64 && Dv <= 64 && units < 384 ? 64 : 128;
       const dim3 pg((unsigned)(((long)max_q * R + rows - 1) / rows), G, B);

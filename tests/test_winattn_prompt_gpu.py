@@ -16,13 +16,16 @@ CASES = [  # H, G, D, Dv, bs, window, keep, options
     (8, 1, 128, 80, 64, 300, 33, ("gate", "cap")),
     (4, 1, 128, 128, 32, 64, 0, ("freqs", "sink")),
     (4, 2, 64, 64, 64, 1, 0, ()),
-    (32, 8, 64, 64, 64, 0, 0, ("sink",)),             # 608 units of 128 rows: heads of 64 in workgroups of 128 rows
+    (32, 8, 64, 64, 64, 0, 0, ("sink",)),             # heads of 64 in workgroups of 128 rows, as the rows fill the chip
     (32, 8, 64, 48, 32, 200, 10, ("gate", "cap")),
+    (4, 4, 64, 64, 128, 177, 40, ("sink", "slopes", "cap")),
+    (4, 2, 64, 64, 64, 64, 0, ()),
 ]
 
 
+@pytest.mark.parametrize("fill", [False, True])          # a few hundred rows, most behind windows in the general form; 192 workgroups' worth, not
 @pytest.mark.parametrize("case", CASES)
-def test_against_fp64(case):
+def test_against_fp64(case, fill):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     from ssd_amd.hip import ops as K
@@ -30,7 +33,7 @@ def test_against_fp64(case):
     R = H // G
     g = torch.Generator().manual_seed(D + Dv + bs + window)
     rnd = lambda *s: torch.randn(*s, generator=g)
-    news, pasts = [128 // R + 1, 600, 65, 1], [0, 213, 700, 90]
+    news, pasts = [128 // R + 1, 192 // G * 128 // R if fill else 600, 65, 1], [0, 213, 700, 90]
     nb = sum(-(-(n + c) // bs) for n, c in zip(news, pasts)) + 1
     order = torch.randperm(nb, generator=g).tolist()
     kc = torch.full((nb, G, bs, D), float("nan")).to(BF)
@@ -84,21 +87,23 @@ def test_against_fp64(case):
             z = torch.cat([s, sinks.double().unsqueeze(1)], 1) if sinks is not None else s
             w = torch.softmax(z, 1)[:, :p + 1]
             o, mag = torch.einsum("hk,khv->hv", w, Vd[:p + 1]), torch.einsum("hk,khv->hv", w, Vd[:p + 1].abs())
+            turn = 0.0
             if freqs is not None:
                 a, hv = p * freqs.double(), Dv // 2
                 o = torch.cat([o[:, :hv] * a.cos() + o[:, hv:] * a.sin(), o[:, hv:] * a.cos() - o[:, :hv] * a.sin()], 1)
-                mag = (mag[:, :hv] + mag[:, hv:]).repeat(1, 2) + 2.0 ** -8       # (an angle of up to 800 in fp32: 800 * 2^-24 of the pair)
+                mag = (mag[:, :hv] + mag[:, hv:]).repeat(1, 2)
+                turn = (p + 1) * 2.0 ** -24 * mag                  # an angle of up to p in fp32 is off by up to p * 2^-24, and the sine and cosine by 2^-24
             if gate is not None:
                 f = torch.sigmoid(gate[t, :H * Dv].double()).view(H, Dv) * osc
                 o, mag = o * f, mag * f
             # bf16 has 8 significant bits: rounding moves a number by half a last place, at most 2^-8 of it.  Once for the output, once for every
             # weight (which their sum does not see), with 1e-4 for scores in fp32 and the hardware exponential
-            tol = 2.0 ** -8 * o.abs() + (2.0 ** -8 + 1e-4) * mag + 1e-5
+            tol = 2.0 ** -8 * o.abs() + (2.0 ** -8 + 1e-4) * mag + turn + 1e-5
             d = (out[t] - o).abs() - tol
             assert bool((d <= 0).all()), (case, b, i, float(d.max()))
 
 
-@pytest.mark.parametrize("H,G,D,Dv,window,keep", [(8, 2, 128, 128, 0, 0), (8, 2, 64, 64, 300, 20), (4, 1, 64, 128, 0, 0), (16, 4, 128, 64, 500, 0)])
+@pytest.mark.parametrize("H,G,D,Dv,window,keep", [(8, 2, 128, 128, 0, 0), (8, 2, 64, 64, 600, 20), (4, 1, 64, 128, 0, 0), (16, 4, 128, 64, 512, 0)])
 def test_single_tokens_beside_a_prompt(H, G, D, Dv, window, keep):
     """Decoded tokens in a prompt's batch give the bits that they give among themselves: the same keys over the same four waves."""
     if not torch.cuda.is_available():
