@@ -574,9 +574,12 @@ extern "C" int ssd_attn_paged(const void* q_rows, const void* k_cache, const voi
   // More than a workgroup's worth of causal rows per kv head: the throughput form (attention_prefill.hip) -- 42 -> 21 us at 512 tokens of 32 heads in
   // 8 groups, 25 -> 15 at 256 tokens of 64 heads.  (It also leads at 128 tokens, 13 -> 10 us; prompts of up to 160 tokens are
   // what the recorded full-size token streams start from, and another order of summation moves their near-ties: they stay with the form above.)
-  // (it scales after it has looked for the largest product, and masks before: scale > 0)
+  // A caller that asks for four waves and more has too few row tiles to fill the chip: the form above splits the keys of each over them, this one does
+  // not (MI355X, the form above | this, us: 8 heads in 1, 300 tokens, 6 waves 11 | 14, behind 4000 keys 64 | 121; 4 heads of 64 in 2, 400 tokens
+  // behind 1000, 8 waves 16 | 34; with 3 waves 16 | 13 .. 123 | 122, with 2 154 | 102; over 700 batches never slower with up to 3).
+  // (It scales after it has looked for the largest product, and masks before: scale > 0.)
   const int G = nh / nkv;
-  if (mode == 0 && splits == 1 && !(flags & 3) && max_q * G > PREFILL_ROWS && T >= PREFILL_MIN_TOKENS && scale > 0.f) {
+  if (mode == 0 && splits == 1 && !(flags & 3) && ((flags >> 8) & 0xf) <= 3 && max_q * G > PREFILL_ROWS && T >= PREFILL_MIN_TOKENS && scale > 0.f) {
     const PrefillAttn a = {p.q, p.kc, p.vc, block_tables, context_lens, cu_q, p.out_rows, p.out_frag, max_blocks, q_per_seq, nh, nkv, p.bs_shift,
                            p.scale_log2e};
     return attn_prefill_launch(a, B, max_q, hd, st);

@@ -68,6 +68,25 @@ def test_prompts(nh, nkv, hd, bs, new, old):
     assert torch.equal(back, rows)
 
 
+@pytest.mark.parametrize("waves", [0, 3, 4, 8])              # the throughput form up to three, the general one from four on
+def test_waves(waves):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ssd_amd.hip import ops as H
+    nh, nkv, hd, bs, new, c = 8, 1, 128, 64, 170, 1000
+    g = torch.Generator().manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(BF).cuda()
+    n = -(-c // bs)
+    q, K, V = rnd(new, nh, hd), rnd(n * bs, nkv, hd), rnd(n * bs, nkv, hd)
+    pages = lambda t: t.view(n, bs, nkv, hd).transpose(1, 2).contiguous()
+    rows = torch.full((new, nh * hd), 7.0, dtype=BF, device="cuda")
+    H.attn_paged(q, pages(K), pages(V), torch.arange(n, dtype=torch.int32, device="cuda").view(1, n), n, torch.tensor([c], dtype=torch.int32).cuda(), 1,
+                 new, new, nh, nkv, hd, bs, hd ** -0.5, cu_q=torch.tensor([0, new], dtype=torch.int32).cuda(), out_rows=rows, waves=waves)
+    ref = reference(q.double(), K[:c].double(), V[:c].double(), hd ** -0.5).flatten(1)
+    d = (rows.double() - ref).abs()
+    assert bool((d <= 2.0 ** -8 * ref.abs() + 2.0 ** -13).all()), float(d.max())          # (bounds as above)
+
+
 @pytest.mark.parametrize("scale,ctx,fixed", [
     (0.125, [0, 30, 200], True), (0.125, [0, 30, 200], False),       # a sequence without keys, one with fewer keys than rows
     (-0.125, [64, 70, 300], False), (0.0, [64, 64, 100], True)])      # scores that fall with the products; equal weights
