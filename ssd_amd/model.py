@@ -257,6 +257,7 @@ class HipDecoder:
     # ---------------------------------------------------------------------------------------------
     PF_MIN_WEIGHT_BYTES = 100 << 20
     PF_ALWAYS_WEIGHT_BYTES = 300 << 20
+    WIDE_OUTPUTS = 48 << 10
     BIG_MIN_ROWS = 160
     AP_WIDE_HEAD_BYTES = 1200 << 20
     PARTS_WIDE_WEIGHT_BYTES = 64 << 20
@@ -272,18 +273,21 @@ class HipDecoder:
     def _gemm_chunk(self, xf, K, w, N, y, m, ldy, epi, bias):
         """At most 128 token rows.  Up to 16: the skinny kernel, which a second 16-row token tile slows down where K is long.
         65..128: gemm_pf for a matrix of 100 MB and more (70B layer GEMMs 611 -> 383 us, 8B gate_up 83 -> 62 at 128 rows), the skinny kernel
-        below.  (The large-tile kernel also wins there for 16..100 MB -- 8B o_proj 26 -> 15 us -- but prompts of that length are what the
-        recorded full-size token streams start from, and another order of summation moves their near-ties.)
+        below.  (The large-tile kernel leads there for 16..100 MB, 8B o_proj 26 -> 15 us, in another order of summation: see _gemm.)
         17..64, by the weight's size (MI355X, us: skinny | gemm_pf | gemm_big): gemm_pf from 300 MB (64 rows of 70B gate_up 248 | 144 | 168; 32
         rows 153 | 139 | 164, down_proj 119 | 80 | 86, 32B gate_up 95 | 86 | 96); the large-tile kernel with its K splits from 16 MB (64 rows of
         8B gate_up 71 | 49 | 45, down_proj 51 | 32 | 28, o_proj 17 | 17 | 14, 1B down_proj 28 | 18 | 14; 32 rows of 8B down_proj
         34 | 29 | 26, 70B o_proj 39 | 31 | 31, 32B qkv 34 | 32 | 27), up to 32 rows not for gate_up, whose K is short (8B 44 | 48 | 51);
-        the skinny one for what it reads in one go (64 rows of 1B qkv 11 | 13 | 11; 4096 x 1024 8 | 12 | 10)."""
-        size = 2 * N * K
-        if m > 16 and self._pf_eligible(N, K) and (m > 64 or size >= self.PF_ALWAYS_WEIGHT_BYTES):
+        the skinny one for what it reads in one go (64 rows of 1B qkv 11 | 13 | 11; 4096 x 1024 8 | 12 | 10).
+        Up to 32 rows the skinny kernel also keeps a gate_up that gemm_pf has to split along K (two shards of 70B, 28672 x 8192: 85 | 89 | 93,
+        16384 x 14336 79 | 94 | 87; 51200 rows fill the chip unsplit), a vocabulary over a short K (128256 x 2048 91 | 99 | --, 51200 x 1536
+        30 | 30 | 32) and eight shards' o_proj, 8192 x 1024 (8 | 11 | 9)."""
+        size, rows, wide = 2 * N * K, epi == H.EPI_ROWS, N >= self.WIDE_OUTPUTS
+        short = wide and K <= 2048 if rows else not wide                    # (up to 32 rows: what gemm_pf does not lead at)
+        if m > 16 and self._pf_eligible(N, K) and (m > 64 or size >= self.PF_ALWAYS_WEIGHT_BYTES and (m > 32 or not short)):
             assert self._ws_pf is not None and self._ws_pf.numel() * 4 >= H.gemm_pf_workspace_bytes(128, N, K), (N, K)
             H.gemm_pf(xf, w, y, m, N, K, ldy, self._ws_pf, epilogue=epi, bias=bias)
-        elif 16 < m <= 64 and K >= 96 and size >= self.BIG_MIN_WEIGHT_BYTES and (m > 32 or epi == H.EPI_ROWS):
+        elif 16 < m <= 64 and K >= 96 and size >= self.BIG_MIN_WEIGHT_BYTES and (m > 32 or rows and not short and (K > 1024 or N > 8192)):
             H.gemm_big(xf, w, y, m, N, K, ldy, epi, bias, self._ws_big)
         else:
             H.gemm(xf, w, y, m, N, K, ldy, epi, bias)

@@ -44,6 +44,32 @@ def test_wide_down_projections_leave_the_slabs_at_two_token_tiles():
         assert [d.parts_plan(T) for T in (1, 16, 17, 32, 33)] == [True, True, rows == 32, rows == 32, False], (h, I)
 
 
+def test_kernels_of_17_to_128_rows(monkeypatch):
+    """Which GEMM a chunk of m rows of an N x K matrix takes: where the measured lines lie (HipDecoder._gemm_chunk)."""
+    import torch
+    import ssd_amd.model as M
+    took = []
+    for n in ("gemm", "gemm_pf", "gemm_big"):
+        monkeypatch.setattr(M.H, n, lambda *a, n=n, **k: took.append(n))
+    monkeypatch.setattr(M.H, "gemm_pf_workspace_bytes", lambda *a: 0)
+    d = HipDecoder.__new__(HipDecoder)
+    d._ws_pf = d._ws_big = torch.zeros(1)
+    rows, silu = M.H.EPI_ROWS, M.H.EPI_SILU_FRAG
+    S, P, B = "gemm", "gemm_pf", "gemm_big"
+    for N, K, epi, want in (                                  # m = 16, 17, 32, 33, 64, 65
+            (4096, 14336, rows, (S, B, B, B, B, P)), (28672, 4096, silu, (S, S, S, B, B, P)),              # 8B down, gate_up
+            (4096, 4096, rows, (S, B, B, B, B, S)), (3072, 2048, rows, (S, S, S, S, S, S)),                # 8B o, 1B qkv
+            (57344, 8192, silu, (S, P, P, P, P, P)), (28672, 8192, silu, (S, S, S, P, P, P)),              # 70B gate_up, of two shards
+            (14336, 8192, silu, (S, S, S, B, B, P)), (8192, 28672, rows, (S, P, P, P, P, P)),              # of four; 70B down
+            (8192, 1024, rows, (S, S, S, B, B, S)), (51200, 5120, silu, (S, P, P, P, P, P)),               # 70B o of eight; 32B gate_up
+            (128256, 2048, rows, (S, S, S, P, P, P)), (151936, 5120, rows, (S, P, P, P, P, P)),            # heads of 1B and 32B
+            (16384, 512, rows, (S, B, B, B, B, S)), (256, 64, rows, (S, S, S, S, S, S))):
+        took.clear()
+        for m in (16, 17, 32, 33, 64, 65):
+            d._gemm_chunk(None, K, None, N, None, m, N, epi, None)
+        assert tuple(took) == want, (N, K, epi, took)
+
+
 def test_peaky_recipe_scales_the_same_tokens_in_target_and_eagle_draft():
     """bench.py --workload c4e builds its EAGLE pair with the "peaky" recipe (ssd_amd/weights.py peaky_rows): the LM-head rows
     of the same few tokens -- draft-vocabulary ids pushed through the draft's d2t -- are scaled in BOTH models, everything
