@@ -572,8 +572,9 @@ extern "C" int ssd_attn_paged(const void* q_rows, const void* k_cache, const voi
   p.ow = nullptr; p.oparts = nullptr; p.oN = 0;
   hipStream_t st = (hipStream_t)stream;
   // More than a workgroup's worth of causal rows per kv head: the throughput form (attention_prefill.hip) -- 42 -> 21 us at 512 tokens of 32 heads in
-  // 8 groups, 25 -> 15 at 256 tokens of 64 heads.  (It also leads at 128 tokens, 13 -> 10 us; prompts of up to 160 tokens are
-  // what the recorded full-size token streams start from, and another order of summation moves their near-ties: they stay with the form above.)
+  // 8 groups, 25 -> 15 at 256 tokens of 64 heads.  It also leads at 128 tokens, 13 -> 10 us: what keeps it from batches of up to 160 tokens is
+  // that the tests' full-size token streams start from single prompts of that length and have near ties there, which another order of
+  // summation moves.
   // A caller that asks for four waves and more has too few row tiles to fill the chip: the form above splits the keys of each over them, this one does
   // not (MI355X, the form above | this, us: 8 heads in 1, 300 tokens, 6 waves 11 | 14, behind 4000 keys 64 | 121; 4 heads of 64 in 2, 400 tokens
   // behind 1000, 8 waves 16 | 34; with 3 waves 16 | 13 .. 123 | 122, with 2 154 | 102; over 700 batches never slower with up to 3).

@@ -1,4 +1,5 @@
-// Prefill GEMM  y[M,N] = x[M,K] . W[N,K]^T  for 32 < M <= 128 token rows (one prefill chunk).  Replaces the cuBLAS
+// Prefill GEMM  y[M,N] = x[M,K] . W[N,K]^T  for 16 < M <= 128 token rows (one prefill chunk; a decoding batch
+// of 17 to 64 rows of a large matrix).  Replaces the cuBLAS
 // F.linear calls of the reference's eager prefill (ssd/layers/linear.py:65,98,196; model_runner.py:602).
 //
 // Still HBM-bound on MI355X (128 FLOP/B against a ridge of ~312), but unlike the skinny kernel (gemm.hip) the x

@@ -390,7 +390,7 @@ gemm_skinny_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __res
 // bytes, the MFMA operand itself, ran at 60 % -- and lane l fetches chunk (l & 7) ^ (l >> 3) of row l >> 3, so that the eight lanes which an LDS
 // read serves at a time find their chunks in different banks.  The rows of a grouped product are gathered by the same loads.  The
 // accumulators go through LDS once more, 16 or 32 token rows at a time: a wave then stores whole runs of a row, whatever the epilogue.
-// Bound by the matrix cores.  MI355X, against the 64 x 64 form below (which re-stages both operands through registers, two barriers per 32-wide
+// Bound by the matrix cores.  MI355X, against the 64 x 64 form above (which re-stages both operands through registers, two barriers per 32-wide
 // k-step): 4000 x 14720 x 4096 1516 -> 418 us (1150 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 35.
 // (The 256 x 256 tile runs sixteen waves of 64 x 64: with eight of 128 x 64 the first took 452 us.)
 // ---------------------------------------------------------------------------------------------------------------------

@@ -1,11 +1,13 @@
 // The main loop of the large-tile bf16 GEMMs (many token rows: prefill): a workgroup owns (WN * NT) 16-row groups of W and (WM * MT)
 // 16-row groups of x, its WN x WM waves NT x MT of them each, and leaves the fp32 products in acc[NT][MT].
 //
-// What bounds it is the matrix cores, as long as they are fed: a wave with 8 x 4 accumulator tiles reads 12 KiB of LDS per 32 MFMAs
-// (96 of the 128 bytes a CU's LDS delivers per cycle), so both operands travel HBM / L2 -> LDS by DMA (loads to LDS: no registers, no
-// LDS write instructions), 1 KiB per instruction, into a ring of STAGES steps of KS x 32 k.  A step's loads are issued STAGES - 1 steps
-// ahead, and ONE barrier per step both publishes the step and frees the buffer of the one before.
-// Every accumulator is one chain over ascending k, whatever the tile: a row's result does not depend on the rows beside it.
+// What bounds it is the matrix cores and the LDS that feeds them: a wave with 4 x 4 accumulator tiles reads 8 KiB of LDS per 16 MFMAs of 16x16x32
+// (16 cycles each), so that at full rate the four SIMDs take 32 KiB in 256 cycles, all of the 128 bytes a CU's LDS delivers per cycle; 3 x 3
+// tiles ask for a third more than that, 4 x 2 for half as much again.  Both operands therefore travel HBM / L2 -> LDS by DMA (loads to LDS: no
+// registers, no LDS write instructions), 1 KiB per instruction, into a ring of STAGES steps of KS x 32 k.  A step's loads are issued
+// STAGES - 1 steps ahead, and ONE barrier per step both publishes the step and frees the buffer of the one before.
+// In bf16 every accumulator is one chain over the ascending k of the range that its workgroup walks, whatever the tile: where the caller does not cut K
+// (gemm_rows.hip), a row's result does not depend on the rows beside it; ssd_gemm_big's K splits go by the number of rows.  fp32: see below.
 #pragma once
 #include "common.h"
 

@@ -308,10 +308,11 @@ class HipDecoder:
         return S
 
     def _gemm(self, xf, K, w, N, y, T, ldy, epi=H.EPI_ROWS, bias=None):
-        # (up to BIG_MIN_ROWS, and a couple of hundred rows of a matrix under 1 MB -- models of a few hundred channels --, prompts walk the
-        #  128-row kernels: the recorded full-size token streams restart from prompts of up to 160 tokens, and another order of summation moves
-        #  their near-ties.  The large-tile kernel leads there too: 130 rows of 8B qkv 42 -> 24 us, of a 512 x 256 toy 9 -> 5.  K < 96: fewer
-        #  k-steps than a ring has stages)
+        # The large-tile kernel from BIG_MIN_ROWS token rows of the batch on, and for matrices under 1 MB (models of a few hundred channels) from 256.
+        # It leads below as well: 130 rows of 8B qkv 42 -> 24 us, of a 512 x 256 toy 9 -> 5.  What keeps it out is the tests' full-size token streams,
+        # which compare tokens that restart from single prompts of up to 160 tokens, and have near ties there that another order of
+        # summation moves; no property of a sequence hangs on it (two prompts of 100 tokens take it, and the last rows of a prompt of
+        # 145 .. 160 take what _gemm_chunk gives 17 .. 32 rows).  K < 96: fewer k-steps than a ring has stages.
         if T > self.BIG_MIN_ROWS and K >= 96 and (T > 256 or 2 * N * K >= self.BIG_SMALLEST_WEIGHT_BYTES):
             H.gemm_big(xf, w, y, T, N, K, ldy, epi, bias, self._ws_big)
             return
