@@ -173,8 +173,9 @@ class HipDecoder:
         # LM-head argmax candidates (csrc/gemm.hip EPI_ROWS_ARGMAX): one (value, index) per token row and workgroup, finished
         # by ssd_argmax_parts* -- on the greedy path for up to 32 logit rows (decode / verify / tree step)
         self.argmax_fused = True
-        # (a head of 1.2 GB and more: up to 16 rows.  From there gemm_pf + the argmax of its rows is faster: 151936 x 5120, 32 rows: 314 us with
-        #  candidates, 253 + 13 without)
+        # (a head of 1.2 GB and more: up to 16 rows.  From there gemm_pf + the argmax of its rows is faster -- MI355X, 32 | 17 rows, candidates -> rows: 151936 x
+        #  5120 321 | 295 -> 271 | 262 us, 128256 x 5120 267 | 247 -> 223 | 216, 128256 x 8192 411 | 378 -> 350 | 342; close at 151936 x 4096, 1187 MiB, 253 |
+        #  235 -> 235 | 229, level at 128256 x 4096 212 | 196 -> 204 | 199, the other way at 128256 x 2048 105 | 100 -> 112 | 112)
         self.ap_rows = min(self.max_logit_rows, 32 if 2 * self.V * self.h < self.AP_WIDE_HEAD_BYTES else 16)
         self.ap_stride = max(H.gemm_argmax_nparts(m, self.V, self.h) for m in ({1, self.ap_rows} if self.ap_rows > 16 else {1}))
         self.ap_val = z(self.ap_rows, self.ap_stride, dtype=torch.float32)
