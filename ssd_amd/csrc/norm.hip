@@ -41,7 +41,8 @@ __device__ __forceinline__ int norm_row() {
 }
 
 // NORM_MAXC: 8-element chunks of a thread.  The sum of squares runs over a thread's chunks, a wave's lanes, the waves, each in order: waves without
-// a chunk add zeros, so H = 4096 needs 512 of the 1024 threads of its class, and the same bits come out.
+// a chunk add zeros, so H = 4096 needs 512 of the 1024 threads of its class, and the same bits come out.  (2900 x 2048 21.0 -> 14.6 us; with the
+// order of the rows 2163 x 4096 33.7 -> 19.3, 4000 x 8192 86 -> 55.)
 template <int NORM_THREADS, int NORM_MAXC, bool PARTS>
 __global__ void __launch_bounds__(NORM_THREADS)
 rmsnorm_kernel(const u32x4_t* __restrict__ x, const u32x4_t* __restrict__ res_in, u32x4_t* __restrict__ res_out,

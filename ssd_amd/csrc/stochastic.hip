@@ -119,8 +119,8 @@ extern "C" int ssd_topk_rows(const void* logits, long ld, int T, int V, int k, i
 constexpr int SAMPLE_THREADS = 256, SAMPLE_DIRECT_VOCAB = 8192;
 
 // One workgroup per row takes 0.6 ns per candidate as long as each has a CU to itself, 1.1 ns with two to a CU, and starts over after 512 rows; slices
-// spread all candidates evenly, 0.0020 ns each (0.0023 from unaligned rows), behind two more launches (3.4 us).  (MI355X, us, direct | slices: 256 rows of 16000 12 | 14, of 128256
-// 76 | 70; 192 of 8200 8 | 10, of 32000 21 | 18; 512 of 8200 12 | 15, of 50257 62 | 70; 300 of 32000 38 | 26.)
+// spread all candidates evenly, 0.0020 ns each (0.0023 from unaligned rows), behind two more launches (3.4 us).  (MI355X, us, direct | slices: 256 rows of
+// 16000 12 | 14, of 128256 76 | 70; 192 of 8200 8 | 10, of 32000 21 | 18; 512 of 8200 12 | 15, of 50257 62 | 70; 300 of 32000 38 | 26.)
 static bool sample_direct(int T, int V, bool aligned) {
   const int rest = T % 512;
   const double row = 1.1e-3 * (T / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.6e-3 : 1.1e-3);
