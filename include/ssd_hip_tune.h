@@ -24,8 +24,8 @@ int ssd_gemm_pf_cfg(const void* x_frag, const void* w_frag, const void* bias, vo
                     int epilogue, void* workspace, int64_t workspace_bytes, int nt, int splits, void* stream);
 
 
-/* ssd_gemm_big with an explicit decomposition: shape = 0 256 x 128, 1 128 x 256, 2 128 x 128, 3 128 x 64, 4 256 x 256 (features x tokens), splits of K
- * (1..8, at least three k-steps of 32 each). */
+/* ssd_gemm_big with an explicit decomposition: shape = 0 256 x 128, 1 128 x 256, 2 128 x 128, 3 128 x 64, 4 256 x 256, 5 256 x 224, 6 256 x 192, 7 256 x 160,
+ * 8 192 x 192, 9 192 x 160, 10 192 x 128 (features x tokens; 8 .. 10 not with SSD_EPI_SILU_FRAG), splits of K (1..8, at least three k-steps of 32 each). */
 int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
                      void* workspace, int64_t workspace_bytes, int shape, int splits, void* stream);
 

@@ -4,9 +4,9 @@
 // The <= 128-row kernels (gemm.hip, gemm_pf.hip) are built to stream W once per launch, so a prompt of T rows streamed every matrix
 // T / 128 times, and matrices under 100 MB ran the skinny kernel at 128 rows (150 TFLOP/s).  Here the products are bound by the matrix
 // cores (gemm_tile.h).  Measured on MI355X, us per product, 128-row chunks -> this kernel:
-//   T = 2594 (Llama-3.2-1B): qkv 3072 x 2048  530 -> 36, gate_up 16384 x 2048  570 -> 160, down 2048 x 8192  960 -> 100
-//   T = 2163 (Llama-3.1-8B): qkv 6144 x 4096  460 -> 110, gate_up 28672 x 4096  875 -> 440, down 4096 x 14336  590 -> 300
-//   T = 16384 (8B): gate_up 6900 -> 2900 (1330 TFLOP/s), down 4600 -> 1400
+//   T = 2594 (Llama-3.2-1B): qkv 3072 x 2048  530 -> 35, gate_up 16384 x 2048  570 -> 149, down 2048 x 8192  960 -> 90
+//   T = 2163 (Llama-3.1-8B): qkv 6144 x 4096  460 -> 94, gate_up 28672 x 4096  875 -> 410, down 4096 x 14336  590 -> 225
+//   T = 16384 (8B): gate_up 6900 -> 2740 (1400 TFLOP/s), down 4600 -> 1355
 #include "common.h"
 #include "gemm_tile.h"
 
@@ -15,7 +15,7 @@ enum { BIG_ROWS = 0, BIG_SILU_FRAG = 1, BIG_PARTS = 2 };
 namespace {
 
 template <int WN, int WM, int NT, int MT, int STAGES, int EPI>
-__global__ void __launch_bounds__(64 * WN * WM, WN * WM <= 8 ? 2 : 4)
+__global__ void __launch_bounds__(64 * WN * WM, 2)
 gemm_big_kernel(const char* __restrict__ Wf, const char* __restrict__ Xf, const bf16_t* __restrict__ bias, void* __restrict__ Yv, int M, int N,
                 int K, int ldy, int tn, int tm, int splits) {
   typedef TileLoop<WN, WM, NT, MT, STAGES> L;
@@ -29,7 +29,7 @@ gemm_big_kernel(const char* __restrict__ Wf, const char* __restrict__ Xf, const 
   uint32_t soff[L::PER];
 #pragma unroll
   for (int i = 0; i < L::PER; ++i) {
-    const int c = wave * L::PER + i;
+    const int c = L::op_of(wave, i);
     soff[i] = (uint32_t)(c < L::WG ? min(c, gl - g0) : min(c - L::WG, hl - h0)) * (uint32_t)KT * 1024u + (uint32_t)kb * 1024u;
   }
   const auto wr = tile_rsrc(Wf + (size_t)g0 * KT * 1024, (uint32_t)(min(L::WG, gl + 1 - g0) * KT) * 1024u);
@@ -37,7 +37,7 @@ gemm_big_kernel(const char* __restrict__ Wf, const char* __restrict__ Xf, const 
   f32x4_t acc[NT][MT];
   const uint32_t at[1] = {(uint32_t)lane * 16u};
   L::run(smem, nk, at, acc, [&](int i, int step, char* lds) {
-    tile_dma(wave * L::PER + i < L::WG ? wr : xr, lane * 16, soff[i] + (uint32_t)step * 1024u, lds);
+    tile_dma(L::op_of(wave, i) < L::WG ? wr : xr, lane * 16, soff[i] + (uint32_t)step * 1024u, lds);
   });
 
   const int wn = wave / WM, wm = wave % WM;
@@ -140,7 +140,7 @@ int go(const void* x, const void* w, const void* bias, void* y, int M, int N, in
                      (const char*)x, (const bf16_t*)bias, OUT, M, N, K, ldy, tn, tm, splits)
   if (splits > 1) GO(BIG_PARTS, ws);
   else if (epilogue == BIG_ROWS) GO(BIG_ROWS, y);
-  else GO(BIG_SILU_FRAG, y);
+  else if constexpr (NT % 2 == 0) GO(BIG_SILU_FRAG, y);          // (the others never get here: ssd_gemm_big_cfg)
 #undef GO
   if (hipGetLastError() != hipSuccess) return SSD_ERR_LAUNCH;
   if (splits > 1) {
@@ -153,33 +153,40 @@ int go(const void* x, const void* w, const void* bias, void* y, int M, int N, in
   return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
 }
 
-// Tile shapes (features x tokens) and what a k-step of 32 takes when n workgroups share a CU, in us (MI355X, operands not in the caches; fits
-// of T = 130 .. 16384 over the 1B / 8B / 70B matrices).  Large tiles read less of L2 and LDS per product -- 256 x 256 on sixteen waves reaches
-// 1.4 PFLOP/s where 256 x 128 on eight stays at 1.28 (16384 x 4096 x 14336: 1390 | 1510 us), but is alone on its CU while it starts and stores
-// (K = 2048 gains nothing) --; small ones leave fewer CUs idle.
-struct Shape { int features, tokens; float step[3], full, ends; };       // step[n - 1] for n <= 3 workgroups on a CU, n * full beyond; filling the ring, storing
-constexpr Shape SHAPES[] = {{256, 128, {0.46f, 0.85f, 1.27f}, 0.42f, 1.0f},
-                            {128, 256, {0.46f, 0.85f, 1.27f}, 0.43f, 1.0f},
-                            {128, 128, {0.29f, 0.44f, 0.75f}, 0.26f, 1.0f},
-                            {128, 64, {0.21f, 0.31f, 0.54f}, 0.20f, 1.0f},
-                            {256, 256, {0.68f, 1.55f, 2.35f}, 0.79f, 4.0f}};
+// Tile shapes (features x tokens) and what a k-step of 32 takes when the fullest CU has n workgroups of it to run, in us (MI355X, operands not in the
+// caches; fits of 900 timings, T = 48 .. 16384 over the 1B / 3B / 8B matrices, rms 9 %).  The largest has the highest rate; a product of a few rounds
+// of tiles is decided by how full the last round is, so there is a shape for every 32 tokens: 2594 x 16384 x 2048 as 768 tiles of 256 x 224, three rounds,
+// 149 us, as 704 of 256 x 256 163; 2163 x 4096 x 14336 in one round of 224 tiles of 256 x 160 225, of 144 256 x 256 tiles 257; 2594 x 2048 x 2048 as 231 of
+// 192 x 128 26, as 336 of 128 x 128 30.  Tiles of 192 features cut (gate, up) pairs of 16-row groups between waves, so gate_up has none of them.
+struct Shape { int features, tokens; float step[3], full, ends; };       // step[n - 1] for n <= 3 workgroups, n * full beyond; filling the ring, storing
+constexpr int SHAPE_COUNT = 11;
+constexpr Shape SHAPES[SHAPE_COUNT] = {{256, 128, {0.435f, 0.796f, 1.225f}, 0.459f, 1.95f}, {128, 256, {0.398f, 0.790f, 1.161f}, 0.460f, 1.63f},
+                                       {128, 128, {0.273f, 0.461f, 0.668f}, 0.228f, 1.40f}, {128, 64, {0.21f, 0.31f, 0.54f}, 0.20f, 1.0f},
+                                       {256, 256, {0.632f, 1.361f, 2.163f}, 0.761f, 2.14f}, {256, 224, {0.601f, 1.225f, 1.967f}, 0.675f, 1.64f},
+                                       {256, 192, {0.536f, 1.078f, 1.632f}, 0.618f, 1.51f}, {256, 160, {0.506f, 0.987f, 1.540f}, 0.554f, 1.23f},
+                                       {192, 192, {0.419f, 0.815f, 1.257f}, 0.492f, 2.22f}, {192, 160, {0.382f, 0.768f, 1.063f}, 0.449f, 1.83f},
+                                       {192, 128, {0.344f, 0.634f, 0.954f}, 0.356f, 2.36f}};
 struct Plan { int shape, splits; };
 
 // The shape and the number of K splits with the least estimated time: k-steps of the fullest CU, plus, for a split product, a launch
 // (5 us) and its slabs' way to memory and back.  A product with fewer tiles than CUs gains from splits as long as the slabs stay small:
-// 500 x 4096 x 14336 runs 134 us unsplit (128 workgroups), 69 us in four (measured), 99 us as 64-token tiles.
-Plan pick(int M, int N, int K, long ws_bytes) {
+// 800 x 4096 x 14336 runs 117 us unsplit (224 tiles of 128 x 128), 105 in two splits of 112 tiles of 256 x 128.  Over the products timed the choice is
+// 0.4 % slower than the best of all shapes and splits (the lines of before, on four shapes: 8 %).
+Plan pick(int M, int N, int K, int epilogue, long ws_bytes) {
   Plan best{0, 1};
   float least = 1e30f;
-  for (int c = 0; c < 5; ++c)
+  for (int c = 0; c < SHAPE_COUNT; ++c) {
+    if (epilogue == BIG_SILU_FRAG && SHAPES[c].features == 192) continue;
     for (int s = 1; s <= 8; ++s) {
       const int steps = (K / 32 + s - 1) / s;
       if (s > 1 && (steps < 8 || (long)s * M * N * 4 > ws_bytes)) break;
       const long tiles = (long)((N + SHAPES[c].features - 1) / SHAPES[c].features) * ((M + SHAPES[c].tokens - 1) / SHAPES[c].tokens) * s;
       const long n = (tiles + 255) / 256;
-      const float est = steps * (n <= 3 ? SHAPES[c].step[n - 1] : n * SHAPES[c].full) + n * SHAPES[c].ends + (s > 1 ? 5.0f + (float)s * M * N * 8 / 5e6f : 0.f);
+      const float run = steps * (n <= 3 ? SHAPES[c].step[n - 1] : n * SHAPES[c].full) + n * SHAPES[c].ends;
+      const float est = run + (s > 1 ? 5.0f + (float)s * M * N * 8 / 5e6f : 0.f);
       if (est < least) { least = est; best = Plan{c, s}; }
     }
+  }
   return best;
 }
 
@@ -191,21 +198,29 @@ extern "C" int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const vo
   if (epilogue != BIG_ROWS && epilogue != BIG_SILU_FRAG) return SSD_ERR_ARG;
   if (M <= 0 || N <= 0 || K < 64 || N % 16 || K % 32 || (epilogue == BIG_SILU_FRAG && N % 64) || K > (1 << 22)) return SSD_ERR_SHAPE;
   if (epilogue == BIG_ROWS && (ldy < N || ldy % 4)) return SSD_ERR_SHAPE;
-  if (shape < 0 || shape > 4 || splits < 1 || splits > 8 || K / 32 / splits < 3) return SSD_ERR_ARG;
+  if (shape < 0 || shape >= SHAPE_COUNT || (epilogue == BIG_SILU_FRAG && SHAPES[shape].features == 192) || splits < 1 || splits > 8 || K / 32 / splits < 3) return SSD_ERR_ARG;
   if (splits > 1 && (!workspace || workspace_bytes < (int64_t)splits * M * N * 4)) return SSD_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
 #define BIG_ARGS x_frag, w_frag, bias, y, M, N, K, ldy, epilogue, splits, workspace, st
-  if (shape == 0) return go<4, 2, 4, 4, 3>(BIG_ARGS);
-  if (shape == 1) return go<2, 4, 4, 4, 3>(BIG_ARGS);
-  if (shape == 2) return go<2, 2, 4, 4, 3>(BIG_ARGS);
-  if (shape == 3) return go<2, 2, 4, 2, 4>(BIG_ARGS);
-  return go<4, 4, 4, 4, 4>(BIG_ARGS);
+  switch (shape) {
+    case 0: return go<4, 2, 4, 4, 5>(BIG_ARGS);
+    case 1: return go<2, 4, 4, 4, 5>(BIG_ARGS);
+    case 2: return go<2, 2, 4, 4, 4>(BIG_ARGS);
+    case 3: return go<2, 2, 4, 2, 4>(BIG_ARGS);
+    case 4: return go<4, 2, 4, 8, 5>(BIG_ARGS);
+    case 5: return go<4, 2, 4, 7, 5>(BIG_ARGS);
+    case 6: return go<4, 2, 4, 6, 5>(BIG_ARGS);
+    case 7: return go<4, 2, 4, 5, 5>(BIG_ARGS);
+    case 8: return go<4, 2, 3, 6, 5>(BIG_ARGS);
+    case 9: return go<4, 2, 3, 5, 5>(BIG_ARGS);
+    default: return go<4, 2, 3, 4, 5>(BIG_ARGS);
+  }
 #undef BIG_ARGS
 }
 
 extern "C" int ssd_gemm_big(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
                             void* workspace, int64_t workspace_bytes, void* stream) {
   if (M <= 0 || N <= 0 || K < 96) return SSD_ERR_SHAPE;
-  const Plan p = pick(M, N, K, workspace ? workspace_bytes : 0);
+  const Plan p = pick(M, N, K, epilogue, workspace ? workspace_bytes : 0);
   return ssd_gemm_big_cfg(x_frag, w_frag, bias, y, M, N, K, ldy, epilogue, workspace, workspace_bytes, p.shape, p.splits, stream);
 }

@@ -388,14 +388,12 @@ gemm_skinny_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __res
 // Large-tile form (bf16, K % 64 == 0; fp32, K % 32 == 0; 16-byte aligned rows, more rows than the skinny form takes: prompts, larger batches): the main loop
 // of gemm_tile.h over row-major operands, k-steps of 64.  An operand's DMA covers 8 rows x 128 bytes -- whole cache lines; 16 rows x 64
 // bytes, the MFMA operand itself, ran at 60 % -- and lane l fetches chunk (l & 7) ^ (l >> 3) of row l >> 3, so that the eight lanes which an LDS
-// read serves at a time find their chunks in different banks.  The rows of a grouped product are gathered by the same loads.  The
-// accumulators go through LDS once more, 16 or 32 token rows at a time: a wave then stores whole runs of a row, whatever the epilogue.
+// read serves at a time find their chunks in different banks.  The rows of a grouped product are gathered by the same loads.
 // Bound by the matrix cores.  MI355X, against the 64 x 64 form above (which re-stages both operands through registers, two barriers per 32-wide
-// k-step): 4000 x 14720 x 4096 1516 -> 418 us (1150 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 35.
-// (The 256 x 256 tile runs sixteen waves of 64 x 64: with eight of 128 x 64 the first took 452 us.)
+// k-step): 4000 x 14720 x 4096 1516 -> 410 us (1180 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 38.
 // ---------------------------------------------------------------------------------------------------------------------
 template <typename T, int WN, int WM, int NT, int MT, int STAGES, bool GROUPED>
-__global__ void __launch_bounds__(64 * WN * WM, WN * WM <= 8 ? 2 : 4)
+__global__ void __launch_bounds__(64 * WN * WM, 2)
 gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
                       const int* __restrict__ offsets, int E, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx,
                       long gsy, GluClamp gc, DecayGate dg, int tn, int tm, bool vec_out) {
@@ -412,7 +410,7 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
   const T* wg = w + (size_t)blockIdx.y * N * K;
   x += (size_t)blockIdx.y * gsx;
   const long ycol = (long)blockIdx.y * gsy;
-  if constexpr (GROUPED) {
+  if (GROUPED && offsets) {
     int tile = t.m, e = 0;
     for (; e < E; ++e) {
       const int nt = (offsets[e + 1] - offsets[e] + L::XG * 16 - 1) / (L::XG * 16);
@@ -426,26 +424,59 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
   }
   // (rows past the edge read the last row again: their products are never stored)
   const auto wr = tile_rsrc(wg + (size_t)n0 * K, (uint32_t)min(L::WG * 16, N - n0) * (uint32_t)K * ROWB);
-  uint32_t woff[L::PER];
-  const T* xp[L::PER];
+  const auto xr = tile_rsrc(x + (size_t)row0 * ldx, GROUPED ? 0u : (uint32_t)min(L::XG * 16, row_end - row0) * (uint32_t)ldx * ROWB);
+  uint32_t off[L::PER];                // from wr or xr
+  const T* xp[GROUPED ? L::PER : 1];
 #pragma unroll
   for (int i = 0; i < L::PER; ++i) {
-    const int c = wave * L::PER + i, r = (c & 1) * 8 + (lane >> 3), k8 = (lane & 7) ^ (lane >> 3);
-    woff[i] = (uint32_t)min((c >> 1) * 16 + r, N - 1 - n0) * (uint32_t)K * ROWB + k8 * 16;
-    const int m = min(row0 + ((c >> 1) < L::WG ? 0 : (c >> 1) - L::WG) * 16 + r, row_end - 1);
-    xp[i] = x + (GROUPED && row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx + k8 * VEC;
+    const int c = L::op_of(wave, i), r = (c >> 1) * 16 + (c & 1) * 8 + (lane >> 3), k8 = (lane & 7) ^ (lane >> 3);
+    const int m = min(row0 + r - L::WG * 16, row_end - 1);
+    off[i] = (r < L::WG * 16 ? (uint32_t)min(r, N - 1 - n0) * (uint32_t)K : (uint32_t)(m - row0) * (uint32_t)ldx) * ROWB + k8 * 16;
+    if constexpr (GROUPED) xp[i] = r < L::WG * 16 ? x : x + (row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx + k8 * VEC;
   }
   const uint32_t at0 = (uint32_t)(((lane >> 3) & 1) * 1024 + ((lane & 7) * 8 + ((lane >> 4) ^ (lane & 7))) * 16), at[2] = {at0, at0 ^ 64u};
   f32x4_t acc[NT][MT];
   L::run(smem, K / (8 * VEC), at, acc, [&](int i, int step, char* lds) {
-    if (wave * L::PER + i < 2 * L::WG)
-      tile_dma(wr, woff[i], (uint32_t)step * 128u, lds);
+    const bool of_w = L::op_of(wave, i) < 2 * L::WG;
+    if (!GROUPED || of_w)
+      tile_dma(of_w ? wr : xr, off[i], (uint32_t)step * 128u, lds);
     else
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp[i] + step * 8 * VEC), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp[GROUPED ? i : 0] + step * 8 * VEC), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
   });
-  __syncthreads();
 
   const int wn = wave / WM, wm = wave % WM;
+  // Whole rows of four outputs without a function of them: straight from the accumulators (a wave's store fills 32 or 64 bytes of sixteen rows).  Code
+  // that unrolls over the accumulators has to stay short -- a workgroup runs it once, out of a cold instruction cache: with every epilogue in it
+  // the kernel took 12 us longer --, so the others go through LDS, 16 or 32 token rows at a time, in a loop.
+  if (vec_out && N % 4 == 0 && (epi < 3 || epi == 8)) {
+    const bool rows32 = F32 || epi == 0 || epi == 8;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int n = n0 + (wn * NT + i) * 16 + (lane >> 4) * 4;
+      if (n >= N) continue;
+      f32x4_t b = {0.f, 0.f, 0.f, 0.f};
+      if (epi == 8) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[e] = dg.bias[n + e];
+      }
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        const int m = row0 + (wm * MT + j) * 16 + (lane & 15);
+        if (m >= row_end) continue;
+        f32x4_t v = acc[i][j];
+        if (epi == 8) v += b;
+        if (epi == 1) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { v[e] = v[e] > 0.f ? v[e] : 0.f; v[e] = v[e] * v[e]; }
+        }
+        const long at = (long)m * ldy + ycol + n;
+        if (rows32) *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(y) + at) = v;
+        else *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(y) + at) = u32x2_t{pack_bf2_hw(v[0], v[1]), pack_bf2_hw(v[2], v[3])};
+      }
+    }
+    return;
+  }
+  __syncthreads();
   float* rows = reinterpret_cast<float*>(smem) + wave * PASS * LDT;
   const bool pairs = epi_pairs(epi);
 #pragma unroll
@@ -499,25 +530,28 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
 
 constexpr int SKINNY_MAX_ROWS = 16, SKINNY_MAX_GROUPED_ROWS = 64;
 
-// The tile shape with the least estimated time: k-steps of the fullest CU, in us per step of 128 bytes of a row when n workgroups share it
-// (MI355X, fits of 20 .. 7000 rows over 2048 .. 14720-wide matrices).  A grouped product's runs leave half a tile empty each.
-//   bf16: 256 x 256 (features x tokens) has the highest rate, 192 x 192 comes next and divides other sizes (4228 x 4096 x 14720: 506 tiles on
-//   256 CUs, 478 us, where 272 of 256 x 256 take 663 and 1088 of 128 x 128 610); 128 x 64 has a third stage, as it is chosen where a CU
-//   has one or two workgroups (500 x 4096 x 4096: 39 -> 33 us).
+// The tile shape with the least estimated time: k-steps of the fullest CU, in us per step of 128 bytes of a row when it has n workgroups to run, and
+// what a workgroup takes to fill its ring and to store (MI355X).  A grouped product's runs leave half a tile empty each.
+//   bf16, fits of 23 products of 40 .. 7000 rows over 2048 .. 14720-wide matrices, rms 8 %: 256 x 256 (features x tokens) has the highest rate, the others fill
+//   the last round of 256 CUs better (4228 x 4096 x 4096: 506 tiles of 192 x 192 137 us, 272 of 256 x 256 199; 2500 x 2048 x 7424: 220 of 192 x 128 79, of 128 x 128
+//   96; 300 x 4096 x 4096: 160 of 128 x 64 29, 66 of 192 x 128 42).  The choice is within 0.1 % of the best shape over these.
 //   fp32, bound by the matrix cores: 64 x 32 fills the chip with a few hundred rows (562 x 2048 x 2048 80 -> 64 us, 568 gathered rows of 8 experts
 //   x 3072 x 2048 146 -> 106).
-struct RowTile { int features, tokens; float step[3], full; };       // step[n - 1] for n <= 3, n * full beyond
-constexpr RowTile TILES_BF16[] = {{256, 256, {1.45f, 3.2f, 4.9f}, 1.66f}, {192, 192, {1.05f, 2.15f, 3.2f}, 1.06f}, {128, 128, {0.70f, 1.03f, 1.5f}, 0.51f},
-                                  {128, 64, {0.48f, 0.75f, 1.15f}, 0.38f}};
-constexpr RowTile TILES_F32[] = {{128, 128, {2.25f, 4.4f, 6.3f}, 2.03f}, {64, 64, {0.77f, 1.27f, 1.8f}, 0.54f}, {64, 32, {0.45f, 0.71f, 1.0f}, 0.33f}};
+struct RowTile { int features, tokens; float step[3], full, ends; };       // step[n - 1] for n <= 3, n * full beyond
+constexpr RowTile TILES_BF16[] = {{256, 256, {1.209f, 2.709f, 4.166f}, 1.526f, 10.5f}, {192, 192, {0.773f, 1.900f, 2.534f}, 0.907f, 7.5f},
+                                  {128, 128, {0.797f, 0.861f, 1.444f}, 0.512f, 1.5f},  {128, 64, {0.433f, 0.728f, 0.951f}, 0.301f, 1.4f},
+                                  {256, 192, {1.104f, 2.384f, 3.590f}, 1.216f, 4.3f},  {256, 160, {0.905f, 2.010f, 3.034f}, 1.036f, 6.5f},
+                                  {256, 128, {0.757f, 1.620f, 2.348f}, 0.869f, 5.8f},  {192, 128, {0.618f, 1.207f, 2.060f}, 0.668f, 4.9f}};
+constexpr RowTile TILES_F32[] = {{128, 128, {2.25f, 4.4f, 6.3f}, 2.03f, 0.f}, {64, 64, {0.77f, 1.27f, 1.8f}, 0.54f, 0.f}, {64, 32, {0.45f, 0.71f, 1.0f}, 0.33f, 0.f}};
+constexpr int CFG_BF16 = 4, CFG_F32 = 3;          // shapes that ssd_gemm_rows_cfg offers
 template <int COUNT>
-int tile_shape(const RowTile (&tiles)[COUNT], int M, int N, int G, int E) {
+int tile_shape(const RowTile (&tiles)[COUNT], int M, int N, int K, int esz, int G, int E) {
   int best = 0;
   float least = 1e30f;
   for (int c = 0; c < COUNT; ++c) {
     const long count = (long)((N + tiles[c].features - 1) / tiles[c].features) * ((M + tiles[c].tokens - 1) / tiles[c].tokens + (E + 1) / 2) * G;
     const long n = (count + 255) / 256;
-    const float est = n <= 3 ? tiles[c].step[n - 1] : n * tiles[c].full;
+    const float est = (float)(K * (long)esz / 128) * (n <= 3 ? tiles[c].step[n - 1] : n * tiles[c].full) + n * tiles[c].ends;
     if (est < least) { least = est; best = c; }
   }
   return best;
@@ -559,7 +593,7 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   // few rows, or few features: 16-row chunks over the grid as long as that is about what the chip holds at once (64 x 2048 x 2048: 49 us as a
   // tile, a serial walk of K by few workgroups; a router's 1000 x 8 x 2048 the same 48 us)
   const int chunks = (M + 15) / 16;
-  if (shape >= 0 && (!tiled || shape >= (f32 ? 3 : 4))) return SSD_ERR_SHAPE;
+  if (shape >= 0 && (!tiled || shape >= (f32 ? CFG_F32 : CFG_BF16))) return SSD_ERR_SHAPE;
   if (shape < 0 && tiled && f32 && (offsets ? M <= SKINNY_MAX_GROUPED_ROWS : M <= SKINNY_MAX_ROWS || (long)chunks * ((N + 15) / 16) * G <= 1024)) {
     SKINNY_GO(float, 4, offsets ? 1 : chunks);
 #undef SKINNY_GO
@@ -568,7 +602,7 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   // (32 features and fewer with a short K: filling a tile's ring and bringing its accumulators round costs more than it saves, and the guarded
   //  kernel gives the same bits -- 8 features of K = 128 and any rows 4.3 us against 5.4, of K = 192 5.4 against 5.8; level at K = 256)
   if (tiled && (f32 || shape >= 0 || N > 32 || K >= 256)) {
-    if (shape < 0) shape = f32 ? tile_shape(TILES_F32, M, N, G, offsets ? E : 0) : tile_shape(TILES_BF16, M, N, G, offsets ? E : 0);
+    if (shape < 0) shape = f32 ? tile_shape(TILES_F32, M, N, K, 4, G, offsets ? E : 0) : tile_shape(TILES_BF16, M, N, K, 2, G, offsets ? E : 0);
     // what a store of four (paired: two) neighbouring outputs needs: their address a multiple of its size
     const bool out32 = f32 || epi == 0 || epi == 8;
     const int width = epi_pairs(epi) ? 4 : (out32 ? 16 : 8), osz = out32 ? 4 : 2;
@@ -586,12 +620,17 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
     if (f32 && shape == 0) TILE_GO(float, 2, 2, 4, 4, 2, GROUPED)           \
     else if (f32 && shape == 1) TILE_GO(float, 2, 2, 2, 2, 2, GROUPED)      \
     else if (f32) TILE_GO(float, 2, 2, 2, 1, 4, GROUPED)                    \
-    else if (shape == 0) TILE_GO(bf16_t, 4, 4, 4, 4, 2, GROUPED)            \
-    else if (shape == 1) TILE_GO(bf16_t, 4, 4, 3, 3, 3, GROUPED)            \
+    else if (shape == 0) TILE_GO(bf16_t, 4, 2, 4, 8, 2, GROUPED)            \
+    else if (shape == 1) TILE_GO(bf16_t, 4, 2, 3, 6, 3, GROUPED)            \
     else if (shape == 2) TILE_GO(bf16_t, 2, 2, 4, 4, 2, GROUPED)            \
-    else TILE_GO(bf16_t, 2, 2, 4, 2, 3, GROUPED)                            \
+    else if (shape == 3) TILE_GO(bf16_t, 2, 2, 4, 2, 3, GROUPED)            \
+    else if (shape == 4) TILE_GO(bf16_t, 4, 2, 4, 6, 2, GROUPED)            \
+    else if (shape == 5) TILE_GO(bf16_t, 4, 2, 4, 5, 3, GROUPED)            \
+    else if (shape == 6) TILE_GO(bf16_t, 4, 2, 4, 4, 3, GROUPED)            \
+    else TILE_GO(bf16_t, 4, 2, 3, 4, 3, GROUPED)                            \
   }
-    if (offsets) TILE_SHAPES(true) else TILE_SHAPES(false)
+    // (a dense product's rows are 32-bit offsets from the tile's first; rows so far apart that they don't reach go like gathered ones, by pointer)
+    if (offsets || 256L * ldx * esz0 > 0x7fffffffL) TILE_SHAPES(true) else TILE_SHAPES(false)
 #undef TILE_SHAPES
 #undef TILE_GO
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;

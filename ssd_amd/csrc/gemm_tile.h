@@ -1,11 +1,15 @@
-// The main loop of the large-tile bf16 GEMMs (many token rows: prefill): a workgroup owns (WN * NT) 16-row groups of W and (WM * MT)
+// The main loop of the large-tile GEMMs (many token rows: prefill): a workgroup owns (WN * NT) 16-row groups of W and (WM * MT)
 // 16-row groups of x, its WN x WM waves NT x MT of them each, and leaves the fp32 products in acc[NT][MT].
 //
-// What bounds it is the matrix cores and the LDS that feeds them: a wave with 4 x 4 accumulator tiles reads 8 KiB of LDS per 16 MFMAs of 16x16x32
-// (16 cycles each), so that at full rate the four SIMDs take 32 KiB in 256 cycles, all of the 128 bytes a CU's LDS delivers per cycle; 3 x 3
-// tiles ask for a third more than that, 4 x 2 for half as much again.  Both operands therefore travel HBM / L2 -> LDS by DMA (loads to LDS: no
-// registers, no LDS write instructions), 1 KiB per instruction, into a ring of STAGES steps of KS x 32 k.  A step's loads are issued
-// STAGES - 1 steps ahead, and ONE barrier per step both publishes the step and frees the buffer of the one before.
+// What bounds it is the matrix cores, and how much of their time the operands' way to them takes.  Both operands travel HBM / L2 -> LDS by DMA (loads
+// to LDS: no registers, no LDS write instructions), 1 KiB per instruction, into a ring of STAGES steps of KS x 32 k, and from there into TWO sets of
+// registers: while a wave multiplies one 32-wide k-block, the next one's operands are on their way from LDS (between its MFMAs, one read for every two or
+// three of them), so that no wave waits for LDS with its matrix core idle.  A step's buffer is free as soon as its last block is in registers, before
+// that block is multiplied: ONE barrier per step publishes the next step and frees this one, and a step's loads are issued STAGES ahead.
+// Eight waves of 4 x 8 tiles make 256 x 256: 12 KiB of LDS reads per 32 MFMAs (sixteen waves of 4 x 4 read a third more, and have no registers for a
+// second set).  Measured, MI355X, 256 x 256, us per k-block of a full chip: everything 0.75, without the DMA 0.62, MFMAs alone 0.55 (the clock that the
+// matrix cores leave: 0.43 at 2.4 GHz), without the MFMAs 0.42; sixteen waves that read a block just before they multiply it 0.80.  16384 x 4096 x 14336
+// 1425 -> 1355 us (1.42 PFLOP/s).  (32x32x16 MFMAs 0.83, s_setprio around them 0.79, waves of 8 x 8 spill.)
 // In bf16 every accumulator is one chain over the ascending k of the range that its workgroup walks, whatever the tile: where the caller does not cut K
 // (gemm_rows.hip), a row's result does not depend on the rows beside it; ssd_gemm_big's K splits go by the number of rows.  fp32: see below.
 #pragma once
@@ -38,28 +42,22 @@ __device__ __forceinline__ f32x4_t mfma_f32(uint32_t a, uint32_t b, f32x4_t c) {
 template <int WN, int WM, int NT, int MT, int STAGES, int KS = 1, bool F32 = false>
 struct TileLoop {
   static constexpr int WAVES = WN * WM, WG = WN * NT, XG = WM * MT;          // waves; 16-row groups of W, of x
-  static constexpr int STEP = (WG + XG) * KS * 1024;                              // LDS bytes of a k-step
-  static constexpr int PER = (WG + XG) * KS / WAVES;                             // 1 KiB operands each wave fetches per k-step
+  static constexpr int OPS = (WG + XG) * KS, STEP = OPS * 1024;                 // 1 KiB operands, LDS bytes of a k-step
+  static constexpr int PER = (OPS + WAVES - 1) / WAVES;                         // operands each wave fetches per k-step (the last ones twice where they don't go round)
   static constexpr int LDS = STAGES * STEP;
-  static_assert((WG + XG) * KS % WAVES == 0, "every wave fetches as many operands");
+  static __device__ __forceinline__ int op_of(int wave, int i) { return OPS % WAVES ? min(wave * PER + i, OPS - 1) : wave * PER + i; }
 
-  // fetch_one(i, step, lds): KiB i of this wave's PER (KiB wave * PER + i of the workgroup's step: W's groups first, KS each, then x's) of
-  // step `step` on its way to LDS.  at[s]: where in a group's KS KiB this lane finds its part of the s-th MFMA operand.
+  // fetch_one(i, step, lds): operand op_of(wave, i) of the workgroup's step (W's groups first, KS each, then x's) of step `step` on its way to
+  // LDS.  at[s]: where in a group's KS KiB this lane finds its part of the s-th MFMA operand.
   template <typename Fetch>
   static __device__ __forceinline__ void run(char* smem, int nk, const uint32_t (&at)[KS], f32x4_t (&acc)[NT][MT], const Fetch& fetch_one) {
+    static_assert(KS == 1 || KS == 2, "register sets go by the parity of a k-block");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave / WM, wm = wave % WM;
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
       for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    auto fetch = [&](int step, uint32_t buf) {
-#pragma unroll
-      for (int i = 0; i < PER; ++i) fetch_one(i, step, smem + buf * STEP + (wave * PER + i) * 1024);
-    };
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) fetch(s < nk ? s : nk - 1, s);
-    uint32_t cur = 0;
     f32x4_t part[F32 ? NT : 1][F32 ? MT : 1];
     if constexpr (F32) {
 #pragma unroll
@@ -67,36 +65,58 @@ struct TileLoop {
 #pragma unroll
         for (int j = 0; j < MT; ++j) part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-    for (int k = 0; k < nk; ++k) {
-      tile_wait<PER * (STAGES - 2)>();                 // this wave's share of step k is in LDS
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // everybody's is, and nobody reads step k - 1 any more
-      // (past the end the last step is fetched again: into the buffer nobody reads, so that the count of loads in flight stays static)
-      const int ahead = k + STAGES - 1;
-      fetch(ahead < nk ? ahead : nk - 1, cur == 0 ? STAGES - 1 : cur - 1);
+    auto fetch = [&](int step, uint32_t buf) {
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const char* a0 = smem + cur * STEP + wn * NT * KS * 1024 + at[s];
-        const char* b0 = smem + cur * STEP + (WG + wm * MT) * KS * 1024 + at[s];
-        u32x4_t a[NT], b[MT];
+      for (int i = 0; i < PER; ++i) fetch_one(i, step, smem + buf * STEP + op_of(wave, i) * 1024);
+    };
+    u32x4_t a[2][NT], b[2][MT];
+    auto read = [&](u32x4_t (&ra)[NT], u32x4_t (&rb)[MT], uint32_t buf, int s) {
+      const char* a0 = smem + buf * STEP + wn * NT * KS * 1024 + at[s];
+      const char* b0 = smem + buf * STEP + (WG + wm * MT) * KS * 1024 + at[s];
 #pragma unroll
-        for (int j = 0; j < MT; ++j) b[j] = *reinterpret_cast<const u32x4_t*>(b0 + j * KS * 1024);
+      for (int i = 0; i < NT; ++i) ra[i] = *reinterpret_cast<const u32x4_t*>(a0 + i * KS * 1024);
 #pragma unroll
-        for (int i = 0; i < NT; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(a0 + i * KS * 1024);
+      for (int j = 0; j < MT; ++j) rb[j] = *reinterpret_cast<const u32x4_t*>(b0 + j * KS * 1024);
+    };
+    auto multiply = [&](const u32x4_t (&ra)[NT], const u32x4_t (&rb)[MT]) {
+      if constexpr (F32) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) part[i][j] = mfma_f32(ra[i][e], rb[j][e], part[i][j]);
+      } else {
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
-          for (int j = 0; j < MT; ++j) {
-            if constexpr (!F32) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
-          }
-        if constexpr (F32) {
+          for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(ra[i], rb[j], acc[i][j]);
+        // the reads of the next block between this one's MFMAs
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int i = 0; i < NT; ++i)
-#pragma unroll
-              for (int j = 0; j < MT; ++j) part[i][j] = mfma_f32(a[i][e], b[j][e], part[i][j]);
+        for (int r = 0; r < NT + MT; ++r) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, NT * MT / (NT + MT), 0);
         }
+        __builtin_amdgcn_sched_group_barrier(0x008, NT * MT, 0);
       }
+    };
+    // (past the end the last step is fetched again, into a buffer that nobody reads for a product, so that the count of loads in flight stays static)
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s) fetch(s < nk ? s : nk - 1, s);
+    tile_wait<PER * (STAGES - 1)>();                   // this wave's share of the first step is in LDS
+    asm volatile("s_barrier" ::: "memory");            // everybody's is
+    uint32_t cur = 0;
+    read(a[0], b[0], 0, 0);
+    // set h holds the last block of step k: step k + 1 becomes visible, k's buffer is filled again, the next block is read and this one multiplied
+    auto last_block = [&](int k, int h) {
+      __builtin_amdgcn_sched_barrier(0);
+      tile_wait<PER * (STAGES - 2)>();                 // this wave's share of step k + 1 is in LDS
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // everybody's is, and nobody reads step k's buffer any more
+      const int ahead = k + STAGES;
+      fetch(ahead < nk ? ahead : nk - 1, cur);
+      cur = cur + 1 == STAGES ? 0 : cur + 1;
+      read(a[h ^ 1], b[h ^ 1], cur, 0);
+      multiply(a[h], b[h]);
       if constexpr (F32) {
         if ((k + 1) % F32_SEG_STEPS == 0 || k + 1 == nk) {
 #pragma unroll
@@ -105,7 +125,19 @@ struct TileLoop {
             for (int j = 0; j < MT; ++j) { acc[i][j] += part[i][j]; part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f}; }
         }
       }
-      cur = cur + 1 == STAGES ? 0 : cur + 1;
+    };
+    if constexpr (KS == 1) {
+      for (int k = 0; k < nk; k += 2) {
+        last_block(k, 0);
+        if (k + 1 < nk) last_block(k + 1, 1);
+      }
+    } else {
+      for (int k = 0; k < nk; ++k) {
+        __builtin_amdgcn_sched_barrier(0);
+        read(a[1], b[1], cur, 1);
+        multiply(a[0], b[0]);
+        last_block(k, 1);
+      }
     }
     tile_wait<0>();                                    // nothing may land in LDS after the workgroup has ended
   }

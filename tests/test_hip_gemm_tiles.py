@@ -1,0 +1,63 @@
+"""Tile shapes of 32-token steps: ssd_gemm_big's by number and as its sizes choose them, ssd_gemm_rows' (csrc/gemm_rows.hip) at sizes that choose each of
+them, against fp64 products; last tiles of one row, odd numbers of k-steps, fewer k-steps than a ring holds."""
+import pytest
+import torch
+
+from tests.test_hip_gemm_big import H, check, frag, operands  # noqa: F401
+from tests.test_hip_gemm_rows_tile import act
+from tests.test_hip_gemm_rows_tile import check as check_rows
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+
+
+@pytest.mark.parametrize("shape", [5, 6, 7, 8, 9, 10])
+@pytest.mark.parametrize("M,N,K,splits", [(1, 16, 96, 1), (225, 272, 96, 1), (193, 208, 352, 3), (161, 512, 1024, 8), (129, 400, 160, 1), (385, 192, 2080, 2)])
+def test_big_rows(H, shape, M, N, K, splits):
+    x, w, b = operands(M, N, K, M + N + K)
+    ws = torch.empty(splits * M * N, dtype=torch.float32, device="cuda")
+    y = torch.full((M, N + 12), 7.0, dtype=BF, device="cuda")
+    H.gemm_big(frag(H, x), frag(H, w), y, M, N, K, N + 12, bias=b.cuda(), workspace=ws, shape=shape, splits=splits)
+    check(y[:, :N], x.double() @ w.double().T + b.double(), (shape, M, N, K, splits))
+    assert bool((y[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("shape", [5, 6, 7])
+def test_big_silu(H, shape):
+    M, I, K = 257, 160, 416
+    x, w, _ = operands(M, 2 * I, K, shape)
+    wf = torch.zeros(2 * I * K, dtype=BF, device="cuda")
+    H.rows_to_frag(w.cuda(), wf, 2 * I, K, mode=1)
+    got = []
+    for s in (shape, 2):
+        out = torch.zeros(H.frag_numel(M, I), dtype=BF, device="cuda")
+        H.gemm_big(frag(H, x), wf, out, M, 2 * I, K, 0, epilogue=H.EPI_SILU_FRAG, shape=s, splits=1)
+        rows = torch.zeros(M, I, dtype=BF, device="cuda")
+        H.frag_to_rows(out, rows, M, I)
+        got.append(rows)
+    assert torch.equal(*got)                # one chain of k per output, whatever the tile
+    from ssd_amd.hip.lib import SsdHipError
+    with pytest.raises(SsdHipError):        # tiles of 192 features cut (gate, up) pairs
+        H.gemm_big(frag(H, x), wf, out, M, 2 * I, K, 0, epilogue=H.EPI_SILU_FRAG, shape=8, splits=1)
+
+
+# rows x features whose fewest rounds of 256 workgroups are, in this order, of 256 x 192, 256 x 160, 256 x 128 and 192 x 128 tiles
+@pytest.mark.parametrize("M,N,K", [(3041, 3074, 1088), (2113, 4098, 1088), (1921, 3080, 2112), (641, 3080, 2112)])
+def test_rows_of_other_shapes(H, M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g).to(BF).cuda(), (torch.randn(N, K, generator=g) / K ** 0.5).to(BF).cuda()
+    z = x.double() @ w.double().T
+    for epi in (0, 1, 2, 3):
+        y = torch.full((M, N // 2 if epi == 3 else N), 7.0, dtype=torch.float32 if epi == 0 else BF, device="cuda")
+        H.gemm_rows(x, w, y, M, N, K, False, epi)
+        ref = {0: z, 1: z.relu() ** 2, 2: z, 3: act(z, 3)}[epi]
+        check_rows(y, ref, (M, N, K, epi), epi != 0, slope=12.0 if epi in (1, 3) else 1.0)
+        if epi != 3:
+            tile = torch.zeros_like(y)
+            H.gemm_rows_cfg(x, w, tile, M, N, K, False, 2, epi)
+            assert torch.equal(y, tile)
+    b = torch.randn(N, device="cuda")
+    y = torch.zeros(M, N, device="cuda")
+    H.gemm_rows_bias(x, w, y, M, N, K, b, False)
+    check_rows(y, z + b.double(), (M, N, K, "bias"), False)
