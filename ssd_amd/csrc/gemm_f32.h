@@ -1,0 +1,85 @@
+// fp32 products on the bf16 matrix cores, and the order of their sums.
+//
+// A float is the sum of three bf16 numbers, exactly: h, the float rounded to nearest; m, the rest x - h rounded to nearest; l, what then remains, at most 8
+// bits.  A product of two floats is h h' + (h m' + m h') + m m' + (h l' + l h') and three products below 2^-24 of it, which are left out; each of the six is exact in fp32 and summed there by 16x16x32 MFMAs.  Six of those take 96 cycles for 32 k, eight
+// 16x16x4 fp32 MFMAs 256, and they round a sum after every 32 k where those round it after every 4.
+// MI355X, relative error against fp64 of N(0, 1) x N(0, 1 / K) products, fp32 MFMAs in segments of 256 k -> this:
+// K = 96 1.8e-7 -> 0.5e-7, K = 1536 2.9e-7 -> 1.0e-7, K = 2048 2.9e-7 -> 1.1e-7, K = 14336 3.2e-7 -> 2.6e-7.
+//
+// The order of a sum is part of what the fp32 mode promises -- a row's result is the same bits whichever kernel computes it -- and is defined here:
+// runs of F32_RUN k are dealt to F32_CHAINS chains in turn.  A chain adds up its runs in order, a block of 32 k at a time, in two accumulators that start
+// from zero: `low` takes the five small products (l h', h l', m m', m h', h m'), `high` takes h h'; its sum is high + low.  The chains' sums are added in
+// their order.  In a block of 32, lane q of a row holds k = 4 q .. 4 q + 3 and 16 + 4 q .. 16 + 4 q + 3.
+//
+// Infinities, NaN and floats that round past the largest bf16 make a rest NaN: a sum that is not finite is computed again as one FMA chain over ascending k, whose result it then is.
+// (Terms below the smallest normal number may be flushed: an error of 2^-126 times the other factor.)
+#pragma once
+#include "common.h"
+
+constexpr int F32_RUN = 64, F32_CHAINS = 8;
+
+struct F32Split { u32x4_t h, m, l; };        // 8 k of a row, three MFMA operands
+
+// the floats of 4 q .. 4 q + 3 and of 16 + 4 q ..: 44 instructions
+__device__ __forceinline__ F32Split f32_split(u32x4_t p, u32x4_t q) {
+  F32Split s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t x0 = i < 2 ? p[2 * i] : q[2 * i - 4], x1 = i < 2 ? p[2 * i + 1] : q[2 * i - 3];
+    const uint32_t h = pack_bf2_hw(__uint_as_float(x0), __uint_as_float(x1));
+    const float r0 = __uint_as_float(x0) - __uint_as_float(h << 16), r1 = __uint_as_float(x1) - __uint_as_float(h & 0xffff0000u);
+    const uint32_t m = pack_bf2_hw(r0, r1);
+    s.h[i] = h;
+    s.m[i] = m;
+    s.l[i] = __builtin_amdgcn_perm(__float_as_uint(r1 - __uint_as_float(m & 0xffff0000u)), __float_as_uint(r0 - __uint_as_float(m << 16)), 0x07060302u);
+  }
+  return s;
+}
+
+// The same with the rests by dot products -- -1 times one half of h and 0 times the other, added to x, exact as above -- in 28 instructions.  They take the matrix
+// core's time: for kernels that wait for memory (16 rows x 2048 x 2048 13.5 -> 12.5 us), not for those that multiply (512 x 2048 x 2048 28 -> 33).
+__device__ __forceinline__ float f32_rest(uint32_t hs, uint32_t minus_one, float x) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, hs), __builtin_bit_cast(bf16x2_t, minus_one), x, false);
+}
+__device__ __forceinline__ F32Split f32_split_dot(u32x4_t p, u32x4_t q) {
+  uint32_t low = 0x0000bf80u, high = 0xbf800000u;
+  asm("" : "+s"(low), "+s"(high));             // (in registers: an inline constant of a packed operand is neither of the two)
+  F32Split s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t x0 = i < 2 ? p[2 * i] : q[2 * i - 4], x1 = i < 2 ? p[2 * i + 1] : q[2 * i - 3];
+    const uint32_t h = pack_bf2_hw(__uint_as_float(x0), __uint_as_float(x1));
+    const float r0 = f32_rest(h, low, __uint_as_float(x0)), r1 = f32_rest(h, high, __uint_as_float(x1));
+    const uint32_t m = pack_bf2_hw(r0, r1);
+    s.h[i] = h;
+    s.m[i] = m;
+    s.l[i] = __builtin_amdgcn_perm(__float_as_uint(f32_rest(m, high, r1)), __float_as_uint(f32_rest(m, low, r0)), 0x07060302u);
+  }
+  return s;
+}
+
+// the products of NT groups of 16 features with one of tokens: term by term, so that neighbouring MFMAs have different accumulators
+template <int NT>
+__device__ __forceinline__ void f32_block(const F32Split (&a)[NT], const F32Split& b, f32x4_t (&high)[NT], f32x4_t (&low)[NT]) {
+#pragma unroll
+  for (int i = 0; i < NT; ++i) low[i] = mfma16(a[i].l, b.h, low[i]);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) low[i] = mfma16(a[i].h, b.l, low[i]);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) low[i] = mfma16(a[i].m, b.m, low[i]);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) low[i] = mfma16(a[i].m, b.h, low[i]);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) low[i] = mfma16(a[i].h, b.m, low[i]);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) high[i] = mfma16(a[i].h, b.h, high[i]);
+}
+
+__device__ __forceinline__ bool f32_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
+
+// what a sum that is not finite is instead
+static __device__ __noinline__ float f32_plain(const float* a, const float* b, int K) {
+  float s = 0.f;
+  for (int k = 0; k < K; ++k) s = fmaf(a[k], b[k], s);
+  return s;
+}

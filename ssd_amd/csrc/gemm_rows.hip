@@ -1,4 +1,4 @@
-// Row-major GEMM for ANY M, N, K, in bf16 (MFMA 16x16x32, fp32 accumulation) or in true fp32 (MFMA 16x16x4, or FMA), dense or grouped:
+// Row-major GEMM for ANY M, N, K, in bf16 (MFMA 16x16x32, fp32 accumulation) or in true fp32 (gemm_f32.h, or FMA), dense or grouped:
 //   y[m][n] = sum_k x[row(m)][k] * w[g(m)][n][k]
 // The skinny / prefill GEMMs of gemm.hip, gemm_pf.hip and gemm_big.hip need fragment-major operands with N % 16 == 0 and K % 32 == 0; models
 // whose sizes do not meet that, grouped (per-expert) products over gathered token rows, and the fp32 arithmetic mode use this file:
@@ -6,7 +6,7 @@
 // follows: a 256-thread workgroup owns a 64 x 64 output tile; a K step of 32 is staged through LDS with bounds guards (rows or columns past the
 // edge read as zero), so no operand needs padding; wave w multiplies token rows 16w..16w+15 by the tile's four 16-feature groups.
 // In the tile forms every bf16 output element is the sum over k in ascending 32-wide steps, whatever M, the tile or the group is; in fp32 the order
-// (gemm_tile.h; FMA chains in the guarded kernel) is a function of K and the alignment alone: a row's result does not depend on which other
+// (gemm_f32.h; FMA chains in the guarded kernel) is a function of K and the alignment alone: a row's result does not depend on which other
 // rows share its launch.
 //   grouped: offsets[E+1] cuts the (sorted) rows into E runs, run e multiplies by w + e * N * K; row_idx (optional) names the x row
 //   of every sorted row as row_idx[r] / idx_div; tiles never straddle two runs (blockIdx.y walks a list of at most
@@ -14,6 +14,7 @@
 //   batched: G independent products in one launch (blockIdx.z / blockIdx.y = g): x + g * gsx with row stride ldx, w + g * N * K,
 //   y + g * gsy with row stride ldy -- per-head products whose operands are column slices of token-major rows.
 #include "common.h"
+#include "gemm_f32.h"
 #include "gemm_tile.h"
 
 namespace {
@@ -215,10 +216,10 @@ gemm_rows_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restr
 // multiplies.)  With four waves two workgroups share a CU, one's loads covering the other's start and end; where no CU gets a second one, eight waves
 // halve the chain of stages.  Deeper rings gained nothing.
 //   bf16: a wave's runs are one chain of 16x16x32 MFMAs, the waves' sums are added in wave order.
-//   fp32: a run is a segment of gemm_tile.h's order; after every round of four, wave 0 adds the segments' sums in theirs.
+//   fp32: a stage is a run of gemm_f32.h's order; four waves have two chains each, eight have one.
 // MI355X, weights not in the caches, direct loads -> four waves: bf16, 4 rows: 14720 x 4096 36.6 -> 21.3 us (5.7 TB/s), 4096 x 14720 31.5 -> 19.3,
-// 2048 x 7424 18.9 -> 8.8; fp32, 4 rows: 32000 x 2048 77 -> 40 us (6.6 TB/s), 3088 x 2048 11.4 -> 6.8, 2048 x 3072 16.9 -> 8.8.  fp32 error against
-// fp64, relative: 3e-7 at K = 2048 .. 4096.
+// 2048 x 7424 18.9 -> 8.8; fp32, 4 rows: 32000 x 2048 77 -> 40 us (6.6 TB/s).  fp32, weights of many matrices in turn, fp32 MFMAs on four waves
+// -> this, by 1 .. 4 rows | 16: 3088 x 2048 11.9 -> 8.7 | 12.9 -> 10.8, 2048 x 3072 16.0 -> 10.0 | 17.2 -> 12.9.
 // Weights of many matrices in turn (partly from the Infinity Cache), one row, direct loads with 16 waves | four | eight waves: N = 8, K = 4096 7.7 | 8.1 |
 // 5.6 us, K = 14720 16.3 | 25.6 | 14.6; 4096 x 4096 10.3 | 11.3 | 9.4, 4096 x 14720 30.4 | 32.5 | 22.7, 64 x 2048 6.7 | 5.4 | 4.7; direct loads with
 // eight, four, eight: 4096 x 1280 5.2 | 5.8 | 5.0, 64 x 1536 4.6 | 5.0 | 4.2.
@@ -227,14 +228,17 @@ gemm_rows_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restr
 template <typename T, int NW>             // NW waves
 struct Skinny {
   static constexpr bool F32 = sizeof(T) == 4;
-  static constexpr int SPR = F32 ? F32_SEG * 4 / 256 : 2;                    // stages of a run
+  static constexpr int SPR = F32 ? F32_RUN * 4 / 256 : 2;                    // stages of a run
+  static constexpr int CH = F32 ? F32_CHAINS / NW : 1;                          // fp32: chains of gemm_f32.h that a wave has, its stages their runs in turn
+  static_assert(!F32 || (F32_CHAINS % NW == 0 && CH <= 2 && SPR == 1), "");
+  static constexpr int SUMS = F32 ? F32_CHAINS : NW;                          // that are added up
   static constexpr int RING = 16 * 1024;                                      // LDS bytes of a wave's ring: the largest of stages() x stage_bytes()
   static constexpr int stage_bytes(int xi) { return (4 + xi) * 1024; }
   static constexpr int stages(int xi) { return xi == 1 ? 3 : 2; }
 
   // Up to 4 * XI token rows at xr (this lane's four-row pieces) against the 16 weight rows at wr: wave 0 returns the sums.
   template <int XI>
-  static __device__ __forceinline__ f32x4_t chunk(char* ring, f32x4_t (*red)[NW][64], uint32_t& turn, const char* const (&wr)[4],
+  static __device__ __forceinline__ f32x4_t chunk(char* ring, f32x4_t (*red)[SUMS][64], uint32_t& turn, const char* const (&wr)[4],
                                                   const char* const (&xr)[XI], long row_bytes) {
     constexpr int R = stages(XI), STAGE = stage_bytes(XI), PER = 4 + XI;
     static_assert(R * STAGE <= RING, "the ring holds the stages");
@@ -262,57 +266,71 @@ struct Skinny {
 #pragma unroll
     for (int s = 0; s < R - 1; ++s)
       if (s < n) fetch(s, s);
-    f32x4_t total = {0.f, 0.f, 0.f, 0.f};
-    int cur = 0, l = 0;
-    const int rounds = F32 ? (runs + NW - 1) / NW : 1;
-    for (int round = 0; round < rounds; ++round, ++turn) {
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-      const int end = F32 ? min(n, (round + 1) * SPR) : n;
-      for (; l < end; ++l) {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                   // (the stage before is in registers)
-        const int ahead = n - 1 - l;
-        if (ahead >= R - 1) {
-          fetch(l + R - 1, cur == 0 ? R - 1 : cur - 1);
-          tile_wait<(R - 1) * PER>();
-        } else if (R > 2 && ahead == 1) {
-          tile_wait<PER>();
-        } else {
-          tile_wait<0>();
-        }
-        const char* p = ring + cur * STAGE;
-        cur = cur + 1 == R ? 0 : cur + 1;
-        u32x4_t a[4], b[4];
+    f32x4_t total = {0.f, 0.f, 0.f, 0.f}, acc = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t low[CH][1] = {}, high[CH][1] = {};                               // (fp32)
+    int cur = 0;
+    auto stage = [&](int l, int chain) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                     // (the stage before is in registers)
+      const int ahead = n - 1 - l;
+      if (ahead >= R - 1) {
+        fetch(l + R - 1, cur == 0 ? R - 1 : cur - 1);
+        tile_wait<(R - 1) * PER>();
+      } else if (R > 2 && ahead == 1) {
+        tile_wait<PER>();
+      } else {
+        tile_wait<0>();
+      }
+      const char* p = ring + cur * STAGE;
+      cur = cur + 1 == R ? 0 : cur + 1;
+      u32x4_t a[4], b[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          a[j] = *reinterpret_cast<const u32x4_t*>(p + r * 256 + ((j * 4 + qd) ^ r) * 16);
-          b[j] = *reinterpret_cast<const u32x4_t*>(p + 4096 + xrow * 256 + ((j * 4 + qd) ^ xrow) * 16);
-        }
-        const long left = row_bytes - (long)stage_of(l) * 256;               // bytes of the rows from this stage on
-        if (ragged && left < 256) {
+      for (int j = 0; j < 4; ++j) {
+        a[j] = *reinterpret_cast<const u32x4_t*>(p + r * 256 + ((j * 4 + qd) ^ r) * 16);
+        b[j] = *reinterpret_cast<const u32x4_t*>(p + 4096 + xrow * 256 + ((j * 4 + qd) ^ xrow) * 16);
+      }
+      const long left = row_bytes - (long)stage_of(l) * 256;                 // bytes of the rows from this stage on
+      if (ragged && left < 256) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if ((j * 4 + qd) * 16 >= left) a[j] = b[j] = u32x4_t{0u, 0u, 0u, 0u};
+        for (int j = 0; j < 4; ++j)
+          if ((j * 4 + qd) * 16 >= left) a[j] = b[j] = u32x4_t{0u, 0u, 0u, 0u};
+      }
+      if constexpr (F32) {
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+          if (j && j * 64 >= left) break;
+          const F32Split as[1] = {f32_split_dot(a[j], a[j + 1])};
+          f32_block<1>(as, f32_split_dot(b[j], b[j + 1]), high[chain], low[chain]);
         }
+      } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           if (j && j * 64 >= left) break;
-          if constexpr (F32) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc = mfma_f32(a[j][e], b[j][e], acc);
-          } else {
-            acc = mfma16(a[j], b[j], acc);
-          }
+          acc = mfma16(a[j], b[j], acc);
         }
       }
-      // (two sets of sums in turn: one barrier per round both publishes a set and tells that the one before has been read)
-      red[turn & 1][wave][lane] = acc;
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (wave == 0) {
-#pragma unroll
-        for (int v = 0; v < NW; ++v)
-          if (round * NW + v < runs) total += red[turn & 1][v][lane];
+    };
+    if constexpr (F32) {
+      for (int l = 0; l < n; l += CH) {
+        stage(l, 0);
+        if (CH == 2 && l + 1 < n) stage(l + 1, CH - 1);
       }
+    } else {
+      for (int l = 0; l < n; ++l) stage(l, 0);
     }
+    // (two sets of sums in turn: one barrier per chunk both publishes a set and tells that the one before has been read)
+    if constexpr (F32) {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) red[turn & 1][c * NW + wave][lane] = high[c][0] + low[c][0];
+    } else {
+      red[turn & 1][wave][lane] = acc;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (wave == 0) {
+#pragma unroll
+      for (int v = 0; v < SUMS; ++v)
+        if (v < runs) total += red[turn & 1][v][lane];
+    }
+    ++turn;
     return total;
   }
 };
@@ -324,7 +342,7 @@ gemm_skinny_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __res
                    long gsy, GluClamp gc, DecayGate dg) {
   typedef Skinny<T, NW> L;
   __shared__ __attribute__((aligned(1024))) char smem[NW * L::RING];
-  __shared__ f32x4_t red[2][NW][64];
+  __shared__ f32x4_t red[2][L::SUMS][64];
   const int lane = threadIdx.x & 63, r = lane & 15, qd = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = blockIdx.x * 16;
@@ -377,7 +395,12 @@ gemm_skinny_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __res
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int n = n0 + qd * 4 + e;
-          if (n < N) store_out<T>(y, mrow, ldy, ycol + n, sum[e], epi, dg);
+          if (n >= N) continue;
+          if constexpr (L::F32) {
+            if (!f32_finite(sum[e]))
+              sum[e] = f32_plain(w + ((size_t)blockIdx.y * N + n) * K, x + (row_idx ? (long)(row_idx[mrow] / idx_div) : (long)mrow) * ldx, K);
+          }
+          store_out<T>(y, mrow, ldy, ycol + n, sum[e], epi, dg);
         }
       }
     }
@@ -392,14 +415,12 @@ gemm_skinny_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __res
 // Bound by the matrix cores.  MI355X, against the 64 x 64 form above (which re-stages both operands through registers, two barriers per 32-wide
 // k-step): 4000 x 14720 x 4096 1516 -> 410 us (1180 TFLOP/s), 2000 x 4096 x 14720 600 -> 222, 100 x 14720 x 4096 105 -> 38.
 // ---------------------------------------------------------------------------------------------------------------------
-template <typename T, int WN, int WM, int NT, int MT, int STAGES, bool GROUPED>
+template <int WN, int WM, int NT, int MT, int STAGES, bool GROUPED>
 __global__ void __launch_bounds__(64 * WN * WM, 2)
-gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
+gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y, int M, int N, int K, int epi,
                       const int* __restrict__ offsets, int E, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx,
                       long gsy, GluClamp gc, DecayGate dg, int tn, int tm, bool vec_out) {
-  constexpr bool F32 = sizeof(T) == 4;
-  constexpr int VEC = 16 / sizeof(T), ROWB = sizeof(T);              // elements of a 16-byte chunk; bytes of an element
-  typedef TileLoop<WN, WM, NT, MT, STAGES, 2, F32> L;
+  typedef TileLoop<WN, WM, NT, MT, STAGES, 2> L;
   constexpr int LDT = NT * 16 + 4, PASS = MT % 2 == 0 && L::WAVES * 32 * LDT * 4 <= L::LDS ? 32 : 16;                       // a wave's epilogue rows (floats), token rows per pass
   static_assert(MT * 16 % PASS == 0 && L::WAVES * PASS * LDT * 4 <= L::LDS, "the epilogue rows fit the ring");
   __shared__ __attribute__((aligned(1024))) char smem[L::LDS];
@@ -407,7 +428,7 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
   const TileAt t = tile_at(blockIdx.x, tn, tm);
   const int n0 = t.n * L::WG * 16;
   int row0 = t.m * L::XG * 16, row_end = M;
-  const T* wg = w + (size_t)blockIdx.y * N * K;
+  const bf16_t* wg = w + (size_t)blockIdx.y * N * K;
   x += (size_t)blockIdx.y * gsx;
   const long ycol = (long)blockIdx.y * gsy;
   if (GROUPED && offsets) {
@@ -423,25 +444,25 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
     wg = w + (size_t)e * N * K;
   }
   // (rows past the edge read the last row again: their products are never stored)
-  const auto wr = tile_rsrc(wg + (size_t)n0 * K, (uint32_t)min(L::WG * 16, N - n0) * (uint32_t)K * ROWB);
-  const auto xr = tile_rsrc(x + (size_t)row0 * ldx, GROUPED ? 0u : (uint32_t)min(L::XG * 16, row_end - row0) * (uint32_t)ldx * ROWB);
+  const auto wr = tile_rsrc(wg + (size_t)n0 * K, (uint32_t)min(L::WG * 16, N - n0) * (uint32_t)K * 2u);
+  const auto xr = tile_rsrc(x + (size_t)row0 * ldx, GROUPED ? 0u : (uint32_t)min(L::XG * 16, row_end - row0) * (uint32_t)ldx * 2u);
   uint32_t off[L::PER];                // from wr or xr
-  const T* xp[GROUPED ? L::PER : 1];
+  const bf16_t* xp[GROUPED ? L::PER : 1];
 #pragma unroll
   for (int i = 0; i < L::PER; ++i) {
     const int c = L::op_of(wave, i), r = (c >> 1) * 16 + (c & 1) * 8 + (lane >> 3), k8 = (lane & 7) ^ (lane >> 3);
     const int m = min(row0 + r - L::WG * 16, row_end - 1);
-    off[i] = (r < L::WG * 16 ? (uint32_t)min(r, N - 1 - n0) * (uint32_t)K : (uint32_t)(m - row0) * (uint32_t)ldx) * ROWB + k8 * 16;
-    if constexpr (GROUPED) xp[i] = r < L::WG * 16 ? x : x + (row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx + k8 * VEC;
+    off[i] = (r < L::WG * 16 ? (uint32_t)min(r, N - 1 - n0) * (uint32_t)K : (uint32_t)(m - row0) * (uint32_t)ldx) * 2u + k8 * 16;
+    if constexpr (GROUPED) xp[i] = r < L::WG * 16 ? x : x + (row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx + k8 * 8;
   }
   const uint32_t at0 = (uint32_t)(((lane >> 3) & 1) * 1024 + ((lane & 7) * 8 + ((lane >> 4) ^ (lane & 7))) * 16), at[2] = {at0, at0 ^ 64u};
   f32x4_t acc[NT][MT];
-  L::run(smem, K / (8 * VEC), at, acc, [&](int i, int step, char* lds) {
+  L::run(smem, K / 64, at, acc, [&](int i, int step, char* lds) {
     const bool of_w = L::op_of(wave, i) < 2 * L::WG;
     if (!GROUPED || of_w)
       tile_dma(of_w ? wr : xr, off[i], (uint32_t)step * 128u, lds);
     else
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp[GROUPED ? i : 0] + step * 8 * VEC), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp[GROUPED ? i : 0] + step * 64), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
   });
 
   const int wn = wave / WM, wm = wave % WM;
@@ -449,7 +470,7 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
   // that unrolls over the accumulators has to stay short -- a workgroup runs it once, out of a cold instruction cache: with every epilogue in it
   // the kernel took 12 us longer --, so the others go through LDS, 16 or 32 token rows at a time, in a loop.
   if (vec_out && N % 4 == 0 && (epi < 3 || epi == 8)) {
-    const bool rows32 = F32 || epi == 0 || epi == 8;
+    const bool rows32 = epi == 0 || epi == 8;
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int n = n0 + (wn * NT + i) * 16 + (lane >> 4) * 4;
@@ -493,7 +514,7 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
       const int m = row0 + wm * MT * 16 + p * PASS + r, n = n0 + wn * NT * 16 + q;
       if (m >= row_end || n >= N) continue;
       const f32x4_t v = *reinterpret_cast<const f32x4_t*>(rows + r * LDT + q);
-      if (!F32 && pairs) {
+      if (pairs) {
         const float rs = epi == 6 && gc.row_scale ? gc.row_scale[row_idx ? row_idx[m] : m] : 1.0f;
         bf16_t* o = reinterpret_cast<bf16_t*>(y) + (long)m * ldy + ycol + (n >> 1);
         const float a = glu_act(v[0], v[1], epi, rs, gc.limit, gc.alpha);
@@ -503,12 +524,11 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
           o[0] = (bf16_t)f2bf(a);
           if (n + 3 < N) o[1] = (bf16_t)f2bf(glu_act(v[2], v[3], epi, rs, gc.limit, gc.alpha));
         }
-      } else if (vec_out && n + 3 < N && (epi == 0 || epi == 8 || (F32 && epi < 3))) {
+      } else if (vec_out && n + 3 < N && (epi == 0 || epi == 8)) {
         f32x4_t o = v;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if (epi == 8) o[e] += dg.bias[n + e];
-          if (epi == 1) { o[e] = o[e] > 0.f ? o[e] : 0.f; o[e] = o[e] * o[e]; }
         }
         *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(y) + (long)m * ldy + ycol + n) = o;
       } else if (vec_out && n + 3 < N && (epi == 1 || epi == 2)) {
@@ -521,10 +541,137 @@ gemm_rows_tile_kernel(const T* __restrict__ x, const T* __restrict__ w, void* __
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (n + e < N) store_out<T>(y, m, ldy, ycol + n + e, v[e], epi, dg);
+          if (n + e < N) store_out<bf16_t>(y, m, ldy, ycol + n + e, v[e], epi, dg);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// fp32, more rows than the skinny form takes (K % 32 == 0, 16-byte aligned rows): 64 features x 16 * MT tokens to a workgroup, whose eight waves own the eight
+// chains of gemm_f32.h -- each the whole tile for its runs of K, through a stage of its own that DMA fills (no barrier), and at the end an eighth of the
+// tile, for which it adds the chains' sums up.  So a product of a few hundred rows fills the chip with tiles that still multiply every operand they have
+// split sixteen times: 96 MFMAs (1536 cycles of the matrix core) and 352 vector instructions (1408) for a step of 64 x 64 x 32.  The two waves of a SIMD
+// take turns with them; one alone runs them one after the other (four waves with two stages each, splitting a step ahead: half the rate; v_dot2 for the
+// rests, 28 instructions an operand instead of 44, keeps the matrix core waiting).  A step's operands go from the stage to registers at once, so that the
+// next step's loads have all of it to arrive.
+// MI355X, against 16x16x4 fp32 MFMAs on tiles that a workgroup's waves share: 160 x 2048 x 2048 31 -> 18 us, 512 x 2048 x 2048 45 -> 27, 1356 x 2048 x 3072 171 -> 107,
+// 3000 x 3088 x 2048 325 -> 235 (160 TFLOP/s; the fp32 MFMAs' peak is 157).  The MFMAs alone take 0.83 us a step (chip full), splits and reads 0.65, the DMA
+// 0.3: together 1.8, whichever wave does what when, as long as the chip is full; larger tiles would split less often, and do not fit the registers.
+// ---------------------------------------------------------------------------------------------------------------------
+template <int MT, bool GROUPED>
+__global__ void __launch_bounds__(512, 2)
+gemm_rows_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int M, int N, int K, int epi,
+                     const int* __restrict__ offsets, int E, const int* __restrict__ row_idx, int idx_div, long ldx, long ldy, long gsx, long gsy,
+                     DecayGate dg, int tn, int tm, bool vec_out) {
+  constexpr int NT = 4, PER = 2 * (NT + MT), STEP = PER * 1024;          // 1 KiB pieces (8 rows x 128 bytes), bytes of a step of 32 k
+  static_assert(F32_CHAINS == 8 && F32_RUN == 64, "a wave is a chain, two of its steps a run");
+  __shared__ __attribute__((aligned(1024))) char smem[F32_CHAINS * STEP];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const TileAt t = tile_at(blockIdx.x, tn, tm);
+  const int n0 = t.n * NT * 16;
+  int row0 = t.m * MT * 16, row_end = M;
+  const float* wg = w + (size_t)blockIdx.y * N * K;
+  x += (size_t)blockIdx.y * gsx;
+  const long ycol = (long)blockIdx.y * gsy;
+  if (GROUPED && offsets) {
+    int tile = t.m, e = 0;
+    for (; e < E; ++e) {
+      const int nt = (offsets[e + 1] - offsets[e] + MT * 16 - 1) / (MT * 16);
+      if (tile < nt) break;
+      tile -= nt;
+    }
+    if (e >= E) return;
+    row0 = offsets[e] + tile * MT * 16;
+    row_end = offsets[e + 1];
+    wg = w + (size_t)e * N * K;
+  }
+  // piece i: rows 8 i .. 8 i + 7 of the tile's features, then of its tokens (rows past the edge read the last row again: their products are never stored);
+  // lane l fetches chunk (l & 7) ^ (l >> 3) of row l >> 3, see above
+  const auto wr = tile_rsrc(wg + (size_t)n0 * K, (uint32_t)min(NT * 16, N - n0) * (uint32_t)K * 4u);
+  const auto xr = tile_rsrc(x + (size_t)row0 * ldx, GROUPED ? 0u : (uint32_t)min(MT * 16, row_end - row0) * (uint32_t)ldx * 4u);
+  uint32_t woff[2 * NT], xoff[GROUPED ? 1 : 2 * MT];
+  const float* xp[GROUPED ? 2 * MT : 1];
+  const int k4 = (lane & 7) ^ (lane >> 3);
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i) woff[i] = (uint32_t)min(i * 8 + (lane >> 3), N - 1 - n0) * (uint32_t)K * 4u + k4 * 16;
+#pragma unroll
+  for (int i = 0; i < 2 * MT; ++i) {
+    const int m = min(row0 + i * 8 + (lane >> 3), row_end - 1);
+    if constexpr (GROUPED) xp[i] = x + (row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx + k4 * 4;
+    else xoff[i] = (uint32_t)(m - row0) * (uint32_t)ldx * 4u + k4 * 16;
+  }
+  const int S = K / 32, runs = (S + 1) / 2, mine = runs > wave ? (runs - wave + 7) / 8 : 0;
+  const int n = 2 * mine - (mine && (S & 1) && (runs - 1) % 8 == wave ? 1 : 0);          // this wave's steps
+  char* stage = smem + wave * STEP;
+  auto fetch = [&](int l) {
+    const uint32_t step = (uint32_t)(((l >> 1) * 8 + wave) * 2 + (l & 1));
+#pragma unroll
+    for (int i = 0; i < 2 * NT; ++i) tile_dma(wr, woff[i], step * 128u, stage + i * 1024);
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) {
+      char* lds = stage + (2 * NT + i) * 1024;
+      if constexpr (GROUPED)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xp[i] + step * 32), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+      else
+        tile_dma(xr, xoff[i], step * 128u, lds);
+    }
+  };
+  const uint32_t at0 = (uint32_t)(((lane >> 3) & 1) * 1024 + ((lane & 7) * 8 + ((lane >> 4) ^ (lane & 7))) * 16), at1 = at0 ^ 64u;
+  u32x4_t raw[NT + MT][2];
+  f32x4_t high[MT][NT], low[MT][NT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) high[j][i] = low[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (n > 0) fetch(0);
+  for (int l = 0; l < n; ++l) {
+    tile_wait<0>();
+#pragma unroll
+    for (int i = 0; i < NT + MT; ++i) {
+      raw[i][0] = *reinterpret_cast<const u32x4_t*>(stage + i * 2048 + at0);
+      raw[i][1] = *reinterpret_cast<const u32x4_t*>(stage + i * 2048 + at1);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");               // the stage is free
+    if (l + 1 < n) fetch(l + 1);
+    F32Split a[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) a[i] = f32_split(raw[i][0], raw[i][1]);
+#pragma unroll
+    for (int j = 0; j < MT; ++j) f32_block<NT>(a, f32_split(raw[NT + j][0], raw[NT + j][1]), high[j], low[j]);
+  }
+  __syncthreads();                                                   // nobody reads his stage any more, and nothing lands there
+  f32x4_t* red = reinterpret_cast<f32x4_t*>(smem);
+#pragma unroll
+  for (int j = 0; j < MT; ++j)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) red[((wave * MT + j) * NT + i) * 64 + lane] = high[j][i] + low[j][i];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < (NT * MT + 7) / 8; ++u) {
+    const int at = u * 8 + wave, f = n0 + (at % NT) * 16 + (lane >> 4) * 4, m = row0 + (at / NT) * 16 + (lane & 15);
+    if (at >= NT * MT || m >= row_end || f >= N) continue;
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < F32_CHAINS; ++c) v += red[(c * MT * NT + at) * 64 + lane];
+    if (!(f32_finite(v[0]) && f32_finite(v[1]) && f32_finite(v[2]) && f32_finite(v[3]))) {
+      const float* xm = x + (GROUPED && row_idx ? (long)(row_idx[m] / idx_div) : (long)m) * ldx;
+#pragma unroll 1
+      for (int e = 0; e < 4 && f + e < N; ++e)
+        if (!f32_finite(v[e])) v[e] = f32_plain(wg + (size_t)(f + e) * K, xm, K);
+    }
+    if (vec_out && f + 3 < N && (epi < 3 || epi == 8)) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (epi == 8) v[e] += dg.bias[f + e];
+        if (epi == 1) { v[e] = v[e] > 0.f ? v[e] : 0.f; v[e] = v[e] * v[e]; }
+      }
+      *reinterpret_cast<f32x4_t*>(y + (long)m * ldy + ycol + f) = v;
+    } else {
+#pragma unroll 1
+      for (int e = 0; e < 4 && f + e < N; ++e) store_out<float>(y, m, ldy, ycol + f + e, v[e], epi, dg);
+    }
   }
 }
 
@@ -535,14 +682,14 @@ constexpr int SKINNY_MAX_ROWS = 16, SKINNY_MAX_GROUPED_ROWS = 64;
 //   bf16, fits of 23 products of 40 .. 7000 rows over 2048 .. 14720-wide matrices, rms 8 %: 256 x 256 (features x tokens) has the highest rate, the others fill
 //   the last round of 256 CUs better (4228 x 4096 x 4096: 506 tiles of 192 x 192 137 us, 272 of 256 x 256 199; 2500 x 2048 x 7424: 220 of 192 x 128 79, of 128 x 128
 //   96; 300 x 4096 x 4096: 160 of 128 x 64 29, 66 of 192 x 128 42).  The choice is within 0.1 % of the best shape over these.
-//   fp32, bound by the matrix cores: 64 x 32 fills the chip with a few hundred rows (562 x 2048 x 2048 80 -> 64 us, 568 gathered rows of 8 experts
-//   x 3072 x 2048 146 -> 106).
+//   fp32, fits of 20 .. 3000 rows over 512 .. 4096-wide matrices: 48 or 32 tokens where tiles of 64 leave a round half empty (560 x 2048 x 2048: 384 tiles of
+//   64 x 48 40 us, 288 of 64 x 64 49; 250 x 2048 x 2048: 256 of 64 x 32 18, 128 of 64 x 64 25).
 struct RowTile { int features, tokens; float step[3], full, ends; };       // step[n - 1] for n <= 3, n * full beyond
 constexpr RowTile TILES_BF16[] = {{256, 256, {1.209f, 2.709f, 4.166f}, 1.526f, 10.5f}, {192, 192, {0.773f, 1.900f, 2.534f}, 0.907f, 7.5f},
                                   {128, 128, {0.797f, 0.861f, 1.444f}, 0.512f, 1.5f},  {128, 64, {0.433f, 0.728f, 0.951f}, 0.301f, 1.4f},
                                   {256, 192, {1.104f, 2.384f, 3.590f}, 1.216f, 4.3f},  {256, 160, {0.905f, 2.010f, 3.034f}, 1.036f, 6.5f},
                                   {256, 128, {0.757f, 1.620f, 2.348f}, 0.869f, 5.8f},  {192, 128, {0.618f, 1.207f, 2.060f}, 0.668f, 4.9f}};
-constexpr RowTile TILES_F32[] = {{128, 128, {2.25f, 4.4f, 6.3f}, 2.03f, 0.f}, {64, 64, {0.77f, 1.27f, 1.8f}, 0.54f, 0.f}, {64, 32, {0.45f, 0.71f, 1.0f}, 0.33f, 0.f}};
+constexpr RowTile TILES_F32[] = {{64, 64, {0.33f, 0.68f, 0.97f}, 0.335f, 4.5f}, {64, 32, {0.225f, 0.445f, 0.625f}, 0.212f, 2.5f}, {64, 48, {0.275f, 0.55f, 0.80f}, 0.266f, 3.5f}};
 constexpr int CFG_BF16 = 4, CFG_F32 = 3;          // shapes that ssd_gemm_rows_cfg offers
 template <int COUNT>
 int tile_shape(const RowTile (&tiles)[COUNT], int M, int N, int K, int esz, int G, int E) {
@@ -590,12 +737,14 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
   //  depend on sizes and alignment that do not change with the number of rows only)
   const bool tiled = (f32 ? K % 32 == 0 && K >= 64 : K % 64 == 0 && K >= 128) && K <= (1 << 22) && x_vec && (uintptr_t)w % 16 == 0;
   const int id = idx_div < 1 ? 1 : idx_div;
-  // few rows, or few features: 16-row chunks over the grid as long as that is about what the chip holds at once (64 x 2048 x 2048: 49 us as a
-  // tile, a serial walk of K by few workgroups; a router's 1000 x 8 x 2048 the same 48 us)
+  // few rows, or few features: 16-row chunks over the grid as long as that is about what the chip holds at once (fp32: 512
+  // chunks of 16 x 16 outputs; 64 x 2048 x 2048 16 us, 17 as tiles, 80 rows 25 | 17; 250 x 512 x 2048 13 | 16, 300 rows 23 | 16)
   const int chunks = (M + 15) / 16;
   if (shape >= 0 && (!tiled || shape >= (f32 ? CFG_F32 : CFG_BF16))) return SSD_ERR_SHAPE;
-  if (shape < 0 && tiled && f32 && (offsets ? M <= SKINNY_MAX_GROUPED_ROWS : M <= SKINNY_MAX_ROWS || (long)chunks * ((N + 15) / 16) * G <= 1024)) {
-    SKINNY_GO(float, 4, offsets ? 1 : chunks);
+  if (shape < 0 && tiled && f32 && (offsets ? M <= SKINNY_MAX_GROUPED_ROWS : M <= SKINNY_MAX_ROWS || (long)chunks * ((N + 15) / 16) * G <= 512)) {
+    // (eight waves, a chain each, where no CU gets a second workgroup, as above; the same bits)
+    if ((long)((N + 15) / 16) * (offsets ? (M < E ? M : E) : (long)chunks * G) <= 256 && K > 1024) SKINNY_GO(float, 8, offsets ? 1 : chunks);
+    else SKINNY_GO(float, 4, offsets ? 1 : chunks);
 #undef SKINNY_GO
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
@@ -607,32 +756,39 @@ int launch(const void* x, const void* w, void* y, int M, int N, int K, int epi, 
     const bool out32 = f32 || epi == 0 || epi == 8;
     const int width = epi_pairs(epi) ? 4 : (out32 ? 16 : 8), osz = out32 ? 4 : 2;
     const bool vec_out = (uintptr_t)y % width == 0 && (size_t)ldy * osz % width == 0 && (size_t)gsy * osz % width == 0;
-#define TILE_GO(T, WN, WM, NT, MT, STAGES, GROUPED)                                                                                       \
+#define TILE_GO(WN, WM, NT, MT, STAGES, GROUPED)                                                                                          \
   {                                                                                                                                   \
-    typedef TileLoop<WN, WM, NT, MT, STAGES, 2, sizeof(T) == 4> L;                                                                    \
+    typedef TileLoop<WN, WM, NT, MT, STAGES, 2> L;                                                                                    \
     const int tn = (N + L::WG * 16 - 1) / (L::WG * 16), tm = (M + L::XG * 16 - 1) / (L::XG * 16) + (offsets ? E : 0);                 \
-    hipLaunchKernelGGL((gemm_rows_tile_kernel<T, WN, WM, NT, MT, STAGES, GROUPED>), dim3(tn * tm, G), dim3(64 * L::WAVES), 0,                 \
-                       (hipStream_t)stream, (const T*)x, (const T*)w, y, M, N, K, epi, offsets, E, row_idx, id, ldx, ldy, gsx, gsy,   \
+    hipLaunchKernelGGL((gemm_rows_tile_kernel<WN, WM, NT, MT, STAGES, GROUPED>), dim3(tn * tm, G), dim3(64 * L::WAVES), 0,                \
+                       (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)w, y, M, N, K, epi, offsets, E, row_idx, id, ldx, ldy, gsx, gsy,   \
                        gc, dg, tn, tm, vec_out);                                                                                      \
+  }
+#define F32_GO(MT, GROUPED)                                                                                                               \
+  {                                                                                                                                   \
+    const int tn = (N + 63) / 64, tm = (M + MT * 16 - 1) / (MT * 16) + (offsets ? E : 0);                                             \
+    hipLaunchKernelGGL((gemm_rows_f32_kernel<MT, GROUPED>), dim3(tn * tm, G), dim3(512), 0, (hipStream_t)stream, (const float*)x,          \
+                       (const float*)w, (float*)y, M, N, K, epi, offsets, E, row_idx, id, ldx, ldy, gsx, gsy, dg, tn, tm, vec_out);    \
   }
 #define TILE_SHAPES(GROUPED)                                                \
   {                                                                         \
-    if (f32 && shape == 0) TILE_GO(float, 2, 2, 4, 4, 2, GROUPED)           \
-    else if (f32 && shape == 1) TILE_GO(float, 2, 2, 2, 2, 2, GROUPED)      \
-    else if (f32) TILE_GO(float, 2, 2, 2, 1, 4, GROUPED)                    \
-    else if (shape == 0) TILE_GO(bf16_t, 4, 2, 4, 8, 2, GROUPED)            \
-    else if (shape == 1) TILE_GO(bf16_t, 4, 2, 3, 6, 3, GROUPED)            \
-    else if (shape == 2) TILE_GO(bf16_t, 2, 2, 4, 4, 2, GROUPED)            \
-    else if (shape == 3) TILE_GO(bf16_t, 2, 2, 4, 2, 3, GROUPED)            \
-    else if (shape == 4) TILE_GO(bf16_t, 4, 2, 4, 6, 2, GROUPED)            \
-    else if (shape == 5) TILE_GO(bf16_t, 4, 2, 4, 5, 3, GROUPED)            \
-    else if (shape == 6) TILE_GO(bf16_t, 4, 2, 4, 4, 3, GROUPED)            \
-    else TILE_GO(bf16_t, 4, 2, 3, 4, 3, GROUPED)                            \
+    if (f32 && shape == 0) F32_GO(4, GROUPED)                               \
+    else if (f32 && shape == 1) F32_GO(2, GROUPED)                          \
+    else if (f32) F32_GO(3, GROUPED)                                        \
+    else if (shape == 0) TILE_GO(4, 2, 4, 8, 2, GROUPED)                    \
+    else if (shape == 1) TILE_GO(4, 2, 3, 6, 3, GROUPED)                    \
+    else if (shape == 2) TILE_GO(2, 2, 4, 4, 2, GROUPED)                    \
+    else if (shape == 3) TILE_GO(2, 2, 4, 2, 3, GROUPED)                    \
+    else if (shape == 4) TILE_GO(4, 2, 4, 6, 2, GROUPED)                    \
+    else if (shape == 5) TILE_GO(4, 2, 4, 5, 3, GROUPED)                    \
+    else if (shape == 6) TILE_GO(4, 2, 4, 4, 3, GROUPED)                    \
+    else TILE_GO(4, 2, 3, 4, 3, GROUPED)                                    \
   }
     // (a dense product's rows are 32-bit offsets from the tile's first; rows so far apart that they don't reach go like gathered ones, by pointer)
     if (offsets || 256L * ldx * esz0 > 0x7fffffffL) TILE_SHAPES(true) else TILE_SHAPES(false)
 #undef TILE_SHAPES
 #undef TILE_GO
+#undef F32_GO
     return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
   }
   const int tiles_m = (M + BM - 1) / BM + (offsets ? E : 0);

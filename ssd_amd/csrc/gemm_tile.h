@@ -1,4 +1,4 @@
-// The main loop of the large-tile GEMMs (many token rows: prefill): a workgroup owns (WN * NT) 16-row groups of W and (WM * MT)
+// The main loop of the large-tile bf16 GEMMs (many token rows: prefill): a workgroup owns (WN * NT) 16-row groups of W and (WM * MT)
 // 16-row groups of x, its WN x WM waves NT x MT of them each, and leaves the fp32 products in acc[NT][MT].
 //
 // What bounds it is the matrix cores, and how much of their time the operands' way to them takes.  Both operands travel HBM / L2 -> LDS by DMA (loads
@@ -10,8 +10,8 @@
 // second set).  Measured, MI355X, 256 x 256, us per k-block of a full chip: everything 0.75, without the DMA 0.62, MFMAs alone 0.55 (the clock that the
 // matrix cores leave: 0.43 at 2.4 GHz), without the MFMAs 0.42; sixteen waves that read a block just before they multiply it 0.80.  16384 x 4096 x 14336
 // 1425 -> 1355 us (1.42 PFLOP/s).  (32x32x16 MFMAs 0.83, s_setprio around them 0.79, waves of 8 x 8 spill.)
-// In bf16 every accumulator is one chain over the ascending k of the range that its workgroup walks, whatever the tile: where the caller does not cut K
-// (gemm_rows.hip), a row's result does not depend on the rows beside it; ssd_gemm_big's K splits go by the number of rows.  fp32: see below.
+// Every accumulator is one chain over the ascending k of the range that its workgroup walks, whatever the tile: where the caller does not cut K
+// (gemm_rows.hip), a row's result does not depend on the rows beside it; ssd_gemm_big's K splits go by the number of rows.
 #pragma once
 #include "common.h"
 
@@ -29,17 +29,7 @@ __device__ __forceinline__ void tile_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// fp32 products (mfma 16x16x4: a lane holds ONE k of its row; peak 157 TFLOP/s, twice the vector unit's without packed fp32).  The order of
-// a sum is part of what the fp32 mode promises -- a row's result is the same bits whichever kernel computes it -- and is defined here:
-// segments of F32_SEG k (the last one shorter), each a chain from zero over its blocks of 16 k, a block being four MFMAs, the e-th over
-// k = e, 4 + e, 8 + e, 12 + e (lane q of a row holds 4 consecutive k: one 16-byte load); the segments' sums are added in order, from zero.
-constexpr int F32_SEG = 256, F32_SEG_STEPS = F32_SEG / 32;
-__device__ __forceinline__ f32x4_t mfma_f32(uint32_t a, uint32_t b, f32x4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a), __uint_as_float(b), c, 0, 0, 0);
-}
-
-// F32: operands are floats, a step is 32 k (KS = 2), `acc` the sum over segments.
-template <int WN, int WM, int NT, int MT, int STAGES, int KS = 1, bool F32 = false>
+template <int WN, int WM, int NT, int MT, int STAGES, int KS = 1>
 struct TileLoop {
   static constexpr int WAVES = WN * WM, WG = WN * NT, XG = WM * MT;          // waves; 16-row groups of W, of x
   static constexpr int OPS = (WG + XG) * KS, STEP = OPS * 1024;                 // 1 KiB operands, LDS bytes of a k-step
@@ -58,13 +48,6 @@ struct TileLoop {
     for (int i = 0; i < NT; ++i)
 #pragma unroll
       for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    f32x4_t part[F32 ? NT : 1][F32 ? MT : 1];
-    if constexpr (F32) {
-#pragma unroll
-      for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
     auto fetch = [&](int step, uint32_t buf) {
 #pragma unroll
       for (int i = 0; i < PER; ++i) fetch_one(i, step, smem + buf * STEP + op_of(wave, i) * 1024);
@@ -79,26 +62,17 @@ struct TileLoop {
       for (int j = 0; j < MT; ++j) rb[j] = *reinterpret_cast<const u32x4_t*>(b0 + j * KS * 1024);
     };
     auto multiply = [&](const u32x4_t (&ra)[NT], const u32x4_t (&rb)[MT]) {
-      if constexpr (F32) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+      for (int i = 0; i < NT; ++i)
 #pragma unroll
-          for (int i = 0; i < NT; ++i)
+        for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(ra[i], rb[j], acc[i][j]);
+      // the reads of the next block between this one's MFMAs
 #pragma unroll
-            for (int j = 0; j < MT; ++j) part[i][j] = mfma_f32(ra[i][e], rb[j][e], part[i][j]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-          for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(ra[i], rb[j], acc[i][j]);
-        // the reads of the next block between this one's MFMAs
-#pragma unroll
-        for (int r = 0; r < NT + MT; ++r) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, NT * MT / (NT + MT), 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, NT * MT, 0);
+      for (int r = 0; r < NT + MT; ++r) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, NT * MT / (NT + MT), 0);
       }
+      __builtin_amdgcn_sched_group_barrier(0x008, NT * MT, 0);
     };
     // (past the end the last step is fetched again, into a buffer that nobody reads for a product, so that the count of loads in flight stays static)
 #pragma unroll
@@ -117,14 +91,6 @@ struct TileLoop {
       cur = cur + 1 == STAGES ? 0 : cur + 1;
       read(a[h ^ 1], b[h ^ 1], cur, 0);
       multiply(a[h], b[h]);
-      if constexpr (F32) {
-        if ((k + 1) % F32_SEG_STEPS == 0 || k + 1 == nk) {
-#pragma unroll
-          for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int j = 0; j < MT; ++j) { acc[i][j] += part[i][j]; part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f}; }
-        }
-      }
     };
     if constexpr (KS == 1) {
       for (int k = 0; k < nk; k += 2) {

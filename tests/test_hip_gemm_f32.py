@@ -1,0 +1,94 @@
+"""fp32 products on the bf16 matrix cores (csrc/gemm_f32.h, the fp32 forms of csrc/gemm_rows.hip) against fp64: every tile shape and both few-row forms
+where K is less than a round of the chains, a part of one, and many; floats at the ends of their range; infinities and NaN as plain fp32 products give them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def H():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ssd_amd.hip import ops
+    return ops
+
+
+def operands(M, N, K, seed=0):
+    g = torch.Generator().manual_seed(M + N + K + seed)
+    return torch.randn(M, K, generator=g).cuda(), (torch.randn(N, K, generator=g) / K ** 0.5).cuda()
+
+
+# What is left out of a product is below 3 * 2^-24 of it; a sum's roundings are one per 32 k in a chain of K / 8, of partial sums below 6: for K <= 2^13,
+# 2^-24 * (3 * sum |x w| + 6 * (K / 256 + 8)) with sum |x w| below sqrt(K)
+def bound(K):
+    return 2.0 ** -24 * (3 * K ** 0.5 + 6 * (K / 256 + 8))
+
+
+@pytest.mark.parametrize("K", [64, 96, 480, 512, 544, 1056, 2080, 7424])
+def test_forms(H, K):
+    N = 130
+    for M in (1, 5, 16, 33, 65):
+        x, w = operands(M, N, K)
+        ref = x.double() @ w.double().T
+        y = torch.full((M, N), 7.0, device="cuda")
+        H.gemm_rows(x, w, y, M, N, K, True, 0)
+        assert float((y.double() - ref).abs().max()) <= bound(K), (M, K)
+        for shape in range(3):
+            z = torch.full((M, N), 7.0, device="cuda")
+            H.gemm_rows_cfg(x, w, z, M, N, K, True, shape, 0)
+            assert torch.equal(z, y), (M, K, shape)
+
+
+def test_wide_weights_few_rows(H):
+    """Four waves with two chains each (many workgroups) and eight with one (few) give a row the same bits."""
+    K = 2048
+    x, w = operands(3, 8192, K)
+    wide, narrow = torch.zeros(3, 8192, device="cuda"), torch.zeros(3, 1024, device="cuda")
+    H.gemm_rows(x, w, wide, 3, 8192, K, True, 0)
+    H.gemm_rows(x, w[:1024].contiguous(), narrow, 3, 1024, K, True, 0)
+    assert torch.equal(wide[:, :1024], narrow)
+    assert float((wide.double() - x.double() @ w.double().T).abs().max()) <= bound(K)
+
+
+@pytest.mark.parametrize("M", [3, 70])
+def test_not_finite(H, M):
+    """One infinity, NaN (its payload in the low bits), a pair of infinities of either sign, an overflow: where the plain sum is finite the product is, where it
+    is an infinity it is that one, where it is NaN it is NaN; other rows keep their bits."""
+    N, K = 70, 256
+    x, w = operands(M, N, K)
+    clean = torch.zeros(M, N, device="cuda")
+    H.gemm_rows(x, w, clean, M, N, K, True, 0)
+    x[0, 5] = float("inf")
+    x[1, 7:8].view(torch.int32).fill_(0x7f800001)
+    x[2, 9], x[2, 10] = float("inf"), float("-inf")
+    w[3, :] = 0.0
+    w[4, 11] = float("-inf")
+    if M > 3:
+        x[M - 1, 20], w[5, 20] = 2e38, 4.0
+    y = torch.zeros(M, N, device="cuda")
+    H.gemm_rows(x, w, y, M, N, K, True, 0)
+    want = x.double().cpu() @ w.double().cpu().T                     # (overflow to fp32 infinities happens on the conversion)
+    want = want.float()
+    got = y.cpu()
+    assert bool((got.isnan() == want.isnan()).all())
+    assert bool((got.isinf() == want.isinf()).all()) and bool((got[want.isinf()] == want[want.isinf()]).all())
+    cols = [n for n in range(N) if n not in (3, 4, 5)]
+    assert torch.equal(y[3:M - 1][:, cols], clean[3:M - 1][:, cols])
+
+
+def test_ends_of_the_range(H):
+    """Floats just below the largest (which round past the largest bf16) times tiny ones, products of moderate size; and tiny ones alone, whose parts below
+    the smallest normal number may be lost."""
+    M, N, K = 40, 33, 64
+    x, w = operands(M, N, K)
+    big = x.sign() * 3.4e38
+    tiny = w * 1e-38
+    y = torch.zeros(M, N, device="cuda")
+    H.gemm_rows(big, tiny, y, M, N, K, True, 0)
+    ref = big.double() @ tiny.double().T
+    # (terms of about 3.4 * K^-1/2; parts of a weight of 1e-38 that are flushed: 2^-126 of it lost at most, times 3.4e38)
+    assert float((y.double() - ref).abs().max()) <= 4 * bound(K) * 3.4 + K * 3.4e38 * 2.0 ** -126
+    small = x * 1e-20
+    H.gemm_rows(small, small[:N].contiguous(), y, M, N, K, True, 0)
+    assert float((y.double() - small.double() @ small[:N].double().T).abs().max()) <= K * 2.0 ** -126
