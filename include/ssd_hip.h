@@ -31,7 +31,7 @@ extern "C" {
 
 /* Bumped whenever a signature or a semantic of this header changes; ssd_abi_version() returns the value the library was built
  * with, so a consumer compiled against another header can tell (tests/abi_consumer.c does). */
-#define SSD_HIP_ABI_VERSION 9
+#define SSD_HIP_ABI_VERSION 10
 
 #define SSD_OK 0
 #define SSD_ERR_SHAPE (-1)
@@ -323,6 +323,12 @@ int ssd_fork_topf_split(const void* logits_rows, long ld, int V, const int64_t* 
  * r = req_keys[r][0..2] (int64 [B][3]: seq id, accepted length - 1, recovery token), or -1. */
 int ssd_cache_lookup(const int64_t* req_keys, const int64_t* cache_seq, const int32_t* cache_j, const int64_t* cache_forks,
                      int B, int Bc, int W, int32_t* out_idx, void* stream);
+
+/* Up to ten copies between pinned host memory (hipHostMalloc) and device memory in one launch, in either direction: the host-to-device copies of
+ * prepare_decode_tensors_from_seqs / prepare_prefill_tensors_from_seqs (ssd/engine/helpers/runner_helpers.py:50-180) and a step's read-back.  Segment i:
+ * words[i] 4-byte words (0: none; fewer than 2^29) from src[i] to dst[i], both 16-byte aligned.  The three arrays are read before the call returns; a host
+ * buffer may be rewritten, or read, once the stream has passed the launch. */
+int ssd_copy_segments(const void* const* src, void* const* dst, const int32_t* words, int n, void* stream);
 
 /* Device-side replacement for the host loop body of SpeculatorSync.speculate --
  * ssd/engine/speculator_sync.py:47-66 (+ runner_helpers.py:59-75): append the sampled token, bump

@@ -103,6 +103,52 @@ extern "C" int ssd_store_step_rows(const void* src_rows, long src_ld, void* dst,
 }
 
 
+// A step's inputs from pinned host memory to the device buffers that the kernels read, or its results back, all of them in one launch: a copy each took
+// 3 to 5 us on the device and a gap before it (six of them before a decoded token: 60 us of 820).  Loads and stores go past the caches, at system scope:
+// pinned memory is rewritten by the host between launches and read by it after them.  Bound by the link's latency (about 3 us) up to a few dozen KiB.
+constexpr int MAX_SEGMENTS = 10;
+struct Segments { const char* src[MAX_SEGMENTS]; char* dst[MAX_SEGMENTS]; int words[MAX_SEGMENTS]; int n; };
+
+__global__ void __launch_bounds__(256) copy_segments_kernel(Segments s) {
+  constexpr int SYSTEM = 17;                             // sc0 | sc1
+  long at = (long)blockIdx.x * 256 + threadIdx.x;        // 16-byte chunk over all segments
+  const long step = (long)gridDim.x * 256;
+  for (int i = 0; i < s.n; ++i) {
+    const long chunks = (s.words[i] + 3) >> 2;
+    const auto from = __builtin_amdgcn_make_buffer_rsrc((void*)s.src[i], 0, s.words[i] * 4, 0x00020000);
+    const auto to = __builtin_amdgcn_make_buffer_rsrc((void*)s.dst[i], 0, s.words[i] * 4, 0x00020000);
+    for (; at < chunks; at += step) {
+      if (at * 4 + 3 < s.words[i]) {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_amdgcn_raw_buffer_load_b128(from, (int)(at * 16), 0, SYSTEM), to, (int)(at * 16), 0, SYSTEM);
+      } else {
+        for (long w = at * 4; w < s.words[i]; ++w)
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_amdgcn_raw_buffer_load_b32(from, (int)(w * 4), 0, SYSTEM), to, (int)(w * 4), 0, SYSTEM);
+      }
+    }
+    at -= chunks;
+  }
+}
+
+extern "C" int ssd_copy_segments(const void* const* src, void* const* dst, const int32_t* words, int n, void* stream) {
+  if (!src || !dst || !words) return SSD_ERR_ARG;
+  if (n < 1 || n > MAX_SEGMENTS) return SSD_ERR_SHAPE;
+  Segments s;
+  long chunks = 0;
+  s.n = 0;
+  for (int i = 0; i < n; ++i) {
+    if (words[i] == 0) continue;
+    if (words[i] < 0 || words[i] >= (1 << 29)) return SSD_ERR_SHAPE;
+    if (!src[i] || !dst[i] || (uintptr_t)src[i] % 16 || (uintptr_t)dst[i] % 16) return SSD_ERR_ARG;
+    s.src[s.n] = (const char*)src[i];
+    s.dst[s.n] = (char*)dst[i];
+    s.words[s.n++] = words[i];
+    chunks += (words[i] + 3) / 4;
+  }
+  if (chunks == 0) return SSD_OK;
+  hipLaunchKernelGGL(copy_segments_kernel, dim3((unsigned)(chunks < 256 * 512 ? (chunks + 255) / 256 : 512)), dim3(256), 0, (hipStream_t)stream, s);
+  return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
+}
+
 // hipGraph capture for a host that is not PyTorch (the reference captures its decode / verify / glue / tree steps with torch.cuda.CUDAGraph,
 // ssd/engine/helpers/cudagraph_helpers.py:20-120; this repo's engine does the same through torch on ROCm, where that IS hipGraph): every
 // entry point of this library only enqueues on `stream`, so whatever sequence of calls lies between begin and end becomes one replayable

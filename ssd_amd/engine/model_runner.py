@@ -53,6 +53,36 @@ def model_class(family: str):
     return HipDecoder
 
 
+class InputStage:
+    """Pinned host regions of a runner's static inputs: put() fills one, send() copies what was filled since to the device, one launch for
+    all of them.  The host may fill them again once the stream has passed the launch."""
+
+    def __init__(self, inputs: dict[str, torch.Tensor]):
+        self._host = {k: torch.zeros(t.shape, dtype=t.dtype).pin_memory() for k, t in inputs.items()}
+        self._view = {k: t.numpy() for k, t in self._host.items()}
+        self._at = {k: i for i, k in enumerate(inputs)}
+        self._copies = H.SegmentCopies([(self._host[k], t) for k, t in inputs.items()])
+
+    def put(self, name: str, values, at: int = 0) -> None:
+        """values -> rows at .. of input `name`; what lies before them has to be filled as well."""
+        v, n = self._view[name], at + len(values)
+        v[at:n] = values
+        self._copies.words[self._at[name]] = n * (v.nbytes // v.shape[0] // 4)
+
+    def put_tables(self, name: str, tables) -> None:
+        """Lists of different lengths -> rows, -1 behind each."""
+        v = self._view[name]
+        for i, t in enumerate(tables):
+            v[i, :len(t)] = t
+            v[i, len(t):] = -1
+        self._copies.words[self._at[name]] = len(tables) * v.shape[1]
+
+    def send(self) -> None:
+        self._copies.launch()
+        for i in range(self._copies.n):
+            self._copies.words[i] = 0
+
+
 class ModelRunner:
     PREFILL_GRAPHS = 4              # prefill shapes kept as hipGraphs
     PREFILL_GRAPH_MAX_T = 1024      # longer prefills are GPU-bound by far: launch overhead does not matter
@@ -143,6 +173,7 @@ class ModelRunner:
         self.d_bt = torch.zeros(B, self.max_blocks, dtype=torch.int32, **dev)
         # recurrent-state slots of the batch's sequences (models with recurrent layers; the block manager hands the slots out)
         self.d_state = torch.zeros(B, dtype=torch.int32, **dev) if getattr(self.model, "state_slots", 0) else None
+        self.d_temps = torch.zeros(B, dtype=torch.float32, **dev)       # temperatures this model samples with
         self.d_next = torch.zeros(max(self.max_decode_tokens, B), dtype=torch.int64, **dev)
         self.d_spec = torch.zeros(B, self.K + 1, dtype=torch.int64, **dev)
         self.d_step = torch.zeros(1, dtype=torch.int32, **dev)
@@ -156,6 +187,15 @@ class ModelRunner:
         watchdog.stage("engine_init")           # (whatever the set-up's outcome: its stage limits end here)
         self._stage: dict = {}
         self._stage_set = 0
+        inputs = dict(ids=self.d_ids, pos=self.d_pos, slots=self.d_slots, ctx=self.d_ctx, cu_q=self.d_cu_q, gather=self.d_gather, bt=self.d_bt,
+                      temps=self.d_temps)
+        if self.d_state is not None:
+            inputs["state"] = self.d_state
+        self._inputs, self._input_stages = inputs, {}
+        # what a step reads back: its tokens or its packed verify result, and the error word of the resident segments
+        err = [(self.model.chain_err, self._chain_err_host)] if self._has_chain_err() else []
+        self._tokens_back = H.SegmentCopies([(self.d_next, self.h_next), *err])
+        self._packed_back = H.SegmentCopies([(self.d_packed, self.h_packed), *err])
         self._ctx_hint = 4096
         self.graphs: dict = {}
         self._prefill_seen: dict = {}      # prefill shapes met once (run eagerly); a shape is captured when it comes back
@@ -211,7 +251,6 @@ class ModelRunner:
         B, K, V = self.seq_cap, max(self.K, 1), self.cfg.vocab_size
         dev = dict(device=self.device)
         self.d_rng = torch.tensor([0x5D5D0000 + (7 if self.is_draft else 3) + 1000 * self.config.weights_seed], dtype=torch.int64, **dev)
-        self.d_temps = torch.zeros(B, dtype=torch.float32, **dev)       # temperatures this model samples with
         self.d_temps_q = torch.zeros(B, dtype=torch.float32, **dev)     # (target) the draft's temperatures
         self.d_ratio = torch.zeros(B, dtype=torch.int32, **dev)
         self.d_lse_p = torch.zeros(B * (K + 1), dtype=torch.float32, **dev)
@@ -225,12 +264,13 @@ class ModelRunner:
             rows = max(B * K, self.max_bs * getattr(self.config, "MQ_LEN", 1))
             self.d_boost = torch.zeros(rows, self.sx_k, dtype=torch.int32, **dev)
 
-    def _check_collectives(self) -> None:
+    def _check_collectives(self, posted: bool = False) -> None:
+        """posted: the error word has come back with the step's results (_read_back)."""
         ar = self.model.custom_ar
         if ar is not None and ar.failed():
             raise RuntimeError("one-shot all-reduce timed out waiting for a peer; results of this step are invalid "
                                "(rerun with SSD_CUSTOM_AR=0 to use RCCL)")
-        if self._has_chain_err() and (int(self._chain_err_host[0]) or int(self.model.chain_err.item())):
+        if self._has_chain_err() and (int(self._chain_err_host[0]) or (not posted and int(self.model.chain_err.item()))):
             self._raise_chain_err()
 
     # The resident layer segments (csrc/chain.hip, csrc/tree_segment.hip) report a given-up bounded wait in a device word.  The
@@ -287,50 +327,53 @@ class ModelRunner:
             stage[:n] = torch.from_numpy(values) if isinstance(values, np.ndarray) else torch.tensor(values, dtype=dtype)
             dst[:n].copy_(stage[:n], non_blocking=True)
 
-    def _upload_block_tables(self, seqs) -> None:
+    def _input_stage(self) -> InputStage:
+        """The pinned regions that the batch being prepared is written to (see _upload for the second set)."""
+        stage = self._input_stages.get(self._stage_set)
+        if stage is None:
+            stage = self._input_stages[self._stage_set] = InputStage(self._inputs)
+        return stage
+
+    def _put_block_tables(self, stage: InputStage, seqs) -> None:
         if self.d_state is not None:
             slots = [s.state_slot for s in seqs]
             assert all(0 <= x < self.model.state_slots for x in slots), "a sequence of a recurrent model runs without a state slot"
-            self._upload(self.d_state, slots, torch.int32)
-        rows = []
-        for s in seqs:
-            t = self._table(s)
-            assert len(t) <= self.max_blocks
-            rows.append(t + [-1] * (self.max_blocks - len(t)))
-        self._upload(self.d_bt, rows, torch.int32)
+            stage.put("state", slots)
+        tables = [self._table(s) for s in seqs]
+        assert all(len(t) <= self.max_blocks for t in tables)
+        stage.put_tables("bt", tables)
 
-    def _prepare_prefill(self, seqs) -> tuple[int, int]:
+    def _prepare_prefill(self, seqs, temps=None) -> tuple[int, int]:
         """prepare_prefill_tensors_from_seqs (runner_helpers.py:123-180): new tokens of each sequence, their
         positions and slots; context length = whole sequence (keys already cached by a prefix hit included).  The device waits for
         this: positions and slots are computed as arrays (16384 tokens: 2.6 -> 0.5 ms)."""
-        ids, pos, slots, ctx, cu, gather = [], [], [], [], [0], []
+        ctx, cu, gather = [], [0], []
         max_q = 0
-        for s in seqs:
-            cached = s.num_draft_cached_tokens if self.is_draft else s.num_cached_tokens
-            n = len(s)
-            assert cached < n, "fully cached prompt: nothing to prefill"
-            table = self._table(s)
-            ids.extend(s[cached:])
-            p = np.arange(cached, n)
-            pos.append(p)
-            slots.append(self._slot(np.array(table, dtype=np.int64), p))
+        cached = [s.num_draft_cached_tokens if self.is_draft else s.num_cached_tokens for s in seqs]
+        assert sum(len(s) - c for s, c in zip(seqs, cached)) <= self.d_ids.numel(), "prefill exceeds max_num_batched_tokens"
+        stage = self._input_stage()
+        for s, c in zip(seqs, cached):
+            n, at = len(s), cu[-1]
+            assert c < n, "fully cached prompt: nothing to prefill"
+            p = np.arange(c, n)
+            stage.put("ids", s[c:], at)
+            stage.put("pos", p, at)
+            stage.put("slots", self._slot(np.array(self._table(s), dtype=np.int64), p), at)
             ctx.append(n)
-            cu.append(cu[-1] + n - cached)
+            cu.append(at + n - c)
             gather.append(cu[-1] - 1)
-            max_q = max(max_q, n - cached)
-        T = len(ids)
-        assert T <= self.d_ids.numel(), "prefill exceeds max_num_batched_tokens"
+            max_q = max(max_q, n - c)
         self._note_ctx(max(ctx))
-        self._upload(self.d_ids, np.array(ids, dtype=np.int64), torch.int64)
-        self._upload(self.d_pos, np.concatenate(pos), torch.int64)
-        self._upload(self.d_slots, np.concatenate(slots), torch.int32)
-        self._upload(self.d_ctx, ctx, torch.int32)
-        self._upload(self.d_cu_q, cu, torch.int32)
-        self._upload(self.d_gather, gather, torch.int32)
-        self._upload_block_tables(seqs)
-        return T, max_q
+        stage.put("ctx", ctx)
+        stage.put("cu_q", cu)
+        stage.put("gather", gather)
+        if temps is not None:
+            stage.put("temps", temps)
+        self._put_block_tables(stage, seqs)
+        stage.send()
+        return cu[-1], max_q
 
-    def _prepare_decode(self, seqs, back: int = 0) -> int:
+    def _prepare_decode(self, seqs, back: int = 0, temps=None) -> int:
         """Single-token decode inputs (runner_helpers.py:59-75).  back = 1 feeds the token BEFORE the last one (the
         deferred KV deposit of a fully accepted draft chain, see deposit_pending)."""
         ids, pos, slots, ctx = [], [], [], []
@@ -343,11 +386,15 @@ class ModelRunner:
             ctx.append(p + 1)
             slots.append(self._slot(self._table(s), p))
         self._note_ctx(max(ctx) + self.K + 1)
-        self._upload(self.d_ids, ids, torch.int64)
-        self._upload(self.d_pos, pos, torch.int64)
-        self._upload(self.d_slots, slots, torch.int32)
-        self._upload(self.d_ctx, ctx, torch.int32)
-        self._upload_block_tables(seqs)
+        stage = self._input_stage()
+        stage.put("ids", ids)
+        stage.put("pos", pos)
+        stage.put("slots", slots)
+        stage.put("ctx", ctx)
+        if temps is not None:
+            stage.put("temps", temps)
+        self._put_block_tables(stage, seqs)
+        stage.send()
         return len(seqs)
 
     def _prepare_verify(self, seqs, ids_from_seq: bool) -> int:
@@ -365,12 +412,14 @@ class ModelRunner:
             slots.extend(self._slot(table, p) for p in range(pos0, pos0 + K + 1))
             ctx.append(len(s))
         self._note_ctx(max(ctx))
+        stage = self._input_stage()
         if ids_from_seq:
-            self._upload(self.d_ids, ids, torch.int64)
-        self._upload(self.d_pos, pos, torch.int64)
-        self._upload(self.d_slots, slots, torch.int32)
-        self._upload(self.d_ctx, ctx, torch.int32)
-        self._upload_block_tables(seqs)
+            stage.put("ids", ids)
+        stage.put("pos", pos)
+        stage.put("slots", slots)
+        stage.put("ctx", ctx)
+        self._put_block_tables(stage, seqs)
+        stage.send()
         return len(seqs) * (K + 1)
 
     # ---------------------------------------------------------------------------------------------
@@ -495,7 +544,8 @@ class ModelRunner:
             return toks
         self._acts_sliced = None
         if is_prefill:
-            T, max_q = self._prepare_prefill(seqs)
+            temps = self._sampling_temps(seqs)
+            T, max_q = self._prepare_prefill(seqs, temps)
 
             def body():
                 self.model.forward(self.d_ids, self.d_pos, T, self._meta("prefill", B, max_q))
@@ -521,7 +571,7 @@ class ModelRunner:
                         del self.graphs[k]
                 self._launch(key, body)             # "captured": the eager warm-up run already produced this call's result
             self._log_margins(B, [(s.seq_id, len(s)) for s in seqs])
-            self._sample_or_argmax(seqs, B)
+            self._sample_or_argmax(temps, B)
             toks = self._read_tokens(B)
             return (toks, self.model.full_logits(B)) if draft_return_logits else toks
         if not last_only:
@@ -530,17 +580,16 @@ class ModelRunner:
                 self._prepare_verify(seqs, ids_from_seq=True)
                 self.graphs[("verify_logits", B, self._ctx_hint)].replay()
             return self.model.full_logits(T)
-        self._prepare_decode(seqs)
-        temps = self._seq_temps(seqs)
+        temps = self._sampling_temps(seqs)
+        self._prepare_decode(seqs, temps=temps)
         # the call that captures a graph has already run the step eagerly (the warm-up).  Models whose memory is cache pages run it
         # once more through the new graph (the same rows land in the same slots); a recurrent state would absorb the token twice,
         # so such models keep the warm-up's result
         rerun = not getattr(self.model, "state_slots", 0)
-        if any(t > 0 for t in temps):       # autoregressive sampling (AutoRegressiveStep at temperature > 0)
+        if temps is not None:               # autoregressive sampling (AutoRegressiveStep at temperature > 0)
             self._ensure_stochastic()
-            self._upload(self.d_temps, temps, torch.float32)
             if self._launch(("decode_s", B), lambda: self._body_decode(B, False, sample=True)) == "captured" and rerun:
-                self._prepare_decode(seqs)
+                self._prepare_decode(seqs, temps=temps)
                 self.graphs[("decode_s", B, self._ctx_hint)].replay()
         elif self._launch(("decode", B), lambda: self._body_decode(B, False)) == "captured" and rerun:
             self._prepare_decode(seqs)
@@ -603,11 +652,15 @@ class ModelRunner:
         return [float(s.draft_temperature) if (self.is_draft and s.draft_temperature is not None) else float(s.temperature)
                 for s in seqs]
 
-    def _sample_or_argmax(self, seqs, B: int) -> None:
+    def _sampling_temps(self, seqs) -> list[float] | None:
+        """The batch's temperatures, None where all of them are 0 (greedy)."""
         temps = self._seq_temps(seqs)
-        if any(t > 0 for t in temps):
+        return temps if any(t > 0 for t in temps) else None
+
+    def _sample_or_argmax(self, temps, B: int) -> None:
+        """temps: those that the inputs were prepared with (_sampling_temps)."""
+        if temps is not None:
             self._ensure_stochastic()
-            self._upload(self.d_temps, temps, torch.float32)
             V = self.cfg.vocab_size
             H.sample_rows(self.model.full_logits(B), V, B, V, self.d_temps, 1, self.d_rng, 3, self.d_next)
             H.rng_advance(self.d_rng)
@@ -615,10 +668,17 @@ class ModelRunner:
             self.model.argmax(B, self.d_next)
 
     def _read_tokens(self, n: int) -> list[int]:
-        self.h_next[:n].copy_(self.d_next[:n], non_blocking=True)
+        self._read_back(self._tokens_back, 2 * n)
         torch.cuda.current_stream().synchronize()
-        self._check_collectives()
+        self._check_collectives(posted=True)
         return self.h_next[:n].tolist()
+
+    def _read_back(self, copies, words: int) -> None:
+        """A step's results, and the error word, on their way to pinned memory (in one launch)."""
+        copies.words[0] = words
+        if copies.n > 1:
+            copies.words[1] = 1
+        copies.launch()
 
     # ---- fast path of synchronous speculation: no host sync until the verify result ----
     @torch.inference_mode()
@@ -636,11 +696,9 @@ class ModelRunner:
             self._ensure_stochastic()
 
         def stage():
-            self._prepare_decode(seqs)
+            self._prepare_decode(seqs, temps=temps if sample else None)
             self.d_step.zero_()
             self.d_spec[:B, 0].copy_(self.d_ids[:B])
-            if sample:
-                self._upload(self.d_temps, temps, torch.float32)
 
         def chain():                     # all K forwards in ONE hipGraph: no host gap between them
             for _ in range(K):
@@ -705,14 +763,14 @@ class ModelRunner:
             stage()
             self.graphs[(*key, self._ctx_hint)].replay()
         self._log_margins(B * (K + 1), [(s.seq_id, s.num_tokens - (K + 1) + j + 1) for s in seqs for j in range(K + 1)])
-        self.h_packed[:B].copy_(self.d_packed[:B], non_blocking=True)
+        self._read_back(self._packed_back, 2 * B * (K + 3))
         # the verify is in flight and the host is about to block on it: the moment for a co-located draft server to
         # enqueue its next round on its own stream (engine/draft_runner.py run_deferred)
         hook = getattr(self, "overlap_hook", None)
         if hook is not None:
             hook()
         torch.cuda.current_stream().synchronize()
-        self._check_collectives()
+        self._check_collectives(posted=True)
         rows = self.h_packed[:B].tolist()
         suffixes = [r[2:3 + r[0]] for r in rows]
         recovery = [r[1] for r in rows]

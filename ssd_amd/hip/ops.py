@@ -6,6 +6,8 @@ hipGraph-capturable).  No function in this module computes anything in torch.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from .lib import load_library, SsdHipError
@@ -346,6 +348,23 @@ def fork_topf_split(logits, ld: int, V: int, returned, counts, offsets, B: int, 
     """ssd_fork_topf spread over the chip (per-slice candidates + merge): bit-equal, ~10x shorter on the draft's critical path."""
     _check(load_library().ssd_fork_topf_split(_p(logits), ld, V, _p(returned), _p(counts), _p(offsets), B, K, mq, _p(workspace), _p(out),
                                               _stream()), "ssd_fork_topf_split")
+
+
+class SegmentCopies:
+    """Up to ten fixed (source, destination) pairs, one of each pair in pinned host memory, copied in one launch; the tensors stay alive here."""
+
+    def __init__(self, pairs):
+        n = len(pairs)
+        assert 0 < n <= 10 and all((a.is_cuda or a.is_pinned()) and (b.is_cuda or b.is_pinned()) and a.is_contiguous() and b.is_contiguous()
+                                  and a.nbytes == b.nbytes and a.nbytes % 4 == 0 for a, b in pairs)
+        self.pairs, self.n = list(pairs), n
+        self.words = (ctypes.c_int32 * n)()
+        self._src = (ctypes.c_void_p * n)(*(a.data_ptr() for a, _ in pairs))
+        self._dst = (ctypes.c_void_p * n)(*(b.data_ptr() for _, b in pairs))
+
+    def launch(self):
+        """words[i] (at most the pair's size) of pair i on the current stream."""
+        _check(load_library().ssd_copy_segments(self._src, self._dst, self.words, self.n, _stream()), "ssd_copy_segments")
 
 
 def cache_lookup(req_keys, cache_seq, cache_j, cache_forks, B: int, Bc: int, W: int, out_idx):
