@@ -104,28 +104,37 @@ extern "C" int ssd_store_step_rows(const void* src_rows, long src_ld, void* dst,
 
 
 // A step's inputs from pinned host memory to the device buffers that the kernels read, or its results back, all of them in one launch: a copy each took
-// 3 to 5 us on the device and a gap before it (six of them before a decoded token: 60 us of 820).  Loads and stores go past the caches, at system scope:
-// pinned memory is rewritten by the host between launches and read by it after them.  Bound by the link's latency (about 3 us) up to a few dozen KiB.
+// 3 to 5 us on the device and a gap before it (six of them before a decoded token: 60 us of 820).  Loads and stores are volatile (system scope, past the
+// caches): pinned memory is rewritten by the host between launches and read by it after them.  Bound by the link's latency (about 3 us) up to a few dozen KiB.
 constexpr int MAX_SEGMENTS = 10;
 struct Segments { const char* src[MAX_SEGMENTS]; char* dst[MAX_SEGMENTS]; int words[MAX_SEGMENTS]; int n; };
 
-__global__ void __launch_bounds__(256) copy_segments_kernel(Segments s) {
-  constexpr int SYSTEM = 17;                             // sc0 | sc1
-  long at = (long)blockIdx.x * 256 + threadIdx.x;        // 16-byte chunk over all segments
-  const long step = (long)gridDim.x * 256;
-  for (int i = 0; i < s.n; ++i) {
-    const long chunks = (s.words[i] + 3) >> 2;
-    const auto from = __builtin_amdgcn_make_buffer_rsrc((void*)s.src[i], 0, s.words[i] * 4, 0x00020000);
-    const auto to = __builtin_amdgcn_make_buffer_rsrc((void*)s.dst[i], 0, s.words[i] * 4, 0x00020000);
-    for (; at < chunks; at += step) {
-      if (at * 4 + 3 < s.words[i]) {
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_amdgcn_raw_buffer_load_b128(from, (int)(at * 16), 0, SYSTEM), to, (int)(at * 16), 0, SYSTEM);
-      } else {
-        for (long w = at * 4; w < s.words[i]; ++w)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_amdgcn_raw_buffer_load_b32(from, (int)(w * 4), 0, SYSTEM), to, (int)(w * 4), 0, SYSTEM);
-      }
+__global__ void __launch_bounds__(256) copy_segments_kernel(Segments s, long total) {
+  for (long at = (long)blockIdx.x * 256 + threadIdx.x; at < total; at += (long)gridDim.x * 256) {
+    // whose 16-byte chunk `at` is; then one load for all lanes (a load per segment waits for the link as many times: 15 us instead of 4)
+    long c = at;
+    int i = 0;
+    for (; i < s.n - 1 && c >= (s.words[i] + 3) >> 2; ++i) c -= (s.words[i] + 3) >> 2;
+    const char* from = s.src[0];
+    char* to = s.dst[0];
+    int words = s.words[0];
+#pragma unroll
+    for (int j = 1; j < MAX_SEGMENTS; ++j)
+      if (i == j) { from = s.src[j]; to = s.dst[j]; words = s.words[j]; }
+    const volatile u32x4_t* src = reinterpret_cast<const volatile u32x4_t*>(from) + c;
+    volatile u32x4_t* dst = reinterpret_cast<volatile u32x4_t*>(to) + c;
+    if (c * 4 + 3 < words) {
+      *dst = *src;
+    } else {
+      const int left = words - (int)c * 4;               // 1 .. 3, all of them fetched before the first is stored
+      uint32_t v[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (k < left) v[k] = reinterpret_cast<const volatile uint32_t*>(src)[k];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (k < left) reinterpret_cast<volatile uint32_t*>(dst)[k] = v[k];
     }
-    at -= chunks;
   }
 }
 
@@ -145,7 +154,7 @@ extern "C" int ssd_copy_segments(const void* const* src, void* const* dst, const
     chunks += (words[i] + 3) / 4;
   }
   if (chunks == 0) return SSD_OK;
-  hipLaunchKernelGGL(copy_segments_kernel, dim3((unsigned)(chunks < 256 * 512 ? (chunks + 255) / 256 : 512)), dim3(256), 0, (hipStream_t)stream, s);
+  hipLaunchKernelGGL(copy_segments_kernel, dim3((unsigned)(chunks < 256 * 512 ? (chunks + 255) / 256 : 512)), dim3(256), 0, (hipStream_t)stream, s, chunks);
   return hipGetLastError() == hipSuccess ? SSD_OK : SSD_ERR_LAUNCH;
 }
 
