@@ -118,7 +118,10 @@ int ssd_gemm_pf(const void* x_frag, const void* w_frag, const void* bias, void* 
                 int epilogue, void* workspace, int64_t workspace_bytes, int splits, void* stream);
 /* The same F.linear for many token rows (csrc/gemm_big.hip): large LDS tiles, any M; N % 16 == 0 (% 64 with SSD_EPI_SILU_FRAG), K % 32 == 0,
  * K >= 96, ldy % 4 == 0.  `workspace` (may be NULL): room for the fp32 slabs of products with too few tiles to fill the chip, which are
- * split along K as far as workspace_bytes allow. */
+ * split along K as far as workspace_bytes allow.  epilogue 2 (no bias; y and ldy are not looked at): the slabs [splits][M][N] in `workspace` ARE the
+ * output, for ssd_rmsnorm_parts / ssd_rope_store_kv_parts to add up instead of a launch behind the product -- the same bits; splits =
+ * ssd_gemm_big_splits(M, N, K, workspace_bytes), and refused (SSD_ERR_SHAPE) where that is 1. */
+int ssd_gemm_big_splits(int M, int N, int K, int64_t workspace_bytes);
 int ssd_gemm_big(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
                  void* workspace, int64_t workspace_bytes, void* stream);
 /* Fused decode-layer GEMM for M <= 16 (csrc/gemm_fused.hip): [residual add + RMSNorm] -> F.linear ->

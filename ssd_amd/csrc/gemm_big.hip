@@ -143,7 +143,7 @@ int go(const void* x, const void* w, const void* bias, void* y, int M, int N, in
   else if constexpr (NT % 2 == 0) GO(BIG_SILU_FRAG, y);          // (the others never get here: ssd_gemm_big_cfg)
 #undef GO
   if (hipGetLastError() != hipSuccess) return SSD_ERR_LAUNCH;
-  if (splits > 1) {
+  if (splits > 1 && epilogue != BIG_PARTS) {
     const unsigned blocks = (unsigned)(((size_t)M * (epilogue == BIG_ROWS ? N : N / 2) / 4 + 255) / 256);
     if (epilogue == BIG_ROWS)
       hipLaunchKernelGGL((gemm_big_sum_kernel<BIG_ROWS>), dim3(blocks), dim3(256), 0, st, (const float*)ws, (const bf16_t*)bias, y, M, N, splits, ldy);
@@ -190,12 +190,9 @@ Plan pick(int M, int N, int K, int epilogue, long ws_bytes) {
   return best;
 }
 
-}  // namespace
-
-extern "C" int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
-                                void* workspace, int64_t workspace_bytes, int shape, int splits, void* stream) {
-  if (!x_frag || !w_frag || !y) return SSD_ERR_ARG;
-  if (epilogue != BIG_ROWS && epilogue != BIG_SILU_FRAG) return SSD_ERR_ARG;
+// Every entry point's checks, and the launch.
+int run(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue, void* workspace,
+        int64_t workspace_bytes, int shape, int splits, void* stream) {
   if (M <= 0 || N <= 0 || K < 64 || N % 16 || K % 32 || (epilogue == BIG_SILU_FRAG && N % 64) || K > (1 << 22)) return SSD_ERR_SHAPE;
   if (epilogue == BIG_ROWS && (ldy < N || ldy % 4)) return SSD_ERR_SHAPE;
   if (shape < 0 || shape >= SHAPE_COUNT || (epilogue == BIG_SILU_FRAG && SHAPES[shape].features == 192) || splits < 1 || splits > 8 || K / 32 / splits < 3) return SSD_ERR_ARG;
@@ -218,9 +215,30 @@ extern "C" int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const vo
 #undef BIG_ARGS
 }
 
+}  // namespace
+
+extern "C" int ssd_gemm_big_cfg(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
+                                void* workspace, int64_t workspace_bytes, int shape, int splits, void* stream) {
+  if (!x_frag || !w_frag || !y) return SSD_ERR_ARG;
+  if (epilogue != BIG_ROWS && epilogue != BIG_SILU_FRAG) return SSD_ERR_ARG;
+  return run(x_frag, w_frag, bias, y, M, N, K, ldy, epilogue, workspace, workspace_bytes, shape, splits, stream);
+}
+
+extern "C" int ssd_gemm_big_splits(int M, int N, int K, int64_t workspace_bytes) {
+  if (M <= 0 || N <= 0 || K < 96 || N % 16 || K % 32) return SSD_ERR_SHAPE;
+  return pick(M, N, K, BIG_ROWS, workspace_bytes).splits;
+}
+
 extern "C" int ssd_gemm_big(const void* x_frag, const void* w_frag, const void* bias, void* y, int M, int N, int K, int ldy, int epilogue,
                             void* workspace, int64_t workspace_bytes, void* stream) {
   if (M <= 0 || N <= 0 || K < 96) return SSD_ERR_SHAPE;
+  if (epilogue == BIG_PARTS) {
+    // (the consumer adds the slabs up: bias and rows have no place here)
+    if (!x_frag || !w_frag || bias || !workspace) return SSD_ERR_ARG;
+    const Plan p = pick(M, N, K, BIG_ROWS, workspace_bytes);
+    if (p.splits < 2) return SSD_ERR_SHAPE;
+    return run(x_frag, w_frag, nullptr, nullptr, M, N, K, N, epilogue, workspace, workspace_bytes, p.shape, p.splits, stream);
+  }
   const Plan p = pick(M, N, K, epilogue, workspace ? workspace_bytes : 0);
   return ssd_gemm_big_cfg(x_frag, w_frag, bias, y, M, N, K, ldy, epilogue, workspace, workspace_bytes, p.shape, p.splits, stream);
 }

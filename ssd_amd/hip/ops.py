@@ -13,7 +13,7 @@ import torch
 from .lib import load_library, SsdHipError
 
 EPI_ROWS, EPI_SILU_FRAG, EPI_ROWS_F32 = 0, 1, 2
-PF_EPI_PARTIALS = 2          # ssd_gemm_pf only: leave the split-K partials in the workspace for ssd_rmsnorm_parts
+PF_EPI_PARTIALS = 2          # ssd_gemm_pf, ssd_gemm_big: leave the split-K partials in the workspace for ssd_rmsnorm_parts / ssd_rope_store_kv_parts
 MODE_CAUSAL, MODE_TREE = 0, 1
 
 
@@ -117,6 +117,11 @@ def gemm_pf(x_frag, w_frag, y, M: int, N: int, K: int, ldy: int, workspace, epil
     else:
         _check(load_library().ssd_gemm_pf(_p(x_frag), _p(w_frag), _p(bias), _p(y), M, N, K, ldy, epilogue, _p(workspace),
                                           wb, splits, _stream()), "ssd_gemm_pf")
+
+
+def gemm_big_splits(M: int, N: int, K: int, workspace) -> int:
+    """Slabs that gemm_big splits this product into (1: none)."""
+    return load_library().ssd_gemm_big_splits(M, N, K, 0 if workspace is None else workspace.numel() * workspace.element_size())
 
 
 def gemm_big(x_frag, w_frag, y, M: int, N: int, K: int, ldy: int, epilogue: int = EPI_ROWS, bias=None, workspace=None, shape: int = -1,

@@ -283,30 +283,50 @@ class HipDecoder:
         Up to 32 rows the skinny kernel also keeps a gate_up that gemm_pf has to split along K (two shards of 70B, 28672 x 8192: 85 | 89 | 93,
         16384 x 14336 79 | 94 | 87; 51200 rows fill the chip unsplit), a vocabulary over a short K (128256 x 2048 91 | 99 | --, 51200 x 1536
         30 | 30 | 32) and eight shards' o_proj, 8192 x 1024 (8 | 11 | 9)."""
-        size, rows, wide = 2 * N * K, epi == H.EPI_ROWS, N >= self.WIDE_OUTPUTS
-        short = wide and K <= 2048 if rows else not wide                    # (up to 32 rows: what gemm_pf does not lead at)
-        if m > 16 and self._pf_eligible(N, K) and (m > 64 or size >= self.PF_ALWAYS_WEIGHT_BYTES and (m > 32 or not short)):
+        kind = self._chunk_kind(N, m, K, epi)
+        if kind == "pf":
             assert self._ws_pf is not None and self._ws_pf.numel() * 4 >= H.gemm_pf_workspace_bytes(128, N, K), (N, K)
             H.gemm_pf(xf, w, y, m, N, K, ldy, self._ws_pf, epilogue=epi, bias=bias)
-        elif 16 < m <= 64 and K >= 96 and size >= self.BIG_MIN_WEIGHT_BYTES and (m > 32 or rows and not short and (K > 1024 or N > 8192)):
+        elif kind == "big":
             H.gemm_big(xf, w, y, m, N, K, ldy, epi, bias, self._ws_big)
         else:
             H.gemm(xf, w, y, m, N, K, ldy, epi, bias)
 
-    def _pf_partials_ok(self, T: int, N: int, K: int) -> bool:
-        """o_proj / down_proj of ONE prefill chunk may leave their split-K partials in the workspace for the norm that follows."""
-        return self.pf_parts and not self.use_coll and 32 < T <= 128 and self._pf_eligible(N, K) and self._ws_pf is not None
+    def _chunk_kind(self, N: int, m: int, K: int, epi) -> str:
+        size, rows, wide = 2 * N * K, epi == H.EPI_ROWS, N >= self.WIDE_OUTPUTS
+        short = wide and K <= 2048 if rows else not wide                    # (up to 32 rows: what gemm_pf does not lead at)
+        if m > 16 and self._pf_eligible(N, K) and (m > 64 or size >= self.PF_ALWAYS_WEIGHT_BYTES and (m > 32 or not short)):
+            return "pf"
+        if 16 < m <= 64 and K >= 96 and size >= self.BIG_MIN_WEIGHT_BYTES and (m > 32 or rows and not short and (K > 1024 or N > 8192)):
+            return "big"
+        return "skinny"
 
-    @staticmethod
-    def _pf_splits(T: int, N: int, K: int) -> int:
-        return H.gemm_pf_workspace_bytes(T, N, K) // (4 * T * N)
+    def _takes_big(self, T: int, N: int, K: int) -> bool:
+        """A batch of T rows is one large-tile product (see _gemm)."""
+        return T > self.BIG_MIN_ROWS and K >= 96 and (T > 256 or 2 * N * K >= self.BIG_SMALLEST_WEIGHT_BYTES)
 
-    def _gemm_pf_partials(self, xf, K, w, N, T) -> int:
-        """Prefill GEMM stopped after its split-K stage (csrc/gemm_pf.hip PF_EPI_PARTIALS): fp32 slabs [S][T][N] in the workspace;
-        returns S.  The consumer is ssd_rmsnorm_parts -- one launch per GEMM less."""
-        S = H.gemm_pf_workspace_bytes(T, N, K) // (4 * T * N)
+    def _slab_plan(self, T: int, N: int, K: int) -> tuple[str, int] | None:
+        """(kernel, slabs) where the row product of T x K by N x K may stop after its split-K stage, for the norm or the RoPE / KV-store kernel that
+        follows to add its slabs up -- a launch less (48 rows of 8B: qkv and o_proj 4.7 us each), the same bits.  One chunk of gemm_pf's, or what
+        the large-tile kernel splits."""
+        if not self.pf_parts or self.use_coll:
+            return None
+        if self._takes_big(T, N, K) or T <= 64 and self._chunk_kind(N, T, K, H.EPI_ROWS) == "big":
+            S = H.gemm_big_splits(T, N, K, self._ws_big)
+            return ("big", S) if S > 1 else None
+        if 32 < T <= 128 and self._pf_eligible(N, K) and self._ws_pf is not None:
+            S = H.gemm_pf_workspace_bytes(T, N, K) // (4 * T * N)
+            return ("pf", S)
+        return None
+
+    def _gemm_slabs(self, plan, xf, K, w, N, T):
+        """The product of a _slab_plan, stopped after its split-K stage: (fp32 slabs [S][T][N], S)."""
+        kind, S = plan
+        if kind == "big":
+            H.gemm_big(xf, w, None, T, N, K, N, H.PF_EPI_PARTIALS, None, self._ws_big)
+            return self._ws_big, S
         H.gemm_pf(xf, w, None, T, N, K, N, self._ws_pf, epilogue=H.PF_EPI_PARTIALS)
-        return S
+        return self._ws_pf, S
 
     def _gemm(self, xf, K, w, N, y, T, ldy, epi=H.EPI_ROWS, bias=None):
         # The large-tile kernel from BIG_MIN_ROWS token rows of the batch on, and for matrices under 1 MB (models of a few hundred channels) from 256.
@@ -314,7 +334,7 @@ class HipDecoder:
         # which compare tokens that restart from single prompts of up to 160 tokens, and have near ties there that another order of
         # summation moves; no property of a sequence hangs on it (two prompts of 100 tokens take it, and the last rows of a prompt of
         # 145 .. 160 take what _gemm_chunk gives 17 .. 32 rows).  K < 96: fewer k-steps than a ring has stages.
-        if T > self.BIG_MIN_ROWS and K >= 96 and (T > 256 or 2 * N * K >= self.BIG_SMALLEST_WEIGHT_BYTES):
+        if self._takes_big(T, N, K):
             H.gemm_big(xf, w, y, T, N, K, ldy, epi, bias, self._ws_big)
             return
         if T <= 128:
@@ -521,7 +541,7 @@ class HipDecoder:
                            self.tree_ws, self.chain_gen, self.chain_err, h_out=self.buf_h if last else None, **nxt)
 
     def launch_qkv(self, li: int, T: int, positions, slot_mapping, gemm_only: bool = False, pre_normed: bool = False,
-                   parts: bool | None = None, pf_src: int = 0) -> None:
+                   parts: bool | None = None, slabs=None) -> None:
         """gemm_only: skip the separate add+RMSNorm / RoPE launches of the unfused variants (kernel timing).
         pre_normed: buf_xf / buf_res already hold this layer's normalised input and residual (written by the fused
         all-reduce + add + RMSNorm that closed the previous layer)."""
@@ -541,8 +561,8 @@ class HipDecoder:
             return
         # residual is None on layer 0 (llama3.py:187-190): residual := embeddings, x := norm(embeddings)
         if not gemm_only and not pre_normed:
-            if pf_src:       # the previous layer's down_proj left pf_src split-K slabs [pf_src][T][h] in the prefill workspace
-                H.rmsnorm_parts(self._ws_pf, pf_src, T, w[p + "input_layernorm.weight"], cfg.rms_norm_eps, T, self.h,
+            if slabs:        # the previous layer's down_proj left (fp32 slabs [S][T][h], S)
+                H.rmsnorm_parts(*slabs, T, w[p + "input_layernorm.weight"], cfg.rms_norm_eps, T, self.h,
                                 res_in=res, res_out=res, out_frag=xf)
             elif parts:
                 H.rmsnorm_parts(self.buf_parts_d, self._parts("d", T)[0], T, w[p + "input_layernorm.weight"], cfg.rms_norm_eps, T, self.h,
@@ -553,12 +573,12 @@ class HipDecoder:
         if small or (16 < T <= 32 and not cfg.qk_norm):      # T in 17..32 (tree-decode step): the two-token-tile variant
             H.gemm_fused(w[p + "self_attn.qkv_proj.weight"], T, self.qkv_n, self.h, H.FEPI_QKV_ROPE, x_frag=xf,
                          bias=w.get(p + "self_attn.qkv_proj.bias"), **rope)
-        elif (not gemm_only and w.get(p + "self_attn.qkv_proj.bias") is None and self._pf_partials_ok(T, self.qkv_n, self.h)
-              and self._pf_splits(T, self.qkv_n, self.h) > 1):
-            # single-chunk prefill of a big QKV matrix: its split-K slabs stay in the workspace and the RoPE / KV-store kernel
+        elif (not gemm_only and w.get(p + "self_attn.qkv_proj.bias") is None and (plan := self._slab_plan(T, self.qkv_n, self.h)) is not None
+              and plan[1] > 1):
+            # a QKV product that is split along K: its slabs stay in the workspace and the RoPE / KV-store kernel
             # sums them (bit-identical to the GEMM's epilogue launch + rope_store_kv; one launch less per layer)
-            S = self._gemm_pf_partials(xf, self.h, w[p + "self_attn.qkv_proj.weight"], self.qkv_n, T)
-            H.rope_store_kv_parts(self._ws_pf, S, positions, self.cos_sin, slot_mapping, self.buf_q, kc, vc, T, self.nh, self.nkv,
+            ws, S = self._gemm_slabs(plan, xf, self.h, w[p + "self_attn.qkv_proj.weight"], self.qkv_n, T)
+            H.rope_store_kv_parts(ws, S, positions, self.cos_sin, slot_mapping, self.buf_q, kc, vc, T, self.nh, self.nkv,
                                   self.hd, self.block_size, q_norm_w=w.get(p + "self_attn.q_norm.weight"),
                                   k_norm_w=w.get(p + "self_attn.k_norm.weight"), eps=cfg.rms_norm_eps, qkv_perm=1)
         else:
@@ -570,20 +590,20 @@ class HipDecoder:
                             self.hd, self.block_size, q_norm_w=w.get(p + "self_attn.q_norm.weight"),
                             k_norm_w=w.get(p + "self_attn.k_norm.weight"), eps=cfg.rms_norm_eps, qkv_perm=1)
 
-    def launch_o(self, li: int, T: int, parts: bool | None = None, pf_partials: bool = False) -> int:
-        """Returns the number of split-K slabs left in the prefill workspace (pf_partials), else 0."""
+    def launch_o(self, li: int, T: int, parts: bool | None = None, leave_slabs: bool = False):
+        """Returns what it left for the norm to add up (_gemm_slabs), or None: rows in buf_h."""
         w = self.w[f"model.layers.{li}.self_attn.o_proj.weight"]
-        if pf_partials and self._pf_partials_ok(T, self.h, self.qn):
-            return self._gemm_pf_partials(self.buf_af, self.qn, w, self.h, T)
+        if leave_slabs and (plan := self._slab_plan(T, self.h, self.qn)) is not None:
+            return self._gemm_slabs(plan, self.buf_af, self.qn, w, self.h, T)
         if self.parts_plan(T) if parts is None else parts:
             S, wv = self._parts("o", T)
             H.gemm_parts(self.buf_af, w, T, self.h, self.qn, parts=self.buf_parts_o, splits=S, waves=wv)
         else:
             self._gemm(self.buf_af, self.qn, w, self.h, self.buf_h, T, self.h)
-        return 0
+        return None
 
     def launch_gate_up(self, li: int, T: int, gemm_only: bool = False, pre_normed: bool = False, parts: bool | None = None,
-                       o_splits: int | None = None, pf_src: int = 0) -> None:
+                       o_splits: int | None = None, slabs=None) -> None:
         """o_splits: slabs o_proj left in buf_parts_o (default: the split-K GEMM's; the fused attention + o_proj leaves nkv)."""
         cfg, w = self.cfg, self.w
         p = f"model.layers.{li}."
@@ -597,8 +617,8 @@ class HipDecoder:
                          eps=cfg.rms_norm_eps, y=self.buf_actf, waves=8, **src)     # profiles/micro/fused_probe.py: 13.2 us vs 16.4 (16 waves)
         else:
             if not gemm_only and not pre_normed:
-                if pf_src:       # o_proj left pf_src split-K slabs in the prefill workspace
-                    H.rmsnorm_parts(self._ws_pf, pf_src, T, w[p + "post_attention_layernorm.weight"], cfg.rms_norm_eps,
+                if slabs:        # o_proj left (fp32 slabs, S)
+                    H.rmsnorm_parts(*slabs, T, w[p + "post_attention_layernorm.weight"], cfg.rms_norm_eps,
                                     T, self.h, res_in=self.buf_res, res_out=self.buf_res, out_frag=self.buf_xf)
                 elif parts:
                     H.rmsnorm_parts(self.buf_parts_o, So, T, w[p + "post_attention_layernorm.weight"], cfg.rms_norm_eps,
@@ -608,16 +628,16 @@ class HipDecoder:
                               res_in=self.buf_res, res_out=self.buf_res, out_frag=self.buf_xf)
             self._gemm(self.buf_xf, self.h, w[p + "mlp.gate_up_proj.weight"], 2 * self.I, self.buf_actf, T, 0, epi=H.EPI_SILU_FRAG)
 
-    def launch_down(self, li: int, T: int, parts: bool | None = None, pf_partials: bool = False) -> int:
+    def launch_down(self, li: int, T: int, parts: bool | None = None, leave_slabs: bool = False):
         w = self.w[f"model.layers.{li}.mlp.down_proj.weight"]
-        if pf_partials and self._pf_partials_ok(T, self.h, self.I):
-            return self._gemm_pf_partials(self.buf_actf, self.I, w, self.h, T)
+        if leave_slabs and (plan := self._slab_plan(T, self.h, self.I)) is not None:
+            return self._gemm_slabs(plan, self.buf_actf, self.I, w, self.h, T)
         if self.parts_plan(T) if parts is None else parts:
             S, wv = self._parts("d", T)
             H.gemm_parts(self.buf_actf, w, T, self.h, self.I, parts=self.buf_parts_d, splits=S, waves=wv)
         else:
             self._gemm(self.buf_actf, self.I, w, self.h, self.buf_h, T, self.h)
-        return 0
+        return None
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, T: int, meta: AttnMeta) -> None:
         """Runs all layers; leaves the final (pre-norm) hidden state in buf_h and the residual in buf_res."""
@@ -648,15 +668,15 @@ class HipDecoder:
         fuse = self.use_coll and ar is not None and self.fuse_ar_norm and ar.fits_rows(T, self.h)
         eps, res, xf = cfg.rms_norm_eps, self.buf_res, self.buf_xf
         L = cfg.num_layers
-        pf_d = 0            # split-K slabs the previous layer's down_proj left for this layer's input norm (single-chunk prefill)
+        slabs_d = None      # what the previous layer's down_proj left for this layer's input norm to add up
         for li in range(L):
-            self.launch_qkv(li, T, positions, meta.slot_mapping, pre_normed=fuse and li > 0, parts=parts, pf_src=pf_d)
+            self.launch_qkv(li, T, positions, meta.slot_mapping, pre_normed=fuse and li > 0, parts=parts, slabs=slabs_d)
             if self.taps is not None and li in self.taps:
                 # launch_qkv has just written x + residual: to buf_res2 on the fused-prologue path, to buf_res otherwise
                 src = self.buf_res2 if self.fusion_plan(T)[1] else res
                 i = self.taps.index(li)
                 self.acts[:T, i * self.h:(i + 1) * self.h].copy_(src[:T])
-            pf_o = 0
+            slabs_o = None
             if fuse_ao:
                 H.attn_oproj_parts(self.buf_q, self.kv_cache[li, 0], self.kv_cache[li, 1], meta.block_tables, self.max_blocks,
                                    meta.context_lens, T, self.nh, self.nkv, self.hd, self.block_size, scale,
@@ -667,14 +687,14 @@ class HipDecoder:
                              cu_q=meta.cu_q, q_per_seq=meta.q_per_seq, mode=meta.mode, tree_K=meta.tree_K, tree_mq=meta.tree_mq,
                              tree_step=meta.tree_step, tree_F=meta.tree_F, tree_jidx=meta.tree_jidx, splits=splits,
                              flags=attn_flags, ws_o=self.ws_o, ws_ml=self.ws_ml, out_frag=self.buf_af, waves=attn_waves)
-                pf_o = self.launch_o(li, T, parts=parts, pf_partials=not parts)
+                slabs_o = self.launch_o(li, T, parts=parts, leave_slabs=not parts)
             if fuse:
                 ar.all_reduce_add_rmsnorm(h, res, res, w[f"model.layers.{li}.post_attention_layernorm.weight"], eps, T, self.h, out_frag=xf)
             else:
                 self._allreduce(h[:T])
-            self.launch_gate_up(li, T, pre_normed=fuse, parts=parts, o_splits=self.nkv if fuse_ao else None, pf_src=pf_o)
+            self.launch_gate_up(li, T, pre_normed=fuse, parts=parts, o_splits=self.nkv if fuse_ao else None, slabs=slabs_o)
             # (the last layer's down_proj keeps its epilogue: compute_logits' last-token gather reads rows)
-            pf_d = self.launch_down(li, T, parts=parts, pf_partials=not parts and li + 1 < L)
+            slabs_d = self.launch_down(li, T, parts=parts, leave_slabs=not parts and li + 1 < L)
             if fuse and li + 1 < L:
                 ar.all_reduce_add_rmsnorm(h, res, res, w[f"model.layers.{li + 1}.input_layernorm.weight"], eps, T, self.h, out_frag=xf)
             else:

@@ -61,3 +61,31 @@ def test_rows_of_other_shapes(H, M, N, K):
     y = torch.zeros(M, N, device="cuda")
     H.gemm_rows_bias(x, w, y, M, N, K, b, False)
     check_rows(y, z + b.double(), (M, N, K, "bias"), False)
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 4096, 2048), (48, 1024, 4096), (200, 1024, 8224)])
+def test_big_slabs(H, M, N, K):
+    """A split product that stops before its sum: the slabs, added up in order and rounded, are the rows' bits.  What is not split, or has a bias, is refused."""
+    from ssd_amd.hip.lib import SsdHipError
+    x, w, b = operands(M, N, K, M)
+    xf, wf = frag(H, x), frag(H, w)
+    ws = torch.full((8 * M * N + 64,), 7.0, device="cuda")
+    S = H.gemm_big_splits(M, N, K, ws)
+    assert S > 1
+    rows = torch.zeros(M, N, dtype=BF, device="cuda")
+    H.gemm_big(xf, wf, rows, M, N, K, N, workspace=ws)
+    ws.fill_(7.0)
+    H.gemm_big(xf, wf, None, M, N, K, N, epilogue=H.PF_EPI_PARTIALS, workspace=ws)
+    assert bool((ws[S * M * N:] == 7.0).all())
+    slabs = ws[:S * M * N].view(S, M, N)
+    total = slabs[0].clone()
+    for s in range(1, S):
+        total += slabs[s]
+    assert torch.equal(total.to(BF), rows)
+    with pytest.raises(SsdHipError):
+        H.gemm_big(xf, wf, None, M, N, K, N, epilogue=H.PF_EPI_PARTIALS, bias=b.cuda(), workspace=ws)
+    assert H.gemm_big_splits(M, N, K, None) == 1
+    with pytest.raises(SsdHipError):
+        H.gemm_big(xf, wf, None, M, N, K, N, epilogue=H.PF_EPI_PARTIALS, workspace=None)
+    with pytest.raises(SsdHipError):
+        H.gemm_big(xf, wf, None, M, N, K, N, epilogue=H.PF_EPI_PARTIALS, workspace=ws[:16])
