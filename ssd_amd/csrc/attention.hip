@@ -55,7 +55,13 @@ constexpr int attn_region_bytes() { return RT * 16 * HD * 4 + RT * 16 * 8; }
 // normalised bf16 output of its heads in LDS as an MFMA B operand and multiplies: slab h of the split-K partial sums of
 // o_proj, summed by the consumer like ssd_gemm_parts' slabs.  The weight stream hides behind the attention latency chain and
 // one kernel boundary per layer disappears (a 1B draft decode layer: 6.6 us attention + 3.9 us o_proj as two launches).
-template <int HD, int RT, int KT, bool OPROJ = false>
+// What bounds a wave is the instructions of a tile and the LDS round trips between them, not the keys' way from memory (one wave over 3000 keys: 2.2 us a
+// tile of 32): tiles that every row sees in full are not masked, probabilities are rounded by the converter, all of V's operands are fetched before
+// the first product.  MI355X, us: 3000 keys, one wave 201 -> 83, eight 38 -> 32; 48 sequences of up to 3000 keys 61 -> 55 (4 TB/s), 32 of up to 500 13 -> 11,
+// seven rows over 707 keys 15.5 -> 12.8.  (Non-temporal loads, or two tiles in flight per wave: level or worse.)
+// PLAIN: V by transpose reads and P in two terms, what every caller asks for; the flags for less of either (ssd_attn_paged, bits 0 and 1) take an
+// instantiation that looks at them for every output tile and waits for LDS as often.
+template <int HD, int RT, int KT, bool OPROJ = false, bool PLAIN = true>
 __global__ void __launch_bounds__(512) attn_kernel(const AttnParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int KTS = OPROJ ? 7 : 6;        // trace slot (profiling builds only)
@@ -114,6 +120,7 @@ __global__ void __launch_bounds__(512) attn_kernel(const AttnParams p) {
     const int last_row = min(rows - 1, (tile_base + RT) * 16 - 1);
     kmax = ctx - (Tq - 1 - last_row / G);
   }
+  const int all_see = p.mode == 0 ? ctx - (Tq - 1) : ctx - (p.tree_K + 1) - (p.tree_step + 1) * p.tree_mq;      // keys before this: visible to every row
   const int stride = p.splits * W * 32;
   int k0 = (z * W + wave) * 32;
 
@@ -234,15 +241,16 @@ __global__ void __launch_bounds__(512) attn_kernel(const AttnParams p) {
     const int k0t = kt;
     // -- mask + online softmax; P^T stays in the accumulator layout --
     u32x4_t pf[RT], pl[RT];
+    const bool open = k0t + 32 <= all_see;      // every key of the tile is visible to every row (wave-uniform): nothing to mask
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       float s[8];
-      float tmax = -INFINITY;
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf)
+      for (int i = 0; i < 8; ++i) s[i] = st[i >> 2][rt][i & 3] * p.scale_log2e;
+      if (!open) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = k0t + hf * 16 + g4 * 4 + r;
+        for (int i = 0; i < 8; ++i) {
+          const int key = k0t + (i >> 2) * 16 + g4 * 4 + (i & 3);
           bool ok = rvalid[rt] && key < kmax;
           if (p.mode == 0) {
             ok = ok && key < lim[rt];
@@ -254,61 +262,78 @@ __global__ void __launch_bounds__(512) attn_kernel(const AttnParams p) {
             vis = vis || (rel > p.tree_K && ((rel - p.tree_K - 1) % p.tree_mq) == tl[rt]);  // own branch diagonal
             ok = ok && vis;
           }
-          const float v = ok ? st[hf][rt][r] * p.scale_log2e : -INFINITY;
-          s[hf * 4 + r] = v;
-          tmax = fmaxf(tmax, v);
+          s[i] = ok ? s[i] : -INFINITY;
         }
+      }
+      float tmax = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
       tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
       tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
       const float mnew = fmaxf(m[rt], tmax);
       const float msafe = (mnew == -INFINITY) ? 0.f : mnew;
-      const float alpha = exp2f(m[rt] - msafe);
+      const float alpha = __builtin_amdgcn_exp2f(m[rt] - msafe);          // (arguments <= 0: weights below 2^-126 become zero)
       float ps = 0.f;
       float pv[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) { pv[i] = exp2f(s[i] - msafe); ps += pv[i]; }
+      for (int i = 0; i < 8; ++i) { pv[i] = __builtin_amdgcn_exp2f(s[i] - msafe); ps += pv[i]; }
       lsum[rt] = lsum[rt] * alpha + ps;
       m[rt] = mnew;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) o[rt][dt] *= alpha;
-      pf[rt] = u32x4_t{pack_bf2(pv[0], pv[1]), pack_bf2(pv[2], pv[3]), pack_bf2(pv[4], pv[5]), pack_bf2(pv[6], pv[7])};
       // P = P_hi + P_lo (two bf16 terms, ~2^-17 relative): P.V then tracks an fp32-softmax reference instead of
       // carrying FlashAttention's 2^-9 probability rounding; costs one extra MFMA per output tile.
-      float pr[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) pr[i] = pv[i] - round_bf(pv[i]);
-      pl[rt] = u32x4_t{pack_bf2(pr[0], pr[1]), pack_bf2(pr[2], pr[3]), pack_bf2(pr[4], pr[5]), pack_bf2(pr[6], pr[7])};
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t hi = pack_bf2(pv[2 * i], pv[2 * i + 1]);
+        pf[rt][i] = hi;
+        pl[rt][i] = pack_bf2(pv[2 * i] - bf2f(hi & 0xffffu), pv[2 * i + 1] - __uint_as_float(hi & 0xffff0000u));
+      }
     }
     // the V tile is private to this wave: LDS ops of one wave execute in order, so a wave-level fence (no
     // s_barrier -- waves have different trip counts) is all the write->transpose-read hand-off needs
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     // -- O^T += V^T . P^T ; V^T fragments by transpose-read from the staged tile --
+    // lane (r16, g4) supplies the address of row 4*g4 + (r16 >> 2), column quad (r16 & 3) of the
+    // [32 keys][16 d] sub-tile; the hardware returns column r16 of rows 4*g4 .. 4*g4+3.
+    auto v_frag = [&](int dt) {
+      const bf16_t* a0 = vlds + (dt * 32 + g4 * 4 + (r16 >> 2)) * 16 + (r16 & 3) * 4;
+      typedef s16x4_t __attribute__((address_space(3))) * lds_v4_t;
+      const u32x2_t lo = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(a0)));
+      const u32x2_t hi = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(a0 + 16 * 16)));
+      return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+    };
+    if constexpr (PLAIN) {
+      u32x4_t vf[DT];          // all of them on their way before the first product
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      u32x4_t vf;
-      if (p.use_tr) {
-        // lane (r16, g4) supplies the address of row 4*g4 + (r16 >> 2), column quad (r16 & 3) of the
-        // [32 keys][16 d] sub-tile; the hardware returns column r16 of rows 4*g4 .. 4*g4+3.
-        const bf16_t* a0 = vlds + (dt * 32 + g4 * 4 + (r16 >> 2)) * 16 + (r16 & 3) * 4;
-        typedef s16x4_t __attribute__((address_space(3))) * lds_v4_t;
-        const s16x4_t t0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(a0));
-        const s16x4_t t1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4_t)(a0 + 16 * 16));
-        u32x2_t lo = __builtin_bit_cast(u32x2_t, t0), hi = __builtin_bit_cast(u32x2_t, t1);
-        vf = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
-      } else {
-        uint32_t e[8];
+      for (int dt = 0; dt < DT; ++dt) vf[dt] = v_frag(dt);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int key = (i < 4) ? (g4 * 4 + i) : (16 + g4 * 4 + (i - 4));
-          e[i] = vlds[(dt * 32 + key) * 16 + r16];
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) o[rt][dt] = mfma16(vf[dt], pf[rt], o[rt][dt]);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) o[rt][dt] = mfma16(vf[dt], pl[rt], o[rt][dt]);
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        u32x4_t vf;
+        if (p.use_tr) {
+          vf = v_frag(dt);
+        } else {
+          uint32_t e[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int key = (i < 4) ? (g4 * 4 + i) : (16 + g4 * 4 + (i - 4));
+            e[i] = vlds[(dt * 32 + key) * 16 + r16];
+          }
+          vf = u32x4_t{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
         }
-        vf = u32x4_t{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-      }
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        o[rt][dt] = mfma16(vf, pf[rt], o[rt][dt]);
-        if (p.p_split) o[rt][dt] = mfma16(vf, pl[rt], o[rt][dt]);
+        for (int rt = 0; rt < RT; ++rt) {
+          o[rt][dt] = mfma16(vf, pf[rt], o[rt][dt]);
+          if (p.p_split) o[rt][dt] = mfma16(vf, pl[rt], o[rt][dt]);
+        }
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
@@ -474,7 +499,7 @@ __global__ void attn_combine_kernel(const float* __restrict__ ws_o, const float*
 template <int HD, int RT, int KT>
 static int attn_launch_rt(const AttnParams& p, dim3 grid, int waves, hipStream_t st) {
   const int lds = waves * attn_region_bytes<HD, RT>();
-  auto kern = attn_kernel<HD, RT, KT, false>;
+  auto kern = p.use_tr && p.p_split ? attn_kernel<HD, RT, KT, false> : attn_kernel<HD, RT, KT, false, false>;
   if (lds > 64 * 1024 &&
       hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return SSD_ERR_LAUNCH;

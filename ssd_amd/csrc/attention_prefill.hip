@@ -152,11 +152,11 @@ attn_prefill_kernel(const PrefillAttn p) {
           w[e] = __builtin_amdgcn_exp2f(fmaf(st[kb][rt][e], p.scale_log2e, -ref));
           sum += w[e];
         }
-        const uint32_t h0 = pack_bf2_hw(w[0], w[1]), h1 = pack_bf2_hw(w[2], w[3]);
+        const uint32_t h0 = pack_bf2(w[0], w[1]), h1 = pack_bf2(w[2], w[3]);
         ph[kb / 2][rt][(kb & 1) * 2] = h0;
         ph[kb / 2][rt][(kb & 1) * 2 + 1] = h1;
-        pl[kb / 2][rt][(kb & 1) * 2] = pack_bf2_hw(w[0] - __uint_as_float(h0 << 16), w[1] - __uint_as_float(h0 & 0xffff0000u));
-        pl[kb / 2][rt][(kb & 1) * 2 + 1] = pack_bf2_hw(w[2] - __uint_as_float(h1 << 16), w[3] - __uint_as_float(h1 & 0xffff0000u));
+        pl[kb / 2][rt][(kb & 1) * 2] = pack_bf2(w[0] - __uint_as_float(h0 << 16), w[1] - __uint_as_float(h0 & 0xffff0000u));
+        pl[kb / 2][rt][(kb & 1) * 2 + 1] = pack_bf2(w[2] - __uint_as_float(h1 << 16), w[3] - __uint_as_float(h1 & 0xffff0000u));
       }
       lsum[rt] += sum;
     }
@@ -191,7 +191,7 @@ attn_prefill_kernel(const PrefillAttn p) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const int d = dt * 16 + g4 * 4;
-      const u32x2_t v = {pack_bf2_hw(o[rt][dt][0] * inv, o[rt][dt][1] * inv), pack_bf2_hw(o[rt][dt][2] * inv, o[rt][dt][3] * inv)};
+      const u32x2_t v = {pack_bf2(o[rt][dt][0] * inv, o[rt][dt][1] * inv), pack_bf2(o[rt][dt][2] * inv, o[rt][dt][3] * inv)};
       if (p.out_rows) *reinterpret_cast<u32x2_t*>(p.out_rows + ((size_t)tok * p.nh + head) * HD + d) = v;
       if (p.out_frag) {
         const int kcol = head * HD + d;

@@ -404,8 +404,8 @@ __device__ __forceinline__ void win_finish(f32x4_t (&acc)[MV], float mx, float l
   for (int i = 0; i < MV; ++i)
     if (i < DVT) {
       u32x2_t o2;
-      o2[0] = pack_bf2_hw(acc[i][0], acc[i][1]);
-      o2[1] = pack_bf2_hw(acc[i][2], acc[i][3]);
+      o2[0] = pack_bf2(acc[i][0], acc[i][1]);
+      o2[1] = pack_bf2(acc[i][2], acc[i][3]);
       *reinterpret_cast<u32x2_t*>(orow + i * 16) = o2;
     }
 }
@@ -537,8 +537,8 @@ win_rows(float* __restrict__ smem, const bf16_t* __restrict__ q, const bf16_t* _
     ls = ls * c + psum;
     mx = mn;
     u32x4_t pb;
-    pb[0] = pack_bf2_hw(pv[0], pv[1]); pb[1] = pack_bf2_hw(pv[2], pv[3]);
-    pb[2] = pack_bf2_hw(pv[4], pv[5]); pb[3] = pack_bf2_hw(pv[6], pv[7]);
+    pb[0] = pack_bf2(pv[0], pv[1]); pb[1] = pack_bf2(pv[2], pv[3]);
+    pb[2] = pack_bf2(pv[4], pv[5]); pb[3] = pack_bf2(pv[6], pv[7]);
 #pragma unroll
     for (int i = 0; i < MV; ++i)
       if (i < DVT) {
@@ -796,8 +796,8 @@ winattn_prompt_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
           w[e] = __builtin_amdgcn_exp2f(st[kb][t][e] - ref);
           sum += w[e];
         }
-        pb[kb / 2][t][(kb & 1) * 2] = pack_bf2_hw(w[0], w[1]);
-        pb[kb / 2][t][(kb & 1) * 2 + 1] = pack_bf2_hw(w[2], w[3]);
+        pb[kb / 2][t][(kb & 1) * 2] = pack_bf2(w[0], w[1]);
+        pb[kb / 2][t][(kb & 1) * 2 + 1] = pack_bf2(w[2], w[3]);
       }
       lsum[t] += sum;
     }

@@ -20,24 +20,15 @@ constexpr int SSD_MAX_DEVICES = 16;  // per-device host-side caches (function at
 
 __device__ __forceinline__ float bf2f(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
 
-// fp32 -> bf16, round-to-nearest-even (the rounding every torch bf16 store performs).
-__device__ __forceinline__ uint32_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;  // quiet NaN
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return u >> 16;
-}
-__device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) { return f2bf(lo) | (f2bf(hi) << 16); }
-
-// The same conversion on gfx950's converter (v_cvt_pk_bf16_f32: one instruction for two values instead of ~12): round-to-nearest-even,
-// bit-identical to f2bf on every non-NaN input (checked exhaustively over all 2^32 patterns on the MI355X by ssd_selftest_bf16_cvt,
-// tests/test_hip_ops.py); used where a kernel converts tens of values per thread (csrc/tree_segment.hip).
+// fp32 -> bf16, round-to-nearest-even (the rounding every torch bf16 store performs), on gfx950's converter (v_cvt_pk_bf16_f32: two values in one
+// instruction, where integer arithmetic takes a dozen and a branch around NaN): the same bits as the integer form on every non-NaN input, NaN for NaN
+// (all 2^32 patterns: ssd_selftest_bf16_cvt, misc.hip).
 typedef __attribute__((ext_vector_type(2))) float f32x2_t;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
-__device__ __forceinline__ uint32_t pack_bf2_hw(float lo, float hi) {
+__device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
 }
-__device__ __forceinline__ float round_bf_hw(float f) { return bf2f(pack_bf2_hw(f, 0.f) & 0xffffu); }
+__device__ __forceinline__ uint32_t f2bf(float f) { return pack_bf2(f, 0.f) & 0xffffu; }
 
 // Round an fp32 value through bf16 (models "store bf16, reload" between two reference kernels).
 __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }

@@ -65,7 +65,7 @@ gemm_big_kernel(const char* __restrict__ Wf, const char* __restrict__ Xf, const 
       for (int j = 0; j < MT; ++j) {
         const int m = m0 + j * 16;
         if (m < M) {
-          const u32x2_t v = {pack_bf2_hw(acc[i][j][0] + bb[0], acc[i][j][1] + bb[1]), pack_bf2_hw(acc[i][j][2] + bb[2], acc[i][j][3] + bb[3])};
+          const u32x2_t v = {pack_bf2(acc[i][j][0] + bb[0], acc[i][j][1] + bb[1]), pack_bf2(acc[i][j][2] + bb[2], acc[i][j][3] + bb[3])};
           *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(Yv) + (size_t)m * ldy + n) = v;
         }
       }
@@ -88,10 +88,10 @@ gemm_big_kernel(const char* __restrict__ Wf, const char* __restrict__ Xf, const 
         float o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float g = round_bf_hw(acc[i][j][r] + bg[r]), u = round_bf_hw(acc[i + 1][j][r] + bu[r]);
+          const float g = round_bf(acc[i][j][r] + bg[r]), u = round_bf(acc[i + 1][j][r] + bu[r]);
           o[r] = (g / (1.0f + __expf(-g))) * u;
         }
-        if (m < M) out[frag_chunk(m, f >> 3, KT2) * 2 + ((f >> 2) & 1)] = u32x2_t{pack_bf2_hw(o[0], o[1]), pack_bf2_hw(o[2], o[3])};
+        if (m < M) out[frag_chunk(m, f >> 3, KT2) * 2 + ((f >> 2) & 1)] = u32x2_t{pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3])};
       }
     }
   }
@@ -115,7 +115,7 @@ gemm_big_sum_kernel(const float* __restrict__ ws, const bf16_t* __restrict__ bia
     if (i4 >= MN) return;
     const int m = (int)(i4 / N), n = (int)(i4 % N);
     const f32x4_t s = sum(i4, n);
-    *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(Yv) + (size_t)m * ldy + n) = u32x2_t{pack_bf2_hw(s[0], s[1]), pack_bf2_hw(s[2], s[3])};
+    *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(Yv) + (size_t)m * ldy + n) = u32x2_t{pack_bf2(s[0], s[1]), pack_bf2(s[2], s[3])};
   } else {
     const int half = N >> 1;
     if (i4 >= (size_t)M * half) return;
@@ -124,10 +124,10 @@ gemm_big_sum_kernel(const float* __restrict__ ws, const bf16_t* __restrict__ bia
     float o[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float a = round_bf_hw(g[r]), b = round_bf_hw(u[r]);
+      const float a = round_bf(g[r]), b = round_bf(u[r]);
       o[r] = (a / (1.0f + __expf(-a))) * b;
     }
-    reinterpret_cast<u32x2_t*>(Yv)[frag_chunk(m, f >> 3, half >> 5) * 2 + ((f >> 2) & 1)] = u32x2_t{pack_bf2_hw(o[0], o[1]), pack_bf2_hw(o[2], o[3])};
+    reinterpret_cast<u32x2_t*>(Yv)[frag_chunk(m, f >> 3, half >> 5) * 2 + ((f >> 2) & 1)] = u32x2_t{pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3])};
   }
 }
 

@@ -26,9 +26,9 @@ __device__ __forceinline__ F32Split f32_split(u32x4_t p, u32x4_t q) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t x0 = i < 2 ? p[2 * i] : q[2 * i - 4], x1 = i < 2 ? p[2 * i + 1] : q[2 * i - 3];
-    const uint32_t h = pack_bf2_hw(__uint_as_float(x0), __uint_as_float(x1));
+    const uint32_t h = pack_bf2(__uint_as_float(x0), __uint_as_float(x1));
     const float r0 = __uint_as_float(x0) - __uint_as_float(h << 16), r1 = __uint_as_float(x1) - __uint_as_float(h & 0xffff0000u);
-    const uint32_t m = pack_bf2_hw(r0, r1);
+    const uint32_t m = pack_bf2(r0, r1);
     s.h[i] = h;
     s.m[i] = m;
     s.l[i] = __builtin_amdgcn_perm(__float_as_uint(r1 - __uint_as_float(m & 0xffff0000u)), __float_as_uint(r0 - __uint_as_float(m << 16)), 0x07060302u);
@@ -48,9 +48,9 @@ __device__ __forceinline__ F32Split f32_split_dot(u32x4_t p, u32x4_t q) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t x0 = i < 2 ? p[2 * i] : q[2 * i - 4], x1 = i < 2 ? p[2 * i + 1] : q[2 * i - 3];
-    const uint32_t h = pack_bf2_hw(__uint_as_float(x0), __uint_as_float(x1));
+    const uint32_t h = pack_bf2(__uint_as_float(x0), __uint_as_float(x1));
     const float r0 = f32_rest(h, low, __uint_as_float(x0)), r1 = f32_rest(h, high, __uint_as_float(x1));
-    const uint32_t m = pack_bf2_hw(r0, r1);
+    const uint32_t m = pack_bf2(r0, r1);
     s.h[i] = h;
     s.m[i] = m;
     s.l[i] = __builtin_amdgcn_perm(__float_as_uint(f32_rest(m, high, r1)), __float_as_uint(f32_rest(m, low, r0)), 0x07060302u);

@@ -492,7 +492,7 @@ gemm_rows_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w
         }
         const long at = (long)m * ldy + ycol + n;
         if (rows32) *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(y) + at) = v;
-        else *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(y) + at) = u32x2_t{pack_bf2_hw(v[0], v[1]), pack_bf2_hw(v[2], v[3])};
+        else *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(y) + at) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
       }
     }
     return;

@@ -4,15 +4,21 @@
 
 extern "C" int ssd_abi_version(void) { return SSD_HIP_ABI_VERSION; }
 
-// Diagnostic: the hardware fp32 -> bf16 conversion (common.h pack_bf2_hw) against the integer form (f2bf) over ALL 2^32 fp32 bit
+// Diagnostic: the hardware fp32 -> bf16 conversion (common.h pack_bf2) against integer round-to-nearest-even over ALL 2^32 fp32 bit
 // patterns.  counts[0] = mismatches on non-NaN inputs (must be 0), counts[1] = NaN inputs whose result is not a NaN (must be 0).
+__device__ __forceinline__ uint32_t f2bf_integer(float f) {
+  uint32_t u = __float_as_uint(f);
+  if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;  // quiet NaN
+  u += 0x7fffu + ((u >> 16) & 1u);
+  return u >> 16;
+}
 __global__ void bf16_cvt_selftest_kernel(unsigned long long* counts) {
   unsigned long long bad = 0, badnan = 0;
   const uint32_t base = (blockIdx.x * blockDim.x + threadIdx.x) << 12;
   for (uint32_t i = 0; i < 4096u; ++i) {
     const uint32_t u = base + i;
     const float f = __uint_as_float(u);
-    const uint32_t sw = f2bf(f), hw = pack_bf2_hw(f, 0.f) & 0xffffu, hw2 = pack_bf2_hw(0.f, f) >> 16;
+    const uint32_t sw = f2bf_integer(f), hw = pack_bf2(f, 0.f) & 0xffffu, hw2 = pack_bf2(0.f, f) >> 16;
     if ((u & 0x7fffffffu) > 0x7f800000u) badnan += ((hw & 0x7fffu) <= 0x7f80u) || ((hw2 & 0x7fffu) <= 0x7f80u);
     else bad += (sw != hw) || (sw != hw2);
   }

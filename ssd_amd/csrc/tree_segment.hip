@@ -208,7 +208,7 @@ __device__ __forceinline__ void ts_store_rows(const f32x4_t* cred, int mt, ts_rs
   f32x4_t s = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int w = 0; w < TS_WAVES; ++w) s += cred[(w * MT + mt) * 64 + lane];
-  const unsigned lo0 = pack_bf2_hw(s[0], s[1]), lo1 = pack_bf2_hw(s[2], s[3]);
+  const unsigned lo0 = pack_bf2(s[0], s[1]), lo1 = pack_bf2(s[2], s[3]);
   const unsigned hi0 = __shfl_down(lo0, 16, 64), hi1 = __shfl_down(lo1, 16, 64);
   const int q4 = lane >> 4, m = mt * 16 + (lane & 15);
   if ((q4 & 1) == 0 && (q4 >> 1) == half && m < M)
@@ -268,13 +268,13 @@ __device__ __forceinline__ void ts_add_norm(const TsParams& p, u32x4_t* xlds, in
         for (int j = 0; j < CPL; ++j) {
           const int c = j * 64 + lane;
           if (c == b) {
-            const u32x4_t ro = {pack_bf2_hw(x[j][0], x[j][1]), pack_bf2_hw(x[j][2], x[j][3]), pack_bf2_hw(x[j][4], x[j][5]), pack_bf2_hw(x[j][6], x[j][7])};
+            const u32x4_t ro = {pack_bf2(x[j][0], x[j][1]), pack_bf2(x[j][2], x[j][3]), pack_bf2(x[j][4], x[j][5]), pack_bf2(x[j][6], x[j][7])};
             ts_store<FIRST ? TS_SC1 : TS_PLAIN>(ro, rdst, (unsigned)c * 16u, __builtin_amdgcn_readfirstlane((unsigned)row * rowb));
           }
           u32x4_t o;
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            o[e] = pack_bf2_hw((x[j][2 * e] * rs) * bf2f(wv[j][e] & 0xffffu), (x[j][2 * e + 1] * rs) * bf2f(wv[j][e] >> 16));
+            o[e] = pack_bf2((x[j][2 * e] * rs) * bf2f(wv[j][e] & 0xffffu), (x[j][2 * e + 1] * rs) * bf2f(wv[j][e] >> 16));
           xlds[c * pitch + row] = o;
         }
       }
@@ -352,10 +352,10 @@ __global__ void __launch_bounds__(TS_THREADS) tree_segment_kernel(const TsParams
         float o[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float gb = round_bf_hw(gs[r]), ub = round_bf_hw(us[r]);
+          const float gb = round_bf(gs[r]), ub = round_bf(us[r]);
           o[r] = (gb / (1.0f + __expf(-gb))) * ub;
         }
-        const unsigned lo0 = pack_bf2_hw(o[0], o[1]), lo1 = pack_bf2_hw(o[2], o[3]);
+        const unsigned lo0 = pack_bf2(o[0], o[1]), lo1 = pack_bf2(o[2], o[3]);
         const unsigned hi0 = __shfl_down(lo0, 16, 64), hi1 = __shfl_down(lo1, 16, 64);
         // activation feature n = pr * 16 + q4 * 4 + r of token m: chunk (m, n / 8) of the fragment-major [MT * 16][I] image
         if ((q4 & 1) == 0 && mt * 16 + mcol < M) {
@@ -421,12 +421,12 @@ __global__ void __launch_bounds__(TS_THREADS) tree_segment_kernel(const TsParams
         for (int w = 0; w < TS_WAVES; ++w) s += cred[(w * MT + mt) * 64 + lane];
         float x[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) x[r] = round_bf_hw(s[r]);   // the reference stores qkv as bf16 before RoPE
+        for (int r = 0; r < 4; ++r) x[r] = round_bf(s[r]);   // the reference stores qkv as bf16 before RoPE
         if (p.qkv_rows) {
           // Qwen3: RMSHeadNorm sits between the projection and the rotation and needs a whole head (8 row groups = 8 workgroups here):
           // the rows leave as the projection wrote them (rotation-paired order) and ssd_rope_store_kv goes on
           if (m < M)
-            *reinterpret_cast<u32x2_t*>(p.qkv_rows + (size_t)m * p.qkv_n + grp * 16 + nrow) = u32x2_t{pack_bf2_hw(x[0], x[1]), pack_bf2_hw(x[2], x[3])};
+            *reinterpret_cast<u32x2_t*>(p.qkv_rows + (size_t)m * p.qkv_n + grp * 16 + nrow) = u32x2_t{pack_bf2(x[0], x[1]), pack_bf2(x[2], x[3])};
         } else if (grp < qk_groups) {
           const int head = grp / gph, j = grp % gph;
           float other[4];
@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(TS_THREADS) tree_segment_kernel(const TsParams
             for (int r = 0; r < 4; ++r)
               yv[r] = hi ? __fadd_rn(__fmul_rn(x[r], c4[r]), __fmul_rn(other[r], s4[r]))
                          : __fsub_rn(__fmul_rn(x[r], c4[r]), __fmul_rn(other[r], s4[r]));
-            const u32x2_t v = {pack_bf2_hw(yv[0], yv[1]), pack_bf2_hw(yv[2], yv[3])};
+            const u32x2_t v = {pack_bf2(yv[0], yv[1]), pack_bf2(yv[2], yv[3])};
             const int dim = hi * half + d;
             if (head < p.nh) {
               *reinterpret_cast<u32x2_t*>(p.q_out + ((size_t)m * p.nh + head) * p.hd + dim) = v;
@@ -460,7 +460,7 @@ __global__ void __launch_bounds__(TS_THREADS) tree_segment_kernel(const TsParams
           const int slot = p.slots[m];
           if (slot >= 0) {
             const size_t rowi = ((size_t)(slot / p.bs) * p.nkv + kvh) * p.bs + (slot % p.bs);
-            const u32x2_t v = {pack_bf2_hw(x[0], x[1]), pack_bf2_hw(x[2], x[3])};
+            const u32x2_t v = {pack_bf2(x[0], x[1]), pack_bf2(x[2], x[3])};
             *reinterpret_cast<u32x2_t*>(p.v_cache + rowi * p.hd + dim) = v;
           }
         }
