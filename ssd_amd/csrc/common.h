@@ -74,6 +74,16 @@ __device__ __forceinline__ float col_sum(float v) {
   return v;
 }
 
+// Workgroup of a recurrent scan -> (sequence, head, column block) of a grid (sequences, heads, column blocks): heads fastest, sequences last.  A
+// workgroup lives as long as its sequence, and workgroup id % 8 is the XCD: with the sequences fastest, four unequal ones kept two XCDs each, and the
+// chip waited for the two of the longest (MI355X, 1800 + 118 + 1594 + 716 tokens, memory_scan, 32 heads of 128 x 128 627 -> 423 us, 16 heads with
+// gates 535 -> 303, delta_scan, 32 heads 687 -> 477, lightning_scan 810 -> 728; equal lengths and single sequences level).
+struct ScanAt { int b, h, block; };
+__device__ __forceinline__ ScanAt scan_at() {
+  const uint32_t id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), r = id / gridDim.y;
+  return ScanAt{(int)(r / gridDim.z), (int)(id % gridDim.y), (int)(r % gridDim.z)};
+}
+
 // Threads per row of the RMSNorm kernels (norm.hip rmsnorm_kernel and comm.hip allreduce_add_rmsnorm_kernel MUST agree: the
 // chunk -> thread mapping fixes the fp32 summation order, and the fused all-reduce + norm is bit-identical to the unfused
 // pair).  A row is a latency chain (load, reduce, scale, store): hidden sizes >= 4096 get 1024 threads, i.e. at most two

@@ -99,7 +99,8 @@ delta_scan_kernel(const float4* __restrict__ qk, const float* __restrict__ vrows
   constexpr int F4 = (TB * D4 + 255) / 256, FV = (TB * COLS + 255) / 256;
   __shared__ float4 sk[TB * D4], sq[TB * D4], sg[CH ? TB * D4 : 1], ss[TB];
   __shared__ float sv[TB * COLS], so[TB * COLS];
-  const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * COLS, tid = threadIdx.x;
+  const ScanAt at = scan_at();
+  const int b = at.b, h = at.h, c0 = at.block * COLS, tid = threadIdx.x;
   const int col = tid / P, p = tid % P, e = c0 + col;
   const int grp = h / (H / G);
   const int row0 = cu_q ? cu_q[b] : b * q_per_seq;
@@ -218,7 +219,7 @@ delta_scan_kernel(const float4* __restrict__ qk, const float* __restrict__ vrows
     for (int j = 0; j < NJ; ++j) sp[P * j] = s[j];
   }
   if (cs.taps > 1) {           // the slot's saved convolution inputs: every workgroup of the sequence saves its share of the channels
-    const int wg = h * gridDim.z + blockIdx.z, nwg = H * gridDim.z, chunk = (cs.C + nwg - 1) / nwg;
+    const int wg = h * gridDim.z + at.block, nwg = H * gridDim.z, chunk = (cs.C + nwg - 1) / nwg;
     save_conv_state(cs.proj, cs.ld, cs.off, cs.C, cs.state, cs.taps, slot, row0, row1, p0, wg * chunk, min(cs.C, (wg + 1) * chunk));
   }
 }

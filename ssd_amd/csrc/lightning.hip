@@ -37,7 +37,8 @@ lightning_scan_kernel(const float* __restrict__ proj, long ld, int q_off, int k_
   float* sk = sq + D;                     // [D]
   float* sv = sk + D;                     // [Dv]
   float* po = sv + Dv;                    // [NG][Dv]
-  const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const ScanAt at = scan_at();
+  const int b = at.b, h = at.h, tid = threadIdx.x;
   const int row0 = cu_q ? cu_q[b] : b * q_per_seq;
   const int row1 = cu_q ? cu_q[b + 1] : (b + 1) * q_per_seq;
   if (row1 <= row0) return;
@@ -92,7 +93,8 @@ lightning_scan_reg_kernel(const float* __restrict__ proj, long ld, int q_off, in
   __shared__ float sq[TB][D], sk[TB][D];
   __shared__ float sv[TB][CB];
   __shared__ float po[TB][NG][CB];
-  const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * CB, tid = threadIdx.x;
+  const ScanAt at = scan_at();
+  const int b = at.b, h = at.h, c0 = at.block * CB, tid = threadIdx.x;
   const int g = tid >> 5, e = tid & 31;
   const int row0 = cu_q ? cu_q[b] : b * q_per_seq;
   const int row1 = cu_q ? cu_q[b + 1] : (b + 1) * q_per_seq;

@@ -105,7 +105,7 @@ memory_gates_kernel(const float* __restrict__ proj, long ld, Gating gt, const in
 
 struct Rows { const float* proj; long ld; int q_off, k_off, v_off; float q_scale; };
 
-// grid = (sequences, heads, column blocks)
+// grid = (sequences, heads, column blocks), dealt by scan_at
 template <int P, int NJ, int TB, int MODE>
 __global__ void __launch_bounds__(256)
 memory_scan_kernel(Rows in, const float* __restrict__ decay, const float4* __restrict__ gates, Gating gt,
@@ -122,7 +122,8 @@ memory_scan_kernel(Rows in, const float* __restrict__ decay, const float4* __res
   __shared__ float sz[2][TB], so[TB * COLS];        // exp(-m) (the batches alternate: read while the next batch is staged); read-outs
   __shared__ float2 pair[MODE == MODE_INLINE ? TB : 1];
   __shared__ float top[MODE == MODE_INLINE ? TB + 1 : 1];
-  const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * COLS, tid = threadIdx.x;
+  const ScanAt at = scan_at();
+  const int b = at.b, h = at.h, c0 = at.block * COLS, tid = threadIdx.x;
   const int col = tid / P, p = tid % P, e = c0 + col;
   const int NC = MODE == MODE_DECAY ? Dv : Dv + 1;
   const int row0 = cu_q ? cu_q[b] : b * q_per_seq;
@@ -134,7 +135,7 @@ memory_scan_kernel(Rows in, const float* __restrict__ decay, const float4* __res
   float4 s[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) s[j] = (fresh || e >= NC) ? float4{0.f, 0.f, 0.f, 0.f} : sp[P * j];
-  float* mp = MODE == MODE_INLINE ? m_state + ((size_t)slot * H + h) * ld_m + blockIdx.z : nullptr;
+  float* mp = MODE == MODE_INLINE ? m_state + ((size_t)slot * H + h) * ld_m + at.block : nullptr;
   float m = MODE == MODE_INLINE && !fresh ? *mp : 0.f;          // every column block keeps a copy: none reads what another one writes
   const float fixed = MODE == MODE_DECAY ? decay[h] : 0.f;
   const float bg = MODE == MODE_INLINE ? (tid < 32 ? gt.bias_f[h] : gt.bias_i[h]) : 0.f;

@@ -95,7 +95,8 @@ wkv_scan_kernel(const float* __restrict__ proj, long ld, int r_off, int k_off, i
   float* su = sd + D;
   float* sv = su + D;
   float* po = sv + D;                     // [NG][D]
-  const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const ScanAt at = scan_at();
+  const int b = at.b, h = at.h, tid = threadIdx.x;
   const int row0 = cu_q ? cu_q[b] : b * q_per_seq;
   const int row1 = cu_q ? cu_q[b + 1] : (b + 1) * q_per_seq;
   if (row1 <= row0) return;
@@ -153,7 +154,8 @@ ssd_scan_kernel(const float* __restrict__ xbc, long ldx, int x_off, int b_off, i
   float* sd = sk + N;
   float* sv = sd + N;                     // [Dv]
   float* po = sv + Dv;                    // [NG][Dv]
-  const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const ScanAt at = scan_at();
+  const int b = at.b, h = at.h, tid = threadIdx.x;
   const int grp = h / (H / G);
   const int row0 = cu_q ? cu_q[b] : b * q_per_seq;
   const int row1 = cu_q ? cu_q[b + 1] : (b + 1) * q_per_seq;
@@ -208,7 +210,8 @@ scan_reg_kernel(WkvArgs wa, SsdArgs sa, const int64_t* __restrict__ positions, c
   __shared__ float sq[TB][D], sk[TB][D], sd[TB][MODE == 0 ? D : 1];
   __shared__ float sv[TB][CB];
   __shared__ float po[TB][NG][CB];
-  const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * CB, tid = threadIdx.x;
+  const ScanAt at = scan_at();
+  const int b = at.b, h = at.h, c0 = at.block * CB, tid = threadIdx.x;
   const int g = tid >> 5, e = tid & 31;
   const int row0 = cu_q ? cu_q[b] : b * q_per_seq;
   const int row1 = cu_q ? cu_q[b + 1] : (b + 1) * q_per_seq;
@@ -305,7 +308,7 @@ scan_reg_kernel(WkvArgs wa, SsdArgs sa, const int64_t* __restrict__ positions, c
 #pragma unroll
   for (int n = 0; n < EPT; ++n) sp[(size_t)(g + NG * n) * Dv] = S[n];
   // the slot's saved rows (token shift / convolution inputs): every workgroup of the sequence saves its share of the columns
-  const int wg = h * gridDim.z + blockIdx.z, nwg = H * gridDim.z;
+  const int wg = h * gridDim.z + at.block, nwg = H * gridDim.z;
   if (MODE == 0) {
     const int chunk = (W + nwg - 1) / nwg;
     for (int c = wg * chunk + tid; c < min(W, (wg + 1) * chunk); c += 256)
