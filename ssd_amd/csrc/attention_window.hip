@@ -623,12 +623,16 @@ winattn_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
 // 16) rows shares every 64-key tile of K and V through LDS, filled by DMA one tile ahead, one barrier per tile; a row keeps its reference maximum until
 // some score exceeds it by 2^8 (exact: sum and denominator both carry it); only tiles at a row's first or last key are masked.  A key's 16-byte
 // chunks of K are rotated by its index, a value column's chunks of 8 keys by the column, so that operand reads hit different banks.
-// Bound by the exponentials and conversions between the two products.  (The form above reads every K and V tile once per 16 rows from L2.)
+// Bound by a tile's instructions, the exponentials and conversions between the two products first, and by how long the longest scan takes alone (1800
+// keys: 29 tiles of 2.8 us).  So the options are looked at per tile, not per score: without a cap and slopes nothing stands between the products but
+// maximum, multiply-add, exponential and sum; keys that were never stored are zeroed in LDS, in the one tile that has any.  (The form above reads every K
+// and V tile once per 16 rows from L2.)
 // A sequence of at most 16 rows beside prompts (a decoded token) would leave one wave to scan its whole context: its workgroup takes the form above,
 // the steps over all four waves.  MI355X, 32 heads of 128 in 8 groups, the form above alone | one wave | this: 300 tokens and one at key 16000
 // 420 | 1149 | 391 us, 512 tokens and two at keys 2000 and 1500 87 | 151 | 58.
 // MI355X, 32 heads of 128 in 8 groups, the form above -> this: prompts of 1800, 1500, 600 and 328 tokens 610 -> 201 us, behind a window of 512
-// 340 -> 101, 500 tokens 52 -> 43, 16384 tokens 23.1 -> 4.9 ms; 32 heads of 64 in 8, 2000 tokens 316 -> 116 us.
+// 340 -> 101, 500 tokens 52 -> 43, 16384 tokens 23.1 -> 4.9 ms; 32 heads of 64 in 8, 2000 tokens 316 -> 116 us; with the options looked at per score ->
+// per tile: 1800, 118, 1594 and 716 tokens 217 -> 179, behind a window of 1024 181 -> 148, 6000 tokens 877 -> 607, heads of 64 138 -> 118.
 // ---------------------------------------------------------------------------------------------------------------------
 constexpr int WP_KEYS = 64;
 
@@ -739,11 +743,20 @@ winattn_prompt_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
     for (int i = 0; i < MV; ++i) acc[t][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   const float inv_cap = cap > 0.f ? 1.0f / cap : 0.f;
+  const bool bent = cap > 0.f || slopes || !(scale > 0.f);        // (the scale is applied after the largest product is known: it has to keep the order)
+  const float unit = bent ? 1.0f : scale * LOG2E;
   if (tiles > 0) fetch(0, 0);
   for (int it = 0; it < tiles; ++it) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");       // the tile is in LDS; nobody reads the one before any more
     if (it + 1 < tiles) fetch(it + 1, (it + 1) & 1);
     const int k0 = key_of(it);
+    if (k0 + WP_KEYS - 1 > kmax && k0 <= kmax) {
+      // keys past the last row's position were never stored: whatever lies there must not meet a zero weight
+      const int n = kmax + 1 - k0, key = lane;
+      for (int col = wave; col < Dv && key >= n; col += 4)
+        *reinterpret_cast<bf16_t*>(wsm + (it & 1) * TILE + KB + col * 128 + (((key >> 3) ^ (col & 7)) << 4) + (key & 7) * 2) = 0;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
     if (k0 > wmax || (k0 + WP_KEYS <= wmin && k0 >= keep_first)) continue;             // (a wave without rows here still meets the barriers)
     const char* kl = wsm + (it & 1) * TILE;
     const char* vl = kl + KB;
@@ -759,7 +772,32 @@ winattn_prompt_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
         for (int t = 0; t < RT; ++t) st[kb][t] = mfma16(a, qf[t][ks], st[kb][t]);
       }
     }
-    const bool edge = k0 + WP_KEYS - 1 > wlast || k0 < wfirst;
+    // a cap, slopes: every score in log2 units here; else the scale rides the exponent's multiply-add.  The options are looked at once per tile
+    if (bent) {
+#pragma unroll
+      for (int kb = 0; kb < WP_KEYS / 16; ++kb)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float v = st[kb][t][e];
+            if (cap > 0.f) v = cap * LOG2E * (1.0f - 2.0f / (1.0f + __expf(2.0f * (v * scale) * inv_cap)));
+            else v *= scale * LOG2E;
+            if (slopes) v -= slope[t] * (float)(pos[t] - (k0 + kb * 16 + qd * 4 + e));
+            st[kb][t][e] = v;
+          }
+    }
+    if (k0 + WP_KEYS - 1 > wlast || k0 < wfirst) {
+#pragma unroll
+      for (int kb = 0; kb < WP_KEYS / 16; ++kb)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int key = k0 + kb * 16 + qd * 4 + e;
+            if (!(key <= pos[t] && (key >= first[t] || key < keep_first))) st[kb][t][e] = -INFINITY;
+          }
+    }
     u32x4_t pb[WP_KEYS / 32][RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
@@ -767,16 +805,8 @@ winattn_prompt_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
 #pragma unroll
       for (int kb = 0; kb < WP_KEYS / 16; ++kb)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float v = st[kb][t][e];
-          const int key = k0 + kb * 16 + qd * 4 + e;
-          if (cap > 0.f) v = cap * LOG2E * (1.0f - 2.0f / (1.0f + __expf(2.0f * (v * scale) * inv_cap)));
-          else v *= scale * LOG2E;
-          if (slopes) v -= slope[t] * (float)(pos[t] - key);
-          if (edge) v = key <= pos[t] && (key >= first[t] || key < keep_first) ? v : -INFINITY;
-          st[kb][t][e] = v;
-          top = fmaxf(top, v);
-        }
+        for (int e = 0; e < 4; ++e) top = fmaxf(top, st[kb][t][e]);
+      top *= unit;
       if (__any(top > m[t] + 8.0f)) {
         top = fmaxf(top, __shfl_xor(top, 16, 64));
         top = fmaxf(m[t], fmaxf(top, __shfl_xor(top, 32, 64)));
@@ -793,7 +823,7 @@ winattn_prompt_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
         float w[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          w[e] = __builtin_amdgcn_exp2f(st[kb][t][e] - ref);
+          w[e] = __builtin_amdgcn_exp2f(fmaf(st[kb][t][e], unit, -ref));
           sum += w[e];
         }
         pb[kb / 2][t][(kb & 1) * 2] = pack_bf2(w[0], w[1]);
@@ -801,27 +831,31 @@ winattn_prompt_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
       }
       lsum[t] += sum;
     }
+    auto values = [&](int c, int i) {
+      const char* row = vl + (i * 16 + r) * 128 + (qd & 1) * 8;
+      const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(row + (((c * 4 + (qd >> 1)) ^ (r & 7)) * 16));
+      const u32x2_t hi = *reinterpret_cast<const u32x2_t*>(row + (((c * 4 + 2 + (qd >> 1)) ^ (r & 7)) * 16));
+      return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+    };
 #pragma unroll
     for (int c = 0; c < WP_KEYS / 32; ++c) {
       if (!needed(k0 + c * 32)) continue;
-      // keys past the last row's position were never stored: whatever lies there must not meet a zero weight
-      const int ka = k0 + c * 32 + qd * 4;
-      const bool past = k0 + c * 32 + 31 > kmax;
-      const uint32_t l0 = (ka <= kmax ? 0xffffu : 0u) | (ka + 1 <= kmax ? 0xffff0000u : 0u);
-      const uint32_t l1 = (ka + 2 <= kmax ? 0xffffu : 0u) | (ka + 3 <= kmax ? 0xffff0000u : 0u);
-      const uint32_t u0 = (ka + 16 <= kmax ? 0xffffu : 0u) | (ka + 17 <= kmax ? 0xffff0000u : 0u);
-      const uint32_t u1 = (ka + 18 <= kmax ? 0xffffu : 0u) | (ka + 19 <= kmax ? 0xffff0000u : 0u);
+      if (DVT == MV) {
 #pragma unroll
-      for (int i = 0; i < MV; ++i)
-        if (i < DVT) {
-          const char* row = vl + (i * 16 + r) * 128 + (qd & 1) * 8;
-          const u32x2_t lo = *reinterpret_cast<const u32x2_t*>(row + (((c * 4 + (qd >> 1)) ^ (r & 7)) * 16));
-          const u32x2_t hi = *reinterpret_cast<const u32x2_t*>(row + (((c * 4 + 2 + (qd >> 1)) ^ (r & 7)) * 16));
-          u32x4_t va = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
-          if (past) { va[0] &= l0; va[1] &= l1; va[2] &= u0; va[3] &= u1; }
+        for (int i = 0; i < MV; ++i) {
+          const u32x4_t va = values(c, i);
 #pragma unroll
           for (int t = 0; t < RT; ++t) acc[t][i] = mfma16(va, pb[c][t], acc[t][i]);
         }
+      } else {
+#pragma unroll
+        for (int i = 0; i < MV; ++i)
+          if (i < DVT) {
+            const u32x4_t va = values(c, i);
+#pragma unroll
+            for (int t = 0; t < RT; ++t) acc[t][i] = mfma16(va, pb[c][t], acc[t][i]);
+          }
+      }
     }
   }
   auto finish = [&](f32x4_t (&o)[MV], float mx, float sum, int at, int t) {
