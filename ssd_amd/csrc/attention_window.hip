@@ -193,14 +193,40 @@ winattn_store_conv_rope_kernel(const float* __restrict__ proj, long ld, int col_
 
 // Per head: x' = w * x / rms(x) over the head's D entries (one weight vector for all q heads, one for all k heads), then the pair (i, i + half)
 // turns by pos * qk_freqs[i].  One wave per head vector, the pairs' sines and cosines once per workgroup.  G = 0: no keys and values.
+// The cache holds the values by column, a page's keys side by side.  In batches of 256 tokens on, the workgroups past the tokens' turn 64 tokens x 64
+// columns through LDS: a wave writes a column's 64 keys, wherever each lies, in one instruction.  (2 bytes a line from each token's workgroup: MI355X,
+// 32 heads of 128 in 8 groups, 4228 tokens 77 -> 63 us, 50 of them the queries'; 600 tokens 26 -> 20, 256 tokens 20 -> 18; 8 heads in 2 groups, 4000 tokens
+// 27.4 -> 26.6; fewer columns than VT_VALUES gain nothing: 8 heads of 64 in 2, 1000 tokens 12.7 either way.)
+constexpr int VT_TOKENS = 64, VT_COLS = 64, VT_VALUES = 256;
+
 template <typename T>
 __global__ void __launch_bounds__(256)
 winattn_store_norm_rope_kernel(const float* __restrict__ qkv, long ld, const T* __restrict__ wq, const T* __restrict__ wk, float eps,
                                const int64_t* __restrict__ positions, const float* __restrict__ qk_freqs, int rot_dims,
-                               const int32_t* __restrict__ slots, T* __restrict__ q_out, T* __restrict__ kc, T* __restrict__ vc, int H, int G,
-                               int D, int Dv, int bs) {
+                               const int32_t* __restrict__ slots, T* __restrict__ q_out, T* __restrict__ kc, T* __restrict__ vc, int tokens, int H,
+                               int G, int D, int Dv, int bs) {
   __shared__ float sn[512], cs[512];
-  const int t = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ T tile[VT_TOKENS][VT_COLS + 2];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if ((int)blockIdx.x >= tokens) {
+    const int tiles = (tokens + VT_TOKENS - 1) / VT_TOKENS, id = blockIdx.x - tokens, t0 = id % tiles * VT_TOKENS, c0 = id / tiles * VT_COLS;
+    const int n = min(tokens - t0, VT_TOKENS), cols = min(G * Dv - c0, VT_COLS);
+    const float* v = qkv + (size_t)t0 * ld + (size_t)(H + G) * D + c0;
+#pragma unroll
+    for (int i = wave; i < VT_TOKENS; i += 4)
+      if (i < n && lane < cols) stf<T>(&tile[i][lane], v[(size_t)i * ld + lane]);
+    __syncthreads();
+    const int slot = lane < n ? slots[t0 + lane] : -1;
+    if (slot < 0) return;
+    const long blk = slot / bs;
+    const int off = slot % bs;
+    for (int i = wave; i < cols; i += 4) {
+      const int c = c0 + i, g = c / Dv, d = c % Dv;
+      vc[(((size_t)blk * G + g) * Dv + d) * bs + off] = tile[lane][i];
+    }
+    return;
+  }
+  const int t = blockIdx.x;
   const int half = rot_dims >> 1, per = D - half;          // items of a head: `half` pairs, then the entries that do not turn
   const float pos = (float)positions[t];
   for (int i = threadIdx.x; i < half; i += 256) sincosf(pos * qk_freqs[i], &sn[i], &cs[i]);
@@ -229,7 +255,7 @@ winattn_store_norm_rope_kernel(const float* __restrict__ qkv, long ld, const T* 
       }
     }
   }
-  if (slot >= 0) {
+  if (slot >= 0 && (int)gridDim.x == tokens) {
     const float* v = row + (size_t)(H + G) * D;
     for (int c = blockIdx.y * 256 + threadIdx.x; c < G * Dv; c += 256 * gridDim.y) {
       const int g = c / Dv, d = c % Dv;
@@ -966,15 +992,16 @@ extern "C" int ssd_winattn_store_norm_rope(const void* qkv_rows, long ld, const 
       rot_dims > 1024 || ld < (long)(H + G) * D + (long)G * Dv)
     return SSD_ERR_SHAPE;
   const int units = (H + G + 3) / 4;
-  const dim3 grid(T, T >= 256 ? 1 : (units < 16 ? units : 16));
+  const int turned = T >= 256 && (long)G * Dv >= VT_VALUES ? (T + VT_TOKENS - 1) / VT_TOKENS * ((G * Dv + VT_COLS - 1) / VT_COLS) : 0;      // workgroups
+  const dim3 grid(T + turned, T >= 256 ? 1 : (units < 16 ? units : 16));
   if (f32)
     hipLaunchKernelGGL(winattn_store_norm_rope_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, (const float*)qkv_rows, ld,
                        (const float*)q_norm_w, (const float*)k_norm_w, eps, positions, qk_freqs, rot_dims, slots, (float*)q_out,
-                       (float*)k_cache, (float*)v_cache, H, G, D, Dv, block_size);
+                       (float*)k_cache, (float*)v_cache, T, H, G, D, Dv, block_size);
   else
     hipLaunchKernelGGL(winattn_store_norm_rope_kernel<bf16_t>, grid, dim3(256), 0, (hipStream_t)stream, (const float*)qkv_rows, ld,
                        (const bf16_t*)q_norm_w, (const bf16_t*)k_norm_w, eps, positions, qk_freqs, rot_dims, slots, (bf16_t*)q_out,
-                       (bf16_t*)k_cache, (bf16_t*)v_cache, H, G, D, Dv, block_size);
+                       (bf16_t*)k_cache, (bf16_t*)v_cache, T, H, G, D, Dv, block_size);
   return LAUNCH_OK();
 }
 
