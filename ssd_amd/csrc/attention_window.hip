@@ -455,6 +455,8 @@ __device__ __forceinline__ void win_finish(f32x4_t (&acc)[MV], float mx, float l
 //            weights, and winattn_merge_kernel joins them in slice order: a long context of few sequences fills the chip.
 // V of keys past the last row's position is zeroed (a weight of zero times whatever an unwritten slot holds must stay zero).
 // The sink joins the denominator at the end.  The cap's tanh is 1 - 2 / (1 + exp(2x)) on the fast exponential.
+// A decode step is a chain of round trips and of a few hundred instructions: heads of exactly 64 and 128 have kernels of their own, whose loads and
+// products no branch divides (MI355X, four sequences of up to 1800 keys, 32 heads of 128 in 8 groups 16.3 -> 13.9 us).
 // ---------------------------------------------------------------------------------------------------------------------
 // One wave's part of it: the 16 rows from row0 (split: the workgroup's, of which this wave takes every fourth step of its slice).
 template <int MK, int MV>        // upper bounds of D / 32 and Dv / 16 (register arrays)
@@ -537,14 +539,21 @@ win_rows(float* __restrict__ smem, const bf16_t* __restrict__ q, const bf16_t* _
         if (ks < KS) sc[hg] = mfma16(kreg[hg][ks], qreg[ks], sc[hg]);
     }
     // lane (row r, keys k0 + hg * 16 + qd * 4 + i)
+#pragma unroll
+    for (int hg = 0; hg < 2; ++hg) sc[hg] *= scale;
+    if (cap > 0.f) {
+#pragma unroll
+      for (int hg = 0; hg < 2; ++hg)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc[hg][i] = cap * (1.0f - 2.0f / (1.0f + __expf(2.0f * sc[hg][i] * inv_cap)));
+    }
     float sv[8], smax = -INFINITY;
 #pragma unroll
     for (int hg = 0; hg < 2; ++hg)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int key = k0 + hg * 16 + qd * 4 + i;
-        float s = sc[hg][i] * scale;
-        if (cap > 0.f) s = cap * (1.0f - 2.0f / (1.0f + __expf(2.0f * s * inv_cap)));
+        float s = sc[hg][i];
         s -= slope * (float)(pos - key);
         s = (key <= pos && (key >= first || key < keep_first)) ? s : -INFINITY;
         sv[hg * 4 + i] = s;
@@ -622,15 +631,16 @@ win_rows(float* __restrict__ smem, const bf16_t* __restrict__ q, const bf16_t* _
                    out_scale, out + (size_t)token * ldo + head * Dv);
 }
 
-template <int MK, int MV>
+template <int MK, int MV, bool FULL = false>            // FULL: D = 32 MK, Dv = 16 MV
 __global__ void __launch_bounds__(256)
 winattn_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vt,
                     const float* __restrict__ slopes, const float* __restrict__ sinks, const int32_t* __restrict__ bt, int max_blocks,
-                    const int64_t* __restrict__ positions, const int32_t* __restrict__ cu_q, int q_per_seq, int H, int G, int D, int Dv,
+                    const int64_t* __restrict__ positions, const int32_t* __restrict__ cu_q, int q_per_seq, int H, int G, int D_, int Dv_,
                     int bs, int window, int keep_first, float scale, float cap, const float* __restrict__ out_freqs,
                     const float* __restrict__ gate, long ldg, float out_scale, bf16_t* __restrict__ out, long ldo, int dtiles,
                     float* __restrict__ part) {
   extern __shared__ float smem[];
+  const int D = FULL ? 32 * MK : D_, Dv = FULL ? 16 * MV : Dv_;
   const int wave = threadIdx.x >> 6, b = blockIdx.z, g = blockIdx.y, R = H / G;
   const int tok0 = cu_q ? cu_q[b] : b * q_per_seq;
   const int nrows = (cu_q ? cu_q[b + 1] - tok0 : q_per_seq) * R;
@@ -1088,12 +1098,14 @@ extern "C" int ssd_winattn_paged(const void* q_rows, const void* k_cache, const 
       grid.x = (unsigned)(dtiles * slices);
     }
     const size_t lds = (4 * 16 * (size_t)Dv + 128) * sizeof(float);
-#define WIN_MFMA(MK, MV)                                                                                                            \
-  hipLaunchKernelGGL((winattn_mfma_kernel<MK, MV>), grid, dim3(256), lds, (hipStream_t)stream, (const bf16_t*)q_rows,               \
+#define WIN_MFMA(...)                                                                                                               \
+  hipLaunchKernelGGL((winattn_mfma_kernel<__VA_ARGS__>), grid, dim3(256), lds, (hipStream_t)stream, (const bf16_t*)q_rows,               \
                      (const bf16_t*)k_cache, (const bf16_t*)v_cache, slopes, sinks, block_tables, max_blocks, positions, cu_q,      \
                      q_per_seq, H, G, D, Dv, block_size, window, keep_first, scale, cap, out_freqs, gate_rows, ldg, out_scale,        \
                      (bf16_t*)out_rows, ldo, dtiles, (float*)workspace)
-    if (D <= 64 && Dv <= 64) WIN_MFMA(2, 4);
+    if (D == 64 && Dv == 64) WIN_MFMA(2, 4, true);
+    else if (D == 128 && Dv == 128) WIN_MFMA(4, 8, true);
+    else if (D <= 64 && Dv <= 64) WIN_MFMA(2, 4);
     else if (D <= 128 && Dv <= 128) WIN_MFMA(4, 8);
     else {
       if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)winattn_mfma_kernel<8, 16>, hipFuncAttributeMaxDynamicSharedMemorySize,
